@@ -572,7 +572,7 @@ def split_calls(case, device, routings: int, steps: int, warmup: int, label: str
             kernel("stage_send_resolve_kernel", us.get("send", []), lambda j: T * (2 * H + 4 * K) + T * row_d),
         ],
         "dispatch_recv": [
-            kernel("stage_recv_first_kernel", us.get(("recv", 0), []), lambda j: 2 * int(rows_of[j][0]) * row_d),
+            kernel("stage_recv_kernel, behind stage_layout_kernel", us.get(("recv", 0), []), lambda j: 2 * int(rows_of[j][0]) * row_d),
             seq_kernel("stage_recv_kernel", later, later_seq),
         ],
         "combine_send": [seq_kernel("combine_send_kernel", csend, csend_seq)],

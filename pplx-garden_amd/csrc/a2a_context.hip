@@ -300,6 +300,15 @@ uint32_t rows_upper_bound(const a2a_ctx *ctx) {
     return (uint32_t)(rows < cap ? rows : cap);
 }
 
+// Bytes the sends of this step staged.
+uint64_t staged_bytes(const a2a_ctx *ctx) {
+    uint64_t tokens = 0;
+    for (uint32_t g = 0; g < ctx->cfg.world_size; ++g) {
+        if (ctx->sent_mask >> g & 1) tokens += ctx->num_tokens[g];
+    }
+    return tokens * ctx->staging.disp_stride;
+}
+
 // The one-launch routing pass recounts earlier chunks in every chunk workgroup
 // and all entries in every receiver workgroup: quadratic in the chunks of a
 // source.  Measured at 8 entries per token: 2 us faster than the two-launch
@@ -1048,6 +1057,7 @@ int a2a_dispatch_recv(a2a_ctx *ctx, uint32_t rank, int32_t *out_num_tokens, void
     rv.row_bytes = (uint32_t)row_bytes_of(c);
     rv.hidden_dim_scale = c.hidden_dim_scale;
     rv.max_rows = rows_upper_bound(ctx);
+    rv.staged_bytes = staged_bytes(ctx);
     // The first recv of a step lays out every receiver: once per step, as the reference's host
     // worker does (a2a_worker.rs:526-703), not once per recv launch.
     rv.valid_mask = ctx->sent_mask & ~ctx->empty_mask;

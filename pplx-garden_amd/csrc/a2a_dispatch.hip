@@ -30,14 +30,6 @@ constexpr int kMaxLdsScales = 1024;
 // Arguments travel by value; a launch can carry 4 KB of them.
 static_assert(sizeof(PushArgs) + sizeof(FinalizeArgs) + sizeof(Workspace) <= 4096, "kernel arguments too large");
 
-// The 16-byte store of a dispatched copy, at device scope (`sc1`): the line is written through
-// instead of staying dirty in the L2 of the storing die.  Measured on the 4096-token pack against
-// the other policies of the store: non-temporal 62 us, ordinary 50.3 us, device scope 49.7 us
-// (plain kernels of the same shape: 63 / 48.5 / 47.4 us).
-__device__ __forceinline__ void store_copy(u32x4 v, u32x4 *p) {
-    asm volatile("global_store_dwordx4 %0, %1, off sc1" ::"v"(p), "v"(v) : "memory");
-}
-
 // Moves the row of `token` to its copies.  Lanes 0..K-1 of EVERY wavefront hold
 // the row pointer, scale pointer and scale stride of route k (0 = no copy).
 // The row is loaded here, AFTER the routes are known, unless the caller passes

@@ -54,6 +54,14 @@ struct StageSendArgs {
     uint32_t resolver_wave;   // resolving send: wavefront that resolves the routes (set by the launcher)
 };
 
+// A grid of wavefronts over the pieces (64 sixteen-byte chunks) of a receiver's rows.
+struct PieceGrid {
+    uint32_t pieces;          // of a row
+    uint32_t magic;           // n / pieces = mulhi(n, magic) for the wavefronts of a grid (0 for one piece a row)
+    uint32_t step_rows;       // wavefronts of the grid = step_rows * pieces + step_pieces
+    uint32_t step_pieces;
+};
+
 struct StageRecvArgs {
     PushDst dst;
     int32_t *out_num_tokens;  // rows per local expert for the caller, may be null
@@ -61,12 +69,13 @@ struct StageRecvArgs {
     uint32_t row_bytes;
     uint32_t hidden_dim_scale;
     uint32_t max_rows;        // upper bound of received rows known to the host
-    uint32_t team_waves;      // wavefronts that share a row (set by the launcher)
+    uint64_t staged_bytes;    // what the step's sends staged
+    PieceGrid grid;           // set by the launcher
     // the first recv of a step only: it lays out every receiver
     uint32_t valid_mask;      // sources that sent tokens in this step (the others count as empty)
     uint32_t max_private;     // rows per source in the private part of a receive region (a2a_worker.rs:646-656)
-    uint32_t copy_blocks;     // workgroups that serve the caller's rank; the others lay out the other receivers (launcher)
-    uint32_t slices;          // workgroups per other receiver (set by the launcher)
+    uint32_t copy_blocks;     // few rows: workgroups that serve the caller's rank; the others lay out the other receivers (launcher)
+    uint32_t slices;          // workgroups per receiver that is laid out for later recvs (launcher)
 };
 
 struct CombineSendArgs {
@@ -76,7 +85,7 @@ struct CombineSendArgs {
     uint32_t rank;
     uint32_t row_bytes;
     uint32_t max_rows;
-    uint32_t team_waves;      // wavefronts that share a row (set by the launcher)
+    PieceGrid grid;           // set by the launcher
 };
 
 struct CombineRecvArgs {
@@ -109,8 +118,7 @@ hipError_t launch_stage_send_single(const StageSendArgs &args, const Workspace &
 // The send of a large step after launch_route_accumulate(..., for_send = true).
 hipError_t launch_stage_send_resolve(const StageSendArgs &args, const Workspace &ws, const Staging &st,
                                      bool quantize, hipStream_t stream, KernelTiming timing = KernelTiming());
-// `first_of_step`: no recv has run since the step's sends; this launch also lays out the other receivers.
-// Steps with few rows (a workgroup per row) take kernels of their own, here and in the combine-send.
+// `first_of_step`: no recv has run since the step's sends; all receivers are laid out first.
 hipError_t launch_stage_recv(const StageRecvArgs &args, const Workspace &ws, const Staging &st, bool first_of_step,
                              hipStream_t stream, KernelTiming timing = KernelTiming());
 hipError_t launch_combine_send(const CombineSendArgs &args, const Workspace &ws, const Staging &st,

@@ -949,6 +949,8 @@ __global__ __launch_bounds__(1024) void stage_send_resolve_kernel(const StageSen
     stage_row<QUANT>(args, st, g, token, staging_threads);
 }
 
+constexpr uint32_t kPieceThreads = 256;   // threads of a workgroup of the kernels that copy rows in pieces
+
 // A team of `team` threads (one or more whole wavefronts) copies a row of
 // `num_chunks` 16-byte pieces: eight loads per thread in flight, non-temporal
 // both ways (rows are read once and written once).
@@ -989,30 +991,27 @@ __device__ __forceinline__ void copy_received_row(const uint8_t *src, uint32_t p
 }
 
 // ---------------------------------------------------------------------------
-// dispatch recv.  The receivers of a step are laid out ONCE per step, by the
-// launch of the step's first recv (the reference's host worker runs
-// process_routing_info once per rank and step, a2a_worker.rs:526-703).
+// dispatch recv.  The receivers of a step are laid out ONCE per step, by the step's
+// first recv (the reference's host worker runs process_routing_info once per rank
+// and step, a2a_worker.rs:526-703).  A layout is made in LDS from the published
+// per-source counts of a receiver's experts (a2a_worker.rs:577-606,621-694: rows per
+// expert, padded first row of every expert, first row of every (source, expert) run
+// inside it, and the order in which the runs ARRIVE: sources in the worker's order,
+// experts inside a source); then one thread per received row writes the row's
+// metadata (padded_index, source_rank, source position and the two offset tables:
+// a2a_worker.rs:636-671) and the staged row it comes from (the token behind its
+// position in the sender's order).
 //
-// stage_recv_first_kernel is that launch.  Its first workgroups serve the rank
-// that called: each lays the receiver out in LDS from the published per-source
-// counts of its experts (a2a_worker.rs:577-606,621-694: rows per expert, padded
-// first row of every expert, first row of every (source, expert) run inside it,
-// and the order in which the runs ARRIVE: sources in the worker's order,
-// experts inside a source), then teams of wavefronts share the received rows:
-// the row's metadata is written (padded_index, source_rank, source position and
-// the two offset tables: a2a_worker.rs:636-671) and payload and scales are
-// copied from the sender's staged token (a2a_dispatch_recv.cu:139-155).  A rank
-// on a GPU of its own would launch only these.  The workgroups behind them lay
-// out the OTHER receivers, in the shadow of that copy: the same layout in LDS,
-// then one thread per received row writes the row's metadata and the staged row
-// it comes from (the token behind its position in the sender's order).
+// stage_layout_kernel does that for every receiver, in front of the first recv's
+// copy.  Where the rows are few, stage_recv_first_few_kernel does layout and copy in
+// one launch: its first workgroups lay out the OTHER receivers, those behind them
+// lay the calling rank out, each for the row it copies.
 //
-// stage_recv_kernel is the launch of every later recv of the step.  It only
-// copies: a team of wavefronts per received row reads where the row comes from
-// and where it goes (one trip for both) and moves payload and scales; its first
-// workgroup hands the receiver's counts to the caller.
+// stage_recv_kernel is the copy: where a row comes from and where it goes is read
+// from the tables (a2a_dispatch_recv.cu:139-155); its first workgroup hands the
+// receiver's counts to the caller.
 //
-// Dynamic LDS of a layout: 4 * G * Le + 1 + 3 * G words.
+// Dynamic LDS of a layout: 5 * G * Le + 1 + 3 * G + Le words.
 // ---------------------------------------------------------------------------
 struct ReceiverTables {   // in LDS, see lay_out_receiver
     uint32_t *tot;       // [g][le]  copies source g sends to local expert le
@@ -1024,156 +1023,10 @@ struct ReceiverTables {   // in LDS, see lay_out_receiver
     uint32_t *grp_cnt;   // [g]      rows this receiver gets from source g
     const uint8_t *order;  // [i]    the i-th source this receiver lays out
     uint32_t rows;       // rows received
-    // only with lay_out_receiver_spread (w = i * Le + le is the run of the i-th source visited and local expert le):
+    // (w = i * Le + le is the run of the i-th source visited and local expert le)
     uint32_t *pos;       // [w]      position of the run in the sender's expert-sorted order (excl, by run)
     uint32_t own_g, own_pos, own_seg, own_end, own_row;   // run w = threadIdx.x of this thread (if there is one), in registers
 };
-
-// Lays out receiver `r` in LDS.  Whole workgroup.  `publish`: this workgroup also writes the
-// receiver's tables to memory and (if given) its counts to the caller.  Returns false, before the
-// expensive part, when the workgroup's first row `first_row` lies beyond the rows received and it
-// does not publish: the host sizes grids for an upper bound, a receiver typically gets 1/N of it.
-__device__ __forceinline__ bool lay_out_receiver(uint32_t valid_mask, const Workspace &ws, const Staging &st, uint32_t r,
-                                                 bool publish, uint32_t first_row, int32_t *out_num_tokens,
-                                                 uint32_t out_rows, uint32_t *s_recv, uint8_t *s_order,
-                                                 ReceiverTables &t) {
-    const uint32_t G = ws.num_groups, E = ws.num_experts, Le = ws.experts_per_rank;
-    const uint32_t first = r * Le;
-    const uint32_t n_local = first >= E ? 0 : (E - first < Le ? E - first : Le);
-    const uint32_t items = G * Le;
-    const uint32_t tid = threadIdx.x;
-    const uint32_t nthreads = blockDim.x;
-    const uint32_t lane = tid & (kWave - 1);
-    uint32_t *tot = t.tot = s_recv;
-    uint32_t *excl = t.excl = tot + items;
-    uint32_t *run_row = t.run_row = excl + items;
-    uint32_t *seg = t.seg = run_row + items;
-    uint32_t *grp_dst = t.grp_dst = seg + items + 1;
-    uint32_t *grp_src = t.grp_src = grp_dst + G;
-    uint32_t *grp_cnt = t.grp_cnt = grp_src + G;
-    t.order = s_order;
-
-    // The order in which this receiver lays out its sources (one byte per source, from the table the
-    // context computed once) travels with the counts and is read from LDS from then on: looked up in
-    // memory where it is used, it put a dependent trip into the layout and one in front of every row.
-    // All loads of a thread are asked for before the first is used (none under a condition of its own:
-    // a word that does not count is read from a valid place and dropped), or each would be waited for
-    // by itself, one trip to memory after the other.
-    const uint32_t order_word = ws.order[r * (kMaxWorld / 4) + (tid < G ? tid >> 2 : 0)];
-    for (uint32_t w = tid; w < items; w += nthreads) {
-        const uint32_t g = Le > 1 ? __umulhi(w, ws.le_magic) : w;
-        const uint32_t le = w - g * Le;
-        const uint32_t e = first + le;
-        const bool live = le < n_local && (valid_mask >> g & 1);
-        const uint32_t at = live ? g * E + e : 0;
-        const uint32_t count = ws.num_routed[at];
-        const uint32_t upto = ws.expert_offsets[at > 0 ? at - 1 : 0];
-        tot[w] = live ? count : 0;
-        excl[w] = live && e > 0 ? upto : 0;
-    }
-    if (tid < G) s_order[tid] = (uint8_t)(order_word >> (8 * (tid & 3)));
-    __syncthreads();
-
-    // Rows this receiver gets from source g (lane g; there are at most kMaxWorld <= 64 sources): the
-    // sender's scan over its experts gives them without a sum.  Every wavefront adds them up by itself.
-    uint32_t from_source = 0;
-    if (lane < G && n_local != 0) {
-        const uint32_t last = lane * Le + n_local - 1;
-        from_source = excl[last] + tot[last] - excl[lane * Le];
-    }
-    const uint32_t from_lower = wave_inclusive_scan(from_source, lane);   // inclusive over the sources
-    const uint32_t rows = t.rows = (uint32_t)__builtin_amdgcn_readlane((int)from_lower, kWave - 1);
-    if (!publish && first_row >= rows) return false;   // uniform
-
-    // The layout is the work of two wavefronts, each by itself (scans on the DPP path, no barrier
-    // inside); the others wait for them.  Done by every wavefront of every workgroup, with workgroup
-    // scans, it was most of the kernel's instructions.
-    const uint32_t wave = tid / kWave;
-    if (wave == 0) {
-        // Per source: where its rows for this receiver begin in its own send order (dst_group_offset,
-        // a2a_worker.rs:571-575) and how many rows the lower-numbered sources send here
-        // (src_group_offset, a2a_worker.rs:582-590: numeric order, not the order of arrival).
-        if (lane < G) {
-            grp_dst[lane] = excl[lane * Le];
-            grp_cnt[lane] = from_source;
-            grp_src[lane] = from_lower - from_source;
-        }
-
-        // Rows per expert, padded offsets, first row of every run.
-        const uint32_t visited = lane < G ? s_order[lane] : 0;   // lane i: the i-th source in the order of the layout
-        const uint32_t pad = ws.expert_padding;
-        uint32_t carry = 0;
-        for (uint32_t l0 = 0; l0 < Le; l0 += kWave) {
-            const uint32_t le = l0 + lane;
-            const bool mine = le < n_local;
-            uint32_t tpe = 0;
-            if (mine) {
-                for (uint32_t g = 0; g < G; ++g) tpe += tot[g * Le + le];
-            }
-            const uint32_t padded = (tpe + pad - 1) / pad * pad;
-            const uint32_t scan = wave_inclusive_scan(mine ? padded : 0, lane);
-            if (mine) {
-                const uint32_t poff = carry + scan - padded;
-                const uint32_t e = first + le;
-                uint32_t running = poff;
-                uint32_t g = (uint32_t)__builtin_amdgcn_readlane((int)visited, 0);
-                uint32_t next = tot[g * Le + le];
-                for (uint32_t i = 0; i < G; ++i) {
-                    // the count of the source after this one is asked for before this one's is used
-                    const uint32_t count = next;
-                    const uint32_t g_next = (uint32_t)__builtin_amdgcn_readlane((int)visited, (int)(i + 1 < G ? i + 1 : i));
-                    next = tot[g_next * Le + le];
-                    run_row[i * Le + le] = running;
-                    if (publish) ws.slot_base[g * E + e] = running;
-                    running += count;
-                    g = g_next;
-                }
-                if (publish) {
-                    ws.tokens_per_expert[e] = tpe;
-                    ws.padded_offset[e] = poff;
-                    if (out_num_tokens != nullptr) out_num_tokens[le] = (int32_t)tpe;
-                    if (poff + tpe > out_rows) atomicOr(ws.err, A2A_DEV_RECV_OVERFLOW);
-                }
-            }
-            carry += (uint32_t)__builtin_amdgcn_readlane((int)scan, kWave - 1);
-        }
-    }
-    if (wave == (nthreads > kWave ? 1u : 0u)) {
-        // Arrival order: sources as the worker visits them, local experts inside a source.  Lane i has
-        // the rows that arrive before those of the i-th source visited; inside a source the sender's
-        // scan over its experts says how many rows precede those of a local expert.  No sum, no scan
-        // over the runs.
-        const uint32_t visited = lane < G ? s_order[lane] : 0;
-        const uint32_t theirs = (uint32_t)__shfl((int)from_source, (int)visited);   // every lane takes part
-        const uint32_t arrive = lane < G ? theirs : 0;
-        const uint32_t before = wave_inclusive_scan(arrive, lane) - arrive;
-        for (uint32_t b = 0; b < items; b += kWave) {
-            const uint32_t s = b + lane;
-            const uint32_t i = s < items ? (Le > 1 ? __umulhi(s, ws.le_magic) : s) : 0;
-            const uint32_t base = (uint32_t)__shfl((int)before, (int)i);
-            const uint32_t count = (uint32_t)__shfl((int)arrive, (int)i);
-            if (s < items) {
-                const uint32_t le = s - i * Le;
-                const uint32_t g = s_order[i];
-                seg[s] = base + (le < n_local ? excl[g * Le + le] - excl[g * Le] : count);
-            }
-        }
-        if (lane == 0) {
-            seg[items] = rows;
-            if (publish) {
-                if (rows > st.max_recv) atomicOr(ws.err, A2A_DEV_RECV_OVERFLOW);
-                st.num_recv[2 * r] = rows;
-            }
-        }
-    }
-    __syncthreads();
-    if (publish && tid == 0) {
-        // rows that come from other nodes (num_efa_tokens, a2a_worker.rs:681-687)
-        const uint32_t remote_segs = (ws.world / ws.node_size - 1) * (ws.node_size / ws.dp_size) * Le;
-        st.num_recv[2 * r + 1] = remote_segs < items ? seg[remote_segs] : rows;
-    }
-    return true;
-}
 
 // What the receiver's tables say of arrival `row` of run `s` (seg[s] <= row < seg[s + 1]).
 struct RowMeta {
@@ -1181,18 +1034,6 @@ struct RowMeta {
     uint32_t pos;      // position in the source's expert-sorted order
     uint32_t dst_row;  // row in the receiver's buffer
 };
-
-__device__ __forceinline__ RowMeta row_of_run(const ReceiverTables &t, const Workspace &ws, uint32_t s, uint32_t row) {
-    const uint32_t Le = ws.experts_per_rank;
-    const uint32_t i = Le > 1 ? __umulhi(s, ws.le_magic) : s;
-    const uint32_t le = s - i * Le;
-    RowMeta m;
-    m.g = t.order[i];
-    const uint32_t j = row - t.seg[s];
-    m.pos = t.excl[m.g * Le + le] + j;
-    m.dst_row = t.run_row[s] + j;
-    return m;
-}
 
 // Writes the five per-row tables of the reference's host worker for arrival `row` of receiver `r`
 // (a2a_worker.rs:633-671).  One thread.
@@ -1224,86 +1065,12 @@ __device__ __forceinline__ void write_row_tables(const ReceiverTables &t, const 
     st.combine_send_offset[at] = cso;
 }
 
-__global__ __launch_bounds__(1024) void stage_recv_first_kernel(const StageRecvArgs args, const Workspace ws,
-                                                                const Staging st) {
-    extern __shared__ uint32_t s_recv[];
-    __shared__ uint8_t s_order[kMaxWorld];
-    const uint32_t tid = threadIdx.x;
-    const uint32_t nthreads = blockDim.x;
-    const uint32_t lane = tid & (kWave - 1);
-    const uint32_t items = ws.num_groups * ws.experts_per_rank;
-    ReceiverTables t;
-
-    if (blockIdx.x >= args.copy_blocks) {
-        // ---- one of the other receivers: layout, then one thread per received row ----
-        const uint32_t w = blockIdx.x - args.copy_blocks;
-        uint32_t r = w / args.slices;
-        const uint32_t slice = w - r * args.slices;
-        if (r >= args.rank) ++r;   // the caller's rank is served by the first workgroups
-        if (!lay_out_receiver(args.valid_mask, ws, st, r, slice == 0, slice * nthreads, nullptr, 0xFFFFFFFFu, s_recv,
-                              s_order, t))
-            return;
-        const uint32_t total = t.rows < st.max_recv ? t.rows : st.max_recv;   // beyond: flagged and dropped
-        for (uint32_t row = slice * nthreads + tid; row < total; row += args.slices * nthreads) {
-            // the run this arrival belongs to: the last one with seg[s] <= row (runs without rows share
-            // their first arrival with the run after them, so the last such run is the one with rows)
-            uint32_t lo = 0, hi = items;   // seg[lo] <= row < seg[hi]
-            while (hi - lo > 1) {
-                const uint32_t mid = (lo + hi) / 2;
-                if (t.seg[mid] <= row) lo = mid; else hi = mid;
-            }
-            const RowMeta m = row_of_run(t, ws, lo, row);
-            // the token behind the position: asked for first, used last
-            const uint32_t token = m.pos < ws.max_tk ? st.pos_token[(size_t)m.g * ws.max_tk + m.pos] : 0;
-            write_row_tables(t, ws, st, r, row, m, args.max_private);
-            st.source_row[(size_t)r * st.max_recv + row] = m.g * st.max_tokens + token;
-        }
-        return;
-    }
-
-    // ---- the caller's rank: layout, then a team of wavefronts per received row ----
-    const uint32_t r = args.rank;
-    const uint32_t team_threads = args.team_waves * kWave;
-    const uint32_t teams = nthreads / team_threads;
-    if (!lay_out_receiver(args.valid_mask, ws, st, r, blockIdx.x == 0, blockIdx.x * teams, args.out_num_tokens,
-                          args.dst.out_rows, s_recv, s_order, t))
-        return;
-    // From here on the workgroup is split into teams that work alone (no barrier): one received row
-    // per team at a time.  Every wavefront of a team finds the row's run by itself.
-    const PushDst &dst = args.dst;
-    const uint32_t num_chunks = args.row_bytes / 16;
-    const uint32_t member = tid % team_threads;
-    for (uint32_t row = blockIdx.x * teams + tid / team_threads; row < t.rows; row += args.copy_blocks * teams) {
-        // the run this arrival belongs to: the one non-empty run with seg[s] <= row < seg[s + 1]
-        uint32_t s = 0;
-        for (uint32_t s0 = 0; s0 < items; s0 += kWave) {
-            const uint32_t cand = s0 + lane;
-            const uint64_t hit = __ballot(cand < items && t.seg[cand] <= row && row < t.seg[cand + 1]);
-            if (hit != 0) {
-                s = s0 + (uint32_t)__builtin_ctzll(hit);
-                break;
-            }
-        }
-        const RowMeta m = row_of_run(t, ws, s, row);
-        if (row >= st.max_recv) continue;   // flagged by the layout: more rows than the receive region was sized for
-        const uint32_t token = st.pos_token[(size_t)m.g * ws.max_tk + m.pos];
-        if (member == 0) {
-            write_row_tables(t, ws, st, r, row, m, args.max_private);
-            st.source_row[(size_t)r * st.max_recv + row] = m.g * st.max_tokens + token;
-        }
-        if (dst.out_x == nullptr) continue;
-        if (m.dst_row >= dst.out_rows) {
-            if (member == 0) atomicOr(ws.err, A2A_DEV_RECV_OVERFLOW);
-            continue;
-        }
-        const uint8_t *src = st.send_buf + ((size_t)m.g * st.max_tokens + token) * st.disp_stride;
-        copy_received_row(src, st.payload_bytes, num_chunks, args.hidden_dim_scale, dst, m.dst_row, member, team_threads);
-    }
-}
-
-// The same layout for the steps with few rows (stage_recv_first_few_kernel), where the layout is most of
-// what a recv waits for.  In the tables run_row and seg (and pos) a run is w = i * Le + le, i the
-// source's place in the order of the layout, as in lay_out_receiver.
+// Lays out receiver `r` in LDS.  Whole workgroup.  `publish`: this workgroup also writes the
+// receiver's tables to memory and (if given) its counts to the caller.  Returns false, before the
+// expensive part, when the workgroup's first row `first_row` lies beyond the rows received and it
+// does not publish: the host sizes grids for an upper bound, a receiver typically gets 1/N of it.
+// In the tables run_row, seg and pos a run is w = i * Le + le, i the source's place in the order of
+// the layout.
 //
 // The work is spread over all threads, one run (source in the order of the layout, local expert)
 // each, and what counts is the number of dependent LDS trips and barriers between the arrival of the
@@ -1313,7 +1080,7 @@ __global__ __launch_bounds__(1024) void stage_recv_first_kernel(const StageRecvA
 // After the last barrier inside, a thread's OWN runs (w = tid, tid + blockDim.x, ...) are complete in
 // LDS and the first of them is in t.own_*; `all_visible` adds the barrier after which every thread
 // may read every run.
-__device__ __forceinline__ bool lay_out_receiver_spread(uint32_t valid_mask, const Workspace &ws, const Staging &st, uint32_t r,
+__device__ __forceinline__ bool lay_out_receiver(uint32_t valid_mask, const Workspace &ws, const Staging &st, uint32_t r,
                                                  bool publish, uint32_t first_row, int32_t *out_num_tokens,
                                                  uint32_t out_rows, uint32_t *s_recv, uint8_t *s_order,
                                                  ReceiverTables &t, bool all_visible) {
@@ -1532,8 +1299,8 @@ __device__ __forceinline__ bool lay_out_receiver_spread(uint32_t valid_mask, con
     return true;
 }
 
-// What the spread tables say of arrival `row` of run `s` (seg[s] <= row < seg[s + 1]): one LDS trip.
-__device__ __forceinline__ RowMeta row_of_run_spread(const ReceiverTables &t, const Workspace &ws, uint32_t s, uint32_t row) {
+// What the tables say of arrival `row` of run `s` (seg[s] <= row < seg[s + 1]): one LDS trip.
+__device__ __forceinline__ RowMeta row_of_run(const ReceiverTables &t, const Workspace &ws, uint32_t s, uint32_t row) {
     const uint32_t Le = ws.experts_per_rank;
     const uint32_t i = Le > 1 ? __umulhi(s, ws.le_magic) : s;
     RowMeta m;
@@ -1544,9 +1311,36 @@ __device__ __forceinline__ RowMeta row_of_run_spread(const ReceiverTables &t, co
     return m;
 }
 
+// Slice `slice` of the work that lays out receiver `r`: the layout in LDS, then one thread per received
+// row writes the row's tables and the staged row it comes from.
+__device__ __forceinline__ void lay_out_rows(const StageRecvArgs &args, const Workspace &ws, const Staging &st, uint32_t r,
+                                             uint32_t slice, uint32_t *s_recv, uint8_t *s_order) {
+    const uint32_t tid = threadIdx.x;
+    const uint32_t nthreads = blockDim.x;
+    ReceiverTables t;
+    if (!lay_out_receiver(args.valid_mask, ws, st, r, slice == 0, slice * nthreads, nullptr, 0xFFFFFFFFu,
+                                 s_recv, s_order, t, true))
+        return;
+    const uint32_t total = t.rows < st.max_recv ? t.rows : st.max_recv;   // beyond: flagged and dropped
+    for (uint32_t row = slice * nthreads + tid; row < total; row += args.slices * nthreads) {
+        // the run this arrival belongs to: the last one with seg[s] <= row (runs without rows share
+        // their first arrival with the run after them, so the last such run is the one with rows)
+        uint32_t lo = 0, hi = ws.num_groups * ws.experts_per_rank;   // seg[lo] <= row < seg[hi]
+        while (hi - lo > 1) {
+            const uint32_t mid = (lo + hi) / 2;
+            if (t.seg[mid] <= row) lo = mid; else hi = mid;
+        }
+        const RowMeta m = row_of_run(t, ws, lo, row);
+        // the token behind the position: asked for first, used last
+        const uint32_t token = m.pos < ws.max_tk ? st.pos_token[(size_t)m.g * ws.max_tk + m.pos] : 0;
+        write_row_tables(t, ws, st, r, row, m, args.max_private);
+        st.source_row[(size_t)r * st.max_recv + row] = m.g * st.max_tokens + token;
+    }
+}
+
 // The step's first recv when the step has few rows (the host gave every row a workgroup as wide as the
-// row): the same work as stage_recv_first_kernel with the layout spread over the threads, and the
-// whole workgroup serves one row at a time: the thread whose run holds the row says so to the others.
+// row): layout and copy in one launch; the whole workgroup serves one row at a time, and the thread whose
+// run holds the row says so to the others.
 // Dynamic LDS: 5 * G * Le + 1 + 3 * G + Le words.
 __global__ __launch_bounds__(1024) void stage_recv_first_few_kernel(const StageRecvArgs args, const Workspace ws,
                                                                     const Staging st) {
@@ -1564,28 +1358,10 @@ __global__ __launch_bounds__(1024) void stage_recv_first_few_kernel(const StageR
     const uint32_t other_blocks = gridDim.x - args.copy_blocks;
     if (blockIdx.x < other_blocks) {
         // ---- one of the other receivers: layout, then one thread per received row ----
-        const uint32_t w = blockIdx.x;
-        uint32_t r = w / args.slices;
-        const uint32_t slice = w - r * args.slices;
+        uint32_t r = blockIdx.x / args.slices;
+        const uint32_t slice = blockIdx.x - r * args.slices;
         if (r >= args.rank) ++r;   // the caller's rank is served by the workgroups behind these
-        if (!lay_out_receiver_spread(args.valid_mask, ws, st, r, slice == 0, slice * nthreads, nullptr, 0xFFFFFFFFu,
-                                     s_recv, s_order, t, true))
-            return;
-        const uint32_t total = t.rows < st.max_recv ? t.rows : st.max_recv;   // beyond: flagged and dropped
-        for (uint32_t row = slice * nthreads + tid; row < total; row += args.slices * nthreads) {
-            // the run this arrival belongs to: the last one with seg[s] <= row (runs without rows share
-            // their first arrival with the run after them, so the last such run is the one with rows)
-            uint32_t lo = 0, hi = items;   // seg[lo] <= row < seg[hi]
-            while (hi - lo > 1) {
-                const uint32_t mid = (lo + hi) / 2;
-                if (t.seg[mid] <= row) lo = mid; else hi = mid;
-            }
-            const RowMeta m = row_of_run_spread(t, ws, lo, row);
-            // the token behind the position: asked for first, used last
-            const uint32_t token = m.pos < ws.max_tk ? st.pos_token[(size_t)m.g * ws.max_tk + m.pos] : 0;
-            write_row_tables(t, ws, st, r, row, m, args.max_private);
-            st.source_row[(size_t)r * st.max_recv + row] = m.g * st.max_tokens + token;
-        }
+        lay_out_rows(args, ws, st, r, slice, s_recv, s_order);
         return;
     }
 
@@ -1594,7 +1370,7 @@ __global__ __launch_bounds__(1024) void stage_recv_first_few_kernel(const StageR
     const PushDst &dst = args.dst;
     const uint32_t num_chunks = args.row_bytes / 16;
     const uint32_t block = blockIdx.x - other_blocks;
-    if (!lay_out_receiver_spread(args.valid_mask, ws, st, r, block == 0, block, args.out_num_tokens,
+    if (!lay_out_receiver(args.valid_mask, ws, st, r, block == 0, block, args.out_num_tokens,
                                  args.dst.out_rows, s_recv, s_order, t, false))
         return;
     for (uint32_t row = block; row < t.rows; row += args.copy_blocks) {
@@ -1607,7 +1383,7 @@ __global__ __launch_bounds__(1024) void stage_recv_first_few_kernel(const StageR
         for (uint32_t w = tid + nthreads; w < items; w += nthreads) {
             // (a thread's own runs are complete, and every run's first arrival is there)
             if (t.seg[w] <= row && row < t.seg[w + 1]) {
-                const RowMeta mine = row_of_run_spread(t, ws, w, row);
+                const RowMeta mine = row_of_run(t, ws, w, row);
                 s_meta[0] = mine.g;
                 s_meta[1] = mine.pos;
                 s_meta[2] = mine.dst_row;
@@ -1635,80 +1411,66 @@ __global__ __launch_bounds__(1024) void stage_recv_first_few_kernel(const StageR
     }
 }
 
-__global__ __launch_bounds__(1024) void stage_recv_kernel(const StageRecvArgs args, const Workspace ws,
-                                                          const Staging st) {
-    // everything a wavefront takes from the argument block, asked for in one go
-    A2A_PIN(args.dst.out_x);
-    A2A_PIN(args.dst.out_scale);
-    A2A_PIN(args.dst.out_stride);
-    A2A_PIN(args.dst.os_stride_elem);
-    A2A_PIN(args.dst.os_stride_token);
-    A2A_PIN(args.dst.out_rows);
-    A2A_PIN(args.rank);
-    A2A_PIN(args.row_bytes);
-    A2A_PIN(args.hidden_dim_scale);
-    A2A_PIN(args.team_waves);
-    A2A_PIN(st.send_buf);
-    A2A_PIN(st.padded_index);
-    A2A_PIN(st.source_row);
-    A2A_PIN(st.num_recv);
-    A2A_PIN(st.disp_stride);
-    A2A_PIN(st.payload_bytes);
-    A2A_PIN(st.max_recv);
-    const uint32_t r = args.rank;
-    const uint32_t tid = threadIdx.x;
-    const PushDst &dst = args.dst;
-    const uint32_t num_chunks = args.row_bytes / 16;
-    const uint32_t team = args.team_waves * kWave;   // threads that share a row
-    const uint32_t teams = blockDim.x / team;
-    const uint32_t member = tid % team;
-    const uint32_t *padded_index = st.padded_index + (size_t)r * st.max_recv;
-    const uint32_t *source_row = st.source_row + (size_t)r * st.max_recv;
-    // The first row's two table words are asked for together with the number of rows received
-    // (a row index the tables do not hold reads entry 0 and is dropped by the loop's bound).
-    uint32_t row = blockIdx.x * teams + tid / team;
-    const uint32_t probe = row < st.max_recv ? row : 0;
-    uint32_t dst_row = padded_index[probe];
-    uint32_t from = source_row[probe];
-    uint32_t total = st.num_recv[2 * r];
-    if (total > st.max_recv) total = st.max_recv;   // flagged by the layout: more rows than the region was sized for
-
-    if (blockIdx.x == 0) {
-        // the receiver's counts for the caller (a2a_dispatch_recv.cu:220-224)
-        const uint32_t E = ws.num_experts, Le = ws.experts_per_rank;
-        const uint32_t first = r * Le;
-        const uint32_t n_local = first >= E ? 0 : (E - first < Le ? E - first : Le);
-        for (uint32_t le = tid; le < n_local; le += blockDim.x) {
-            const uint32_t tpe = ws.tokens_per_expert[first + le];
-            if (args.out_num_tokens != nullptr) args.out_num_tokens[le] = (int32_t)tpe;
-            if (ws.padded_offset[first + le] + tpe > dst.out_rows) atomicOr(ws.err, A2A_DEV_RECV_OVERFLOW);
-        }
-    }
-    if (dst.out_x == nullptr) return;
-
-    const uint32_t stride = gridDim.x * teams;
-    while (row < total) {
-        // the next row's words travel while this one is copied
-        const uint32_t next = row + stride;
-        const uint32_t next_probe = next < total ? next : row;
-        const uint32_t next_dst = padded_index[next_probe];
-        const uint32_t next_from = source_row[next_probe];
-        if (dst_row >= dst.out_rows) {
-            if (member == 0) atomicOr(ws.err, A2A_DEV_RECV_OVERFLOW);
-        } else {
-            const uint8_t *src = st.send_buf + (size_t)from * st.disp_stride;
-            copy_received_row(src, st.payload_bytes, num_chunks, args.hidden_dim_scale, dst, dst_row, member, team);
-        }
-        row = next;
-        dst_row = next_dst;
-        from = next_from;
+// The receiver's counts for the caller (a2a_dispatch_recv.cu:220-224).  One workgroup of a recv that did
+// not lay the receiver out itself.
+__device__ __forceinline__ void hand_over_counts(const StageRecvArgs &args, const Workspace &ws, uint32_t out_rows) {
+    const uint32_t E = ws.num_experts, Le = ws.experts_per_rank;
+    const uint32_t first = args.rank * Le;
+    const uint32_t n_local = first >= E ? 0 : (E - first < Le ? E - first : Le);
+    for (uint32_t le = threadIdx.x; le < n_local; le += blockDim.x) {
+        const uint32_t tpe = ws.tokens_per_expert[first + le];
+        if (args.out_num_tokens != nullptr) args.out_num_tokens[le] = (int32_t)tpe;
+        if (ws.padded_offset[first + le] + tpe > out_rows) atomicOr(ws.err, A2A_DEV_RECV_OVERFLOW);
     }
 }
 
-// A later recv of a step with few rows: the host gave every row a workgroup as wide as the row, so a
-// workgroup is one team and has one row, seldom two; nothing is divided and no row is asked for ahead.
-__global__ __launch_bounds__(1024) void stage_recv_few_kernel(const StageRecvArgs args, const Workspace ws,
-                                                              const Staging st) {
+// Lays out every receiver of a step whose rows are copied by the kernels below (the first recv of the
+// step launches it in front of its copy): the same layout as above, then one thread per received row.
+// Dynamic LDS as stage_recv_first_few_kernel.
+__global__ __launch_bounds__(1024) void stage_layout_kernel(const StageRecvArgs args, const Workspace ws,
+                                                            const Staging st) {
+    extern __shared__ uint32_t s_recv[];
+    __shared__ __align__(16) uint8_t s_order[kMaxWorld];
+    const uint32_t r = blockIdx.x / args.slices;
+    lay_out_rows(args, ws, st, r, blockIdx.x - r * args.slices, s_recv, s_order);
+}
+
+// Rows cut into pieces of 64 sixteen-byte chunks, a wavefront each: wavefront w of the grid takes the
+// pieces w, w + wavefronts, ... of all rows counted through.
+struct PieceWalk {
+    uint32_t row, piece;
+
+    __device__ __forceinline__ void start(const PieceGrid &grid, uint32_t unit) {
+        row = grid.pieces > 1 ? __umulhi(unit, grid.magic) : unit;
+        piece = unit - row * grid.pieces;
+    }
+    __device__ __forceinline__ void advance(const PieceGrid &grid) {
+        row += grid.step_rows;
+        piece += grid.step_pieces;
+        if (piece >= grid.pieces) {
+            piece -= grid.pieces;
+            ++row;
+        }
+    }
+};
+
+// A recv that did not lay the receivers out.  It only moves rows, and what bounds it is the write side of
+// HBM while the reads can come from the Infinity Cache: every staged row is read by the recvs of all the
+// ranks its token was routed to.  Hence
+//  - the rows are walked in the order of arrival by a grid of wavefronts, one 16-byte chunk a lane, so that
+//    reads and writes each advance as ONE front through memory.  A wavefront per row with eight chunks a
+//    lane in flight kept 4096 rows half open at a time: rows of 7392 bytes, 16384 a launch (8 ranks x 2048
+//    tokens), 52.1 us = 4.65 TB/s of reads and writes then, 42.1 us in this order;
+//  - staged rows are loaded with ordinary loads, which keep them in that cache, and from 32 MB of staged rows
+//    on (STREAM) the copies are stored non-temporally, which keeps THEM out of it: 37.0 us = 6.5 TB/s (rows of
+//    14 KB, 235 MB staged: 84.3 -> 69.3 us; 470 MB staged, more than the cache holds: 172 -> 143 us with
+//    non-temporal loads as the other side).  Below that everything fits and the copies are
+//    worth keeping for whoever reads them next (8 x 512 tokens: 10.6 us either way).
+// A row's scales travel with its first pieces; they are 3 us of the 42 (rows of scales are not whole cache
+// lines: their ends are written by two wavefronts at different times).
+template <bool STREAM>
+__global__ __launch_bounds__(kPieceThreads) void stage_recv_kernel(const StageRecvArgs args, const Workspace ws,
+                                                                   const Staging st) {
     // everything a wavefront takes from the argument block, asked for in one go
     A2A_PIN(args.dst.out_x);
     A2A_PIN(args.dst.out_scale);
@@ -1719,6 +1481,10 @@ __global__ __launch_bounds__(1024) void stage_recv_few_kernel(const StageRecvArg
     A2A_PIN(args.rank);
     A2A_PIN(args.row_bytes);
     A2A_PIN(args.hidden_dim_scale);
+    A2A_PIN(args.grid.pieces);
+    A2A_PIN(args.grid.magic);
+    A2A_PIN(args.grid.step_rows);
+    A2A_PIN(args.grid.step_pieces);
     A2A_PIN(st.send_buf);
     A2A_PIN(st.padded_index);
     A2A_PIN(st.source_row);
@@ -1728,60 +1494,79 @@ __global__ __launch_bounds__(1024) void stage_recv_few_kernel(const StageRecvArg
     A2A_PIN(st.max_recv);
     const uint32_t r = args.rank;
     const uint32_t tid = threadIdx.x;
+    const uint32_t lane = tid & (kWave - 1);
     const PushDst &dst = args.dst;
     const uint32_t num_chunks = args.row_bytes / 16;
     const uint32_t *padded_index = st.padded_index + (size_t)r * st.max_recv;
     const uint32_t *source_row = st.source_row + (size_t)r * st.max_recv;
-    // The row's two table words are asked for together with the number of rows received (a row
-    // index the tables do not hold reads entry 0 and is dropped by the loop's bound).
-    uint32_t row = blockIdx.x;
-    const uint32_t probe = row < st.max_recv ? row : 0;
+    // The first piece's two table words are asked for together with the number of rows received
+    // (a row index the tables do not hold reads entry 0 and is dropped by the loop's bound).
+    PieceWalk at;
+    at.start(args.grid, __builtin_amdgcn_readfirstlane(blockIdx.x * (kPieceThreads / kWave) + tid / kWave));
+    const uint32_t probe = at.row < st.max_recv ? at.row : 0;
     uint32_t dst_row = padded_index[probe];
     uint32_t from = source_row[probe];
     uint32_t total = st.num_recv[2 * r];
     if (total > st.max_recv) total = st.max_recv;   // flagged by the layout: more rows than the region was sized for
 
-    if (blockIdx.x == 0) {
-        // the receiver's counts for the caller (a2a_dispatch_recv.cu:220-224)
-        const uint32_t E = ws.num_experts, Le = ws.experts_per_rank;
-        const uint32_t first = r * Le;
-        const uint32_t n_local = first >= E ? 0 : (E - first < Le ? E - first : Le);
-        for (uint32_t le = tid; le < n_local; le += blockDim.x) {
-            const uint32_t tpe = ws.tokens_per_expert[first + le];
-            if (args.out_num_tokens != nullptr) args.out_num_tokens[le] = (int32_t)tpe;
-            if (ws.padded_offset[first + le] + tpe > dst.out_rows) atomicOr(ws.err, A2A_DEV_RECV_OVERFLOW);
-        }
-    }
+    if (blockIdx.x == 0) hand_over_counts(args, ws, dst.out_rows);
     if (dst.out_x == nullptr) return;
 
-    while (row < total) {
-        if (dst_row >= dst.out_rows) {
-            if (tid == 0) atomicOr(ws.err, A2A_DEV_RECV_OVERFLOW);
-        } else {
-            const uint8_t *src = st.send_buf + (size_t)from * st.disp_stride;
-            copy_received_row(src, st.payload_bytes, num_chunks, args.hidden_dim_scale, dst, dst_row, tid, blockDim.x);
+    while (at.row < total) {
+        const uint8_t *src = st.send_buf + (size_t)from * st.disp_stride;
+        const uint32_t c = at.piece * kWave + lane;
+        const bool fits = dst_row < dst.out_rows;
+        const bool active = fits && c < num_chunks;
+                const bool scaled = fits && dst.out_scale != nullptr && c < args.hidden_dim_scale;
+        u32x4 v = {0, 0, 0, 0};
+        float scale = 0.0f;
+        if (active) v = reinterpret_cast<const u32x4 *>(src)[c];
+        if (scaled) scale = reinterpret_cast<const float *>(src + st.payload_bytes)[c];
+        // the next piece's words travel while this one is copied
+        PieceWalk next = at;
+        next.advance(args.grid);
+        const uint32_t next_probe = next.row < total ? next.row : at.row;
+        const uint32_t next_dst = padded_index[next_probe];
+        const uint32_t next_from = source_row[next_probe];
+        if (active) {
+            u32x4 *const to = reinterpret_cast<u32x4 *>(dst.out_x + (size_t)dst_row * dst.out_stride) + c;
+            if constexpr (STREAM) __builtin_nontemporal_store(v, to); else store_copy(v, to);
         }
-        row += gridDim.x;
-        if (row < total) {
-            dst_row = padded_index[row];
-            from = source_row[row];
+        if (scaled) dst.out_scale[(size_t)dst_row * dst.os_stride_token + (size_t)c * dst.os_stride_elem] = scale;
+        if (fits && dst.out_scale != nullptr) {
+            // rows with more scales than pieces have lanes
+            for (uint32_t q = c + args.grid.pieces * kWave; q < args.hidden_dim_scale; q += args.grid.pieces * kWave) {
+                dst.out_scale[(size_t)dst_row * dst.os_stride_token + (size_t)q * dst.os_stride_elem] =
+                    reinterpret_cast<const float *>(src + st.payload_bytes)[q];
+            }
         }
+        if (!fits && at.piece == 0 && lane == 0) atomicOr(ws.err, A2A_DEV_RECV_OVERFLOW);
+        at = next;
+        dst_row = next_dst;
+        from = next_from;
     }
 }
 
 // ---------------------------------------------------------------------------
 // combine send: copy expert_y[padded_index[i]] to the staging row of the copy
 // it answers, i.e. row `source_position[i]` of sender `source_rank[i]`
-// (a2a_combine_send.cu:124-136,196-205).
+// (a2a_combine_send.cu:124-136,196-205).  Walked in pieces as stage_recv_kernel is, and for the same
+// reason: in the order of arrival the rows written are consecutive per source and the rows read per
+// (source, expert), so both sides are fronts through memory.  16384 rows of 14 KB: 105.5 us = 4.45 TB/s
+// with a wavefront per row, 76.5 us = 6.1 TB/s in this order (a plain copy between two arrays in the
+// same order: 74 us; both sides come from and go to HBM, so loads and stores keep nothing).
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(1024) void combine_send_kernel(const CombineSendArgs args,
-                                                            const Workspace ws, const Staging st) {
+__global__ __launch_bounds__(kPieceThreads) void combine_send_kernel(const CombineSendArgs args, const Workspace ws,
+                                                                     const Staging st) {
     // everything a wavefront takes from the argument block, asked for in one go
     A2A_PIN(args.y);
     A2A_PIN(args.y_stride);
     A2A_PIN(args.y_rows);
     A2A_PIN(args.row_bytes);
-    A2A_PIN(args.team_waves);
+    A2A_PIN(args.grid.pieces);
+    A2A_PIN(args.grid.magic);
+    A2A_PIN(args.grid.step_rows);
+    A2A_PIN(args.grid.step_pieces);
     A2A_PIN(ws.dp_size);
     A2A_PIN(ws.max_tk);
     A2A_PIN(st.comb_buf);
@@ -1791,75 +1576,41 @@ __global__ __launch_bounds__(1024) void combine_send_kernel(const CombineSendArg
     A2A_PIN(st.comb_stride);
     A2A_PIN(st.max_recv);
     const uint32_t r = args.rank;
-    uint32_t total = st.num_recv[2 * r];
-    if (total > st.max_recv) total = st.max_recv;
-    const uint32_t num_chunks = args.row_bytes / 16;
-    const uint32_t team = args.team_waves * kWave;   // threads that share a row
-    const uint32_t teams = blockDim.x / team;
-    const uint32_t member = threadIdx.x % team;
-    for (uint32_t i = blockIdx.x * teams + threadIdx.x / team; i < total; i += gridDim.x * teams) {
-        const uint32_t row = st.padded_index[(size_t)r * st.max_recv + i];
-        // every member of the source's dp group reads the same staging rows
-        const uint32_t g = st.source_rank[(size_t)r * st.max_recv + i] / ws.dp_size;
-        const uint32_t pos = st.source_position[(size_t)r * st.max_recv + i];
-        if (row >= args.y_rows || pos >= ws.max_tk) {
-            if (member == 0) atomicOr(ws.err, A2A_DEV_BAD_SLOT);
-            continue;
-        }
-        copy_row_by_team(reinterpret_cast<const u32x4 *>(args.y + (size_t)row * args.y_stride),
-                         reinterpret_cast<u32x4 *>(st.comb_buf + ((size_t)g * ws.max_tk + pos) * st.comb_stride),
-                         num_chunks, member, team);
-    }
-}
-
-// The combine-send of a step with few rows: the host gave every row a workgroup as wide as the row, so
-// a workgroup is one team and has one row, seldom two.  The row's three table words are asked for
-// together with the number of rows received (a row index the tables do not hold reads entry 0 and is
-// dropped by the loop's bound), and nothing is divided: 128 tokens, 3.3 -> 3.1 us per launch.  (The same
-// in the kernel of the large steps made its launches at 4096 tokens 1.5 to 4 % slower.)
-__global__ __launch_bounds__(1024) void combine_send_few_kernel(const CombineSendArgs args,
-                                                                const Workspace ws, const Staging st) {
-    // everything a wavefront takes from the argument block, asked for in one go
-    A2A_PIN(args.y);
-    A2A_PIN(args.y_stride);
-    A2A_PIN(args.y_rows);
-    A2A_PIN(args.row_bytes);
-    A2A_PIN(ws.dp_size);
-    A2A_PIN(ws.max_tk);
-    A2A_PIN(st.comb_buf);
-    A2A_PIN(st.padded_index);
-    A2A_PIN(st.source_rank);
-    A2A_PIN(st.source_position);
-    A2A_PIN(st.comb_stride);
-    A2A_PIN(st.max_recv);
-    const uint32_t r = args.rank;
+    const uint32_t lane = threadIdx.x & (kWave - 1);
     const uint32_t num_chunks = args.row_bytes / 16;
     const uint32_t *padded_index = st.padded_index + (size_t)r * st.max_recv;
     const uint32_t *source_rank = st.source_rank + (size_t)r * st.max_recv;
     const uint32_t *source_position = st.source_position + (size_t)r * st.max_recv;
-    uint32_t i = blockIdx.x;
-    const uint32_t probe = i < st.max_recv ? i : 0;
+    PieceWalk at;
+    at.start(args.grid, __builtin_amdgcn_readfirstlane(blockIdx.x * (kPieceThreads / kWave) + threadIdx.x / kWave));
+    const uint32_t probe = at.row < st.max_recv ? at.row : 0;
     uint32_t row = padded_index[probe];
     uint32_t peer = source_rank[probe];
     uint32_t pos = source_position[probe];
     uint32_t total = st.num_recv[2 * r];
     if (total > st.max_recv) total = st.max_recv;
-    while (i < total) {
+    while (at.row < total) {
+        const uint32_t c = at.piece * kWave + lane;
+        const bool fits = row < args.y_rows && pos < ws.max_tk;
+        const bool active = fits && c < num_chunks;
+        u32x4 v = {0, 0, 0, 0};
+        if (active) v = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(args.y + (size_t)row * args.y_stride) + c);
+        // the next piece's words travel while this one is copied
+        PieceWalk next = at;
+        next.advance(args.grid);
+        const uint32_t next_probe = next.row < total ? next.row : at.row;
+        const uint32_t next_row = padded_index[next_probe];
+        const uint32_t next_peer = source_rank[next_probe];
+        const uint32_t next_pos = source_position[next_probe];
         // every member of the source's dp group reads the same staging rows
         const uint32_t g = ws.dp_size > 1 ? peer / ws.dp_size : peer;
-        if (row >= args.y_rows || pos >= ws.max_tk) {
-            if (threadIdx.x == 0) atomicOr(ws.err, A2A_DEV_BAD_SLOT);
-        } else {
-            copy_row_by_team(reinterpret_cast<const u32x4 *>(args.y + (size_t)row * args.y_stride),
-                             reinterpret_cast<u32x4 *>(st.comb_buf + ((size_t)g * ws.max_tk + pos) * st.comb_stride),
-                             num_chunks, threadIdx.x, blockDim.x);
-        }
-        i += gridDim.x;
-        if (i < total) {
-            row = padded_index[i];
-            peer = source_rank[i];
-            pos = source_position[i];
-        }
+        if (active)
+            store_copy(v, reinterpret_cast<u32x4 *>(st.comb_buf + ((size_t)g * ws.max_tk + pos) * st.comb_stride) + c);
+        if (!fits && at.piece == 0 && lane == 0) atomicOr(ws.err, A2A_DEV_BAD_SLOT);
+        at = next;
+        row = next_row;
+        peer = next_peer;
+        pos = next_pos;
     }
 }
 
@@ -1870,46 +1621,41 @@ uint32_t block_for_chunks(uint32_t chunks) {
     return threads;
 }
 
-// How the rows of a receiver are shared out: the wider the team of wavefronts that shares a row, the
-// shorter the life of a row (what counts when there are few rows), the narrower, the more rows are in
-// flight (what counts when there are many).  The host knows an upper bound of the rows (every copy of
-// every sender); a receiver typically gets 1/N of it, and the team is sized so that those rows give
-// about 4096 wavefronts, as many as the GPU holds at this kernel's occupancy: one wavefront per row from
-// about 4096 rows per receiver on, 2 at 2048, 4 at 1024, up to a team as wide as the row below that
-// (then one workgroup per row).  Measured per step of 8 receivers, rows of 7 KB in / 14 KB back
-// (recv / combine-send, us): 4096 tokens 122 / 198 with one wavefront per row (138 / 210 with two);
-// 2048 tokens 83 / 97 with two (93 / 137 with one, 90 / 123 with four); 1024 tokens 59 / 65 with four
-// (78 / 105 with one, 65 / 77 with two); 512 tokens 50-53 / 48-53 with four to seven (70 / 97 with one);
-// 128 tokens 34 / 31 with the full width (39 / 41 with four).
-constexpr uint32_t kMaxRowWorkgroups = 2048;
-constexpr uint32_t kFewRowWorkgroups = 512;
-constexpr uint32_t kWavefrontsWanted = 4096;
+// The rows of a receiver are copied in pieces by a grid of wavefronts that walks all pieces of all rows in
+// order.  The host knows an upper bound of the rows (every copy of every sender); a receiver typically gets
+// 1/N of it.
+//   - recv: at most 2048 workgroups, the wavefronts that fit the GPU at once (4096 and 8192 workgroups: 43.7 and
+//     43.9 us against 42.1 at 16384 rows of 7 KB).
+//   - combine-send (`in_order`): more workgroups than fit, so that a wavefront of the typical receiver has three
+//     pieces and the hardware, which starts workgroups in order, keeps the front of its 14 KB rows tight: 16384
+//     rows (57344 workgroups' worth of pieces) 88.0 / 86.7 / 82.8 / 78.9 us with 2048 / 4096 / 8192 / 16384 workgroups.
+//     Not more, because the grid is sized for the upper bound and workgroups without rows cost as well:
+//     4096 rows 21.0 / 20.4 / 21.0 / 24.0.
+constexpr uint32_t kPieceWorkgroups = 2048;
+constexpr uint32_t kPiecesInOrder = 3;
+constexpr uint64_t kStreamBytes = 32u << 20;   // staged bytes of a step from which its recvs store past the cache
 
-struct RowLaunch {
-    uint32_t blocks, threads, team_waves;
-};
-
-RowLaunch row_launch(uint32_t max_rows, uint32_t chunks, uint32_t world) {
-    RowLaunch l;
-    const uint32_t width = block_for_chunks(chunks) / kWave;          // wavefronts that cover a row at one piece a lane
-    const uint32_t typical = (max_rows + world - 1) / world;
-    uint32_t want = 1;
-    while (want < width && want * typical < kWavefrontsWanted) want *= 2;
-    if (want >= width) {
-        // few rows: one workgroup per row, as wide as the row needs
-        l.threads = width * kWave;
-        l.team_waves = width;
-        l.blocks = max_rows < kFewRowWorkgroups ? max_rows : kFewRowWorkgroups;
-        return l;
-    }
-    l.team_waves = want;
-    const uint32_t waves = want < 4 ? 4 : want;                       // wavefronts of a workgroup
-    l.threads = waves * kWave;
-    const uint32_t teams = waves / want;
-    const uint32_t blocks = (max_rows + teams - 1) / teams;
-    l.blocks = blocks < kMaxRowWorkgroups ? blocks : kMaxRowWorkgroups;
-    return l;
+uint32_t piece_grid(uint32_t max_rows, uint32_t world, uint32_t chunks, bool in_order, PieceGrid &grid) {
+    constexpr uint32_t waves = kPieceThreads / kWave;
+    grid.pieces = (chunks + kWave - 1) / kWave;
+    const uint64_t most = ((uint64_t)max_rows * grid.pieces + waves - 1) / waves;
+    uint64_t blocks = kPieceWorkgroups;
+    if (in_order && most / world / kPiecesInOrder > blocks) blocks = most / world / kPiecesInOrder;
+    if (blocks > 1u << 16) blocks = 1u << 16;   // (keeps wavefront numbers far below 2^32 / pieces)
+    if (blocks > most) blocks = most;
+    if (blocks < 1) blocks = 1;
+    grid.magic = grid.pieces > 1 ? 0xFFFFFFFFu / grid.pieces + 1 : 0;
+    grid.step_rows = (uint32_t)blocks * waves / grid.pieces;
+    grid.step_pieces = (uint32_t)blocks * waves % grid.pieces;
+    return (uint32_t)blocks;
 }
+
+// The first recv of a step with few rows is ONE launch that lays the receivers out and copies the caller's
+// rows, a workgroup per row; otherwise the layout is a launch in front of the copy.  Whole steps of 8 ranks
+// at the GPU's own pace, hidden 7168, one launch / two: 1 token a rank 91.1 / 93.1 us, 16 tokens (128 rows a
+// receiver) 108.0 / 109.4, 64 tokens (512 rows) 133.7 / 132.7, 128 tokens 180.1 / 177.4.
+constexpr uint32_t kFewRows = 256;
+constexpr uint32_t kFewRowWorkgroups = 512;
 
 }  // namespace
 
@@ -2177,53 +1923,52 @@ hipError_t launch_stage_send_resolve(const StageSendArgs &args, const Workspace 
 
 hipError_t launch_stage_recv(const StageRecvArgs &args, const Workspace &ws, const Staging &st, bool first_of_step,
                              hipStream_t stream, KernelTiming timing) {
-    RowLaunch l = row_launch(args.max_rows, args.row_bytes / 16, ws.world);
-    if (l.blocks == 0) l.blocks = 1;    // the counts are handed over even when nothing was sent
-    StageRecvArgs a = args;
-    a.team_waves = l.team_waves;
-    if (!first_of_step) {
-        if (l.team_waves * kWave == l.threads) {   // few rows: a workgroup per row
-            hipExtLaunchKernelGGL(stage_recv_few_kernel, dim3(l.blocks), dim3(l.threads), 0, stream, timing.start,
-                                  timing.stop, 0, a, ws, st);
-        } else {
-            hipExtLaunchKernelGGL(stage_recv_kernel, dim3(l.blocks), dim3(l.threads), 0, stream, timing.start,
-                                  timing.stop, 0, a, ws, st);
-        }
-        return hipGetLastError();
-    }
-    // Behind the caller's workgroups: a few per other receiver, enough threads for the rows a receiver
-    // typically gets (1/N of the host's upper bound); each repeats that receiver's layout in LDS.
-    a.copy_blocks = l.blocks;
-    const uint32_t typical = (args.max_rows + ws.world - 1) / ws.world;
-    a.slices = (typical + l.threads - 1) / l.threads;
-    if (a.slices < 1) a.slices = 1;
-    if (a.slices > 16) a.slices = 16;
-    const uint32_t blocks = l.blocks + (ws.world - 1) * a.slices;
+    const uint32_t chunks = args.row_bytes / 16;
     const size_t items = (size_t)ws.num_groups * ws.experts_per_rank;
-    if (l.team_waves * kWave == l.threads) {   // few rows: a workgroup per row
-        const size_t lds = (5 * items + 1 + 3 * (size_t)ws.num_groups + ws.experts_per_rank) * sizeof(uint32_t);
-        hipExtLaunchKernelGGL(stage_recv_first_few_kernel, dim3(blocks), dim3(l.threads), lds, stream, timing.start,
-                              timing.stop, 0, a, ws, st);
+    const size_t lds = (5 * items + 1 + 3 * (size_t)ws.num_groups + ws.experts_per_rank) * sizeof(uint32_t);
+    const uint32_t typical = (args.max_rows + ws.world - 1) / ws.world;
+    StageRecvArgs a = args;
+    if (first_of_step && typical <= kFewRows) {
+        const uint32_t threads = block_for_chunks(chunks);
+        uint32_t blocks = args.max_rows < kFewRowWorkgroups ? args.max_rows : kFewRowWorkgroups;
+        if (blocks == 0) blocks = 1;    // the counts are handed over even when nothing was sent
+        // Beside the caller's workgroups: a few per other receiver, enough threads for the rows a receiver
+        // typically gets (1/N of the host's upper bound); each repeats that receiver's layout in LDS.
+        a.copy_blocks = blocks;
+        a.slices = (typical + threads - 1) / threads;
+        if (a.slices < 1) a.slices = 1;
+        if (a.slices > 16) a.slices = 16;
+        hipExtLaunchKernelGGL(stage_recv_first_few_kernel, dim3(blocks + (ws.world - 1) * a.slices), dim3(threads),
+                              lds, stream, timing.start, timing.stop, 0, a, ws, st);
         return hipGetLastError();
     }
-    const size_t lds = (4 * items + 1 + 3 * (size_t)ws.num_groups) * sizeof(uint32_t);
-    hipExtLaunchKernelGGL(stage_recv_first_kernel, dim3(blocks), dim3(l.threads), lds, stream, timing.start,
-                          timing.stop, 0, a, ws, st);
+    if (first_of_step) {
+        constexpr uint32_t threads = 512;
+        a.slices = (typical + threads - 1) / threads;
+        if (a.slices < 1) a.slices = 1;
+        if (a.slices > 32) a.slices = 32;
+        hipLaunchKernelGGL(stage_layout_kernel, dim3(ws.world * a.slices), dim3(threads), lds, stream, a, ws, st);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    const uint32_t blocks = piece_grid(args.max_rows, ws.world, chunks, false, a.grid);
+    if (args.staged_bytes >= kStreamBytes) {
+        hipExtLaunchKernelGGL(stage_recv_kernel<true>, dim3(blocks), dim3(kPieceThreads), 0, stream, timing.start,
+                              timing.stop, 0, a, ws, st);
+    } else {
+        hipExtLaunchKernelGGL(stage_recv_kernel<false>, dim3(blocks), dim3(kPieceThreads), 0, stream, timing.start,
+                              timing.stop, 0, a, ws, st);
+    }
     return hipGetLastError();
 }
 
 hipError_t launch_combine_send(const CombineSendArgs &args, const Workspace &ws, const Staging &st,
                                hipStream_t stream, KernelTiming timing) {
     if (args.max_rows == 0) return hipSuccess;
-    const RowLaunch l = row_launch(args.max_rows, args.row_bytes / 16, ws.world);
+    const uint32_t chunks = args.row_bytes / 16;
     CombineSendArgs a = args;
-    a.team_waves = l.team_waves;
-    if (l.team_waves * kWave == l.threads) {   // few rows: a workgroup per row
-        hipExtLaunchKernelGGL(combine_send_few_kernel, dim3(l.blocks), dim3(l.threads), 0, stream, timing.start,
-                              timing.stop, 0, a, ws, st);
-        return hipGetLastError();
-    }
-    hipExtLaunchKernelGGL(combine_send_kernel, dim3(l.blocks), dim3(l.threads), 0, stream, timing.start, timing.stop,
+    const uint32_t blocks = piece_grid(args.max_rows, ws.world, chunks, true, a.grid);
+    hipExtLaunchKernelGGL(combine_send_kernel, dim3(blocks), dim3(kPieceThreads), 0, stream, timing.start, timing.stop,
                           0, a, ws, st);
     return hipGetLastError();
 }

@@ -11,6 +11,8 @@ import a2a_oracle as oracle
 from a2a_cases import C0, C1, C2, C4, Case, make_world, scaled
 from a2a_harness import (assert_combine_close, assert_dispatch_equal, make_ops, rows_needed, run_gpu,
                          run_oracle, SENTINEL)
+from a2a_transport import RefConfig, check, make_ref_rank, rows_for
+from a2a_transport import run_gpu as run_gpu_rows
 from pplx_garden_amd.native import p2p_all_to_all as native
 
 pytestmark = pytest.mark.gpu
@@ -35,6 +37,28 @@ def test_split_parity(case, sources, device):
     got = run_gpu(case, world, rows, device, split=True)
     assert_dispatch_equal(case, got, want)
     assert_combine_close(case, got, want)
+
+
+F32, BF16, FP8 = torch.float32, torch.bfloat16, torch.float8_e4m3fn
+PIECES = [
+    # the recv's and the combine-send's rows are cut into pieces of 64 chunks of 16 bytes
+    RefConfig("last-piece-not-full", 2, 1, 300, 16, 2944, 23, 4, FP8, BF16, F32),
+    RefConfig("one-chunk-rows", 4, 1, 500, 16, 8, None, 4, BF16, BF16, None),
+    RefConfig("more-scales-than-lanes", 2, 1, 400, 8, 512, 128, 2, FP8, BF16, F32),
+    # a receiver typically gets max_num_tokens * K rows here: one launch up to 256, layout and copy apart from there on
+    RefConfig("256-rows", 2, 1, 64, 16, 1024, 8, 4, FP8, BF16, F32),
+    RefConfig("257-rows", 2, 1, 257, 16, 1024, None, 1, BF16, BF16, None),
+    # 7168 + 112 + 16 bytes at a stride of 7424: 32 MB staged are 4520 tokens; a step on either side
+    RefConfig("kept-in-cache", 2, 1, 2200, 8, 7168, 28, 2, FP8, BF16, F32),
+    RefConfig("past-the-cache", 2, 1, 2300, 8, 7168, 28, 2, FP8, BF16, F32),
+]
+
+
+@pytest.mark.parametrize("cfg", PIECES, ids=lambda c: c.name)
+def test_rows_in_pieces(cfg, device):
+    world = [make_ref_rank(cfg, r) for r in range(cfg.world_size)]
+    rows = rows_for(cfg, world)
+    check(cfg, world, rows, run_gpu_rows(cfg, world, rows, device, True))
 
 
 QUICK_SENDS = [
