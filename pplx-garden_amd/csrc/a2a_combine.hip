@@ -11,15 +11,25 @@
 // Design for CDNA4: one wavefront per (token, slab of 64 sixteen-byte chunks);
 // a lane owns 16 bytes of every source row, so K independent 16-byte loads are
 // in flight per lane before the first multiply-add.  Row pointers and weights
-// are resolved once by the first K lanes and read back as wave-uniform scalars
-// (SGPR base + VGPR offset addressing).  Accumulation is an explicit float fused multiply-add
-// chain, k ascending, then one round-to-nearest-even to the output type
-// (combine_utils.cuh:108-114,14-23).
+// are resolved once by the first K lanes and read back as wave-uniform scalars:
+// each row is a buffer descriptor (uniform base, one offset register for all
+// rows) whose bound stands in for every condition.  Accumulation is an explicit
+// float fused multiply-add chain, k ascending, then one round-to-nearest-even to
+// the output type (combine_utils.cuh:108-114,14-23).
+//
+// What bounds it is HBM: reads alone of the 4096-token shape take 69 us, the
+// output adds what 59 MB of writes cost between them.  4096 tokens of 14 KB
+// rows, K = 8: 91.3 -> 89.7 us (5.9 TB/s) against loads under a condition each (means
+// of several runs, which differ by 1.5 us); for float rows the compiler made
+// copies of all rows' registers at each such condition and waited for every
+// load by itself: 228.9 -> 101.4 us (4096 tokens of 16 KB rows).  Loads and stores are non-temporal (ordinary loads 127 us,
+// device-scope stores 100 us), and so is the load of what a combine
+// accumulates onto (6000 tokens of 8 KB rows, K = 6: 76.5 -> 67.4 us).
+#include "a2a_device.h"
 #include "a2a_internal.h"
 
 namespace a2a {
 
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 struct Bf16 {};
@@ -36,19 +46,19 @@ template <> struct Elem<F32> { static constexpr int kSize = 4; };
 template <typename T> constexpr int vec_elems() { return 16 / Elem<T>::kSize; }
 
 template <typename T, int V>
-__device__ __forceinline__ void load_elems(const uint8_t *p, float (&f)[V], bool streaming) {
+__device__ __forceinline__ void load_elems(const uint8_t *p, float (&f)[V]) {
     if constexpr (Elem<T>::kSize == 4) {
         static_assert(V == 4 || V == 8, "");
 #pragma unroll
         for (int h = 0; h < V / 4; ++h) {
             const u32x4 *q = reinterpret_cast<const u32x4 *>(p) + h;
-            const u32x4 v = streaming ? __builtin_nontemporal_load(q) : *q;
+            const u32x4 v = __builtin_nontemporal_load(q);
 #pragma unroll
             for (int j = 0; j < 4; ++j) f[4 * h + j] = __uint_as_float(v[j]);
         }
     } else if constexpr (V == 8) {
         const u32x4 *q = reinterpret_cast<const u32x4 *>(p);
-        const u32x4 v = streaming ? __builtin_nontemporal_load(q) : *q;
+        const u32x4 v = __builtin_nontemporal_load(q);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             if constexpr (__is_same(T, Bf16)) {
@@ -61,7 +71,7 @@ __device__ __forceinline__ void load_elems(const uint8_t *p, float (&f)[V], bool
         }
     } else {  // V == 4, 16-bit type: 8 bytes
         const u32x2 *q = reinterpret_cast<const u32x2 *>(p);
-        const u32x2 v = streaming ? __builtin_nontemporal_load(q) : *q;
+        const u32x2 v = __builtin_nontemporal_load(q);
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
             if constexpr (__is_same(T, Bf16)) {
@@ -111,10 +121,14 @@ __device__ __forceinline__ void store_elems(uint8_t *p, const float (&f)[V]) {
     }
 }
 
-__device__ __forceinline__ uint64_t read_lane64c(uint64_t v, uint32_t lane) {
-    const uint32_t lo = __builtin_amdgcn_readlane((int)(uint32_t)v, (int)lane);
-    const uint32_t hi = __builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), (int)lane);
-    return ((uint64_t)hi << 32) | lo;
+constexpr int kNonTemporal = 2;   // cache policy bit of a buffer load
+
+// 16 bytes at `offset` of the `bytes` long row at `row`, non-temporally (each row is read once); zeros
+// beyond the row's end, and everywhere for a row that is not there (address 0).
+__device__ __forceinline__ u32x4 load_row_chunk(uint64_t row, uint32_t bytes, uint32_t offset) {
+    __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void *>(row), 0,
+                                                                    row != 0 ? (int)bytes : 0, 0x00020000);
+    return __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)offset, 0, kNonTemporal);
 }
 
 // Convert one 16-byte source chunk (raw) and fuse it into the accumulators.
@@ -140,23 +154,22 @@ __device__ __forceinline__ void fma_chunk(const u32x4 raw, float w, float (&acc)
     }
 }
 
-constexpr int kCombineWaves = 1;    // wavefronts per workgroup; each works on its own
-constexpr int kCombineChunks = 1;   // 16-byte chunks of a row per lane
-constexpr int kSlabChunks = kWave * kCombineChunks;
+constexpr uint32_t kTokensPerLayer = 32768;    // tokens in one layer of the grid
 constexpr uint32_t kOneRankMaxTokens = 2048;   // largest step that takes the ONE_RANK variant of the gather
 
 // T: type of the expert_y rows, U: type of out_tokens.  One WAVEFRONT handles
 // one slab of 64 sixteen-byte chunks of one token; wavefronts share nothing, so
 // a compute unit keeps many of them in flight and the latency of resolving a
-// token's routes is hidden by the loads of its neighbours.  KFIX > 0 unrolls
-// the route loop (all K loads issued before the first use).  ONE_RANK: one rank
+// token's routes is hidden by the loads of its neighbours.  GROUP routes are
+// loaded before the first is used: the smallest of 1, 2, 4, 8 that holds K, or
+// groups of 8 (a load that fills a group up costs its issue only, but at K = 1
+// three of them were 10 %: 96.7 -> 106.4 us for 16000 tokens).  ONE_RANK: one rank
 // alone has tokens and the step is small; its descriptor is read from a fixed
 // place in the argument block, which takes two dependent scalar loads out of
 // the head of every wavefront (0.1-0.4 us of a step of 128 to 1024 tokens; a
 // 4096-token step hides them and is 0.3 us faster without the variant).
-template <typename T, typename U, int KFIX, bool ONE_RANK>
-__global__ __launch_bounds__(kCombineWaves * kWave) void combine_gather_kernel(const CombArgs args,
-                                                                              const Workspace ws) {
+template <typename T, typename U, int GROUP, bool ONE_RANK>
+__global__ __launch_bounds__(kWave) void combine_gather_kernel(const CombArgs args, const Workspace ws) {
     constexpr int V = vec_elems<T>();
     if constexpr (ONE_RANK) {
         // everything the head of a wavefront needs from the argument block, asked for in one go
@@ -199,24 +212,35 @@ __global__ __launch_bounds__(kCombineWaves * kWave) void combine_gather_kernel(c
         A2A_PIN(ws.route_slot);
         A2A_PIN(ws.err);
     }
-    const uint32_t lane = threadIdx.x & (kWave - 1);
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const uint32_t lane = threadIdx.x;
     const uint32_t E = ws.num_experts;
-    const uint32_t K = KFIX > 0 ? (uint32_t)KFIX : ws.topk;
+    const uint32_t K = ws.topk;
     const uint32_t num_chunks = args.hidden_dim / V;
-    const uint32_t slabs = (num_chunks + kSlabChunks - 1) / kSlabChunks;
-
-    const uint32_t unit = blockIdx.x * kCombineWaves + wave;
-    const uint32_t token_global = unit / slabs;
-    const uint32_t slab = unit - token_global * slabs;
+    // the grid: slabs of a token side by side, then its tokens (no division stands in front of the loads)
+    const uint32_t token_global = blockIdx.z * kTokensPerLayer + blockIdx.y;
+    const uint32_t slab = blockIdx.x;
     uint32_t g = 0, token = token_global;
     if constexpr (ONE_RANK) {
         if (token_global >= args.token_start[kMaxWorld]) return;   // the total, at a fixed place
         g = args.single_rank - 1;
     } else {
         if (token_global >= args.token_start[ws.world]) return;
-        while (g + 1 < ws.world && token_global >= args.token_start[g + 1]) ++g;
-        token = token_global - args.token_start[g];
+        // the last rank that starts at or before this token, eight starts at a time asked for together
+        // (the array is non-decreasing and ends in copies of the total)
+        uint32_t start = 0;
+        for (uint32_t r0 = 1; r0 < ws.world; r0 += 8) {
+#pragma unroll
+            for (uint32_t i = 0; i < 8; ++i) {
+                if (r0 + i < (uint32_t)kMaxWorld) {
+                    const uint32_t first = args.token_start[r0 + i];
+                    if (token_global >= first) {
+                        g = r0 + i;
+                        start = first;
+                    }
+                }
+            }
+        }
+        token = token_global - start;
     }
     const CombDst &dst = ONE_RANK ? args.single : args.dst[g];
     const uint32_t group = g / ws.dp_size;   // the routing tables belong to the rank's dp group
@@ -262,62 +286,42 @@ __global__ __launch_bounds__(kCombineWaves * kWave) void combine_gather_kernel(c
         if (!ok && slab == 0) atomicOr(ws.err, A2A_DEV_BAD_SLOT);
     }
 
-    uint32_t c[kCombineChunks];
-    bool active[kCombineChunks];
-    uint8_t *out_chunk[kCombineChunks];
-    float acc[kCombineChunks][V];
+    const uint32_t chunk = slab * kWave + lane;
+    const bool active = chunk < num_chunks;
+    uint8_t *const out_chunk = dst.out + (size_t)token * dst.out_stride + (size_t)chunk * V * Elem<U>::kSize;
+    float acc[V];
 #pragma unroll
-    for (int u = 0; u < kCombineChunks; ++u) {
-        c[u] = slab * kSlabChunks + u * kWave + lane;
-        active[u] = c[u] < num_chunks;
-        out_chunk[u] = dst.out + (size_t)token * dst.out_stride + (size_t)c[u] * V * Elem<U>::kSize;
-#pragma unroll
-        for (int j = 0; j < V; ++j) acc[u][j] = 0.0f;
-        if (args.accumulate && active[u]) load_elems<U, V>(out_chunk[u], acc[u], false);
-    }
+    for (int j = 0; j < V; ++j) acc[j] = 0.0f;
+    if (args.accumulate && active) load_elems<U, V>(out_chunk, acc);
 
-    if constexpr (KFIX > 0) {
-        u32x4 raw[kCombineChunks][KFIX];
-        float w[KFIX];
-        bool present[KFIX];
+    // GROUP routes at a time, all their loads asked for before the first is used.  A row is read through
+    // a buffer descriptor of its own: uniform base, one offset register for all rows, and the descriptor's
+    // bound takes the place of every condition (lanes past the row's end and rows that are not there read
+    // zeros without touching memory).
+    const uint64_t there = __ballot(row_ptr != 0);
+    const uint32_t row_bytes = num_chunks * 16;
+    for (uint32_t k0 = 0; k0 < K; k0 += GROUP) {
+        u32x4 raw[GROUP];
+        float w[GROUP];
 #pragma unroll
-        for (int k = 0; k < KFIX; ++k) {
-            const uint64_t row = read_lane64c(row_ptr, k);
-            w[k] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(weight), k));
-            present[k] = row != 0;
-#pragma unroll
-            for (int u = 0; u < kCombineChunks; ++u) {
-                raw[u][k] = u32x4{0, 0, 0, 0};
-                if (present[k] && active[u]) {
-                    raw[u][k] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(row) + c[u]);
-                }
-            }
+        for (int k = 0; k < GROUP; ++k) {
+            const uint64_t row = read_lane64(row_ptr, k0 + k);
+            w[k] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(weight), (int)(k0 + k)));
+            raw[k] = load_row_chunk(row, row_bytes, chunk * 16);
         }
+        const uint32_t have = (uint32_t)(there >> k0) & ((1u << GROUP) - 1);
+        if (have == (1u << GROUP) - 1) {
 #pragma unroll
-        for (int u = 0; u < kCombineChunks; ++u) {
+            for (int k = 0; k < GROUP; ++k) fma_chunk<T, V>(raw[k], w[k], acc);
+        } else {
+            // (a row that is not there adds nothing, also with a weight that is not finite)
 #pragma unroll
-            for (int k = 0; k < KFIX; ++k) {
-                if (present[k]) fma_chunk<T, V>(raw[u][k], w[k], acc[u]);
-            }
-        }
-    } else {
-        for (uint32_t k = 0; k < K; ++k) {
-            const uint64_t row = read_lane64c(row_ptr, k);
-            const float wk = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(weight), (int)k));
-            if (row != 0) {
-#pragma unroll
-                for (int u = 0; u < kCombineChunks; ++u) {
-                    u32x4 raw = {0, 0, 0, 0};
-                    if (active[u]) raw = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(row) + c[u]);
-                    fma_chunk<T, V>(raw, wk, acc[u]);
-                }
+            for (int k = 0; k < GROUP; ++k) {
+                if (have >> k & 1) fma_chunk<T, V>(raw[k], w[k], acc);
             }
         }
     }
-#pragma unroll
-    for (int u = 0; u < kCombineChunks; ++u) {
-        if (active[u]) store_elems<U, V>(out_chunk[u], acc[u]);
-    }
+    if (active) store_elems<U, V>(out_chunk, acc);
 }
 
 template <typename T, typename U>
@@ -335,17 +339,21 @@ static hipError_t launch_typed(const CombArgs &given, const Workspace &ws, uint3
     if (ranks_with_tokens != 1 || total_tokens > kOneRankMaxTokens) args.single_rank = 0;
     if (args.single_rank != 0) args.single = given.dst[args.single_rank - 1];
     const uint32_t chunks = args.hidden_dim / V;
-    const uint32_t slabs = (chunks + kSlabChunks - 1) / kSlabChunks;
-    const uint64_t units = (uint64_t)total_tokens * slabs;
-    const uint32_t blocks = (uint32_t)((units + kCombineWaves - 1) / kCombineWaves);
-#define A2A_LAUNCH_GATHER(KFIX, ONE)                                                                           \
-    hipExtLaunchKernelGGL((combine_gather_kernel<T, U, KFIX, ONE>), dim3(blocks), dim3(kCombineWaves * kWave), 0, \
-                          stream, timing.start, timing.stop, 0, args, ws)
-    if (ws.topk == 8) {
-        if (args.single_rank != 0) A2A_LAUNCH_GATHER(8, true); else A2A_LAUNCH_GATHER(8, false);
-    } else {
-        if (args.single_rank != 0) A2A_LAUNCH_GATHER(0, true); else A2A_LAUNCH_GATHER(0, false);
-    }
+    const uint32_t slabs = (chunks + kWave - 1) / kWave;
+    const uint32_t layers = (total_tokens + kTokensPerLayer - 1) / kTokensPerLayer;
+    const dim3 grid(slabs, layers > 1 ? kTokensPerLayer : total_tokens, layers);
+#define A2A_LAUNCH_GATHER(GROUP, ONE)                                                                          \
+    hipExtLaunchKernelGGL((combine_gather_kernel<T, U, GROUP, ONE>), grid, dim3(kWave), 0, stream,             \
+                          timing.start, timing.stop, 0, args, ws)
+#define A2A_LAUNCH_GATHER_RANKS(GROUP)                                                                         \
+    do {                                                                                                       \
+        if (args.single_rank != 0) A2A_LAUNCH_GATHER(GROUP, true); else A2A_LAUNCH_GATHER(GROUP, false);       \
+    } while (0)
+    if (ws.topk > 4) A2A_LAUNCH_GATHER_RANKS(8);
+    else if (ws.topk > 2) A2A_LAUNCH_GATHER_RANKS(4);
+    else if (ws.topk > 1) A2A_LAUNCH_GATHER_RANKS(2);
+    else A2A_LAUNCH_GATHER_RANKS(1);
+#undef A2A_LAUNCH_GATHER_RANKS
 #undef A2A_LAUNCH_GATHER
     return hipGetLastError();
 }

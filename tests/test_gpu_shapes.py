@@ -54,3 +54,26 @@ def test_repeated_experts_inside_a_token(split):
     got = run_gpu(case, world, rows, torch.device("cuda:0"), split=split)
     assert_dispatch_equal(case, got, want)
     assert_combine_close(case, got, want)
+
+
+# The combine loads its rows in groups of 1, 2, 4 or 8 (the smallest that holds K, then groups of 8), 64 chunks of
+# 16 bytes per wavefront, with 32768 tokens to a layer of its grid.
+GATHERS = [
+    Case("k1", 70, 640, 8, 2, 1, 7101),
+    Case("k2", 70, 1152, 8, 2, 2, 7102),
+    Case("k3", 70, 512, 12, 4, 3, 7103),
+    Case("k5", 70, 128, 12, 4, 5, 7104),
+    Case("k7", 70, 640, 16, 4, 7, 7105),
+    Case("k9", 70, 512, 16, 4, 9, 7106),
+    Case("k16", 40, 640, 32, 4, 16, 7107),
+    Case("second_layer", 16500, 128, 16, 2, 2, 7108),        # 33000 tokens of two ranks
+]
+
+
+@pytest.mark.parametrize("case", GATHERS, ids=lambda c: c.name)
+def test_gather_groups(case):
+    world = make_world(case, "all")
+    rows = rows_needed(case, world)
+    want = run_oracle(case, world, rows)
+    got = run_gpu(case, world, rows, torch.device("cuda:0"), split=False)
+    assert_combine_close(case, got, want)
