@@ -3,8 +3,10 @@
     python pplx-garden_amd/build.py
 
 Compiles every file under csrc/ with hipcc into
-pplx_garden_amd/lib/liba2a_mi355.so, examples/selftest.cpp (a C++ caller of
-the C ABI) into pplx_garden_amd/lib/a2a_selftest and examples/ceilings.hip (what
+pplx_garden_amd/lib/liba2a_mi355.so, csrc/a2a_torch.cpp (the operator's host
+path, on torch's tensors) into pplx_garden_amd/lib/_a2a_torch.so,
+examples/selftest.cpp (a C++ caller of the C ABI) into
+pplx_garden_amd/lib/a2a_selftest and examples/ceilings.hip (what
 the memory system sustains for the step's access shapes, without the library)
 into pplx_garden_amd/lib/a2a_ceilings.  hipcc cross-compiles without a GPU.
 """
@@ -14,6 +16,7 @@ from __future__ import annotations
 import os
 import subprocess
 import sys
+import sysconfig
 from pathlib import Path
 
 ROOT = Path(__file__).resolve().parent
@@ -38,6 +41,10 @@ HIPCC_FLAGS = [
 
 def library_path() -> Path:
     return OUT_DIR / LIB_NAME
+
+
+def extension_path() -> Path:
+    return OUT_DIR / "_a2a_torch.so"
 
 
 def selftest_path() -> Path:
@@ -81,6 +88,20 @@ def build(verbose: bool = True) -> Path:
     if verbose:
         print(" ".join(link), flush=True)
     subprocess.run(link, check=True)
+    # The operator's host path: host code only, against torch's headers.  The libraries it needs are those of the
+    # torch that is imported before it; the library of the kernels lies beside it.
+    import torch
+    torch_root = Path(torch.__file__).resolve().parent
+    rocm = Path(hipcc).resolve().parent.parent
+    extension = [hipcc, "-x", "c++", "-O2", "-std=c++17", "-fPIC", "-shared", "-DUSE_ROCM", "-D__HIP_PLATFORM_AMD__=1",
+                 "-Wno-unused-command-line-argument", "-I", str(REPO / "include"), "-I", sysconfig.get_paths()["include"],
+                 "-I", str(torch_root / "include"), "-I", str(torch_root / "include" / "torch" / "csrc" / "api" / "include"),
+                 "-I", str(rocm / "include"), str(CSRC / "a2a_torch.cpp"), "-o", str(extension_path()),
+                 "-L", str(torch_root / "lib"), "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python",
+                 "-L", str(OUT_DIR), "-la2a_mi355", "-Wl,-rpath,$ORIGIN"]
+    if verbose:
+        print(" ".join(extension), flush=True)
+    subprocess.run(extension, check=True)
     # A caller of the C ABI with nothing but the HIP runtime around it (no Python, no torch).
     selftest = [hipcc, "-O2", "-std=c++17", "-I", str(REPO / "include"), str(ROOT / "examples" / "selftest.cpp"),
                 "-o", str(selftest_path()), "-L", str(OUT_DIR), "-la2a_mi355", "-Wl,-rpath,$ORIGIN"]

@@ -107,7 +107,9 @@ class LoopbackWorld:
 
     def post(self, key: Tuple, kind: str, rank: int, payload: Any) -> Optional[List[Any]]:
         """Record `rank`'s arguments for collective `kind`.  Returns the
-        arguments of all ranks, in rank order, once the last rank has posted."""
+        arguments of all ranks, in rank order, once the last rank has posted.
+        (The operators' own collectives are collected by their native context,
+        by the same rule.)"""
         slot = self._pending.setdefault((key, kind), {})
         if rank in slot:
             missing = sorted(set(range(self.size)) - set(slot))
@@ -121,4 +123,7 @@ class LoopbackWorld:
         return [slot[r] for r in range(self.size)]
 
     def pending(self, key: Tuple, kind: str) -> List[int]:
-        return sorted(self._pending.get((key, kind), {}))
+        """Ranks that have called collective `kind` of configuration `key` and wait for the others."""
+        context = self._contexts.get(key)
+        native = context.pending(kind) if context is not None else []
+        return sorted({*self._pending.get((key, kind), {}), *native})

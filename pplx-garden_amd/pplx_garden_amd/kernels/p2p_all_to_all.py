@@ -27,18 +27,8 @@ import torch
 
 from pplx_garden_amd.distributed.loopback import LoopbackGroup
 from pplx_garden_amd.kernels.all_to_all import AllToAllKernel
-from pplx_garden_amd.native.p2p_all_to_all import (
-    A2ACombineArgs,
-    A2ADispatchArgs,
-    AllToAllContext,
-)
+from pplx_garden_amd.native.p2p_all_to_all import AllToAllContext, load_extension
 from pplx_garden_amd.utils.math import ceil_div, round_up
-
-QUANT_GROUP = 128
-
-
-def _current_stream(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
 
 
 class P2PAllToAll(AllToAllKernel):
@@ -62,15 +52,10 @@ class P2PAllToAll(AllToAllKernel):
         global_group: LoopbackGroup,
     ) -> None:
         del nets_per_gpu  # no NICs in loopback
-        self._hidden_dim = hidden_dim
-        self._hidden_dim_scale = hidden_dim_scale
-        self._num_experts_per_token = num_experts_per_token
-        self._in_dtype = in_dtype
-        self._out_dtype = out_dtype
-        self._scale_dtype = scale_dtype
         self._device = torch.device(device)
         self._global_group = global_group
         self._all_to_all: Optional[AllToAllContext] = None
+        self._operator = None
 
         if not isinstance(global_group, LoopbackGroup):
             raise TypeError("global_group must be a LoopbackGroup (see LoopbackWorld.group)")
@@ -87,9 +72,6 @@ class P2PAllToAll(AllToAllKernel):
         node_size = node_group.size if node_group is not None else global_group.node_size
         if world_size % node_size != 0:
             raise ValueError(f"node size {node_size} does not divide world size {world_size}")
-        self._rank = rank
-        self._world_size = world_size
-        num_dp_groups = world_size // self._dp_size
         self._num_local_experts = ceil_div(num_experts, world_size)
 
         max_private_tokens, max_recv_tokens = self.receive_capacity(
@@ -137,6 +119,11 @@ class P2PAllToAll(AllToAllKernel):
             )
 
         self._all_to_all = global_group.world.acquire_context(self._key, make_context)
+        # dispatch() and combine() themselves: checks and calls in native code (a2a_torch.cpp)
+        self._operator = load_extension().Operator(
+            self._all_to_all.shared, rank, self._dp_size, hidden_dim,
+            -1 if hidden_dim_scale is None else hidden_dim_scale, self._num_local_experts, num_experts_per_token,
+            in_dtype, out_dtype, scale_dtype is not None, -1 if self._device.index is None else self._device.index)
 
     # ------------------------------------------------------------------
 
@@ -169,14 +156,6 @@ class P2PAllToAll(AllToAllKernel):
         assert self._all_to_all is not None
         return self._all_to_all
 
-    def _is_quantize(self, dp_x: torch.Tensor, dp_x_scale: Optional[torch.Tensor]) -> bool:
-        return (
-            dp_x_scale is None
-            and dp_x.dtype == torch.bfloat16
-            and self._in_dtype == torch.float8_e4m3fn
-            and self._hidden_dim_scale is not None
-        )
-
     def dispatch(
         self,
         out_expert_num_tokens: torch.Tensor,
@@ -190,136 +169,9 @@ class P2PAllToAll(AllToAllKernel):
         do_send: bool = True,
         do_recv: bool = True,
     ) -> None:
-        assert self._all_to_all is not None
-        assert do_send or do_recv
-
-        num_tokens, _ = dp_x.shape
-
-        # Output count buffer (p2p_all_to_all.py:336-340).
-        assert out_expert_num_tokens.shape == (self._num_local_experts,)
-        assert out_expert_num_tokens.stride(0) == 1
-        assert out_expert_num_tokens.dtype == torch.int32
-
-        # Output token buffer (p2p_all_to_all.py:342-348).
-        num_expert_tokens, _ = out_expert_x.shape
-        assert out_expert_x.shape == (num_expert_tokens, self._hidden_dim)
-        assert out_expert_x.stride(1) == 1
-        assert out_expert_x.dtype == self._in_dtype
-        out_x_stride = out_expert_x.stride(0) * out_expert_x.dtype.itemsize
-
-        # Output scale buffer (p2p_all_to_all.py:350-362).
-        if out_expert_x_scale is not None:
-            assert out_expert_x_scale.dtype == self._scale_dtype
-            out_x_scale_ptr = out_expert_x_scale.data_ptr()
-            out_x_scale_stride_elem = out_expert_x_scale.stride(1)
-            out_x_scale_stride_token = out_expert_x_scale.stride(0)
-        else:
-            out_x_scale_ptr = None
-            out_x_scale_stride_elem = None
-            out_x_scale_stride_token = None
-
-        # Input tokens (p2p_all_to_all.py:364-369), plus the quantising mode.
-        quantize = self._is_quantize(dp_x, dp_x_scale)
-        assert dp_x.shape == (num_tokens, self._hidden_dim)
-        assert dp_x.stride(1) == 1
-        if quantize:
-            assert self._hidden_dim % QUANT_GROUP == 0
-            assert self._hidden_dim_scale == self._hidden_dim // QUANT_GROUP
-            assert self._scale_dtype == torch.float32
-            assert out_expert_x_scale is not None
-        else:
-            assert dp_x.dtype == self._in_dtype
-        x_stride = dp_x.stride(0) * dp_x.dtype.itemsize
-
-        # Input scales (p2p_all_to_all.py:371-388).
-        if dp_x_scale is not None:
-            assert self._scale_dtype is not None
-            assert self._hidden_dim_scale is not None
-            assert out_expert_x_scale is not None
-            assert dp_x_scale.dtype == self._scale_dtype
-            x_scale_ptr = dp_x_scale.data_ptr()
-            x_scale_stride_elem = dp_x_scale.stride(1)
-            x_scale_stride_token = dp_x_scale.stride(0)
-        else:
-            if not quantize:
-                assert self._scale_dtype is None
-                assert self._hidden_dim_scale is None
-            x_scale_ptr = None
-            x_scale_stride_elem = None
-            x_scale_stride_token = None
-
-        # Indices and weights (p2p_all_to_all.py:390-402).
-        assert indices.shape == (num_tokens, self._num_experts_per_token)
-        assert indices.stride(1) == 1
-        assert indices.dtype == torch.uint32
-        assert weights.shape == (num_tokens, self._num_experts_per_token)
-        assert weights.stride(1) == 1
-        assert weights.dtype == torch.float32
-
-        # Dynamic bound on the number of tokens (p2p_all_to_all.py:404-411).
-        if bound_m is not None:
-            assert bound_m.numel() == 1
-            assert bound_m.dtype == torch.int32
-            bound_m_ptr = bound_m.data_ptr()
-        else:
-            bound_m_ptr = None
-
-        stream = _current_stream(self._device)
-
-        if do_send and do_recv:
-            args = A2ADispatchArgs(
-                num_tokens=num_tokens, x_ptr=dp_x.data_ptr() or None, x_stride=x_stride,
-                x_scale_ptr=x_scale_ptr, x_scale_stride_elem=x_scale_stride_elem or 0,
-                x_scale_stride_token=x_scale_stride_token or 0,
-                indices=indices.data_ptr() or None, indices_stride=indices.stride(0),
-                weights=weights.data_ptr() or None, weights_stride=weights.stride(0),
-                bound_m=bound_m_ptr, out_num_tokens=out_expert_num_tokens.data_ptr(),
-                out_x=out_expert_x.data_ptr() or None, out_x_stride=out_x_stride,
-                out_x_rows=num_expert_tokens, out_x_scale=out_x_scale_ptr,
-                out_x_scale_stride_elem=out_x_scale_stride_elem or 0,
-                out_x_scale_stride_token=out_x_scale_stride_token or 0)
-            # keep the tensors alive until the collective has been launched
-            keep = (out_expert_num_tokens, out_expert_x, out_expert_x_scale, dp_x, dp_x_scale,
-                    indices, weights, bound_m)
-            posted = self._global_group.world.post(
-                self._key, "dispatch", self._rank, (args, quantize, keep))
-            if posted is not None:
-                modes = {q for _, q, _ in posted}
-                if len(modes) != 1:
-                    raise RuntimeError("every rank must call dispatch() in the same mode")
-                self._all_to_all.dispatch([a for a, _, _ in posted], modes.pop(), stream)
-            return
-
-        if do_send:
-            self._all_to_all.dispatch_send(
-                rank=self._rank,
-                num_tokens=num_tokens,
-                x_ptr=dp_x.data_ptr(),
-                x_stride=x_stride,
-                x_scale_ptr=x_scale_ptr,
-                x_scale_stride_elem=x_scale_stride_elem,
-                x_scale_stride_token=x_scale_stride_token,
-                indices_ptr=indices.data_ptr(),
-                indices_stride=indices.stride(0),
-                weights_ptr=weights.data_ptr(),
-                weights_stride=weights.stride(0),
-                bound_m_ptr=bound_m_ptr,
-                stream=stream,
-                quantize=quantize,
-            )
-
-        if do_recv:
-            self._all_to_all.dispatch_recv(
-                rank=self._rank,
-                out_num_tokens_ptr=out_expert_num_tokens.data_ptr(),
-                out_x_ptr=out_expert_x.data_ptr(),
-                out_x_stride=out_x_stride,
-                out_x_rows=num_expert_tokens,
-                out_x_scale_ptr=out_x_scale_ptr,
-                out_x_scale_stride_elem=out_x_scale_stride_elem,
-                out_x_scale_stride_token=out_x_scale_stride_token,
-                stream=stream,
-            )
+        assert self._operator is not None
+        self._operator.dispatch(out_expert_num_tokens, out_expert_x, out_expert_x_scale, dp_x, dp_x_scale, indices,
+                                weights, bound_m, do_send, do_recv)
 
     def combine(
         self,
@@ -332,91 +184,12 @@ class P2PAllToAll(AllToAllKernel):
         do_recv: bool = True,
         accumulate: bool = False,
     ) -> None:
-        assert self._all_to_all is not None
-        assert do_send or do_recv
-        assert not accumulate or self._dp_size == 1
-
-        num_tokens, _ = indices.shape
-        num_recv_tokens, _ = expert_y.shape
-
-        # p2p_all_to_all.py:463-484
-        assert out_tokens.shape == (num_tokens, self._hidden_dim)
-        assert out_tokens.dtype == self._out_dtype
-        assert out_tokens.stride(1) == 1
-        assert indices.shape == (num_tokens, self._num_experts_per_token)
-        assert indices.stride(1) == 1
-        assert indices.dtype == torch.uint32
-        assert weights.shape == (num_tokens, self._num_experts_per_token)
-        assert weights.stride(1) == 1
-        assert weights.dtype == torch.float32
-        assert expert_y.shape == (num_recv_tokens, self._hidden_dim)
-        assert expert_y.stride(1) == 1
-        expert_y_stride = expert_y.stride(0) * expert_y.dtype.itemsize
-
-        if bound_m is not None:
-            assert bound_m.numel() == 1
-            assert bound_m.dtype == torch.int32
-            bound_m_ptr = bound_m.data_ptr()
-        else:
-            bound_m_ptr = None
-
-        stream = _current_stream(self._device)
-
-        if do_send and do_recv:
-            args = A2ACombineArgs(
-                expert_y=expert_y.data_ptr() or None, expert_y_stride=expert_y_stride,
-                expert_y_rows=num_recv_tokens, num_tokens=num_tokens,
-                out_tokens=out_tokens.data_ptr() or None, out_tokens_stride=out_tokens.stride(0),
-                indices=indices.data_ptr() or None, indices_stride=indices.stride(0),
-                weights=weights.data_ptr() or None, weights_stride=weights.stride(0),
-                bound_m=bound_m_ptr)
-            keep = (out_tokens, indices, weights, expert_y, bound_m)
-            posted = self._global_group.world.post(
-                self._key, "combine", self._rank, (args, expert_y.dtype, bool(accumulate), keep))
-            if posted is not None:
-                dtypes = {d for _, d, _, _ in posted}
-                accs = {a for _, _, a, _ in posted}
-                if len(dtypes) != 1 or len(accs) != 1:
-                    raise RuntimeError(
-                        "every rank must call combine() with the same expert_y dtype and accumulate")
-                self._all_to_all.combine([a for a, _, _, _ in posted], dtypes.pop(), accs.pop(), stream)
-            return
-
-        if expert_y.dtype.itemsize != self._out_dtype.itemsize:
-            # combine-send copies staging rows sized for out_dtype without knowing the type of
-            # expert_y (as the reference's does, a2a_combine_send.cu:261); narrower rows would be over-read
-            raise RuntimeError(
-                f"split combine needs expert_y ({expert_y.dtype}) with the element size of out_dtype "
-                f"({self._out_dtype}); call combine() with do_send and do_recv for mixed types")
-
-        if do_send:
-            self._all_to_all.combine_send(
-                rank=self._rank,
-                expert_x_ptr=expert_y.data_ptr(),
-                expert_x_stride=expert_y_stride,
-                expert_x_rows=num_recv_tokens,
-                stream=stream,
-            )
-
-        if do_recv:
-            self._all_to_all.combine_recv(
-                rank=self._rank,
-                num_tokens=num_tokens,
-                num_recv_tokens=num_recv_tokens,
-                expert_y_dtype=expert_y.dtype,
-                out_tokens_ptr=out_tokens.data_ptr(),
-                out_tokens_stride=out_tokens.stride(0),
-                indices_ptr=indices.data_ptr(),
-                indices_stride=indices.stride(0),
-                weights_ptr=weights.data_ptr(),
-                weights_stride=weights.stride(0),
-                bound_m_ptr=bound_m_ptr,
-                accumulate=accumulate,
-                stream=stream,
-            )
+        assert self._operator is not None
+        self._operator.combine(out_tokens, indices, weights, expert_y, bound_m, do_send, do_recv, accumulate)
 
     def destroy(self) -> None:
         """Release this rank's share of the context; the last rank frees it."""
         if self._all_to_all is not None:
             self._all_to_all = None
+            self._operator = None
             self._global_group.world.release_context(self._key)

@@ -1,4 +1,5 @@
-"""ctypes binding of the compiled library (`liba2a_mi355.so`).
+"""Binding of the compiled library (`liba2a_mi355.so`): ctypes for its C ABI, and the extension
+`_a2a_torch.so` for the calls a step makes (the operator's, and the two group calls).
 
 Plays the part of the reference's pyo3 class `AllToAllContext`
 (python-ext/src/py_p2p_all_to_all.rs:17-205, stub
@@ -7,20 +8,24 @@ python/pplx_garden/native/p2p_all_to_all.pyi:12-98): methods take integers
 (py_p2p_all_to_all.rs:69,73,123-130) and every failure is a `RuntimeError`
 carrying the library's message (py_p2p_all_to_all.rs:133).
 
-There is no fallback: if the library has not been built, importing the context
-raises.
+There is no fallback: if the library or the extension has not been built,
+creating a context raises.
 """
 
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
+import sys
 from ctypes import POINTER, c_char_p, c_int, c_int32, c_size_t, c_uint32, c_uint64, c_void_p
 from pathlib import Path
-from typing import Optional, Sequence
+from typing import List, Optional, Sequence
 
 import torch
 
 _LIB_PATH = Path(__file__).resolve().parent.parent / "lib" / "liba2a_mi355.so"
+_EXTENSION = "_a2a_torch"
 
 # Element type tags in the reference's ScalarType order (rust/torch-lib/src/lib.rs:31-49).
 SCALAR_TYPE = {
@@ -141,6 +146,21 @@ def load_library() -> ctypes.CDLL:
     return lib
 
 
+def load_extension():
+    """Load the extension of the operator's host path once; raise if it has not been built."""
+    module = sys.modules.get(_EXTENSION)
+    if module is None:
+        load_library()
+        path = _LIB_PATH.with_name(_EXTENSION + ".so")
+        if not path.exists():
+            raise ImportError(f"{path} is missing: build it with `python pplx-garden_amd/build.py`")
+        loader = importlib.machinery.ExtensionFileLoader(_EXTENSION, str(path))
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader(_EXTENSION, loader))
+        loader.exec_module(module)
+        sys.modules[_EXTENSION] = module
+    return module
+
+
 def _ptr(value: Optional[int]) -> Optional[int]:
     return None if value in (None, 0) else int(value)
 
@@ -174,6 +194,8 @@ class AllToAllContext:
         self._handle = c_void_p(handle)
         self._config = config
         self._lib = load_library()
+        # what the operators of this context and the group calls go through; closed with the context
+        self.shared = load_extension().Context(handle, config.world_size)
 
     @classmethod
     def create(
@@ -235,6 +257,7 @@ class AllToAllContext:
     def destroy(self) -> None:
         if self._handle:
             handle, self._handle = self._handle, c_void_p()
+            self.shared.close()
             self._check_destroy(self._lib.a2a_ctx_destroy(handle))
 
     @staticmethod
@@ -306,17 +329,19 @@ class AllToAllContext:
 
     def dispatch(self, per_rank, quantize: bool, stream: int) -> None:
         """`per_rank`: one A2ADispatchArgs per rank, or the array from pack_dispatch_args."""
-        self._require_open()
         arr = per_rank if isinstance(per_rank, ctypes.Array) else self.pack_dispatch_args(per_rank)
-        self._check(self._lib.a2a_dispatch(self._handle, arr, int(quantize), _ptr(stream)))
+        self.shared.group_dispatch(arr, quantize, stream)
 
     def combine(self, per_rank, expert_y_dtype: torch.dtype, accumulate: bool, stream: int) -> None:
-        self._require_open()
         if expert_y_dtype not in SCALAR_TYPE:
             raise RuntimeError(f"unsupported expert_y dtype {expert_y_dtype}")
         arr = per_rank if isinstance(per_rank, ctypes.Array) else self.pack_combine_args(per_rank)
-        self._check(self._lib.a2a_combine(
-            self._handle, arr, SCALAR_TYPE[expert_y_dtype], int(bool(accumulate)), _ptr(stream)))
+        self.shared.group_combine(arr, SCALAR_TYPE[expert_y_dtype], accumulate, stream)
+
+    def pending(self, kind: str) -> List[int]:
+        """Ranks whose operators have called collective `kind` ("dispatch" or "combine") and wait for the others."""
+        mask = self.shared.pending(kind)
+        return [r for r in range(self.world_size) if mask >> r & 1]
 
     # -- introspection ------------------------------------------------------
 

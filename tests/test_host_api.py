@@ -266,3 +266,45 @@ int main(void) {
                         "-Wl,--allow-shlib-undefined"], check=True)
         out = subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout.split()
         assert out == ["0.1", "7408", "14336", "2"], out
+
+
+def test_operators_collect_a_collective_in_native_code():
+    """Ranks' calls are collected until the last one (which then needs a live context: this one is closed);
+    a second call of a rank is refused and changes nothing; the checks are the operator's asserts."""
+    module = native.load_extension()
+    context = module.Context(0, 3)
+    ops = [module.Operator(context, r, 1, 128, 1, 2, 4, torch.float8_e4m3fn, torch.bfloat16, True, -1) for r in range(3)]
+    good = [torch.zeros(2, dtype=torch.int32), torch.zeros((8, 128), dtype=torch.float8_e4m3fn), torch.zeros((8, 1)),
+            torch.zeros((5, 128), dtype=torch.bfloat16), None, torch.zeros((5, 4), dtype=torch.int32).view(torch.uint32),
+            torch.zeros((5, 4)), None, True, True]
+    assert ops[2].dispatch(*good) is None and ops[0].dispatch(*good) is None
+    assert context.pending("dispatch") == 0b101 and context.pending("combine") == 0
+    with pytest.raises(RuntimeError, match=r"twice before ranks \[1\]"):
+        ops[0].dispatch(*good)
+    assert context.pending("dispatch") == 0b101
+    for at, bad in [(0, torch.zeros(3, dtype=torch.int32)), (1, good[3]), (2, good[2].double()), (3, good[3].float()),
+                    (4, good[2]), (5, good[5].view(torch.int32)), (6, good[6][:4]), (6, good[6].t().contiguous().t()),
+                    (7, torch.zeros(2, dtype=torch.int32))]:
+        if at == 4:   # scales of the caller with rows that are not fp8
+            bad = torch.zeros((5, 1))
+        with pytest.raises(AssertionError):
+            ops[1].dispatch(*(bad if i == at else v for i, v in enumerate(good)))
+    with pytest.raises(ValueError):
+        ops[1].dispatch(*(good[3][0] if i == 3 else v for i, v in enumerate(good)))
+    with pytest.raises(TypeError):
+        ops[1].dispatch(*(1 if i == 3 else v for i, v in enumerate(good)))
+    with pytest.raises(AssertionError):
+        ops[1].dispatch(*good[:8], False, False)
+    with pytest.raises(RuntimeError, match="destroyed"):
+        ops[1].dispatch(*good)
+    assert context.pending("dispatch") == 0
+    out, y = torch.zeros((5, 128), dtype=torch.bfloat16), torch.zeros((8, 128), dtype=torch.bfloat16)
+    assert ops[1].combine(out, good[5], good[6], y, None, True, True, False) is None
+    assert ops[0].combine(out, good[5], good[6], y, None, True, True, True) is None
+    with pytest.raises(RuntimeError, match="same expert_y dtype and accumulate"):
+        ops[2].combine(out, good[5], good[6], y, None, True, True, False)
+    with pytest.raises(RuntimeError, match="element size"):
+        ops[2].combine(out, good[5], good[6], y.float(), None, True, False, False)
+    assert ops[1].combine(out, good[5], good[6], y, None, True, True, False) is None
+    context.close()
+    assert context.pending("combine") == 0
