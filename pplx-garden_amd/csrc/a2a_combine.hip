@@ -22,8 +22,8 @@
 // rows, K = 8: 91.3 -> 89.7 us (5.9 TB/s) against loads under a condition each (means
 // of several runs, which differ by 1.5 us); for float rows the compiler made
 // copies of all rows' registers at each such condition and waited for every
-// load by itself: 228.9 -> 101.4 us (4096 tokens of 16 KB rows).  Loads and stores are non-temporal (ordinary loads 127 us,
-// device-scope stores 100 us), and so is the load of what a combine
+// load by itself: 228.9 -> 101.4 us (4096 tokens of 16 KB rows).  Loads are non-temporal (ordinary
+// ones 127 us; how the output is written: kStreamedOutput), and so is the load of what a combine
 // accumulates onto (6000 tokens of 8 KB rows, K = 6: 76.5 -> 67.4 us).
 #include "a2a_device.h"
 #include "a2a_internal.h"
@@ -98,37 +98,31 @@ __device__ __forceinline__ uint32_t pack2(float a, float b) {
     }
 }
 
-template <typename U, int V>
-__device__ __forceinline__ void store_elems(uint8_t *p, const float (&f)[V]) {
+typedef int32_t i32x2 __attribute__((ext_vector_type(2)));
+
+// The V elements of chunk `chunk` of the output row at `row`; lanes past the row's end (`bytes`) store nothing.
+template <typename U, int V, int POLICY>
+__device__ __forceinline__ void store_elems(uint64_t row, uint32_t bytes, uint32_t chunk, const float (&f)[V]) {
+    const uint32_t offset = chunk * V * Elem<U>::kSize;
     if constexpr (Elem<U>::kSize == 4) {
 #pragma unroll
         for (int h = 0; h < V / 4; ++h) {
             u32x4 v;
 #pragma unroll
             for (int j = 0; j < 4; ++j) v[j] = __float_as_uint(f[4 * h + j]);
-            __builtin_nontemporal_store(v, reinterpret_cast<u32x4 *>(p) + h);
+            store_row_chunk<POLICY>(v, row, bytes, offset + 16 * h);
         }
     } else if constexpr (V == 8) {
         u32x4 v;
 #pragma unroll
         for (int j = 0; j < 4; ++j) v[j] = pack2<U>(f[2 * j], f[2 * j + 1]);
-        __builtin_nontemporal_store(v, reinterpret_cast<u32x4 *>(p));
+        store_row_chunk<POLICY>(v, row, bytes, offset);
     } else {
-        u32x2 v;
+        i32x2 v;
 #pragma unroll
-        for (int j = 0; j < 2; ++j) v[j] = pack2<U>(f[2 * j], f[2 * j + 1]);
-        __builtin_nontemporal_store(v, reinterpret_cast<u32x2 *>(p));
+        for (int j = 0; j < 2; ++j) v[j] = (int32_t)pack2<U>(f[2 * j], f[2 * j + 1]);
+        __builtin_amdgcn_raw_buffer_store_b64(v, row_descriptor(row, bytes), (int)offset, 0, POLICY);
     }
-}
-
-constexpr int kNonTemporal = 2;   // cache policy bit of a buffer load
-
-// 16 bytes at `offset` of the `bytes` long row at `row`, non-temporally (each row is read once); zeros
-// beyond the row's end, and everywhere for a row that is not there (address 0).
-__device__ __forceinline__ u32x4 load_row_chunk(uint64_t row, uint32_t bytes, uint32_t offset) {
-    __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void *>(row), 0,
-                                                                    row != 0 ? (int)bytes : 0, 0x00020000);
-    return __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)offset, 0, kNonTemporal);
 }
 
 // Convert one 16-byte source chunk (raw) and fuse it into the accumulators.
@@ -157,6 +151,20 @@ __device__ __forceinline__ void fma_chunk(const u32x4 raw, float w, float (&acc)
 constexpr uint32_t kTokensPerLayer = 32768;    // tokens in one layer of the grid
 constexpr uint32_t kOneRankMaxTokens = 2048;   // largest step that takes the ONE_RANK variant of the gather
 
+// How the gather writes where more than one rank has tokens or the step is large, non-temporal / into the Infinity
+// Cache (system scope: written through the caches of the die) / past it:
+//  - outputs of 15 MB behind copies that went past that cache 23.8 / 23.2 / 23.7 us, 29 MB 47.0 / 44.7 / 45.9, 59 MB 91.5 /
+//    86.9 / 89.7, 80 MB 126.0 / 120.4 / 122.1, 88 MB 138 / 140 / 133, 235 MB 371 / 393 / 360.  HBM turns around between
+//    reads and writes, and an output that the cache holds is written back when it suits.
+//  - behind copies that are in the cache themselves: 49 MB 68.0 / 76.0 / -, 27 MB 44.1 / 48.5 / -.
+//  - the ONE_RANK variant's outputs stay non-temporal (15 MB 23.4 / 24.8 / 24.0), and so do those of rows that were
+//    staged (29 MB a launch: 3 us less into the cache, which the copies of the sends that follow lose again).
+// With eight loads a lane, 16 wavefronts a compute unit (19 where outputs go into the cache) are enough to keep HBM busy, and more of
+// them only have more rows open at a time: 470 MB of output 740 -> 670-700 us, 59 MB 86.6 -> 84.5.  The launch asks
+// for LDS that nothing uses to bound them.  (Fewer loads a lane need all wavefronts: K = 2 70.5 -> 80.7 us with 19.)
+constexpr uint64_t kStreamedOutput = 80u << 20;
+constexpr size_t kLds16Waves = 10000, kLds19Waves = 8200;   // of 160 KB
+
 // T: type of the expert_y rows, U: type of out_tokens.  One WAVEFRONT handles
 // one slab of 64 sixteen-byte chunks of one token; wavefronts share nothing, so
 // a compute unit keeps many of them in flight and the latency of resolving a
@@ -168,9 +176,10 @@ constexpr uint32_t kOneRankMaxTokens = 2048;   // largest step that takes the ON
 // place in the argument block, which takes two dependent scalar loads out of
 // the head of every wavefront (0.1-0.4 us of a step of 128 to 1024 tokens; a
 // 4096-token step hides them and is 0.3 us faster without the variant).
-template <typename T, typename U, int GROUP, bool ONE_RANK>
+template <typename T, typename U, int GROUP, bool ONE_RANK, int OUT>
 __global__ __launch_bounds__(kWave) void combine_gather_kernel(const CombArgs args, const Workspace ws) {
     constexpr int V = vec_elems<T>();
+    constexpr int LOAD = OUT == kNonTemporal ? kNonTemporal : kDeviceNonTemporal;
     if constexpr (ONE_RANK) {
         // everything the head of a wavefront needs from the argument block, asked for in one go
         A2A_PIN(args.token_start[kMaxWorld]);
@@ -288,11 +297,11 @@ __global__ __launch_bounds__(kWave) void combine_gather_kernel(const CombArgs ar
 
     const uint32_t chunk = slab * kWave + lane;
     const bool active = chunk < num_chunks;
-    uint8_t *const out_chunk = dst.out + (size_t)token * dst.out_stride + (size_t)chunk * V * Elem<U>::kSize;
+    uint8_t *const out_row = dst.out + (size_t)token * dst.out_stride;
     float acc[V];
 #pragma unroll
     for (int j = 0; j < V; ++j) acc[j] = 0.0f;
-    if (args.accumulate && active) load_elems<U, V>(out_chunk, acc);
+    if (args.accumulate && active) load_elems<U, V>(out_row + (size_t)chunk * V * Elem<U>::kSize, acc);
 
     // GROUP routes at a time, all their loads asked for before the first is used.  A row is read through
     // a buffer descriptor of its own: uniform base, one offset register for all rows, and the descriptor's
@@ -307,7 +316,7 @@ __global__ __launch_bounds__(kWave) void combine_gather_kernel(const CombArgs ar
         for (int k = 0; k < GROUP; ++k) {
             const uint64_t row = read_lane64(row_ptr, k0 + k);
             w[k] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(weight), (int)(k0 + k)));
-            raw[k] = load_row_chunk(row, row_bytes, chunk * 16);
+            raw[k] = load_row_chunk<LOAD>(row, row_bytes, chunk * 16);
         }
         const uint32_t have = (uint32_t)(there >> k0) & ((1u << GROUP) - 1);
         if (have == (1u << GROUP) - 1) {
@@ -321,12 +330,12 @@ __global__ __launch_bounds__(kWave) void combine_gather_kernel(const CombArgs ar
             }
         }
     }
-    if (active) store_elems<U, V>(out_chunk, acc);
+    store_elems<U, V, OUT>((uint64_t)out_row, num_chunks * V * Elem<U>::kSize, chunk, acc);
 }
 
 template <typename T, typename U>
 static hipError_t launch_typed(const CombArgs &given, const Workspace &ws, uint32_t total_tokens,
-                               hipStream_t stream, KernelTiming timing) {
+                               uint64_t copies, hipStream_t stream, KernelTiming timing) {
     constexpr int V = vec_elems<T>();
     CombArgs args = given;
     uint32_t ranks_with_tokens = 0;
@@ -342,12 +351,18 @@ static hipError_t launch_typed(const CombArgs &given, const Workspace &ws, uint3
     const uint32_t slabs = (chunks + kWave - 1) / kWave;
     const uint32_t layers = (total_tokens + kTokensPerLayer - 1) / kTokensPerLayer;
     const dim3 grid(slabs, layers > 1 ? kTokensPerLayer : total_tokens, layers);
-#define A2A_LAUNCH_GATHER(GROUP, ONE)                                                                          \
-    hipExtLaunchKernelGGL((combine_gather_kernel<T, U, GROUP, ONE>), grid, dim3(kWave), 0, stream,             \
+    const bool plain = args.single_rank != 0 || args.staged_base != nullptr;
+    const bool past_cache = !plain && (uint64_t)total_tokens * args.hidden_dim * Elem<U>::kSize >= kStreamedOutput;
+    const bool into_cache = !plain && !past_cache && copies >= kStreamCopies && ws.topk > 2;
+#define A2A_LAUNCH_GATHER(GROUP, ONE, OUT, LDS)                                                                \
+    hipExtLaunchKernelGGL((combine_gather_kernel<T, U, GROUP, ONE, OUT>), grid, dim3(kWave), LDS, stream,      \
                           timing.start, timing.stop, 0, args, ws)
 #define A2A_LAUNCH_GATHER_RANKS(GROUP)                                                                         \
     do {                                                                                                       \
-        if (args.single_rank != 0) A2A_LAUNCH_GATHER(GROUP, true); else A2A_LAUNCH_GATHER(GROUP, false);       \
+        if (args.single_rank != 0) A2A_LAUNCH_GATHER(GROUP, true, kNonTemporal, 0);                            \
+        else if (past_cache) A2A_LAUNCH_GATHER(GROUP, false, kSystemNonTemporal, GROUP == 8 ? kLds16Waves : 0); \
+        else if (into_cache) A2A_LAUNCH_GATHER(GROUP, false, kSystemScope, GROUP == 8 ? kLds19Waves : 0);      \
+        else A2A_LAUNCH_GATHER(GROUP, false, kNonTemporal, 0);                                                 \
     } while (0)
     if (ws.topk > 4) A2A_LAUNCH_GATHER_RANKS(8);
     else if (ws.topk > 2) A2A_LAUNCH_GATHER_RANKS(4);
@@ -359,11 +374,12 @@ static hipError_t launch_typed(const CombArgs &given, const Workspace &ws, uint3
 }
 
 hipError_t launch_combine_gather(const CombArgs &args, const Workspace &ws, uint32_t in_dtype,
-                                 uint32_t out_dtype, uint32_t total_tokens, hipStream_t stream, KernelTiming timing) {
+                                 uint32_t out_dtype, uint32_t total_tokens, uint64_t copies, hipStream_t stream,
+                                 KernelTiming timing) {
     if (total_tokens == 0) return hipSuccess;
 #define A2A_COMBINE_CASE(IN_TAG, IN_T, OUT_TAG, OUT_T) \
     if (in_dtype == IN_TAG && out_dtype == OUT_TAG)    \
-        return launch_typed<IN_T, OUT_T>(args, ws, total_tokens, stream, timing);
+        return launch_typed<IN_T, OUT_T>(args, ws, total_tokens, copies, stream, timing);
     A2A_COMBINE_CASE(A2A_BF16, Bf16, A2A_BF16, Bf16)
     A2A_COMBINE_CASE(A2A_BF16, Bf16, A2A_F32, F32)
     A2A_COMBINE_CASE(A2A_BF16, Bf16, A2A_F16, F16)

@@ -824,7 +824,9 @@ int a2a_combine(a2a_ctx *ctx, const a2a_combine_args *args, uint32_t expert_y_dt
     DeviceGuard guard(c.device);
     const KernelTiming gather_timing = ctx->timing[A2A_KERNEL_GATHER];
     ctx->timing[A2A_KERNEL_GATHER] = KernelTiming();
-    hipError_t e = launch_combine_gather(ca, ctx->ws, expert_y_dtype, c.out_dtype, tokens,
+    // (the ranks of a dp group combine the same tokens)
+    const uint64_t copies = (uint64_t)tokens / ctx->ws.dp_size * c.num_experts_per_token * row_bytes_of(c);
+    hipError_t e = launch_combine_gather(ca, ctx->ws, expert_y_dtype, c.out_dtype, tokens, copies,
                                          static_cast<hipStream_t>(stream), gather_timing);
     if (e != hipSuccess) return hip_fail(ctx, e, "launch combine_gather");
     return A2A_OK;

@@ -16,14 +16,36 @@ __device__ __forceinline__ void lds_barrier() {
 }
 
 // The 16-byte store of a dispatched copy, at device scope (`sc1`): the line is written through
-// instead of staying dirty in the L2 of the storing die.  Measured on the 4096-token pack against
-// the other policies of the store: non-temporal 62 us, ordinary 50.3 us, device scope 49.7 us
-// (plain kernels of the same shape: 63 / 48.5 / 47.4 us).  The wait state behind the store is not optional: a
+// instead of staying dirty in the L2 of the storing die.  The wait state behind the store is not optional: a
 // vector instruction that follows a store of more than 64 bits must not write the registers the store takes
 // its data from in the very next slot, and the compiler, which inserts that state behind stores it knows of,
 // cannot see this one (a loop that cleared the registers for its next piece sent zeros now and then).
 __device__ __forceinline__ void store_copy(u32x4 v, u32x4 *p) {
     asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 0" ::"v"(p), "v"(v) : "memory");
+}
+
+// Cache policies of buffer loads and stores (the sc0, nt and sc1 bits of the instruction).
+constexpr int kOrdinary = 0;
+constexpr int kNonTemporal = 2;
+constexpr int kDeviceScope = 16;
+constexpr int kDeviceNonTemporal = 16 | 2;
+constexpr int kSystemScope = 16 | 1;
+constexpr int kSystemNonTemporal = 16 | 2 | 1;
+
+// A row as a buffer descriptor: `row` is the same in all lanes, and the descriptor's bound takes the place of every
+// condition.  Lanes past the row's end and rows that are not there (address 0) load zeros and store nothing.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t row_descriptor(uint64_t row, uint32_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void *>(row), 0, row != 0 ? (int)bytes : 0, 0x00020000);
+}
+
+template <int POLICY>
+__device__ __forceinline__ u32x4 load_row_chunk(uint64_t row, uint32_t bytes, uint32_t offset) {
+    return __builtin_amdgcn_raw_buffer_load_b128(row_descriptor(row, bytes), (int)offset, 0, POLICY);
+}
+
+template <int POLICY>
+__device__ __forceinline__ void store_row_chunk(u32x4 v, uint64_t row, uint32_t bytes, uint32_t offset) {
+    __builtin_amdgcn_raw_buffer_store_b128(v, row_descriptor(row, bytes), (int)offset, 0, POLICY);
 }
 
 template <int CTRL>

@@ -14,10 +14,9 @@
 // eight scales a wavefront produces are spread over the lanes so that a single
 // store instruction writes them for eight routes at once.  Row pointers are
 // computed once per token by the first K lanes and read back as wave-uniform
-// scalars.  Token rows are loaded non-temporally (each is read once).  The
-// copies are written with cached stores at device scope: measured on this part,
-// non-temporal stores to this many rows at once sustain about two thirds of
-// that rate (see store_copy).
+// scalars.  Token rows are loaded non-temporally (each is read once).  How the
+// copies are written depends on how much of the Infinity Cache they fill (see
+// kStreamCopies).
 #include "a2a_device.h"
 #include "a2a_scan.h"
 
@@ -29,6 +28,24 @@ constexpr int kMaxLdsScales = 1024;
 
 // Arguments travel by value; a launch can carry 4 KB of them.
 static_assert(sizeof(PushArgs) + sizeof(FinalizeArgs) + sizeof(Workspace) <= 4096, "kernel arguments too large");
+
+// Stores one chunk of a row at `offset` of each of its copies (lane k: address of copy k, 0 = none) of `bytes` bytes.
+// The K stores are straight-line code for K = 8: copies that are not there and lanes past the row's end are dropped by
+// the descriptors' bounds, not by branches.
+template <int POLICY>
+__device__ __forceinline__ void store_copies(u32x4 v, uint64_t row_ptr, uint32_t K, uint32_t bytes, uint32_t offset) {
+    if constexpr (POLICY == kOrdinary) {
+        for (uint32_t k = 0; k < K; ++k) {
+            const uint64_t row = read_lane64(row_ptr, k);
+            if (row != 0 && offset < bytes) *reinterpret_cast<u32x4 *>(row + offset) = v;
+        }
+    } else if (K == 8) {
+#pragma unroll
+        for (uint32_t k = 0; k < 8; ++k) store_row_chunk<POLICY>(v, read_lane64(row_ptr, k), bytes, offset);
+    } else {
+        for (uint32_t k = 0; k < K; ++k) store_row_chunk<POLICY>(v, read_lane64(row_ptr, k), bytes, offset);
+    }
+}
 
 // Moves the row of `token` to its copies.  Lanes 0..K-1 of EVERY wavefront hold
 // the row pointer, scale pointer and scale stride of route k (0 = no copy).
@@ -42,7 +59,8 @@ static_assert(sizeof(PushArgs) + sizeof(FinalizeArgs) + sizeof(Workspace) <= 409
 // the workgroup must call (there is a barrier inside); a team without a token
 // passes `live` false.
 // PRE: the thread's first piece of the row was asked for earlier (first_piece) and is passed in.
-template <bool QUANT, bool PRE = false>
+// POLICY: cache policy of the copies' stores.
+template <bool QUANT, bool PRE = false, int POLICY = QUANT ? kDeviceScope : kOrdinary>
 __device__ __forceinline__ void push_rows(const PushArgs &args, const PushSrc &src, uint32_t token, uint32_t K,
                                           uint64_t row_ptr, uint64_t scale_ptr, uint32_t scale_stride,
                                           float *s_scale, uint64_t *s_scale_ptr, uint32_t *s_scale_stride,
@@ -70,12 +88,7 @@ __device__ __forceinline__ void push_rows(const PushArgs &args, const PushSrc &s
             }
             float scale;
             const u32x4 q = quantize16(a, b, &scale);
-            for (uint32_t k = 0; k < K; ++k) {
-                const uint64_t row = read_lane64(row_ptr, k);
-                if (row != 0 && active) {
-                    store_copy(q, reinterpret_cast<u32x4 *>(row + (size_t)c * 16));
-                }
-            }
+            store_copies<POLICY>(q, row_ptr, K, num_chunks * 16, c * 16);
             if (active && (lane & 7) == 0 && c / 8 < kMaxLdsScales) s_scale[c / 8] = scale;
         }
         // The token's scales meet in LDS so that each copy's scale row goes out
@@ -96,12 +109,7 @@ __device__ __forceinline__ void push_rows(const PushArgs &args, const PushSrc &s
         const uint32_t num_chunks = live ? args.row_bytes / 16 : 0;
         for (uint32_t c = tid; c < num_chunks; c += team_threads) {
             const u32x4 v = PRE && c == tid ? pre_a : __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(x_row) + c);
-            for (uint32_t k = 0; k < K; ++k) {
-                const uint64_t row = read_lane64(row_ptr, k);
-                if (row != 0) {
-                    reinterpret_cast<u32x4 *>(row)[c] = v;
-                }
-            }
+            store_copies<POLICY>(v, row_ptr, K, num_chunks * 16, c * 16);
         }
         if (src.x_scale != nullptr && live) {
             const float *xs = src.x_scale + (size_t)token * src.xs_stride_token;
@@ -1584,7 +1592,7 @@ __global__ __launch_bounds__(1024) void dispatch_teams_kernel(const PushArgs arg
 // the grid holds one workgroup per receiver (expert counts for the caller,
 // layout tables) and one per source (its totals and their scan); the last of
 // them hands the totals over to the next step.
-template <bool QUANT>
+template <bool QUANT, int POLICY>
 __global__ __launch_bounds__(1024) void dispatch_resolve_kernel(const PushArgs args, const FinalizeArgs fin,
                                                                 const Workspace ws) {
     __shared__ float s_scale[QUANT ? kMaxLdsScales : 1];
@@ -1737,8 +1745,8 @@ __global__ __launch_bounds__(1024) void dispatch_resolve_kernel(const PushArgs a
         scale_ptr = s_route_scale_ptr[lane];
         scale_stride = s_route_scale_stride[lane];
     }
-    push_rows<QUANT>(args, src, token, K, row_ptr, scale_ptr, scale_stride, s_scale, s_scale_ptr, s_scale_stride,
-                     threadIdx.x, blockDim.x, true);
+    push_rows<QUANT, false, POLICY>(args, src, token, K, row_ptr, scale_ptr, scale_stride, s_scale, s_scale_ptr,
+                                    s_scale_stride, threadIdx.x, blockDim.x, true);
 }
 
 hipError_t launch_dispatch_push(const PushArgs &args, const Workspace &ws, bool quantize,
@@ -1921,6 +1929,10 @@ hipError_t launch_dispatch_single(const PushArgs &args, const FinalizeArgs &fin,
     return hipGetLastError();
 }
 
+// How the copies are written: past the cache from kStreamCopies on.  Smaller steps write quantised rows at device scope,
+// others with ordinary stores (device scope: 1 us less of 24 for 8 KB rows, but 3-5 us more of 33 for rows of 5120
+// bytes).  Rows that are not quantised and have at most two copies take ordinary stores at every size (rows of 2 KB,
+// K = 1: 44.0 us against 46.6 past the cache; 8 KB, K = 2: 91.0 against 94.5).
 hipError_t launch_dispatch_resolve(const PushArgs &args, const FinalizeArgs &fin, const Workspace &ws,
                                    bool quantize, uint32_t total_tokens, hipStream_t stream, KernelTiming timing) {
     uint32_t threads = push_threads(args, quantize);
@@ -1938,13 +1950,17 @@ hipError_t launch_dispatch_resolve(const PushArgs &args, const FinalizeArgs &fin
     }
     if (senders != 1) a.single_source = 0;    // here only "one source has tokens": the rows may be strided
     if (a.single_source != 0) a.single = args.src[a.single_source - 1];
+    const uint64_t copies = (uint64_t)total_tokens * ws.topk * (quantize ? args.hidden_dim : args.row_bytes);
+    const bool stream_copies = copies >= kStreamCopies && (quantize || ws.topk > 2);
+#define A2A_LAUNCH_RESOLVE(Q, P)                                                                                   \
+    hipExtLaunchKernelGGL((dispatch_resolve_kernel<Q, P>), dim3(blocks), dim3(threads), 0, stream, timing.start,  \
+                          timing.stop, 0, a, fin, ws)
     if (quantize) {
-        hipExtLaunchKernelGGL(dispatch_resolve_kernel<true>, dim3(blocks), dim3(threads), 0, stream, timing.start,
-                              timing.stop, 0, a, fin, ws);
+        if (stream_copies) A2A_LAUNCH_RESOLVE(true, kDeviceNonTemporal); else A2A_LAUNCH_RESOLVE(true, kDeviceScope);
     } else {
-        hipExtLaunchKernelGGL(dispatch_resolve_kernel<false>, dim3(blocks), dim3(threads), 0, stream, timing.start,
-                              timing.stop, 0, a, fin, ws);
+        if (stream_copies) A2A_LAUNCH_RESOLVE(false, kDeviceNonTemporal); else A2A_LAUNCH_RESOLVE(false, kOrdinary);
     }
+#undef A2A_LAUNCH_RESOLVE
     return hipGetLastError();
 }
 

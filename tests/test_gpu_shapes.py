@@ -77,3 +77,63 @@ def test_gather_groups(case):
     want = run_oracle(case, world, rows)
     got = run_gpu(case, world, rows, torch.device("cuda:0"), split=False)
     assert_combine_close(case, got, want)
+
+
+# Steps whose copies go past the Infinity Cache (from 104 MB on) and whose combined tokens go into it or, from 80 MB on,
+# past it, at row lengths that end inside a wavefront's slab: the group calls against the split calls, which move
+# every row by other kernels.  (row type, hidden, scales, experts per token, tokens of the two ranks with tokens)
+STREAMED = [
+    (torch.bfloat16, 1000, 0, 5, (10000, 1100)),        # 111 MB of copies, 22 MB of tokens
+    (torch.float16, 1000, 0, 3, (40000, 3001)),         # 258 MB, 86 MB
+    (torch.float32, 1004, 0, 8, (4000, 301)),           # 138 MB, 17 MB
+    (torch.float8_e4m3fn, 1152, 9, 8, (11000, 1000)),   # 111 MB, 28 MB
+    (torch.bfloat16, 1000, 0, 2, (41000, 2100)),        # 172 MB of copies that stay ordinary, 86 MB
+    (torch.bfloat16, 1000, 0, 9, (5800, 7)),            # 105 MB: two groups of rows a token
+]
+
+
+@pytest.mark.parametrize("row,hidden,scales,k,tokens", STREAMED,
+                         ids=lambda v: str(v).replace("torch.", "") if isinstance(v, torch.dtype) else None)
+def test_streamed_copies_and_tokens(row, hidden, scales, k, tokens):
+    from pplx_garden_amd.distributed.loopback import LoopbackWorld
+    from pplx_garden_amd.kernels.p2p_all_to_all import P2PAllToAll
+
+    device, N, E = torch.device("cuda:0"), 3, 24
+    out = torch.bfloat16 if scales else row
+    world = LoopbackWorld(N, device=device)
+    counts = (tokens[0], 0, tokens[1])
+    rows = sum(counts) * k
+    ops = [P2PAllToAll(max_num_tokens=max(counts), num_experts=E, expert_padding=1, hidden_dim=hidden,
+                       hidden_dim_scale=scales or None, in_dtype=row, out_dtype=out,
+                       scale_dtype=torch.float32 if scales else None, num_experts_per_token=k, device=device,
+                       global_group=world.group(r)) for r in range(N)]
+    gen = torch.Generator(device=device).manual_seed(hidden * k)
+    data = []
+    for t in counts:
+        data.append(dict(
+            dp_x=torch.randn((t, hidden), generator=gen, device=device).to(row),
+            dp_x_scale=torch.rand((t, scales), generator=gen, device=device) if scales else None,
+            indices=torch.rand((t, E), generator=gen, device=device).topk(k).indices.to(torch.int32).view(torch.uint32),
+            weights=torch.rand((t, k), generator=gen, device=device)))
+    expert_y = [torch.randn((rows, hidden), generator=gen, device=device).to(out) for _ in range(N)]
+    results = []
+    for halves in ([dict()], [dict(do_recv=False), dict(do_send=False)]):
+        got = [dict(out_expert_num_tokens=torch.zeros(-(-E // N), dtype=torch.int32, device=device),
+                    out_expert_x=torch.zeros((rows, hidden), dtype=torch.uint8 if scales else row, device=device).view(row),
+                    out_expert_x_scale=torch.zeros((rows, scales), device=device) if scales else None) for _ in range(N)]
+        combined = [torch.full((t, hidden), 0.5, dtype=out, device=device) for t in counts]
+        for half in halves:
+            for r in range(N):
+                ops[r].dispatch(**got[r], **data[r], **half)
+        for half in halves:
+            for r in range(N):
+                ops[r].combine(out_tokens=combined[r], indices=data[r]["indices"], weights=data[r]["weights"],
+                               expert_y=expert_y[r], accumulate=True, **half)
+        torch.cuda.synchronize()
+        assert ops[0].context.status() == 0
+        results.append([g[n] for g in got for n in g if g[n] is not None] + combined)
+    assert sum(int(n.sum()) for n in results[0] if n.dtype == torch.int32) == rows
+    for a, b in zip(*results):
+        assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+    for op in ops:
+        op.destroy()
