@@ -1517,7 +1517,7 @@ __global__ __launch_bounds__(kPieceThreads) void stage_recv_kernel(const StageRe
         const uint32_t c = at.piece * kWave + lane;
         const bool fits = dst_row < dst.out_rows;
         const bool active = fits && c < num_chunks;
-                const bool scaled = fits && dst.out_scale != nullptr && c < args.hidden_dim_scale;
+        const bool scaled = fits && dst.out_scale != nullptr && c < args.hidden_dim_scale;
         u32x4 v = {0, 0, 0, 0};
         float scale = 0.0f;
         if (active) v = reinterpret_cast<const u32x4 *>(src)[c];
