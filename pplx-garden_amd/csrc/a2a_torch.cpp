@@ -121,13 +121,18 @@ PyObject *context_pending(PyObject *self, PyObject *kind) {
     return PyLong_FromUnsignedLong(name[0] == 'd' ? c->dispatch->posted : c->combine->posted);
 }
 
-// The arguments of all ranks out of a C array (ctypes) of exactly `world` structures.
+// The arguments of all ranks out of a C array (ctypes) of at least `world` structures.
 template <typename Args>
 bool array_of(PyObject *obj, uint32_t world, Py_buffer *view) {
     if (PyObject_GetBuffer(obj, view, PyBUF_SIMPLE) != 0) return false;
-    if (view->len == (Py_ssize_t)(sizeof(Args) * world)) return true;
+    const bool right_type = view->itemsize == (Py_ssize_t)sizeof(Args);
+    if (right_type && view->len >= (Py_ssize_t)(sizeof(Args) * world)) return true;
     PyBuffer_Release(view);
-    PyErr_Format(PyExc_RuntimeError, "expected arguments of %u ranks", world);
+    if (right_type) {
+        PyErr_Format(PyExc_RuntimeError, "expected arguments of %u ranks", world);
+    } else {
+        PyErr_SetString(PyExc_TypeError, "an array of another call's arguments");
+    }
     return false;
 }
 
@@ -135,13 +140,16 @@ bool array_of(PyObject *obj, uint32_t world, Py_buffer *view) {
 PyObject *context_group_dispatch(PyObject *self, PyObject *const *args, Py_ssize_t n) {
     Context *c = reinterpret_cast<Context *>(self);
     if (n != 3) return PyErr_Format(PyExc_TypeError, "group_dispatch takes 3 arguments");
-    if (!require_open(c)) return nullptr;
     const int quantize = PyObject_IsTrue(args[1]);
     if (quantize < 0) return nullptr;
     void *stream = PyLong_AsVoidPtr(args[2]);
     if (stream == nullptr && PyErr_Occurred()) return nullptr;
     Py_buffer view;
     if (!array_of<a2a_dispatch_args>(args[0], c->world, &view)) return nullptr;
+    if (!require_open(c)) {
+        PyBuffer_Release(&view);
+        return nullptr;
+    }
     a2a_ctx *const ctx = c->ctx;
     int rc;
     Py_BEGIN_ALLOW_THREADS
@@ -156,7 +164,6 @@ PyObject *context_group_dispatch(PyObject *self, PyObject *const *args, Py_ssize
 PyObject *context_group_combine(PyObject *self, PyObject *const *args, Py_ssize_t n) {
     Context *c = reinterpret_cast<Context *>(self);
     if (n != 4) return PyErr_Format(PyExc_TypeError, "group_combine takes 4 arguments");
-    if (!require_open(c)) return nullptr;
     const unsigned long tag = PyLong_AsUnsignedLong(args[1]);
     if (tag == (unsigned long)-1 && PyErr_Occurred()) return nullptr;
     const int accumulate = PyObject_IsTrue(args[2]);
@@ -165,6 +172,10 @@ PyObject *context_group_combine(PyObject *self, PyObject *const *args, Py_ssize_
     if (stream == nullptr && PyErr_Occurred()) return nullptr;
     Py_buffer view;
     if (!array_of<a2a_combine_args>(args[0], c->world, &view)) return nullptr;
+    if (!require_open(c)) {
+        PyBuffer_Release(&view);
+        return nullptr;
+    }
     a2a_ctx *const ctx = c->ctx;
     int rc;
     Py_BEGIN_ALLOW_THREADS

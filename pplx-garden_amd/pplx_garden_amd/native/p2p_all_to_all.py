@@ -330,13 +330,13 @@ class AllToAllContext:
     def dispatch(self, per_rank, quantize: bool, stream: int) -> None:
         """`per_rank`: one A2ADispatchArgs per rank, or the array from pack_dispatch_args."""
         arr = per_rank if isinstance(per_rank, ctypes.Array) else self.pack_dispatch_args(per_rank)
-        self.shared.group_dispatch(arr, quantize, stream)
+        self.shared.group_dispatch(arr, quantize, stream or 0)   # (None: the default stream)
 
     def combine(self, per_rank, expert_y_dtype: torch.dtype, accumulate: bool, stream: int) -> None:
         if expert_y_dtype not in SCALAR_TYPE:
             raise RuntimeError(f"unsupported expert_y dtype {expert_y_dtype}")
         arr = per_rank if isinstance(per_rank, ctypes.Array) else self.pack_combine_args(per_rank)
-        self.shared.group_combine(arr, SCALAR_TYPE[expert_y_dtype], accumulate, stream)
+        self.shared.group_combine(arr, SCALAR_TYPE[expert_y_dtype], accumulate, stream or 0)
 
     def pending(self, kind: str) -> List[int]:
         """Ranks whose operators have called collective `kind` ("dispatch" or "combine") and wait for the others."""

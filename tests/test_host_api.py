@@ -308,3 +308,22 @@ def test_operators_collect_a_collective_in_native_code():
     assert ops[1].combine(out, good[5], good[6], y, None, True, True, False) is None
     context.close()
     assert context.pending("combine") == 0
+
+
+@pytest.mark.parametrize("stream", [None, 0])
+def test_group_calls_take_no_stream_and_longer_arrays(stream):
+    """What the ctypes binding took: None as the default stream, an array with more entries than ranks.  A shorter
+    array and one of the other call's arguments are refused, before the (here closed) context is looked at."""
+    module = native.load_extension()
+    ctx = native.AllToAllContext.__new__(native.AllToAllContext)
+    ctx._handle, ctx.shared = None, module.Context(0, 3)
+    for call, args, other in [(lambda a: ctx.dispatch(a, True, stream), native.A2ADispatchArgs, native.A2ACombineArgs),
+                              (lambda a: ctx.combine(a, torch.bfloat16, False, stream), native.A2ACombineArgs,
+                               native.A2ADispatchArgs)]:
+        for n in (3, 5):
+            with pytest.raises(RuntimeError, match="destroyed"):
+                call((args * n)())
+        with pytest.raises(RuntimeError, match="of 3 ranks"):
+            call((args * 2)())
+        with pytest.raises(TypeError):
+            call((other * 3)())
