@@ -16,12 +16,12 @@ __device__ __forceinline__ void lds_barrier() {
 }
 
 // The 16-byte store of a dispatched copy, at device scope (`sc1`): the line is written through
-// instead of staying dirty in the L2 of the storing die.  The wait state behind the store is not optional: a
-// vector instruction that follows a store of more than 64 bits must not write the registers the store takes
-// its data from in the very next slot, and the compiler, which inserts that state behind stores it knows of,
-// cannot see this one (a loop that cleared the registers for its next piece sent zeros now and then).
+// instead of staying dirty in the L2 of the storing die.  The two wait states behind the store (`s_nop 1`) are not
+// optional: on gfx950 a vector instruction must not write the registers a store of more than 64 bits takes its data
+// from in the two slots that follow it (gfx90a: in the one), and the compiler, which inserts those states behind
+// stores it knows of, cannot see this one (a loop that cleared the registers for its next piece sent zeros now and then).
 __device__ __forceinline__ void store_copy(u32x4 v, u32x4 *p) {
-    asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 0" ::"v"(p), "v"(v) : "memory");
+    asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(p), "v"(v) : "memory");
 }
 
 // Cache policies of buffer loads and stores (the sc0, nt and sc1 bits of the instruction).

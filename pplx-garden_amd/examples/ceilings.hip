@@ -91,7 +91,7 @@ __global__ void copy_sweep(const u32x4 *__restrict__ in, u32x4 *__restrict__ out
 // for the quantised chunk (random in, random out; equal halves give zeros).
 // Stores at device scope, as the library's pack.
 __device__ __forceinline__ void store_sc1(u32x4 v, u32x4 *p) {
-    asm volatile("global_store_dwordx4 %0, %1, off sc1" ::"v"(p), "v"(v) : "memory");
+    asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(p), "v"(v) : "memory");   // (store_copy in a2a_device.h)
 }
 
 __global__ __launch_bounds__(448) void push(const uint8_t *__restrict__ x, uint8_t *__restrict__ out,
