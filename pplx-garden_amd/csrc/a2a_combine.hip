@@ -27,6 +27,7 @@
 // accumulates onto (6000 tokens of 8 KB rows, K = 6: 76.5 -> 67.4 us).
 #include "a2a_device.h"
 #include "a2a_internal.h"
+#include "a2a_rules.h"
 
 namespace a2a {
 
@@ -148,7 +149,6 @@ __device__ __forceinline__ void fma_chunk(const u32x4 raw, float w, float (&acc)
     }
 }
 
-constexpr uint32_t kTokensPerLayer = 32768;    // tokens in one layer of the grid
 constexpr uint32_t kOneRankMaxTokens = 2048;   // largest step that takes the ONE_RANK variant of the gather
 
 // How the gather writes where more than one rank has tokens or the step is large, non-temporal / into the Infinity
@@ -209,6 +209,7 @@ __global__ __launch_bounds__(kWave) void combine_gather_kernel(const CombArgs ar
         // 1.2 us and is left out there.)
         A2A_PIN(args.token_start[0]);
         A2A_PIN(args.token_start[1]);
+        A2A_PIN(args.layer_rows);
         A2A_PIN(args.hidden_dim);
         A2A_PIN(args.accumulate);
         A2A_PIN(args.staged_base);
@@ -226,7 +227,7 @@ __global__ __launch_bounds__(kWave) void combine_gather_kernel(const CombArgs ar
     const uint32_t K = ws.topk;
     const uint32_t num_chunks = args.hidden_dim / V;
     // the grid: slabs of a token side by side, then its tokens (no division stands in front of the loads)
-    const uint32_t token_global = blockIdx.z * kTokensPerLayer + blockIdx.y;
+    const uint32_t token_global = ONE_RANK ? blockIdx.y : blockIdx.z * args.layer_rows + blockIdx.y;
     const uint32_t slab = blockIdx.x;
     uint32_t g = 0, token = token_global;
     if constexpr (ONE_RANK) {
@@ -349,8 +350,9 @@ static hipError_t launch_typed(const CombArgs &given, const Workspace &ws, uint3
     if (args.single_rank != 0) args.single = given.dst[args.single_rank - 1];
     const uint32_t chunks = args.hidden_dim / V;
     const uint32_t slabs = (chunks + kWave - 1) / kWave;
-    const uint32_t layers = (total_tokens + kTokensPerLayer - 1) / kTokensPerLayer;
-    const dim3 grid(slabs, layers > 1 ? kTokensPerLayer : total_tokens, layers);
+    const TokenLayers layers = token_layers(total_tokens);
+    args.layer_rows = layers.rows;
+    const dim3 grid(slabs, layers.rows, layers.layers);
     const bool plain = args.single_rank != 0 || args.staged_base != nullptr;
     const bool past_cache = !plain && (uint64_t)total_tokens * args.hidden_dim * Elem<U>::kSize >= kStreamedOutput;
     const bool into_cache = !plain && !past_cache && copies >= kStreamCopies && ws.topk > 2;

@@ -150,7 +150,7 @@ struct CombArgs {
     // r + 1 when rank r alone has tokens to combine (0 otherwise), and a copy of dst[r] at a fixed place
     // (set by the launcher; see PushArgs::single).
     uint32_t single_rank;
-    uint32_t pad_;
+    uint32_t layer_rows;   // tokens of one layer of the grid (set by the launcher)
     CombDst single;
 };
 

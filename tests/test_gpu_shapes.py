@@ -57,7 +57,7 @@ def test_repeated_experts_inside_a_token(split):
 
 
 # The combine loads its rows in groups of 1, 2, 4 or 8 (the smallest that holds K, then groups of 8), 64 chunks of
-# 16 bytes per wavefront, with 32768 tokens to a layer of its grid.
+# 16 bytes per wavefront, with at most 32768 tokens to a layer of its grid.
 GATHERS = [
     Case("k1", 70, 640, 8, 2, 1, 7101),
     Case("k2", 70, 1152, 8, 2, 2, 7102),
@@ -67,6 +67,7 @@ GATHERS = [
     Case("k9", 70, 512, 16, 4, 9, 7106),
     Case("k16", 40, 640, 32, 4, 16, 7107),
     Case("second_layer", 16500, 128, 16, 2, 2, 7108),        # 33000 tokens of two ranks
+    Case("uneven_layers", 16385, 128, 16, 4, 2, 7109),       # 65540 tokens in three layers, one place empty
 ]
 
 
