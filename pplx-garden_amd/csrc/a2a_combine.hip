@@ -151,19 +151,16 @@ __device__ __forceinline__ void fma_chunk(const u32x4 raw, float w, float (&acc)
 
 constexpr uint32_t kOneRankMaxTokens = 2048;   // largest step that takes the ONE_RANK variant of the gather
 
-// How the gather writes where more than one rank has tokens or the step is large, non-temporal / into the Infinity
-// Cache (system scope: written through the caches of the die) / past it:
-//  - outputs of 15 MB behind copies that went past that cache 23.8 / 23.2 / 23.7 us, 29 MB 47.0 / 44.7 / 45.9, 59 MB 91.5 /
-//    86.9 / 89.7, 80 MB 126.0 / 120.4 / 122.1, 88 MB 138 / 140 / 133, 235 MB 371 / 393 / 360.  HBM turns around between
-//    reads and writes, and an output that the cache holds is written back when it suits.
-//  - behind copies that are in the cache themselves: 49 MB 68.0 / 76.0 / -, 27 MB 44.1 / 48.5 / -.
-//  - the ONE_RANK variant's outputs stay non-temporal (15 MB 23.4 / 24.8 / 24.0), and so do those of rows that were
-//    staged (29 MB a launch: 3 us less into the cache, which the copies of the sends that follow lose again).
-// With eight loads a lane, 16 wavefronts a compute unit (19 where outputs go into the cache) are enough to keep HBM busy, and more of
-// them only have more rows open at a time: 470 MB of output 740 -> 670-700 us, 59 MB 86.6 -> 84.5.  The launch asks
-// for LDS that nothing uses to bound them.  (Fewer loads a lane need all wavefronts: K = 2 70.5 -> 80.7 us with 19.)
-constexpr uint64_t kStreamedOutput = 80u << 20;
-constexpr size_t kLds16Waves = 10000, kLds19Waves = 8200;   // of 160 KB
+// How the gather writes: non-temporally, but past the Infinity Cache where the step's copies went past it
+// (copies_past_cache in a2a_rules.h has the figures) or the tokens themselves are kStreamedOutput bytes or more (behind
+// copies that went past it, non-temporal / past: 80 MB 126.0 / 122.1 us, 88 MB 138 / 133, 235 MB 371 / 360).  The ONE_RANK
+// variant's outputs stay non-temporal (15 MB 23.4 us, past 24.0), and so do those of rows that were staged (they are
+// written between the launches of the other ranks' calls).
+// With eight loads a lane, 16 wavefronts a compute unit are enough to keep HBM busy behind such stores, and more of
+// them only have more rows open at a time: 470 MB of output 740 -> 670-700 us.  The launch asks for LDS that nothing
+// uses to bound them.  (Fewer loads a lane need all wavefronts: K = 2 70.5 -> 80.7 us with 18.)
+constexpr uint64_t kStreamedOutput = 84000000;
+constexpr size_t kLds16Waves = 160 * 1024 / 16;   // of a compute unit's 160 KB, which are given out in blocks of 1280 bytes
 
 // T: type of the expert_y rows, U: type of out_tokens.  One WAVEFRONT handles
 // one slab of 64 sixteen-byte chunks of one token; wavefronts share nothing, so
@@ -336,7 +333,7 @@ __global__ __launch_bounds__(kWave) void combine_gather_kernel(const CombArgs ar
 
 template <typename T, typename U>
 static hipError_t launch_typed(const CombArgs &given, const Workspace &ws, uint32_t total_tokens,
-                               uint64_t copies, hipStream_t stream, KernelTiming timing) {
+                               bool streamed, hipStream_t stream, KernelTiming timing) {
     constexpr int V = vec_elems<T>();
     CombArgs args = given;
     uint32_t ranks_with_tokens = 0;
@@ -346,7 +343,7 @@ static hipError_t launch_typed(const CombArgs &given, const Workspace &ws, uint3
         ++ranks_with_tokens;
         args.single_rank = r + 1;
     }
-    if (ranks_with_tokens != 1 || total_tokens > kOneRankMaxTokens) args.single_rank = 0;
+    if (ranks_with_tokens != 1 || total_tokens > kOneRankMaxTokens || streamed) args.single_rank = 0;
     if (args.single_rank != 0) args.single = given.dst[args.single_rank - 1];
     const uint32_t chunks = args.hidden_dim / V;
     const uint32_t slabs = (chunks + kWave - 1) / kWave;
@@ -354,8 +351,8 @@ static hipError_t launch_typed(const CombArgs &given, const Workspace &ws, uint3
     args.layer_rows = layers.rows;
     const dim3 grid(slabs, layers.rows, layers.layers);
     const bool plain = args.single_rank != 0 || args.staged_base != nullptr;
-    const bool past_cache = !plain && (uint64_t)total_tokens * args.hidden_dim * Elem<U>::kSize >= kStreamedOutput;
-    const bool into_cache = !plain && !past_cache && copies >= kStreamCopies && ws.topk > 2;
+    const bool past_cache =
+        !plain && (streamed || (uint64_t)total_tokens * args.hidden_dim * Elem<U>::kSize >= kStreamedOutput);
 #define A2A_LAUNCH_GATHER(GROUP, ONE, OUT, LDS)                                                                \
     hipExtLaunchKernelGGL((combine_gather_kernel<T, U, GROUP, ONE, OUT>), grid, dim3(kWave), LDS, stream,      \
                           timing.start, timing.stop, 0, args, ws)
@@ -363,7 +360,6 @@ static hipError_t launch_typed(const CombArgs &given, const Workspace &ws, uint3
     do {                                                                                                       \
         if (args.single_rank != 0) A2A_LAUNCH_GATHER(GROUP, true, kNonTemporal, 0);                            \
         else if (past_cache) A2A_LAUNCH_GATHER(GROUP, false, kSystemNonTemporal, GROUP == 8 ? kLds16Waves : 0); \
-        else if (into_cache) A2A_LAUNCH_GATHER(GROUP, false, kSystemScope, GROUP == 8 ? kLds19Waves : 0);      \
         else A2A_LAUNCH_GATHER(GROUP, false, kNonTemporal, 0);                                                 \
     } while (0)
     if (ws.topk > 4) A2A_LAUNCH_GATHER_RANKS(8);
@@ -376,12 +372,12 @@ static hipError_t launch_typed(const CombArgs &given, const Workspace &ws, uint3
 }
 
 hipError_t launch_combine_gather(const CombArgs &args, const Workspace &ws, uint32_t in_dtype,
-                                 uint32_t out_dtype, uint32_t total_tokens, uint64_t copies, hipStream_t stream,
+                                 uint32_t out_dtype, uint32_t total_tokens, bool streamed, hipStream_t stream,
                                  KernelTiming timing) {
     if (total_tokens == 0) return hipSuccess;
 #define A2A_COMBINE_CASE(IN_TAG, IN_T, OUT_TAG, OUT_T) \
     if (in_dtype == IN_TAG && out_dtype == OUT_TAG)    \
-        return launch_typed<IN_T, OUT_T>(args, ws, total_tokens, copies, stream, timing);
+        return launch_typed<IN_T, OUT_T>(args, ws, total_tokens, streamed, stream, timing);
     A2A_COMBINE_CASE(A2A_BF16, Bf16, A2A_BF16, Bf16)
     A2A_COMBINE_CASE(A2A_BF16, Bf16, A2A_F32, F32)
     A2A_COMBINE_CASE(A2A_BF16, Bf16, A2A_F16, F16)

@@ -19,6 +19,7 @@
 #include <vector>
 
 #include "a2a_internal.h"
+#include "a2a_rules.h"
 #include "a2a_staged.h"
 
 using namespace a2a;
@@ -44,6 +45,7 @@ struct a2a_ctx {
     bool group_routing = false;    // the last dispatch was a group call (route_slot is valid)
     uint32_t num_tokens[kMaxWorld] = {};  // tokens of each rank in the last dispatch
     uint32_t quantized = 0;        // mode of the last dispatch
+    bool copies_streamed = false;  // the last group dispatch wrote its copies past the Infinity Cache
 
     Staging staging;               // buffers and tables of the split calls
 
@@ -478,8 +480,12 @@ int plan_dispatch_group(a2a_ctx *ctx, const a2a_config &c, const a2a_dispatch_ar
 }
 
 // Second half: the launches of an accepted plan on the tables of `ws`.
+// `streamed`: whether the pack wrote its copies past the Infinity Cache.  The one-launch packs of small steps never do (at
+// most 8192 entries: the line is rows of 39 KB away), nor does the push behind separate routing launches.
 int launch_dispatch_group(a2a_ctx *ctx, const a2a_config &c, const Workspace &ws, const GroupPlan &plan,
-                          uint32_t quantize, hipStream_t s, KernelTiming pack_timing, KernelTiming route_timing) {
+                          uint32_t quantize, hipStream_t s, KernelTiming pack_timing, KernelTiming route_timing,
+                          bool &streamed) {
+    streamed = false;
     const RouteArgs &ra = plan.ra;
     const FinalizeArgs &fa = plan.fa;
     const PushArgs &pa = plan.pa;
@@ -509,7 +515,9 @@ int launch_dispatch_group(a2a_ctx *ctx, const a2a_config &c, const Workspace &ws
         // workgroups resolve their own rows from them.
         e = launch_route_accumulate(ra, ws, blocks, s, false, route_timing);
         if (e != hipSuccess) return hip_fail(ctx, e, "launch route_hist (accumulating)");
-        e = launch_dispatch_resolve(pa, fa, ws, quantize != 0, tokens, s, pack_timing);
+        streamed = copies_past_cache((uint64_t)tokens * c.num_experts_per_token * row_bytes_of(c), quantize != 0,
+                                     c.num_experts_per_token);
+        e = launch_dispatch_resolve(pa, fa, ws, quantize != 0, tokens, streamed, s, pack_timing);
         if (e != hipSuccess) return hip_fail(ctx, e, "launch dispatch_resolve");
     }
     return A2A_OK;
@@ -709,7 +717,7 @@ int a2a_dispatch(a2a_ctx *ctx, const a2a_dispatch_args *args, uint32_t quantize,
     GroupPlan plan;
     if (int rc = plan_dispatch_group(ctx, ctx->cfg, args, quantize, plan)) return rc;
     if (int rc = launch_dispatch_group(ctx, ctx->cfg, ctx->ws, plan, quantize, static_cast<hipStream_t>(stream),
-                                       pack_timing, route_timing))
+                                       pack_timing, route_timing, ctx->copies_streamed))
         return rc;
     // only an accepted step replaces what the context knows of the previous one
     memcpy(ctx->num_tokens, plan.num_tokens, sizeof ctx->num_tokens);
@@ -763,7 +771,8 @@ int a2a_dispatch_static(const a2a_config *config, const a2a_dispatch_args *args,
     hipLaunchKernelGGL(static_prepare_kernel, dim3(blocks), dim3(1024), 0, s, ws, device_flags == nullptr ? 1u : 0u);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return hip_fail(nullptr, e, "launch static_prepare");
-    return launch_dispatch_group(nullptr, c, ws, plan, quantize, s, KernelTiming(), KernelTiming());
+    bool streamed;   // (there is no combine that follows)
+    return launch_dispatch_group(nullptr, c, ws, plan, quantize, s, KernelTiming(), KernelTiming(), streamed);
 }
 
 int a2a_combine(a2a_ctx *ctx, const a2a_combine_args *args, uint32_t expert_y_dtype,
@@ -824,9 +833,7 @@ int a2a_combine(a2a_ctx *ctx, const a2a_combine_args *args, uint32_t expert_y_dt
     DeviceGuard guard(c.device);
     const KernelTiming gather_timing = ctx->timing[A2A_KERNEL_GATHER];
     ctx->timing[A2A_KERNEL_GATHER] = KernelTiming();
-    // (the ranks of a dp group combine the same tokens)
-    const uint64_t copies = (uint64_t)tokens / ctx->ws.dp_size * c.num_experts_per_token * row_bytes_of(c);
-    hipError_t e = launch_combine_gather(ca, ctx->ws, expert_y_dtype, c.out_dtype, tokens, copies,
+    hipError_t e = launch_combine_gather(ca, ctx->ws, expert_y_dtype, c.out_dtype, tokens, ctx->copies_streamed,
                                          static_cast<hipStream_t>(stream), gather_timing);
     if (e != hipSuccess) return hip_fail(ctx, e, "launch combine_gather");
     return A2A_OK;

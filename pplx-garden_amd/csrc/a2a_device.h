@@ -29,7 +29,6 @@ constexpr int kOrdinary = 0;
 constexpr int kNonTemporal = 2;
 constexpr int kDeviceScope = 16;
 constexpr int kDeviceNonTemporal = 16 | 2;
-constexpr int kSystemScope = 16 | 1;
 constexpr int kSystemNonTemporal = 16 | 2 | 1;
 
 // A row as a buffer descriptor: `row` is the same in all lanes, and the descriptor's bound takes the place of every

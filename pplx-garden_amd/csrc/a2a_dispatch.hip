@@ -16,7 +16,7 @@
 // computed once per token by the first K lanes and read back as wave-uniform
 // scalars.  Token rows are loaded non-temporally (each is read once).  How the
 // copies are written depends on how much of the Infinity Cache they fill (see
-// kStreamCopies).
+// copies_past_cache in a2a_rules.h).
 #include "a2a_device.h"
 #include "a2a_scan.h"
 
@@ -1929,12 +1929,10 @@ hipError_t launch_dispatch_single(const PushArgs &args, const FinalizeArgs &fin,
     return hipGetLastError();
 }
 
-// How the copies are written: past the cache from kStreamCopies on.  Smaller steps write quantised rows at device scope,
-// others with ordinary stores (device scope: 1 us less of 24 for 8 KB rows, but 3-5 us more of 33 for rows of 5120
-// bytes).  Rows that are not quantised and have at most two copies take ordinary stores at every size (rows of 2 KB,
-// K = 1: 44.0 us against 46.6 past the cache; 8 KB, K = 2: 91.0 against 94.5).
-hipError_t launch_dispatch_resolve(const PushArgs &args, const FinalizeArgs &fin, const Workspace &ws,
-                                   bool quantize, uint32_t total_tokens, hipStream_t stream, KernelTiming timing) {
+// How the copies are written: past the Infinity Cache (`streamed`), otherwise quantised rows at device scope and others
+// with ordinary stores (device scope: 1 us less of 24 for 8 KB rows, but 3-5 us more of 33 for rows of 5120 bytes).
+hipError_t launch_dispatch_resolve(const PushArgs &args, const FinalizeArgs &fin, const Workspace &ws, bool quantize,
+                                   uint32_t total_tokens, bool streamed, hipStream_t stream, KernelTiming timing) {
     uint32_t threads = push_threads(args, quantize);
     if (threads < ws.experts_per_rank) {   // a receiver workgroup has one thread per local expert
         threads = (ws.experts_per_rank + kWave - 1) / kWave * kWave;
@@ -1950,15 +1948,13 @@ hipError_t launch_dispatch_resolve(const PushArgs &args, const FinalizeArgs &fin
     }
     if (senders != 1) a.single_source = 0;    // here only "one source has tokens": the rows may be strided
     if (a.single_source != 0) a.single = args.src[a.single_source - 1];
-    const uint64_t copies = (uint64_t)total_tokens * ws.topk * (quantize ? args.hidden_dim : args.row_bytes);
-    const bool stream_copies = copies >= kStreamCopies && (quantize || ws.topk > 2);
 #define A2A_LAUNCH_RESOLVE(Q, P)                                                                                   \
     hipExtLaunchKernelGGL((dispatch_resolve_kernel<Q, P>), dim3(blocks), dim3(threads), 0, stream, timing.start,  \
                           timing.stop, 0, a, fin, ws)
     if (quantize) {
-        if (stream_copies) A2A_LAUNCH_RESOLVE(true, kDeviceNonTemporal); else A2A_LAUNCH_RESOLVE(true, kDeviceScope);
+        if (streamed) A2A_LAUNCH_RESOLVE(true, kDeviceNonTemporal); else A2A_LAUNCH_RESOLVE(true, kDeviceScope);
     } else {
-        if (stream_copies) A2A_LAUNCH_RESOLVE(false, kDeviceNonTemporal); else A2A_LAUNCH_RESOLVE(false, kOrdinary);
+        if (streamed) A2A_LAUNCH_RESOLVE(false, kDeviceNonTemporal); else A2A_LAUNCH_RESOLVE(false, kOrdinary);
     }
 #undef A2A_LAUNCH_RESOLVE
     return hipGetLastError();

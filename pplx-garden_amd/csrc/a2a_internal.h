@@ -172,8 +172,9 @@ hipError_t launch_route_accumulate(const RouteArgs &args, const Workspace &ws, u
                                    KernelTiming timing = KernelTiming());
 // Pack that resolves its rows from the chunk histograms and the step's totals, with the
 // receiver layout and the per-source tables computed by extra workgroups of the same launch.
+// `streamed`: the copies are written past the Infinity Cache (copies_past_cache).
 hipError_t launch_dispatch_resolve(const PushArgs &args, const FinalizeArgs &fin, const Workspace &ws,
-                                   bool quantize, uint32_t total_tokens, hipStream_t stream,
+                                   bool quantize, uint32_t total_tokens, bool streamed, hipStream_t stream,
                                    KernelTiming timing = KernelTiming());
 hipError_t launch_finalize(const FinalizeArgs &args, const Workspace &ws, hipStream_t stream);
 hipError_t launch_route_fused(const RouteArgs &args, const FinalizeArgs &fin, const Workspace &ws,
@@ -194,19 +195,9 @@ bool dispatch_single_fits(const PushArgs &args, const Workspace &ws, bool quanti
 hipError_t launch_dispatch_single(const PushArgs &args, const FinalizeArgs &fin, const Workspace &ws,
                                   bool quantize, uint32_t total_tokens, hipStream_t stream,
                                   KernelTiming timing = KernelTiming());
-// Cache policy of a large step's copies and of its combined tokens, measured on steps whose buffers were not those of
-// the step before (a step that writes the same 235 MB again finds them in the 256 MB Infinity Cache and shows another
-// order).  From this many bytes of copies on the pack sends them past that cache (device scope and non-temporal) and
-// the combine writes its tokens into it.  One goes with the other: tokens written over copies that are still to
-// be written back cost both.  Pack + gather, as smaller steps write / as larger ones, us:
-//   quantised rows of 7168 bytes: 88 MB of copies 58.2 / 59.2, 117 MB 78.1 / 78.0, 176 MB 118.5 / 112.6, 235 MB 157 / 148;
-//   rows of 5120 bytes: 84 MB 57.2 / 56.8, 109 MB 77.4 / 74.9 (one of them alone: 84.2), 168 MB 114.3 / 104.4;
-//   rows of 8 KB: 100 MB 45.5 / 47.2, 134 MB 64.3 / 60.8, 295 MB 141.6 / 130.0.
-constexpr uint64_t kStreamCopies = 104u << 20;
-
-// `copies`: bytes of the rows that the step dispatched (0: not known).
+// `streamed`: the step's copies went past the Infinity Cache (copies_past_cache).
 hipError_t launch_combine_gather(const CombArgs &args, const Workspace &ws, uint32_t in_dtype,
-                                 uint32_t out_dtype, uint32_t total_tokens, uint64_t copies, hipStream_t stream,
+                                 uint32_t out_dtype, uint32_t total_tokens, bool streamed, hipStream_t stream,
                                  KernelTiming timing = KernelTiming());
 
 // Makes a value from the argument block count as used where this stands, so that the scalar loads of

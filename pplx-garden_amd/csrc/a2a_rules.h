@@ -23,4 +23,35 @@ inline TokenLayers token_layers(uint32_t tokens) {
     return t;
 }
 
+// Cache policy of a large step's copies and of its combined tokens.  From kStreamCopies bytes of copies on the pack
+// sends them past the 256 MB Infinity Cache (device scope and non-temporal) and the combine sends its tokens past it
+// too: such a step cannot stay there until it is read, and lines that are not left dirty need not be written back
+// while the next kernels read.  Below the line copies stay where the experts, which read them next, find them.
+// Whole steps, us, copies kept / past the cache, with nothing between dispatch and combine (no user's step; their
+// difference is the writing back that the combine no longer waits for), with a sweep that reads the received rows, and
+// with one that reads them and writes expert_y (buffers not those of the step before):
+//   quantised rows of 7168 bytes, K = 8
+//      117 MB   79.3 /  82.7    136.3 / 139.8     507.2 /  525.3
+//      235 MB  162.1 / 153.8    245.2 / 248.5     954.7 /  958.5
+//      355 MB  240.0 / 228.2    365.1 / 359.6    1392.1 / 1385.7
+//     1879 MB 1251.2 / 1185.0  2377.8 / 2330.1   11770.7 / 11731.8
+//   fp8 rows of 5120 bytes, K = 8
+//      109 MB   81.5 /  78.2    130.3 / 133.1     455.7 /  476.4
+//      307 MB  215.1 / 203.1    329.8 / 324.2    1197.5 / 1188.5
+//      983 MB  648.3 / 595.5    951.3 / 916.9    3409.3 / 3379.9
+//   bf16 rows of 8 KB, K = 6 (the ones that gain least)
+//      201 MB   96.2 /  91.2    158.6 / 166.5     193.3 /  186.0
+//      295 MB  139.1 / 132.3    231.0 / 235.2     276.5 /  270.2
+//      344 MB  158.6 / 150.2    267.4 / 267.3     315.8 /  307.3
+//      786 MB  352.8 / 338.0    585.2 / 593.0     707.9 /  693.7
+//     1573 MB  690.0 / 649.9   1136.0 / 1113.1   1439.6 / 1424.5
+// One goes with the other (copies kept, tokens into the cache instead: up to 11 us more), so the pack decides and the
+// combine follows what the pack did.  Rows that are not quantised and have at most two copies are kept at every size
+// (rows of 2 KB, K = 1: 44.0 us against 46.6 past the cache; 8 KB, K = 2: 91.0 against 94.5).
+constexpr uint64_t kStreamCopies = 320000000;
+
+inline bool copies_past_cache(uint64_t copies, bool quantize, uint32_t topk) {
+    return copies >= kStreamCopies && (quantize || topk > 2);
+}
+
 }  // namespace a2a

@@ -1985,7 +1985,7 @@ hipError_t launch_combine_recv(const CombineRecvArgs &args, const Workspace &ws,
     ca.accumulate = args.accumulate;
     ca.staged_base = st.comb_buf;
     ca.staged_stride = st.comb_stride;
-    return launch_combine_gather(ca, ws, in_dtype, out_dtype, args.dst.num_tokens, 0, stream, timing);
+    return launch_combine_gather(ca, ws, in_dtype, out_dtype, args.dst.num_tokens, false, stream, timing);
 }
 
 }  // namespace a2a

@@ -80,26 +80,33 @@ def test_gather_groups(case):
     assert_combine_close(case, got, want)
 
 
-# Steps whose copies go past the Infinity Cache (from 104 MB on) and whose combined tokens go into it or, from 80 MB on,
-# past it, at row lengths that end inside a wavefront's slab: the group calls against the split calls, which move
-# every row by other kernels.  (row type, hidden, scales, experts per token, tokens of the two ranks with tokens)
+# Steps whose copies go past the Infinity Cache (from 320 MB on; not two copies or fewer of rows that are not quantised),
+# and whose combined tokens go past it with them or, from 84 MB on, by themselves, at row lengths that end inside a
+# wavefront's slab: the group calls against the split calls, which move every row by other kernels.
+# (row type, hidden, scales, experts per token, tokens of the first and third of three ranks, copies go past the cache)
 STREAMED = [
-    (torch.bfloat16, 1000, 0, 5, (10000, 1100)),        # 111 MB of copies, 22 MB of tokens
-    (torch.float16, 1000, 0, 3, (40000, 3001)),         # 258 MB, 86 MB
-    (torch.float32, 1004, 0, 8, (4000, 301)),           # 138 MB, 17 MB
-    (torch.float8_e4m3fn, 1152, 9, 8, (11000, 1000)),   # 111 MB, 28 MB
-    (torch.bfloat16, 1000, 0, 2, (41000, 2100)),        # 172 MB of copies that stay ordinary, 86 MB
-    (torch.bfloat16, 1000, 0, 9, (5800, 7)),            # 105 MB: two groups of rows a token
+    (torch.bfloat16, 1000, 0, 5, (30000, 2200), True),        # 322 MB of copies, 64 MB of tokens
+    (torch.float16, 1000, 0, 3, (52000, 3001), True),         # 330 MB, 110 MB
+    (torch.float32, 1004, 0, 8, (9700, 301), True),           # 321 MB, 40 MB
+    (torch.float8_e4m3fn, 1152, 9, 8, (33000, 1900), True),   # 322 MB, 80 MB
+    (torch.bfloat16, 1000, 0, 9, (17000, 1000), True),        # 324 MB, 36 MB: two groups of rows a token
+    (torch.float32, 1004, 0, 40, (2000, 0), True),            # 321 MB, 8 MB: one sender, few enough tokens for its own gather
+    (torch.bfloat16, 1000, 0, 2, (80000, 2100), False),       # 328 MB of copies that stay ordinary, 164 MB
+    (torch.bfloat16, 1000, 0, 5, (29000, 2000), False),       # 310 MB, 62 MB
 ]
 
 
-@pytest.mark.parametrize("row,hidden,scales,k,tokens", STREAMED,
+def copies_of(row, hidden, k, tokens):
+    return sum(tokens) * k * hidden * row.itemsize
+
+
+@pytest.mark.parametrize("row,hidden,scales,k,tokens,streamed", STREAMED,
                          ids=lambda v: str(v).replace("torch.", "") if isinstance(v, torch.dtype) else None)
-def test_streamed_copies_and_tokens(row, hidden, scales, k, tokens):
+def test_streamed_copies_and_tokens(row, hidden, scales, k, tokens, streamed):
     from pplx_garden_amd.distributed.loopback import LoopbackWorld
     from pplx_garden_amd.kernels.p2p_all_to_all import P2PAllToAll
 
-    device, N, E = torch.device("cuda:0"), 3, 24
+    device, N, E = torch.device("cuda:0"), 3, max(24, k + 2)
     out = torch.bfloat16 if scales else row
     world = LoopbackWorld(N, device=device)
     counts = (tokens[0], 0, tokens[1])

@@ -7,6 +7,8 @@ from pathlib import Path
 
 import pytest
 
+from test_gpu_shapes import STREAMED, copies_of
+
 CSRC = Path(__file__).resolve().parent.parent / "pplx-garden_amd" / "csrc"
 
 SOURCE = """
@@ -14,6 +16,7 @@ SOURCE = """
 extern "C" {
 uint32_t layers(uint32_t tokens) { return a2a::token_layers(tokens).layers; }
 uint32_t layer_rows(uint32_t tokens) { return a2a::token_layers(tokens).rows; }
+int past_cache(uint64_t copies, int quantize, uint32_t k) { return a2a::copies_past_cache(copies, quantize != 0, k); }
 }
 """
 
@@ -27,7 +30,9 @@ def rules(tmp_path_factory):
     (folder / "rules.cpp").write_text(SOURCE)
     subprocess.run([compiler, "-std=c++17", "-Wall", "-Wextra", "-Werror", "-shared", "-fPIC", "-I", str(CSRC),
                     str(folder / "rules.cpp"), "-o", str(folder / "rules.so")], check=True)
-    return ctypes.CDLL(str(folder / "rules.so"))
+    lib = ctypes.CDLL(str(folder / "rules.so"))
+    lib.past_cache.argtypes = [ctypes.c_uint64, ctypes.c_int, ctypes.c_uint32]
+    return lib
 
 
 @pytest.mark.parametrize("tokens", [1, 7, 32767, 32768, 32769, 33000, 65536, 65537, 100001, 1048577, 2147483647])
@@ -36,3 +41,17 @@ def test_the_gathers_grid_has_every_token_and_next_to_no_empty_rows(rules, token
     assert layers * rows >= tokens and rows <= 32768 and layers <= 65536
     assert layers * rows - tokens < layers
     assert layers == -(-tokens // 32768)
+
+
+def test_copies_that_the_infinity_cache_can_hold_stay_there_for_their_reader(rules):
+    """The experts read the copies next: only what the 256 MB cache cannot hold until then goes past it."""
+    for tokens in (1900, 2048, 3072, 4096):      # 109 to 235 MB of quantised rows of 7168 bytes
+        assert not rules.past_cache(tokens * 8 * 7168, 1, 8)
+    assert not rules.past_cache(256 << 20, 1, 8) and not rules.past_cache(256 << 20, 0, 6)
+    assert rules.past_cache(8 * 4096 * 8 * 7168, 1, 8)       # eight ranks of 4096 tokens
+    assert rules.past_cache(1 << 30, 0, 3) and rules.past_cache(1 << 30, 1, 1) and not rules.past_cache(1 << 30, 0, 2)
+
+
+@pytest.mark.parametrize("row,hidden,scales,k,tokens,streamed", STREAMED)
+def test_the_gpu_tests_of_streamed_steps_lie_on_the_side_they_are_meant_for(rules, row, hidden, scales, k, tokens, streamed):
+    assert bool(rules.past_cache(copies_of(row, hidden, k, tokens), 0, k)) == streamed
