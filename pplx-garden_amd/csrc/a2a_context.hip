@@ -302,13 +302,13 @@ uint32_t rows_upper_bound(const a2a_ctx *ctx) {
     return (uint32_t)(rows < cap ? rows : cap);
 }
 
-// Bytes the sends of this step staged.
-uint64_t staged_bytes(const a2a_ctx *ctx) {
+// Bytes of the rows that all recvs of this step receive together.
+uint64_t copies_of_step(const a2a_ctx *ctx) {
     uint64_t tokens = 0;
     for (uint32_t g = 0; g < ctx->cfg.world_size; ++g) {
         if (ctx->sent_mask >> g & 1) tokens += ctx->num_tokens[g];
     }
-    return tokens * ctx->staging.disp_stride;
+    return tokens * ctx->cfg.num_experts_per_token * row_bytes_of(ctx->cfg);
 }
 
 // The one-launch routing pass recounts earlier chunks in every chunk workgroup
@@ -1066,7 +1066,7 @@ int a2a_dispatch_recv(a2a_ctx *ctx, uint32_t rank, int32_t *out_num_tokens, void
     rv.row_bytes = (uint32_t)row_bytes_of(c);
     rv.hidden_dim_scale = c.hidden_dim_scale;
     rv.max_rows = rows_upper_bound(ctx);
-    rv.staged_bytes = staged_bytes(ctx);
+    rv.streamed = received_past_cache(copies_of_step(ctx));
     // The first recv of a step lays out every receiver: once per step, as the reference's host
     // worker does (a2a_worker.rs:526-703), not once per recv launch.
     rv.valid_mask = ctx->sent_mask & ~ctx->empty_mask;

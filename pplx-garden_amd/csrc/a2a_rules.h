@@ -54,4 +54,23 @@ inline bool copies_past_cache(uint64_t copies, bool quantize, uint32_t topk) {
     return copies >= kStreamCopies && (quantize || topk > 2);
 }
 
+// The same for the recvs of the split calls, from kStreamReceived bytes of copies in all of a step's recvs on.  What this
+// keeps in the cache are the STAGED rows, which the recvs of all the ranks a token was routed to read, and the copies of the
+// first recvs are gone anyway by the time the last one has run.  Whole steps, us, copies kept / past the cache, with a
+// sweep that reads the received rows, and with one that reads them and writes expert_y:
+//   fp8 rows of 7168 bytes, K = 8: 184 MB (2 ranks)  320.4 / 332.0   813.3 / 823.1
+//                                  206 MB (1 sender) 416.1 / 411.1  1058.3 / 1052.8
+//                                  229 MB (8 ranks)  503.2 / 494.7  1210.9 / 1196.3
+//                                  940 MB           1804.7 / 1740.6 4332.2 / 4261.9
+//                           K = 4: 161 MB            386.4 / 394.1   858.0 / 863.0
+//                                  206 MB            480.5 / 476.4  1072.1 / 1060.0
+//                           K = 2:  80 MB            267.7 / 265.4   477.3 / 500.2
+//                                  161 MB            432.1 / 431.5   887.5 / 880.6
+//                                  229 MB            571.9 / 554.9  1201.4 / 1179.0
+//   bf16 rows of 14 KB,     K = 4: 184 MB            328.8 / 328.1   353.4 / 348.5
+//                           K = 8: 229 MB            391.1 / 380.1   417.6 / 409.5
+constexpr uint64_t kStreamReceived = 200000000;
+
+inline bool received_past_cache(uint64_t copies) { return copies >= kStreamReceived; }
+
 }  // namespace a2a

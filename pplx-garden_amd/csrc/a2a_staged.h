@@ -69,7 +69,7 @@ struct StageRecvArgs {
     uint32_t row_bytes;
     uint32_t hidden_dim_scale;
     uint32_t max_rows;        // upper bound of received rows known to the host
-    uint64_t staged_bytes;    // what the step's sends staged
+    bool streamed;            // the copies are written past the Infinity Cache (received_past_cache)
     PieceGrid grid;           // set by the launcher
     // the first recv of a step only: it lays out every receiver
     uint32_t valid_mask;      // sources that sent tokens in this step (the others count as empty)

@@ -1461,11 +1461,10 @@ struct PieceWalk {
 //    reads and writes each advance as ONE front through memory.  A wavefront per row with eight chunks a
 //    lane in flight kept 4096 rows half open at a time: rows of 7392 bytes, 16384 a launch (8 ranks x 2048
 //    tokens), 52.1 us = 4.65 TB/s of reads and writes then, 42.1 us in this order;
-//  - staged rows are loaded with ordinary loads, which keep them in that cache, and from 32 MB of staged rows
-//    on (STREAM) the copies are stored non-temporally, which keeps THEM out of it: 37.0 us = 6.5 TB/s (rows of
-//    14 KB, 235 MB staged: 84.3 -> 69.3 us; 470 MB staged, more than the cache holds: 172 -> 143 us with
-//    non-temporal loads as the other side).  Below that everything fits and the copies are
-//    worth keeping for whoever reads them next (8 x 512 tokens: 10.6 us either way).
+//  - staged rows are loaded with ordinary loads, which keep them in that cache, and where the copies of a step
+//    are more than it can keep for their reader (STREAM: received_past_cache in a2a_rules.h) they are stored
+//    non-temporally, which keeps THEM out of it: 37.0 us = 6.5 TB/s (rows of 14 KB, 235 MB staged: 84.3 -> 69.3 us;
+//    470 MB staged, more than the cache holds: 172 -> 143 us with non-temporal loads as the other side).
 // A row's scales travel with its first pieces; they are 3 us of the 42 (rows of scales are not whole cache
 // lines: their ends are written by two wavefronts at different times).
 template <bool STREAM>
@@ -1633,7 +1632,6 @@ uint32_t block_for_chunks(uint32_t chunks) {
 //     4096 rows 21.0 / 20.4 / 21.0 / 24.0.
 constexpr uint32_t kPieceWorkgroups = 2048;
 constexpr uint32_t kPiecesInOrder = 3;
-constexpr uint64_t kStreamBytes = 32u << 20;   // staged bytes of a step from which its recvs store past the cache
 
 uint32_t piece_grid(uint32_t max_rows, uint32_t world, uint32_t chunks, bool in_order, PieceGrid &grid) {
     constexpr uint32_t waves = kPieceThreads / kWave;
@@ -1952,7 +1950,7 @@ hipError_t launch_stage_recv(const StageRecvArgs &args, const Workspace &ws, con
         if (e != hipSuccess) return e;
     }
     const uint32_t blocks = piece_grid(args.max_rows, ws.world, chunks, false, a.grid);
-    if (args.staged_bytes >= kStreamBytes) {
+    if (args.streamed) {
         hipExtLaunchKernelGGL(stage_recv_kernel<true>, dim3(blocks), dim3(kPieceThreads), 0, stream, timing.start,
                               timing.stop, 0, a, ws, st);
     } else {

@@ -48,9 +48,9 @@ PIECES = [
     # a receiver typically gets max_num_tokens * K rows here: one launch up to 256, layout and copy apart from there on
     RefConfig("256-rows", 2, 1, 64, 16, 1024, 8, 4, FP8, BF16, F32),
     RefConfig("257-rows", 2, 1, 257, 16, 1024, None, 1, BF16, BF16, None),
-    # 7168 + 112 + 16 bytes at a stride of 7424: 32 MB staged are 4520 tokens; a step on either side
-    RefConfig("kept-in-cache", 2, 1, 2200, 8, 7168, 28, 2, FP8, BF16, F32),
-    RefConfig("past-the-cache", 2, 1, 2300, 8, 7168, 28, 2, FP8, BF16, F32),
+    # copies of 200 MB are 6975 tokens with four copies of 7168 bytes; a step on either side
+    RefConfig("kept-in-cache", 2, 1, 3450, 8, 7168, 28, 4, FP8, BF16, F32),
+    RefConfig("past-the-cache", 2, 1, 3550, 8, 7168, 28, 4, FP8, BF16, F32),
 ]
 
 

@@ -8,6 +8,7 @@ from pathlib import Path
 import pytest
 
 from test_gpu_shapes import STREAMED, copies_of
+from test_gpu_split import PIECES
 
 CSRC = Path(__file__).resolve().parent.parent / "pplx-garden_amd" / "csrc"
 
@@ -17,6 +18,7 @@ extern "C" {
 uint32_t layers(uint32_t tokens) { return a2a::token_layers(tokens).layers; }
 uint32_t layer_rows(uint32_t tokens) { return a2a::token_layers(tokens).rows; }
 int past_cache(uint64_t copies, int quantize, uint32_t k) { return a2a::copies_past_cache(copies, quantize != 0, k); }
+int received_past_cache(uint64_t copies) { return a2a::received_past_cache(copies); }
 }
 """
 
@@ -32,6 +34,7 @@ def rules(tmp_path_factory):
                     str(folder / "rules.cpp"), "-o", str(folder / "rules.so")], check=True)
     lib = ctypes.CDLL(str(folder / "rules.so"))
     lib.past_cache.argtypes = [ctypes.c_uint64, ctypes.c_int, ctypes.c_uint32]
+    lib.received_past_cache.argtypes = [ctypes.c_uint64]
     return lib
 
 
@@ -55,3 +58,12 @@ def test_copies_that_the_infinity_cache_can_hold_stay_there_for_their_reader(rul
 @pytest.mark.parametrize("row,hidden,scales,k,tokens,streamed", STREAMED)
 def test_the_gpu_tests_of_streamed_steps_lie_on_the_side_they_are_meant_for(rules, row, hidden, scales, k, tokens, streamed):
     assert bool(rules.past_cache(copies_of(row, hidden, k, tokens), 0, k)) == streamed
+
+
+def test_received_rows_that_the_cache_can_keep_stay_there(rules):
+    for tokens, k in ((5600, 2), (5600, 4)):     # 8 x 700 tokens of 7168 bytes: 80 and 161 MB of copies, 42 MB staged
+        assert not rules.received_past_cache(tokens * k * 7168)
+    assert rules.received_past_cache(8 * 2048 * 8 * 7168)
+    sides = {cfg.name: rules.received_past_cache(cfg.world_size * cfg.max_num_tokens * cfg.num_experts_per_token *
+                                                 cfg.hidden_dim * cfg.in_dtype.itemsize) for cfg in PIECES}
+    assert sides.pop("past-the-cache") and not any(sides.values())
