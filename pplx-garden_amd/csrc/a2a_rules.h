@@ -73,4 +73,25 @@ constexpr uint64_t kStreamReceived = 200000000;
 
 inline bool received_past_cache(uint64_t copies) { return copies >= kStreamReceived; }
 
+// The first recv of a step is ONE launch that lays the receivers out and copies the caller's rows, a workgroup per row,
+// where a receiver typically gets at most kFewRows rows, or up to kOneLaunchRows of no more than 8 KB each and
+// kOneLaunchBytes together if every thread of a workgroup has at most one of the `items` runs to lay out; otherwise the
+// layout is a launch in front of the copy.  us, layout apart / one launch, rank 0's four calls with one sender and the whole step:
+//   8 ranks, rows of 7168 bytes:   256 rows  21.8 / 19.5    69.5 /  67.2      512 rows  31.4 / 29.0    89.2 /  86.9
+//                                 1024 rows  49.2 / 47.9   121.5 / 119.9     2048 rows  86.3 / 86.3   220.4 / 220.6
+//     8 senders:                   512 rows       -        133.1 / 131.5     1024 rows       -        166.3 / 165.3
+//   16 ranks, 384 experts:         512 rows  47.0 / 44.6   166.9 / 164.3
+//   32 ranks, 512 experts:         475 rows  72.4 / 74.5   333.4 / 335.6     (512 runs, 448 threads)
+//   rows of 2048 bytes:           1024 rows  24.5 / 23.0    74.8 /  73.0     1400 rows  31.0 / 31.7    84.4 /  85.0
+//   rows of 14 KB:                 256 rows  22.3 / 23.2    71.5 /  72.5      512 rows  33.1 / 33.4    93.9 /  94.1
+//                                 1024 rows  53.5 / 57.0   138.8 / 142.0
+constexpr uint32_t kFewRows = 256, kOneLaunchRows = 1024;
+constexpr uint64_t kOneLaunchBytes = 7500000;
+
+inline bool first_recv_in_one_launch(uint32_t typical_rows, uint32_t row_bytes, uint32_t items, uint32_t threads) {
+    if (typical_rows <= kFewRows) return true;
+    return typical_rows <= kOneLaunchRows && row_bytes <= 8192 &&
+           (uint64_t)typical_rows * row_bytes <= kOneLaunchBytes && items <= threads;
+}
+
 }  // namespace a2a

@@ -1,4 +1,5 @@
 // Kernels of the split calls; see a2a_staged.h for what they mirror.
+#include "a2a_rules.h"
 #include "a2a_staged.h"
 
 #include <cstring>
@@ -951,9 +952,10 @@ __global__ __launch_bounds__(1024) void stage_send_resolve_kernel(const StageSen
 
 constexpr uint32_t kPieceThreads = 256;   // threads of a workgroup of the kernels that copy rows in pieces
 
-// A team of `team` threads (one or more whole wavefronts) copies a row of
-// `num_chunks` 16-byte pieces: eight loads per thread in flight, non-temporal
-// both ways (rows are read once and written once).
+// A team of `team` threads (one or more whole wavefronts) copies a staged row of `num_chunks` 16-byte pieces:
+// eight loads per thread in flight.  Ordinary loads, because the recvs of the other ranks its token was routed to read
+// the row again (non-temporal ones here, in the step's first recv: whole steps of one sender of 512 tokens 86.9 -> 89.7
+// us, of 1024 tokens on 16 ranks 164.3 -> 170.5).
 __device__ __forceinline__ void copy_row_by_team(const u32x4 *src, u32x4 *dst, uint32_t num_chunks, uint32_t member,
                                                  uint32_t team) {
     for (uint32_t c0 = 0; c0 < num_chunks; c0 += 8 * team) {
@@ -961,7 +963,7 @@ __device__ __forceinline__ void copy_row_by_team(const u32x4 *src, u32x4 *dst, u
 #pragma unroll
         for (uint32_t u = 0; u < 8; ++u) {
             const uint32_t c = c0 + u * team + member;
-            if (c < num_chunks) v[u] = __builtin_nontemporal_load(src + c);
+            if (c < num_chunks) v[u] = src[c];
         }
 #pragma unroll
         for (uint32_t u = 0; u < 8; ++u) {
@@ -1648,11 +1650,7 @@ uint32_t piece_grid(uint32_t max_rows, uint32_t world, uint32_t chunks, bool in_
     return (uint32_t)blocks;
 }
 
-// The first recv of a step with few rows is ONE launch that lays the receivers out and copies the caller's
-// rows, a workgroup per row; otherwise the layout is a launch in front of the copy.  Whole steps of 8 ranks
-// at the GPU's own pace, hidden 7168, one launch / two: 1 token a rank 91.1 / 93.1 us, 16 tokens (128 rows a
-// receiver) 108.0 / 109.4, 64 tokens (512 rows) 133.7 / 132.7, 128 tokens 180.1 / 177.4.
-constexpr uint32_t kFewRows = 256;
+// The launch that lays the receivers out and copies the caller's rows (first_recv_in_one_launch in a2a_rules.h).
 constexpr uint32_t kFewRowWorkgroups = 512;
 
 }  // namespace
@@ -1926,8 +1924,8 @@ hipError_t launch_stage_recv(const StageRecvArgs &args, const Workspace &ws, con
     const size_t lds = (5 * items + 1 + 3 * (size_t)ws.num_groups + ws.experts_per_rank) * sizeof(uint32_t);
     const uint32_t typical = (args.max_rows + ws.world - 1) / ws.world;
     StageRecvArgs a = args;
-    if (first_of_step && typical <= kFewRows) {
-        const uint32_t threads = block_for_chunks(chunks);
+    const uint32_t threads = block_for_chunks(chunks);
+    if (first_of_step && first_recv_in_one_launch(typical, args.row_bytes, (uint32_t)items, threads)) {
         uint32_t blocks = args.max_rows < kFewRowWorkgroups ? args.max_rows : kFewRowWorkgroups;
         if (blocks == 0) blocks = 1;    // the counts are handed over even when nothing was sent
         // Beside the caller's workgroups: a few per other receiver, enough threads for the rows a receiver
@@ -1941,11 +1939,11 @@ hipError_t launch_stage_recv(const StageRecvArgs &args, const Workspace &ws, con
         return hipGetLastError();
     }
     if (first_of_step) {
-        constexpr uint32_t threads = 512;
-        a.slices = (typical + threads - 1) / threads;
+        constexpr uint32_t layout_threads = 512;
+        a.slices = (typical + layout_threads - 1) / layout_threads;
         if (a.slices < 1) a.slices = 1;
         if (a.slices > 32) a.slices = 32;
-        hipLaunchKernelGGL(stage_layout_kernel, dim3(ws.world * a.slices), dim3(threads), lds, stream, a, ws, st);
+        hipLaunchKernelGGL(stage_layout_kernel, dim3(ws.world * a.slices), dim3(layout_threads), lds, stream, a, ws, st);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }

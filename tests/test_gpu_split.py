@@ -46,8 +46,15 @@ PIECES = [
     RefConfig("one-chunk-rows", 4, 1, 500, 16, 8, None, 4, BF16, BF16, None),
     RefConfig("more-scales-than-lanes", 2, 1, 400, 8, 512, 128, 2, FP8, BF16, F32),
     # a receiver typically gets max_num_tokens * K rows here: one launch up to 256, layout and copy apart from there on
-    RefConfig("256-rows", 2, 1, 64, 16, 1024, 8, 4, FP8, BF16, F32),
-    RefConfig("257-rows", 2, 1, 257, 16, 1024, None, 1, BF16, BF16, None),
+    # with more (source, expert) runs than a row has chunks (64 and 128 here) ...
+    RefConfig("256-rows", 2, 1, 64, 80, 1024, 8, 4, FP8, BF16, F32),
+    RefConfig("257-rows", 2, 1, 257, 160, 1024, None, 1, BF16, BF16, None),
+    RefConfig("257-rows-one-run-a-thread", 2, 1, 257, 128, 1024, None, 1, BF16, BF16, None),
+    # ... and otherwise one launch up to 1024 rows and 7.5 MB of them, no more than 8 KB each
+    RefConfig("1024-rows", 2, 1, 256, 16, 1024, 8, 4, FP8, BF16, F32),
+    RefConfig("1025-rows", 2, 1, 1025, 16, 1024, None, 1, BF16, BF16, None),
+    RefConfig("915-rows-of-8-KB", 2, 1, 915, 16, 8192, 64, 1, FP8, BF16, F32),
+    RefConfig("916-rows-of-8-KB", 2, 1, 916, 16, 8192, 64, 1, FP8, BF16, F32),
     # copies of 200 MB are 6975 tokens with four copies of 7168 bytes; a step on either side
     RefConfig("kept-in-cache", 2, 1, 3450, 8, 7168, 28, 4, FP8, BF16, F32),
     RefConfig("past-the-cache", 2, 1, 3550, 8, 7168, 28, 4, FP8, BF16, F32),

@@ -19,6 +19,9 @@ uint32_t layers(uint32_t tokens) { return a2a::token_layers(tokens).layers; }
 uint32_t layer_rows(uint32_t tokens) { return a2a::token_layers(tokens).rows; }
 int past_cache(uint64_t copies, int quantize, uint32_t k) { return a2a::copies_past_cache(copies, quantize != 0, k); }
 int received_past_cache(uint64_t copies) { return a2a::received_past_cache(copies); }
+int one_launch(uint32_t rows, uint32_t row_bytes, uint32_t items, uint32_t threads) {
+    return a2a::first_recv_in_one_launch(rows, row_bytes, items, threads);
+}
 }
 """
 
@@ -67,3 +70,19 @@ def test_received_rows_that_the_cache_can_keep_stay_there(rules):
     sides = {cfg.name: rules.received_past_cache(cfg.world_size * cfg.max_num_tokens * cfg.num_experts_per_token *
                                                  cfg.hidden_dim * cfg.in_dtype.itemsize) for cfg in PIECES}
     assert sides.pop("past-the-cache") and not any(sides.values())
+
+
+def test_first_recvs_in_one_launch(rules):
+    # rows a receiver typically gets, bytes of one, (source, expert) runs, threads of a workgroup
+    assert rules.one_launch(512, 7168, 16 * 24, 448)            # 1024 tokens on 16 ranks with 384 experts
+    assert rules.one_launch(1024, 7168, 8 * 32, 448) and rules.one_launch(256, 16384, 1024, 64)
+    assert not rules.one_launch(475, 7168, 32 * 16, 448)        # more runs than threads
+    assert not rules.one_launch(512, 14336, 8 * 16, 896) and not rules.one_launch(1025, 1024, 8, 64)
+    sides = {}
+    for cfg in PIECES:
+        row = cfg.hidden_dim * cfg.in_dtype.itemsize
+        runs = cfg.world_size * -(-cfg.num_experts // cfg.world_size)
+        sides[cfg.name] = rules.one_launch(cfg.max_num_tokens * cfg.num_experts_per_token, row, runs,
+                                           min(max(-(-row // 1024) * 64, 64), 1024))
+    assert [n for n in sides if sides[n]] == ["more-scales-than-lanes", "256-rows", "257-rows-one-run-a-thread",
+                                                  "1024-rows", "915-rows-of-8-KB"]
