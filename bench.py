@@ -484,6 +484,7 @@ def split_calls(case, device, routings: int, steps: int, warmup: int, label: str
         send(j)
         for r in range(1, N):
             empty_send(r)
+        own(native.KERNEL_STAGE_LAYOUT, "layout")
         for r in range(N):
             own(native.KERNEL_STAGE_RECV, ("recv", r))
             recv(r)
@@ -572,13 +573,15 @@ def split_calls(case, device, routings: int, steps: int, warmup: int, label: str
             kernel("stage_send_resolve_kernel", us.get("send", []), lambda j: T * (2 * H + 4 * K) + T * row_d),
         ],
         "dispatch_recv": [
-            kernel("stage_recv_kernel, behind stage_layout_kernel", us.get(("recv", 0), []), lambda j: 2 * int(rows_of[j][0]) * row_d),
+            kernel("stage_layout_kernel", us.get("layout", []), lambda j: 0),
+            kernel("stage_recv_kernel (first of the step)", us.get(("recv", 0), []),
+                   lambda j: 2 * int(rows_of[j][0]) * row_d),
             seq_kernel("stage_recv_kernel", later, later_seq),
         ],
         "combine_send": [seq_kernel("combine_send_kernel", csend, csend_seq)],
         "combine_recv": [kernel("combine_gather_kernel", us.get("combine_recv", []), lambda j: c_bytes)],
     }
-    one_rank_kernels = sum(k["avg_us"] for k in (kernels["dispatch_send"] + kernels["dispatch_recv"][:1]
+    one_rank_kernels = sum(k["avg_us"] for k in (kernels["dispatch_send"] + kernels["dispatch_recv"][:2]
                                                  + kernels["combine_send"] + kernels["combine_recv"]) if k)
     return {
         "workload": label,
@@ -591,7 +594,8 @@ def split_calls(case, device, routings: int, steps: int, warmup: int, label: str
                 "scales per token; a recv reads and writes the rows its rank receives; a combine-send reads and "
                 "writes the bf16 rows of its rank; the combine-recv is the gather of the group call over the "
                 "staging buffer.  one_rank_step = rank 0's four calls (what a rank on a GPU of its own runs; "
-                "its recv is the step's first and also lays out the other receivers); all_ranks_step = the "
+                "its recv is the step's first and lays all receivers out, in a launch in front of its copy that "
+                "one_rank_step_us_kernels counts); all_ranks_step = the "
                 "send, every rank's recv, every rank's combine-send and rank 0's combine-recv (the work of "
                 "the whole group for one sender's tokens, on this GPU).  Kernel durations come from events "
                 f"the launches record themselves, over {sample_steps} steps; wall times from {steps} steps "

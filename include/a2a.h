@@ -328,6 +328,10 @@ int a2a_ctx_read_table(a2a_ctx *ctx, uint32_t rank, uint32_t which,
  *   A2A_KERNEL_GATHER        the gather of the next a2a_combine or a2a_combine_recv
  *   A2A_KERNEL_STAGE_SEND    the staging launch of the next a2a_dispatch_send
  *   A2A_KERNEL_STAGE_RECV    the copy launch of the next a2a_dispatch_recv
+ *   A2A_KERNEL_STAGE_LAYOUT  the launch in front of that copy which lays the receivers
+ *                            out, in the first a2a_dispatch_recv of a large step; the
+ *                            other recvs, and the first of a step that does both in
+ *                            its copy launch, leave those events alone
  *   A2A_KERNEL_COMBINE_SEND  the copy launch of the next a2a_combine_send
  * One-shot: the request is consumed by that call (a call that launches nothing,
  * such as a send without tokens, consumes it too).  Pass two nulls to withdraw
@@ -335,7 +339,8 @@ int a2a_ctx_read_table(a2a_ctx *ctx, uint32_t rank, uint32_t which,
  * the stream or the event). */
 enum {
     A2A_KERNEL_PACK = 0, A2A_KERNEL_GATHER = 1, A2A_KERNEL_ROUTE = 2,
-    A2A_KERNEL_STAGE_SEND = 3, A2A_KERNEL_STAGE_RECV = 4, A2A_KERNEL_COMBINE_SEND = 5
+    A2A_KERNEL_STAGE_SEND = 3, A2A_KERNEL_STAGE_RECV = 4, A2A_KERNEL_COMBINE_SEND = 5,
+    A2A_KERNEL_STAGE_LAYOUT = 6
 };
 int a2a_ctx_time_next_kernel(a2a_ctx *ctx, uint32_t which, void *start_event, void *stop_event);
 

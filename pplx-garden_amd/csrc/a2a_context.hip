@@ -49,7 +49,7 @@ struct a2a_ctx {
 
     Staging staging;               // buffers and tables of the split calls
 
-    KernelTiming timing[6];        // one-shot events for the next launch of each kernel a2a_ctx_time_next_kernel names
+    KernelTiming timing[7];        // one-shot events for the next launch of each kernel a2a_ctx_time_next_kernel names
 };
 
 // Device memory of a2a_dispatch_static: the routing tables of ONE step, in a
@@ -841,7 +841,7 @@ int a2a_combine(a2a_ctx *ctx, const a2a_combine_args *args, uint32_t expert_y_dt
 
 int a2a_ctx_time_next_kernel(a2a_ctx *ctx, uint32_t which, void *start_event, void *stop_event) {
     if (ctx == nullptr) return A2A_ERR_INVALID_ARGUMENT;
-    if (which > A2A_KERNEL_COMBINE_SEND) return fail(ctx, A2A_ERR_INVALID_ARGUMENT, "unknown kernel %u", which);
+    if (which > A2A_KERNEL_STAGE_LAYOUT) return fail(ctx, A2A_ERR_INVALID_ARGUMENT, "unknown kernel %u", which);
     if ((start_event == nullptr) != (stop_event == nullptr))
         return fail(ctx, A2A_ERR_INVALID_ARGUMENT, "pass both events or neither");
     ctx->timing[which].start = static_cast<hipEvent_t>(start_event);
@@ -1072,8 +1072,10 @@ int a2a_dispatch_recv(a2a_ctx *ctx, uint32_t rank, int32_t *out_num_tokens, void
     rv.valid_mask = ctx->sent_mask & ~ctx->empty_mask;
     rv.max_private = c.max_private_tokens;
     const KernelTiming recv_timing = ctx->timing[A2A_KERNEL_STAGE_RECV];
+    const KernelTiming layout_timing = ctx->timing[A2A_KERNEL_STAGE_LAYOUT];
     ctx->timing[A2A_KERNEL_STAGE_RECV] = KernelTiming();
-    const hipError_t e = launch_stage_recv(rv, ctx->ws, ctx->staging, !ctx->recv_seen, s, recv_timing);
+    ctx->timing[A2A_KERNEL_STAGE_LAYOUT] = KernelTiming();
+    const hipError_t e = launch_stage_recv(rv, ctx->ws, ctx->staging, !ctx->recv_seen, s, recv_timing, layout_timing);
     if (e != hipSuccess) return hip_fail(ctx, e, "launch stage_recv");
     ctx->recv_seen = true;
     ctx->staging.recv_mask |= 1u << rank;

@@ -118,9 +118,11 @@ hipError_t launch_stage_send_single(const StageSendArgs &args, const Workspace &
 // The send of a large step after launch_route_accumulate(..., for_send = true).
 hipError_t launch_stage_send_resolve(const StageSendArgs &args, const Workspace &ws, const Staging &st,
                                      bool quantize, hipStream_t stream, KernelTiming timing = KernelTiming());
-// `first_of_step`: no recv has run since the step's sends; all receivers are laid out first.
+// `first_of_step`: no recv has run since the step's sends; all receivers are laid out first (`layout_timing`: where that
+// is a launch of its own).
 hipError_t launch_stage_recv(const StageRecvArgs &args, const Workspace &ws, const Staging &st, bool first_of_step,
-                             hipStream_t stream, KernelTiming timing = KernelTiming());
+                             hipStream_t stream, KernelTiming timing = KernelTiming(),
+                             KernelTiming layout_timing = KernelTiming());
 hipError_t launch_combine_send(const CombineSendArgs &args, const Workspace &ws, const Staging &st,
                                hipStream_t stream, KernelTiming timing = KernelTiming());
 hipError_t launch_combine_recv(const CombineRecvArgs &args, const Workspace &ws, const Staging &st,

@@ -1918,7 +1918,7 @@ hipError_t launch_stage_send_resolve(const StageSendArgs &args, const Workspace 
 }
 
 hipError_t launch_stage_recv(const StageRecvArgs &args, const Workspace &ws, const Staging &st, bool first_of_step,
-                             hipStream_t stream, KernelTiming timing) {
+                             hipStream_t stream, KernelTiming timing, KernelTiming layout_timing) {
     const uint32_t chunks = args.row_bytes / 16;
     const size_t items = (size_t)ws.num_groups * ws.experts_per_rank;
     const size_t lds = (5 * items + 1 + 3 * (size_t)ws.num_groups + ws.experts_per_rank) * sizeof(uint32_t);
@@ -1943,7 +1943,8 @@ hipError_t launch_stage_recv(const StageRecvArgs &args, const Workspace &ws, con
         a.slices = (typical + layout_threads - 1) / layout_threads;
         if (a.slices < 1) a.slices = 1;
         if (a.slices > 32) a.slices = 32;
-        hipLaunchKernelGGL(stage_layout_kernel, dim3(ws.world * a.slices), dim3(layout_threads), lds, stream, a, ws, st);
+        hipExtLaunchKernelGGL(stage_layout_kernel, dim3(ws.world * a.slices), dim3(layout_threads), lds, stream,
+                              layout_timing.start, layout_timing.stop, 0, a, ws, st);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }

@@ -59,6 +59,7 @@ KERNEL_ROUTE = 2
 KERNEL_STAGE_SEND = 3
 KERNEL_STAGE_RECV = 4
 KERNEL_COMBINE_SEND = 5
+KERNEL_STAGE_LAYOUT = 6
 
 
 class A2AConfig(ctypes.Structure):
@@ -362,10 +363,11 @@ class AllToAllContext:
     def time_next_kernel(self, which: int, start_event: Optional[int], stop_event: Optional[int]) -> None:
         """Have the next call that launches kernel `which` (`KERNEL_PACK`, `KERNEL_ROUTE`: the group
         dispatch; `KERNEL_GATHER`: the group combine or the split combine-recv; `KERNEL_STAGE_SEND`,
-        `KERNEL_ROUTE`: the split send; `KERNEL_STAGE_RECV`, `KERNEL_COMBINE_SEND`: those split calls)
+        `KERNEL_ROUTE`: the split send; `KERNEL_STAGE_RECV`, `KERNEL_STAGE_LAYOUT`, `KERNEL_COMBINE_SEND`: those split calls)
         record the two events (raw `hipEvent_t` handles, e.g. `torch.cuda.Event.cuda_event`) at the
         start and end of that kernel itself.  `KERNEL_ROUTE` is the routing launch before the pack or
-        the staging of a large step; a step without such a launch leaves those events alone."""
+        the staging of a large step, `KERNEL_STAGE_LAYOUT` the one before the copy of its first recv; a step
+        without such a launch leaves those events alone."""
         self._require_open()
         self._check(self._lib.a2a_ctx_time_next_kernel(self._handle, which, _ptr(start_event), _ptr(stop_event)))
 

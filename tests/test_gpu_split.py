@@ -68,6 +68,36 @@ def test_rows_in_pieces(cfg, device):
     check(cfg, world, rows, run_gpu_rows(cfg, world, rows, device, True))
 
 
+def test_layout_kernel_own_events(device):
+    """A2A_KERNEL_STAGE_LAYOUT times the launch in front of the first recv's copy, which the events of that copy do not
+    cover; a step that does both in one launch leaves the events alone."""
+    def timed(case):
+        world = make_world(case, "all")
+        _, ops = make_ops(case, device)
+        ev = [torch.cuda.Event(enable_timing=True) for _ in range(4)]
+        for e in ev:
+            e.record()
+        torch.cuda.synchronize(device)
+        before = ev[3].elapsed_time(ev[0])
+        try:
+            ops[0].context.time_next_kernel(native.KERNEL_STAGE_LAYOUT, ev[0].cuda_event, ev[1].cuda_event)
+            run_gpu(case, world, rows_needed(case, world), device, split=True, ops=ops)
+            one_launch = ev[3].elapsed_time(ev[0]) == before
+            ops[0].context.time_next_kernel(native.KERNEL_STAGE_LAYOUT, ev[0].cuda_event, ev[1].cuda_event)
+            ops[0].context.time_next_kernel(native.KERNEL_STAGE_RECV, ev[2].cuda_event, ev[3].cuda_event)
+            run_gpu(case, world, rows_needed(case, world), device, split=True, ops=ops)
+            torch.cuda.synchronize(device)
+            return one_launch, [ev[i].elapsed_time(ev[i + 1]) for i in range(3)]
+        finally:
+            for op in ops:
+                op.destroy()
+
+    one_launch, (layout_ms, gap_ms, copy_ms) = timed(scaled(C1, 200))     # 8 x 200 x 8 rows: 1600 a receiver
+    print(f"layout {layout_ms * 1e3:.1f} us, copy {copy_ms * 1e3:.1f} us", flush=True)
+    assert not one_launch and 0.0 < layout_ms < 1.0 and gap_ms >= 0.0 and 0.0 < copy_ms < 1.0
+    assert timed(scaled(C1, 100))[0]                                      # 800 a receiver
+
+
 QUICK_SENDS = [
     # (tokens, hidden, experts, ranks, top-k, padding, sources, experts may repeat inside a token)
     (1, 2048, 128, 8, 8, 1, "one", False),
