@@ -286,6 +286,16 @@ const Tensor *matrix_of(PyObject *obj, const char *name, PyObject *error) {
     return t;
 }
 
+// Scales: the strides of the first two dimensions are all that is read of their layout; further ones may follow.
+const Tensor *scales_of(PyObject *obj, const char *name) {
+    const Tensor *t = tensor_of(obj, name);
+    if (t != nullptr && t->dim() < 2) {
+        PyErr_Format(PyExc_IndexError, "%s must have at least two dimensions, has %d", name, (int)t->dim());
+        return nullptr;
+    }
+    return t;
+}
+
 bool has_shape(const Tensor &t, int64_t rows, int64_t cols) { return t.size(0) == rows && t.size(1) == cols; }
 
 uint64_t row_bytes(const Tensor &t) { return (uint64_t)t.stride(0) * t.element_size(); }
@@ -375,7 +385,7 @@ PyObject *dispatch(Operator *op, PyObject *const *a, Py_ssize_t n) {
     // Output scale buffer (p2p_all_to_all.py:350-362).
     const Tensor *out_scale = nullptr;
     if (a[2] != Py_None) {
-        out_scale = matrix_of(a[2], "out_expert_x_scale", PyExc_IndexError);
+        out_scale = scales_of(a[2], "out_expert_x_scale");
         if (out_scale == nullptr) return nullptr;
         A2A_REQUIRE(op->has_scale_dtype && out_scale->scalar_type() == ScalarType::Float);
     }
@@ -398,7 +408,7 @@ PyObject *dispatch(Operator *op, PyObject *const *a, Py_ssize_t n) {
     // Input scales (p2p_all_to_all.py:371-388).
     const Tensor *x_scale = nullptr;
     if (a[4] != Py_None) {
-        x_scale = matrix_of(a[4], "dp_x_scale", PyExc_IndexError);
+        x_scale = scales_of(a[4], "dp_x_scale");
         if (x_scale == nullptr) return nullptr;
         A2A_REQUIRE(op->has_scale_dtype && op->hidden_dim_scale >= 0);
         A2A_REQUIRE(out_scale != nullptr);

@@ -310,6 +310,25 @@ def test_operators_collect_a_collective_in_native_code():
     assert context.pending("combine") == 0
 
 
+def test_scales_may_have_more_than_two_dimensions():
+    """Of scales only the first two strides count: (rows, scales, 1), as a view of a blocked layout has them, passes;
+    one dimension has no second stride."""
+    module = native.load_extension()
+    context = module.Context(0, 2)
+    op = module.Operator(context, 0, 1, 128, 1, 2, 4, torch.float8_e4m3fn, torch.bfloat16, True, -1)
+    x = torch.zeros((5, 128), dtype=torch.float8_e4m3fn)
+    args = [torch.zeros(2, dtype=torch.int32), torch.zeros((8, 128), dtype=torch.float8_e4m3fn), torch.zeros((8, 1)), x,
+            torch.zeros((5, 1)), torch.zeros((5, 4), dtype=torch.int32).view(torch.uint32), torch.zeros((5, 4)), None, True,
+            True]
+    for out_scale, x_scale in [(torch.zeros((8, 1, 1)), args[4]), (args[2], torch.zeros((5, 1, 1))),
+                               (torch.zeros((8, 1, 2, 3)), torch.zeros((5, 1, 1)))]:
+        assert op.dispatch(*args[:2], out_scale, x, x_scale, *args[5:]) is None
+        context.close()                                              # forgets what the rank has posted
+    for at in (2, 4):
+        with pytest.raises(IndexError):
+            op.dispatch(*(torch.zeros(8) if i == at else v for i, v in enumerate(args)))
+
+
 @pytest.mark.parametrize("stream", [None, 0])
 def test_group_calls_take_no_stream_and_longer_arrays(stream):
     """What the ctypes binding took: None as the default stream, an array with more entries than ranks.  A shorter
