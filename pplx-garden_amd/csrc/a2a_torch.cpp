@@ -136,14 +136,30 @@ bool array_of(PyObject *obj, uint32_t world, Py_buffer *view) {
     return false;
 }
 
+// A number as int() makes it (numpy's integers too), as the 32 bits of a C argument or as an address.
+bool integer_of(PyObject *obj, uint32_t *out) {
+    PyObject *number = PyNumber_Long(obj);
+    if (number == nullptr) return false;
+    *out = (uint32_t)PyLong_AsUnsignedLongMask(number);
+    Py_DECREF(number);
+    return !PyErr_Occurred();
+}
+
+bool address_of(PyObject *obj, void **out) {
+    PyObject *number = PyNumber_Long(obj);
+    if (number == nullptr) return false;
+    *out = PyLong_AsVoidPtr(number);
+    Py_DECREF(number);
+    return !PyErr_Occurred();
+}
+
 // group_dispatch(array, quantize, stream)
 PyObject *context_group_dispatch(PyObject *self, PyObject *const *args, Py_ssize_t n) {
     Context *c = reinterpret_cast<Context *>(self);
     if (n != 3) return PyErr_Format(PyExc_TypeError, "group_dispatch takes 3 arguments");
-    const int quantize = PyObject_IsTrue(args[1]);
-    if (quantize < 0) return nullptr;
-    void *stream = PyLong_AsVoidPtr(args[2]);
-    if (stream == nullptr && PyErr_Occurred()) return nullptr;
+    uint32_t quantize;
+    void *stream;
+    if (!integer_of(args[1], &quantize) || !address_of(args[2], &stream)) return nullptr;
     Py_buffer view;
     if (!array_of<a2a_dispatch_args>(args[0], c->world, &view)) return nullptr;
     if (!require_open(c)) {
@@ -153,7 +169,7 @@ PyObject *context_group_dispatch(PyObject *self, PyObject *const *args, Py_ssize
     a2a_ctx *const ctx = c->ctx;
     int rc;
     Py_BEGIN_ALLOW_THREADS
-    rc = a2a_dispatch(ctx, static_cast<const a2a_dispatch_args *>(view.buf), (uint32_t)quantize, stream);
+    rc = a2a_dispatch(ctx, static_cast<const a2a_dispatch_args *>(view.buf), quantize, stream);
     Py_END_ALLOW_THREADS
     PyBuffer_Release(&view);
     if (rc != 0) return raise_last_error(ctx, "a2a_dispatch", rc);
@@ -164,12 +180,11 @@ PyObject *context_group_dispatch(PyObject *self, PyObject *const *args, Py_ssize
 PyObject *context_group_combine(PyObject *self, PyObject *const *args, Py_ssize_t n) {
     Context *c = reinterpret_cast<Context *>(self);
     if (n != 4) return PyErr_Format(PyExc_TypeError, "group_combine takes 4 arguments");
-    const unsigned long tag = PyLong_AsUnsignedLong(args[1]);
-    if (tag == (unsigned long)-1 && PyErr_Occurred()) return nullptr;
+    uint32_t tag;
+    void *stream;
+    if (!integer_of(args[1], &tag) || !address_of(args[3], &stream)) return nullptr;
     const int accumulate = PyObject_IsTrue(args[2]);
     if (accumulate < 0) return nullptr;
-    void *stream = PyLong_AsVoidPtr(args[3]);
-    if (stream == nullptr && PyErr_Occurred()) return nullptr;
     Py_buffer view;
     if (!array_of<a2a_combine_args>(args[0], c->world, &view)) return nullptr;
     if (!require_open(c)) {
@@ -179,7 +194,7 @@ PyObject *context_group_combine(PyObject *self, PyObject *const *args, Py_ssize_
     a2a_ctx *const ctx = c->ctx;
     int rc;
     Py_BEGIN_ALLOW_THREADS
-    rc = a2a_combine(ctx, static_cast<const a2a_combine_args *>(view.buf), (uint32_t)tag, (uint32_t)accumulate, stream);
+    rc = a2a_combine(ctx, static_cast<const a2a_combine_args *>(view.buf), tag, (uint32_t)accumulate, stream);
     Py_END_ALLOW_THREADS
     PyBuffer_Release(&view);
     if (rc != 0) return raise_last_error(ctx, "a2a_combine", rc);

@@ -635,6 +635,22 @@ def test_routing_kernel_own_events():
             op.destroy()
 
 
+def test_group_dispatch_refuses_a_quantize_flag_that_is_no_flag():
+    case = C0
+    world = make_world(case, "all")
+    _, ops = make_ops(case, DEV)
+    try:
+        ctx = ops[0].context
+        none = ctx.pack_dispatch_args([native.A2ADispatchArgs() for _ in range(case.world_size)])
+        with pytest.raises(RuntimeError, match="quantize must be 0 or 1"):
+            ctx.dispatch(none, 2, 0)
+        assert_dispatch_equal(case, run_gpu(case, world, rows_needed(case, world), DEV, ops=ops),
+                              run_oracle(case, world, rows_needed(case, world)))
+    finally:
+        for op in ops:
+            op.destroy()
+
+
 def test_operator_reports_the_reference_capacities():
     """`P2PAllToAll.max_recv_tokens` / `max_private_tokens` of live operators on the five baseline
     shapes against the oracle's restatement of python/pplx_garden/kernels/p2p_all_to_all.py:92-114,

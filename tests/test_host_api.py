@@ -346,3 +346,23 @@ def test_group_calls_take_no_stream_and_longer_arrays(stream):
             call((args * 2)())
         with pytest.raises(TypeError):
             call((other * 3)())
+
+
+def test_group_calls_take_numbers_as_the_binding_did():
+    """Stream handles and flags that int() takes (numpy's integers); what int() refuses is a TypeError.  `quantize` is
+    handed on as the number it is, so that the library can refuse a 2."""
+    import numpy as np
+    module = native.load_extension()
+    ctx = native.AllToAllContext.__new__(native.AllToAllContext)
+    ctx._handle, ctx.shared = None, module.Context(0, 3)
+    dispatch, combine = (native.A2ADispatchArgs * 3)(), (native.A2ACombineArgs * 3)()
+    for stream in (0, np.int64(4096), np.uint64(1 << 63)):
+        with pytest.raises(RuntimeError, match="destroyed"):
+            ctx.dispatch(dispatch, np.bool_(True), stream)
+        with pytest.raises(RuntimeError, match="destroyed"):
+            ctx.combine(combine, torch.bfloat16, np.bool_(False), stream)
+    for quantize, stream in ((None, 0), (True, object())):
+        with pytest.raises(TypeError):
+            ctx.dispatch(dispatch, quantize, stream)
+    with pytest.raises(TypeError):
+        ctx.combine(combine, torch.bfloat16, False, object())
