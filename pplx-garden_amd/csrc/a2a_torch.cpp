@@ -16,6 +16,7 @@
 #include <torch/csrc/Dtype.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <cstring>
 #include <string>
 
 #include "a2a.h"
@@ -118,7 +119,9 @@ PyObject *context_pending(PyObject *self, PyObject *kind) {
     Context *c = reinterpret_cast<Context *>(self);
     const char *name = PyUnicode_AsUTF8(kind);
     if (name == nullptr) return nullptr;
-    return PyLong_FromUnsignedLong(name[0] == 'd' ? c->dispatch->posted : c->combine->posted);
+    if (strcmp(name, "dispatch") == 0) return PyLong_FromUnsignedLong(c->dispatch->posted);
+    if (strcmp(name, "combine") == 0) return PyLong_FromUnsignedLong(c->combine->posted);
+    return PyErr_Format(PyExc_ValueError, "no collective %s: \"dispatch\" or \"combine\"", name);
 }
 
 // The arguments of all ranks out of a C array (ctypes) of at least `world` structures.

@@ -329,6 +329,14 @@ def test_scales_may_have_more_than_two_dimensions():
             op.dispatch(*(torch.zeros(8) if i == at else v for i, v in enumerate(args)))
 
 
+def test_pending_knows_two_collectives():
+    context = native.load_extension().Context(0, 3)
+    assert context.pending("dispatch") == 0 and context.pending("combine") == 0
+    for name in ("", "d", "dispatch_send", "recv"):
+        with pytest.raises(ValueError):
+            context.pending(name)
+
+
 @pytest.mark.parametrize("stream", [None, 0])
 def test_group_calls_take_no_stream_and_longer_arrays(stream):
     """What the ctypes binding took: None as the default stream, an array with more entries than ranks.  A shorter
