@@ -9,9 +9,9 @@ group and `world.group(rank)` is what one logical rank passes as
 context, so their buffers and routing tables sit in the same HBM.
 
 A collective is complete when every rank has made the call.  In one process
-the ranks call one after the other, so the world collects the arguments of a
-collective call and the call of the LAST rank launches the work for all of
-them; results are defined once every rank of the world has called.
+the ranks call one after the other, so their shared context collects the
+arguments of a collective call and the call of the LAST rank launches the work
+for all of them; results are defined once every rank of the world has called.
 """
 
 from __future__ import annotations
@@ -65,7 +65,6 @@ class LoopbackWorld:
         self.context_flags = context_flags   # A2A_FLAG_* bits for the contexts created in this world
         self._contexts: Dict[Tuple, Any] = {}
         self._users: Dict[Tuple, int] = {}
-        self._pending: Dict[Tuple[Tuple, str], Dict[int, Any]] = {}
 
     def group(self, rank: int) -> LoopbackGroup:
         if not 0 <= rank < self.size:
@@ -99,31 +98,12 @@ class LoopbackWorld:
         if self._users[key] <= 0:
             ctx = self._contexts.pop(key)
             self._users.pop(key)
-            for pending_key in [k for k in self._pending if k[0] == key]:
-                self._pending.pop(pending_key)
             ctx.destroy()
 
     # -- collectives --------------------------------------------------------
 
-    def post(self, key: Tuple, kind: str, rank: int, payload: Any) -> Optional[List[Any]]:
-        """Record `rank`'s arguments for collective `kind`.  Returns the
-        arguments of all ranks, in rank order, once the last rank has posted.
-        (The operators' own collectives are collected by their native context,
-        by the same rule.)"""
-        slot = self._pending.setdefault((key, kind), {})
-        if rank in slot:
-            missing = sorted(set(range(self.size)) - set(slot))
-            raise RuntimeError(
-                f"rank {rank} called {kind}() twice before ranks {missing} called it: in loopback "
-                "a collective runs when every logical rank has made the call")
-        slot[rank] = payload
-        if len(slot) < self.size:
-            return None
-        del self._pending[(key, kind)]
-        return [slot[r] for r in range(self.size)]
-
     def pending(self, key: Tuple, kind: str) -> List[int]:
-        """Ranks that have called collective `kind` of configuration `key` and wait for the others."""
+        """Ranks that have called collective `kind` ("dispatch" or "combine") of configuration `key` and wait for
+        the others.  Their arguments are with the native context, whose last rank's call runs the collective."""
         context = self._contexts.get(key)
-        native = context.pending(kind) if context is not None else []
-        return sorted({*self._pending.get((key, kind), {}), *native})
+        return context.pending(kind) if context is not None else []

@@ -73,13 +73,14 @@ def make_ops(case: Case, device: torch.device, max_num_tokens: Optional[int] = N
 
 
 def run_gpu(case: Case, world_data: Sequence[RankData], rows: int, device: torch.device,
-            split: bool = False, expert_y_override=None, context_flags: int = 0, ops=None) -> WorldResult:
+            split: bool = False, expert_y_override=None, context_flags: int = 0, ops=None,
+            order: Optional[Sequence[int]] = None) -> WorldResult:
     """dispatch -> 2*dequant -> combine on the GPU through the operator API.
 
     split=False: every rank calls dispatch()/combine() with do_send and do_recv
     (the group calls of the library); split=True: all sends, then all recvs (the
     four split calls).  With `ops` the given operators are used (and kept): several
-    steps on one context."""
+    steps on one context.  `order`: in which the ranks make the group calls."""
     N, H, Hs, Le = case.world_size, case.hidden_dim, case.hidden_dim_scale, case.experts_per_rank
     own_ops = ops is None
     if own_ops:
@@ -108,7 +109,7 @@ def run_gpu(case: Case, world_data: Sequence[RankData], rows: int, device: torch
             for r in range(N):
                 dispatch(r, do_send=False, do_recv=True)
         else:
-            for r in range(N):
+            for r in order or range(N):
                 dispatch(r)
         torch.cuda.synchronize(device)
         flags = ops[0].context.status()
@@ -134,7 +135,7 @@ def run_gpu(case: Case, world_data: Sequence[RankData], rows: int, device: torch
             for r in range(N):
                 combine(r, do_send=False, do_recv=True)
         else:
-            for r in range(N):
+            for r in order or range(N):
                 combine(r)
         torch.cuda.synchronize(device)
         flags = ops[0].context.status()

@@ -35,6 +35,17 @@ def test_group_parity(case, sources, device):
     assert same >= total * 0.9999, (same, total)
 
 
+def test_ranks_may_make_a_collective_call_in_any_order(device):
+    """The context sorts what the ranks pass by rank, whoever calls last."""
+    world = make_world(C0, "ragged")
+    rows = rows_needed(C0, world)
+    want = run_oracle(C0, world, rows)
+    for order in (range(C0.world_size - 1, -1, -1), [*range(1, C0.world_size), 0]):
+        got = run_gpu(C0, world, rows, device, order=order)
+        assert_dispatch_equal(C0, got, want)
+        assert_combine_close(C0, got, want)
+
+
 @pytest.mark.parametrize("split", [False, True], ids=["group", "split"])
 @pytest.mark.parametrize("case,sources", [(C0, "ragged"), (C2, "all"), (C2, "one")],
                          ids=lambda v: v.name if hasattr(v, "name") else v)

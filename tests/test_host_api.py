@@ -163,14 +163,24 @@ def test_loopback_world_runs_a_collective_when_the_last_rank_posts():
     world = LoopbackWorld(3)
     assert [g.rank for g in world.groups] == [0, 1, 2] and world.group(1).size == 3
     key = ("cfg",)
-    assert world.post(key, "dispatch", 1, "b") is None
-    assert world.post(key, "dispatch", 0, "a") is None
+    assert world.pending(key, "dispatch") == []                       # nobody has made a context
+    module = native.load_extension()
+    ctx = native.AllToAllContext.__new__(native.AllToAllContext)      # (its native part has no GPU behind it)
+    ctx._handle, ctx._config, ctx.shared = None, native.A2AConfig(world_size=3), module.Context(0, 3)
+    assert world.acquire_context(key, lambda: ctx) is ctx
+    ops = [module.Operator(ctx.shared, r, 1, 128, -1, 2, 4, torch.bfloat16, torch.bfloat16, False, -1) for r in range(3)]
+    indices, weights = torch.zeros((5, 4), dtype=torch.int32).view(torch.uint32), torch.zeros((5, 4))
+    x, rows = torch.zeros((5, 128), dtype=torch.bfloat16), torch.zeros((8, 128), dtype=torch.bfloat16)
+    dispatch = (torch.zeros(2, dtype=torch.int32), rows, None, x, None, indices, weights, None, True, True)
+    assert ops[1].dispatch(*dispatch) is None and ops[0].dispatch(*dispatch) is None
     assert world.pending(key, "dispatch") == [0, 1]
-    with pytest.raises(RuntimeError, match="twice"):
-        world.post(key, "dispatch", 1, "again")
-    assert world.post(key, "dispatch", 2, "c") == ["a", "b", "c"]      # rank order, not call order
+    with pytest.raises(RuntimeError, match=r"twice before ranks \[2\]"):
+        ops[1].dispatch(*dispatch)
+    with pytest.raises(RuntimeError, match="destroyed"):              # the last rank's call is the one that runs it
+        ops[2].dispatch(*dispatch)
     assert world.pending(key, "dispatch") == []
-    assert world.post(key, "combine", 0, 1) is None                   # kinds do not mix
+    assert ops[0].combine(x, indices, weights, rows, None, True, True, False) is None
+    assert world.pending(key, "combine") == [0] and world.pending(key, "dispatch") == []   # kinds do not mix
     with pytest.raises(ValueError):
         LoopbackWorld(4, node_size=3)
     with pytest.raises(ValueError):
