@@ -17,6 +17,7 @@
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <cstring>
+#include <new>
 #include <string>
 
 #include "a2a.h"
@@ -89,15 +90,19 @@ PyObject *context_new(PyTypeObject *type, PyObject *args, PyObject *) {
     if (c == nullptr) return nullptr;
     c->ctx = reinterpret_cast<a2a_ctx *>(handle);
     c->world = world;
-    c->dispatch = new Pending<a2a_dispatch_args>();
-    c->combine = new Pending<a2a_combine_args>();
+    c->dispatch = new (std::nothrow) Pending<a2a_dispatch_args>();
+    c->combine = new (std::nothrow) Pending<a2a_combine_args>();
+    if (c->dispatch == nullptr || c->combine == nullptr) {
+        Py_DECREF(c);
+        return PyErr_NoMemory();
+    }
     return reinterpret_cast<PyObject *>(c);
 }
 
 void context_dealloc(PyObject *self) {
     Context *c = reinterpret_cast<Context *>(self);
-    c->dispatch->release(0xFFFFFFFFu);
-    c->combine->release(0xFFFFFFFFu);
+    if (c->dispatch != nullptr) c->dispatch->release(0xFFFFFFFFu);
+    if (c->combine != nullptr) c->combine->release(0xFFFFFFFFu);
     delete c->dispatch;
     delete c->combine;
     Py_TYPE(self)->tp_free(self);

@@ -223,6 +223,7 @@ class AllToAllContext:
         (native/p2p_all_to_all.pyi:13-51) minus `rank` (every call names its
         rank) and the transport handles."""
         lib = load_library()
+        load_extension()   # (a context without it could not be used, nor destroyed by its owner)
         if out_dtype not in SCALAR_TYPE:
             raise RuntimeError(f"unsupported out_dtype {out_dtype}")
         cfg = A2AConfig(

@@ -339,6 +339,26 @@ def test_scales_may_have_more_than_two_dimensions():
             op.dispatch(*(torch.zeros(8) if i == at else v for i, v in enumerate(args)))
 
 
+def test_no_context_is_made_that_the_missing_extension_would_leave_behind(monkeypatch):
+    made = []
+
+    class Library:
+        def __getattr__(self, name):
+            return lambda *args: made.append(name) or 0
+
+    def missing():
+        raise ImportError("_a2a_torch.so is missing")
+
+    monkeypatch.setattr(native, "load_library", Library)
+    monkeypatch.setattr(native, "load_extension", missing)
+    with pytest.raises(ImportError):
+        native.AllToAllContext.create(
+            hidden_dim=128, hidden_dim_scale=None, in_elemsize=2, out_elemsize=2, out_dtype=torch.bfloat16,
+            scale_elemsize=None, max_num_tokens=1, max_recv_tokens=1, max_private_tokens=1, num_experts=2,
+            expert_padding=1, num_experts_per_token=1, dp_size=1, node_size=1, world_size=1, device=0)
+    assert made == []
+
+
 def test_pending_knows_two_collectives():
     context = native.load_extension().Context(0, 3)
     assert context.pending("dispatch") == 0 and context.pending("combine") == 0
