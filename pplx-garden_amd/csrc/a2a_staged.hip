@@ -1554,8 +1554,8 @@ __global__ __launch_bounds__(kPieceThreads) void stage_recv_kernel(const StageRe
 // (a2a_combine_send.cu:124-136,196-205).  Walked in pieces as stage_recv_kernel is, and for the same
 // reason: in the order of arrival the rows written are consecutive per source and the rows read per
 // (source, expert), so both sides are fronts through memory.  16384 rows of 14 KB: 105.5 us = 4.45 TB/s
-// with a wavefront per row, 76.5 us = 6.1 TB/s in this order (a plain copy between two arrays in the
-// same order: 74 us; both sides come from and go to HBM, so loads and stores keep nothing).
+// with a wavefront per row, 76.5 us = 6.1 TB/s in this order (a plain copy of as many rows in the same
+// order, examples/ceilings.hip: 67.6 us; both sides come from and go to HBM, so loads and stores keep nothing).
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(kPieceThreads) void combine_send_kernel(const CombineSendArgs args, const Workspace ws,
                                                                      const Staging st) {

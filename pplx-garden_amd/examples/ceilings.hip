@@ -13,9 +13,11 @@
 //   gather     one wavefront per token and 1 KiB piece: 16 bytes from each of
 //              8 rows of 14336 bytes, summed, 16 bytes out, non-temporal (the
 //              combine's shape); once with the output predicated off
-//   row copy   4096 rows picked through a table and written to rows picked
-//              through another, a wavefront per row: rows of 7392 bytes (what a
-//              rank's split recv moves) and of 14336 bytes (its combine-send)
+//   row copy   a wavefront per 1 KiB piece of a row, all pieces of all rows in
+//              order, rows picked through a table and written one after the
+//              other: rows of 7392 bytes (what a rank's split recv moves, from
+//              the staged rows of its tokens) and of 14336 bytes (its
+//              combine-send, from the experts' rows in order)
 //   1024       push and gather over the first 1024 tokens only
 //   launches   what a dependent launch costs by itself: empty kernels of the library's launch shapes
 //              (with 3.8 KB of arguments by value, as the library's) enqueued behind a kernel that
@@ -136,29 +138,16 @@ __global__ __launch_bounds__(64) void gather(const uint8_t *__restrict__ y, uint
     }
 }
 
-// The split calls' row copies without their tables' meaning: row `from[i]` of `in` goes to row `to[i]`
-// of `out`, one wavefront per row, eight 16-byte pieces per lane in flight.
+// The split calls' row copies without their tables' meaning: row `from[i]` of `in` goes to row i of `out`, a wavefront
+// per piece of 64 chunks of 16 bytes.
 __global__ __launch_bounds__(256) void row_copy(const uint8_t *__restrict__ in, uint8_t *__restrict__ out,
-                                                const uint32_t *__restrict__ from, const uint32_t *__restrict__ to,
-                                                uint32_t rows, uint32_t row_bytes) {
-    const uint32_t row = blockIdx.x * 4 + threadIdx.x / 64, lane = threadIdx.x & 63;
-    if (row >= rows) return;
-    const u32x4 *src = reinterpret_cast<const u32x4 *>(in + (size_t)from[row] * row_bytes);
-    u32x4 *dst = reinterpret_cast<u32x4 *>(out + (size_t)to[row] * row_bytes);
-    const uint32_t chunks = row_bytes / 16;
-    for (uint32_t c0 = 0; c0 < chunks; c0 += 512) {
-        u32x4 v[8];
-#pragma unroll
-        for (uint32_t u = 0; u < 8; ++u) {
-            const uint32_t c = c0 + u * 64 + lane;
-            if (c < chunks) v[u] = __builtin_nontemporal_load(src + c);
-        }
-#pragma unroll
-        for (uint32_t u = 0; u < 8; ++u) {
-            const uint32_t c = c0 + u * 64 + lane;
-            if (c < chunks) dst[c] = v[u];
-        }
-    }
+                                                const uint32_t *__restrict__ from, uint32_t rows, uint32_t row_bytes) {
+    const uint32_t chunks = row_bytes / 16, pieces = (chunks + 63) / 64;
+    const uint32_t unit = blockIdx.x * 4 + threadIdx.x / 64, lane = threadIdx.x & 63;
+    const uint32_t row = unit / pieces, c = (unit - row * pieces) * 64 + lane;
+    if (row >= rows || c >= chunks) return;
+    const u32x4 v = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(in + (size_t)from[row] * row_bytes) + c);
+    store_sc1(v, reinterpret_cast<u32x4 *>(out + (size_t)row * row_bytes) + c);
 }
 
 // Write-only sweep in which each workgroup writes `chunk16` consecutive 16-byte pieces and then
@@ -326,28 +315,25 @@ int main() {
     report("  the gather's output alone, 56 MiB striped fill",
            timer.median_us(fill_other, [&] { hipLaunchKernelGGL(write_sweep, dim3(512), dim3(256), 0, s, (u32x4 *)combined, kTokens * kInRow / 16, 9u); }),
            (double)kTokens * kInRow);
-    // The row copies of the split calls: 4096 rows (what one of 8 ranks receives of a 4096-token step),
-    // sources and destinations each a random permutation of 4096 rows of a buffer that holds them all.
-    std::printf("row copies of the split calls (4096 rows, a wavefront per row), after a 600 MiB read:\n");
-    {
-        std::vector<uint32_t> from(kTokens), to(kTokens);
-        std::iota(from.begin(), from.end(), 0u);
-        std::iota(to.begin(), to.end(), 0u);
-        std::shuffle(from.begin(), from.end(), rng);
-        std::shuffle(to.begin(), to.end(), rng);
-        uint32_t *d_from, *d_to;
-        CHECK(hipMalloc(&d_from, kTokens * sizeof(uint32_t)));
-        CHECK(hipMalloc(&d_to, kTokens * sizeof(uint32_t)));
-        CHECK(hipMemcpy(d_from, from.data(), kTokens * sizeof(uint32_t), hipMemcpyHostToDevice));
-        CHECK(hipMemcpy(d_to, to.data(), kTokens * sizeof(uint32_t), hipMemcpyHostToDevice));
-        for (uint32_t row_bytes : {7392u, 14336u}) {   // inside y (4096 x 8 rows of 14336 bytes) and big_b
+    // The row copies of the split calls: 4096 and 16384 rows (what one of 8 ranks receives of a step of 4096 and of
+    // 8 x 2048 tokens); y holds 32768 rows of 14336 bytes and big_b 512 MiB, more than either shape needs.
+    std::printf("row copies of the split calls (a wavefront per piece, in order), after a 600 MiB read:\n");
+    for (uint32_t rows : {4096u, 16384u}) {
+        std::vector<uint32_t> from(rows);
+        uint32_t *d_from;
+        CHECK(hipMalloc(&d_from, rows * sizeof(uint32_t)));
+        for (uint32_t row_bytes : {7392u, 14336u}) {
+            std::iota(from.begin(), from.end(), 0u);
+            if (row_bytes == 7392u) std::shuffle(from.begin(), from.end(), rng);
+            CHECK(hipMemcpy(d_from, from.data(), rows * sizeof(uint32_t), hipMemcpyHostToDevice));
+            const uint32_t units = rows * ((row_bytes / 16 + 63) / 64);
             char name[96];
-            std::snprintf(name, sizeof name, "  rows of %u bytes, read and written", row_bytes);
+            std::snprintf(name, sizeof name, "  %u rows of %u bytes, read and written", rows, row_bytes);
             report(name, timer.median_us(read_other, [&] {
-                       hipLaunchKernelGGL(row_copy, dim3(kTokens / 4), dim3(256), 0, s, (const uint8_t *)y, big_b,
-                                          (const uint32_t *)d_from, (const uint32_t *)d_to, kTokens, row_bytes);
+                       hipLaunchKernelGGL(row_copy, dim3((units + 3) / 4), dim3(256), 0, s, (const uint8_t *)y, big_b,
+                                          (const uint32_t *)d_from, rows, row_bytes);
                    }),
-                   2.0 * kTokens * row_bytes);
+                   2.0 * rows * row_bytes);
         }
     }
 
