@@ -77,7 +77,7 @@ def kernel_sources_sha256() -> str:
 def measured_traffic():
     """HBM bytes per launch from the hardware-counter summary under profiles/, or {} when that
     summary was taken on other kernel sources than the ones this run uses (then it says nothing
-    about this build)."""
+    about them)."""
     try:
         text = TRAFFIC_PROFILE.read_text()
     except OSError:
@@ -89,7 +89,7 @@ def measured_traffic():
     # the other shapes of the baseline: lines "traffic_bytes_<shape>: <kernel>=<bytes>"
     for m in re.finditer(r"^traffic_bytes_(\w+):\s*(\w+)\s*=\s*(\d+)\s*$", text, flags=re.M):
         out.setdefault(m.group(1), {})[m.group(2)] = int(m.group(3))
-    return out, f"FETCH_SIZE and WRITE_SIZE passes of this build, profiles/{TRAFFIC_PROFILE.name}"
+    return out, f"FETCH_SIZE and WRITE_SIZE passes of these kernel sources, profiles/{TRAFFIC_PROFILE.name}"
 
 
 class Workload:
@@ -279,9 +279,9 @@ def time_graph_replay(wl: Workload, steps: int, warmup: int):
 def time_gpu_pace(wl: Workload, batches: int = 5, steps_each: int = 100, step_fn=None):
     """The GPU's own pace per step: `steps_each` steps are enqueued behind a kernel that holds the queue
     for a few milliseconds, so the host is ahead of the GPU for all of them, and two events around them
-    give the time the GPU took.  For steps of about 10 us the host's share of a step (two calls through
-    ctypes and the launches behind them, 7 to 10 us on this pool's hosts) is of the same size as the
-    GPU's, and the wall time of a loop then says which host the box has.  Returns the median over
+    give the time the GPU took.  For steps of about 10 us the host's share of a step (two calls and the
+    launches behind them, 7 to 10 us depending on the host) is of the same size as the GPU's, and the
+    wall time of a loop then says which host the machine has.  Returns the median over
     `batches` in microseconds, or None where torch has no such kernel."""
     import torch
     hold = getattr(torch.cuda, "_sleep", None)
@@ -851,8 +851,8 @@ def main() -> int:
                           "events the launches record themselves, the p50 figures from events around the calls "
                           "of every step (each event adds about 3 us); step_us_gpu_pace is the time per step "
                           "between two events when the steps are enqueued behind a kernel that holds the queue, "
-                          "i.e. with the host ahead of the GPU (the host's share of such a step, two calls "
-                          "through ctypes and their launches, is 7-10 us on this pool's hosts)")
+                          "i.e. with the host ahead of the GPU (the host's share of such a step, two group calls "
+                          "and their launches, is of the same size)")
         qwen = other_shape(C1, device, args.routings, side_steps, args.warmup, ctx_flags, qwen_label)
         kimi = other_shape(C4, device, args.routings, side_steps, args.warmup, ctx_flags, kimi_label, bar_us=37.0)
         kimi_d, kimi_c = algorithmic_bytes(C4.num_tokens, C4.hidden_dim, C4.topk)

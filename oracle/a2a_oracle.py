@@ -3,7 +3,7 @@
 This module restates, in numpy, the algorithm of the reference's p2p-all-to-all
 path so that the HIP kernels can be checked against it.  Nothing in the product
 package may import it: only tests, the smoke check and the benchmark's
-CPU-baseline leg do, and only as the checker.
+CPU-baseline leg do, and only to compare with.
 
 Every function cites the reference file:line it follows (paths relative to the
 reference checkout).  Where the reference leaves something open the choice made

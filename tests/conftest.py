@@ -10,7 +10,7 @@ for p in (REPO, REPO / "pplx-garden_amd", REPO / "pplx-garden_amd" / "benchmarks
 
 
 def pytest_configure(config):
-    config.addinivalue_line("markers", "gpu: needs a real MI355X (run with -m gpu on the GPU box)")
+    config.addinivalue_line("markers", "gpu: needs a real MI355X (run with -m gpu where there is one)")
 
 
 def _has_gpu() -> bool:
