@@ -492,7 +492,12 @@ int launch_dispatch_group(a2a_ctx *ctx, const a2a_config &c, const Workspace &ws
     const uint32_t blocks = plan.blocks, tokens = plan.tokens;
     const uint32_t G = c.world_size / c.dp_size;
     hipError_t e;
-    if (!(c.flags & A2A_FLAG_SEPARATE_ROUTING) && dispatch_small_fits(pa, ws, quantize != 0, tokens)) {
+    const bool past_cache = copies_past_cache((uint64_t)tokens * c.num_experts_per_token * row_bytes_of(c), quantize != 0,
+                                              c.num_experts_per_token);
+    if (!(c.flags & A2A_FLAG_SEPARATE_ROUTING) && !past_cache && dispatch_sources_fits(pa, ws, quantize != 0, tokens)) {
+        e = launch_dispatch_sources(pa, fa, ws, quantize != 0, tokens, s, pack_timing);
+        if (e != hipSuccess) return hip_fail(ctx, e, "launch dispatch_sources");
+    } else if (!(c.flags & A2A_FLAG_SEPARATE_ROUTING) && dispatch_small_fits(pa, ws, quantize != 0, tokens)) {
         e = launch_dispatch_small(pa, fa, ws, quantize != 0, tokens, s, pack_timing);
         if (e != hipSuccess) return hip_fail(ctx, e, "launch dispatch_small");
     } else if (!(c.flags & A2A_FLAG_SEPARATE_ROUTING) && dispatch_single_fits(pa, ws, quantize != 0, tokens)) {
@@ -515,8 +520,7 @@ int launch_dispatch_group(a2a_ctx *ctx, const a2a_config &c, const Workspace &ws
         // workgroups resolve their own rows from them.
         e = launch_route_accumulate(ra, ws, blocks, s, false, route_timing);
         if (e != hipSuccess) return hip_fail(ctx, e, "launch route_hist (accumulating)");
-        streamed = copies_past_cache((uint64_t)tokens * c.num_experts_per_token * row_bytes_of(c), quantize != 0,
-                                     c.num_experts_per_token);
+        streamed = past_cache;
         e = launch_dispatch_resolve(pa, fa, ws, quantize != 0, tokens, streamed, s, pack_timing);
         if (e != hipSuccess) return hip_fail(ctx, e, "launch dispatch_resolve");
     }

@@ -8,6 +8,16 @@ namespace a2a {
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
+// A pointer to memory made from an address that travelled as a number.  Through an ordinary pointer the compiler makes
+// flat accesses of it, which count as LDS operations too: every wait for LDS then waits for them.
+template <typename T>
+using global_t = __attribute__((address_space(1))) T;
+
+template <typename T>
+__device__ __forceinline__ global_t<T> *global_ptr(uint64_t address) {
+    return reinterpret_cast<global_t<T> *>(address);
+}
+
 // A barrier for data that wavefronts of a workgroup hand to each other through LDS: it waits for this
 // wavefront's LDS operations only.  Loads from memory that were asked for earlier stay in flight across
 // it (in front of its own barrier the compiler may wait for every outstanding access to memory).

@@ -1578,6 +1578,435 @@ __global__ __launch_bounds__(1024) void dispatch_teams_kernel(const PushArgs arg
     duties();
 }
 
+// The same division of labour again for steps of SEVERAL sources (up to kSourcesMaxEntries entries with dense index
+// rows, at most eight routes a token), and for steps of one that are too large for the kernel above.  Workgroup 0
+// writes the step's tables, every other one sends up to `per_group` tokens of one source.
+//
+// Such steps are bound by what stands in front of the first row: the general one-launch kernel looks every entry's
+// source up in a table that takes a trip to memory to build and scans all experts with workgroup barriers, and the two
+// launches of larger steps pay a dependent launch and the pack's own look-ups.  us per dispatch at the GPU's own pace,
+// before (general kernel below 3 * 2^19 visits, two launches above) and with this kernel:
+//   8 ranks x 1 token, hidden 7168    8.24 -> 4.67      4 ranks x 64 tokens, hidden 2048, K = 4   7.87 -> 3.77
+//   8 x 16 / 32 / 64 tokens           8.80 -> 4.92 / 9.94 -> 5.95 / 13.95 -> 9.45
+//   8 x 128 (207 MB with the combine) 22.4 -> 15.6 (one source of as many tokens: 15.4)
+//   8 x 192 / 256 tokens              27.0 -> 23.8 / 35.5 -> 30.4
+//   one source of 1100 / 1500 / 2048  23.3 -> 19.3 / 26.3 -> 23.9 / 38.5 -> 35.4
+//   bf16 rows of 8 KB, 8 x 64 / 128   15.2 -> 8.9 / 21.8 -> 15.1
+// Copies go out at device scope, quantised or not (rows of 8 KB, 8 x 128 tokens, ordinary stores: 1.6 us more a step,
+// and 0.5 us more with a sweep in between that reads the received rows).
+//
+// What a route needs of the other sources is how many of their copies lie in front of its own in the receiver's run of
+// rows, and that is one bit per (receiver, other source): whether the receiver lays that source out before mine.  So a
+// token workgroup still keeps ONE word per expert: its low half counts every entry of the step, its high half those
+// that come before the workgroup's first (earlier entries of my source, and all entries of a source that the expert's
+// receiver lays out before mine).  Which of the two a source's entries are is the same for a wavefront's whole chunk of
+// entries up to the receiver, a bit in a mask that the chunk's wavefront holds in scalar registers.  A second table
+// counts the earlier entries of my own source alone (token_offset), an atomic for few of the entries.
+//
+// Workgroup 0 counts per (source, expert) and then writes, a wavefront per job, each receiver's layout and each
+// source's totals: done by workgroups that also send tokens these would need that larger table too.
+//
+// The sources' descriptors are held by the lanes of every wavefront (lane g: source g), so that whoever needs one picks
+// it without another trip to the argument block.  A wavefront counts chunks w, w + counting wavefronts, ... of the
+// sources' entries and moves units (64 pieces of 16 bytes of a copy) u, u + counting wavefronts, ... of the workgroup's
+// rows; both are asked for at the head.
+//
+// Dynamic LDS: max(G, 2) * E words.
+struct SourcesPlan {
+    uint32_t units;          // units of a row
+    uint32_t units_magic;    // ceil(2^32 / units) (0 for one)
+    uint32_t per_group;      // tokens of a workgroup
+    uint32_t chunks;         // of the entries of all sources
+};
+constexpr uint32_t kSourcesMaxEntries = 16384;
+constexpr uint32_t kSourcesChunk = 4 * kWave;    // entries that a wavefront asks for with four loads
+constexpr uint32_t kSourcesMaxTokens = 8;        // of a workgroup
+constexpr uint32_t kSourcesMaxRoutes = 64;
+constexpr uint32_t kSourcesMaxScales = 128;
+constexpr uint32_t kSourcesMaxTable = 12288;     // words of dynamic LDS
+static_assert(sizeof(PushArgs) + sizeof(FinalizeArgs) + sizeof(Workspace) + sizeof(SourcesPlan) <= 4096, "kernel arguments too large");
+
+template <uint32_t NC, uint32_t ROUNDS, bool QUANT>
+__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8))) void dispatch_sources_kernel(
+    const PushArgs args, const FinalizeArgs fin, const Workspace ws, const SourcesPlan plan) {
+    extern __shared__ uint32_t s_cnt[];   // token workgroups: [E] counts, [E] earlier entries of my source; workgroup 0: [G][E]
+    __shared__ float s_scale[kSourcesMaxTokens][kSourcesMaxScales];
+    __shared__ uint64_t s_row_ptr[kSourcesMaxRoutes];
+    __shared__ uint64_t s_scale_ptr[kSourcesMaxRoutes];
+    __shared__ uint32_t s_scale_stride[kSourcesMaxRoutes];
+    __shared__ uint32_t s_route_expert[kSourcesMaxRoutes];
+    __shared__ uint32_t s_counted;        // counting wavefronts whose entries are in the table
+
+    const uint32_t tid = threadIdx.x;
+    const uint32_t lane = tid & (kWave - 1);
+    // Lane g of every wavefront holds source g (beyond the last source: no tokens, and a start behind every workgroup).
+    const bool is_source = lane < (uint32_t)kMaxWorld;
+    const PushSrc &from = args.src[lane & (kMaxWorld - 1)];
+    uint64_t src_x = (uint64_t)from.x, src_x_stride = from.x_stride, src_ids = (uint64_t)from.indices;
+    uint64_t src_bound = (uint64_t)from.bound_m;
+    uint32_t src_tokens = from.num_tokens, src_start = args.token_start[lane & (kMaxWorld - 1)];
+    const uint32_t nthreads = blockDim.x;
+    A2A_PIN(nthreads);
+    A2A_PIN(args.hidden_dim);
+    A2A_PIN(args.hidden_dim_scale);
+    A2A_PIN(args.row_bytes);
+    A2A_PIN(args.topk_magic);
+    A2A_PIN(ws.world);
+    A2A_PIN(ws.num_groups);
+    A2A_PIN(ws.num_experts);
+    A2A_PIN(ws.topk);
+    A2A_PIN(ws.experts_per_rank);
+    A2A_PIN(ws.le_magic);
+    A2A_PIN(ws.expert_padding);
+    A2A_PIN(ws.max_tk);
+    A2A_PIN(ws.laid_before);
+    A2A_PIN(ws.route_slot);
+    A2A_PIN(ws.token_offset);
+    A2A_PIN(ws.err);
+    A2A_PIN(plan.units);
+    A2A_PIN(plan.units_magic);
+    A2A_PIN(plan.per_group);
+    A2A_PIN(plan.chunks);
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid / kWave));
+    const uint32_t waves = nthreads / kWave;
+    const uint32_t movers = waves - 1;                 // wavefronts of a token workgroup that count and move rows
+    const uint32_t G = ws.num_groups, E = ws.num_experts, K = ws.topk, Le = ws.experts_per_rank;
+    const uint32_t pad = ws.expert_padding;
+    const uint32_t num_chunks = QUANT ? args.hidden_dim / 16 : args.row_bytes / 16;   // 16-byte pieces of a copy
+    const uint32_t Hs = args.hidden_dim_scale;
+    auto of_lane = [](uint32_t v, uint32_t l) { return (uint32_t)__builtin_amdgcn_readlane((int)v, (int)l); };
+
+    // (waited for here, all at once, so that none of the loads below waits for the one before it)
+    asm volatile("" : "+v"(src_x), "+v"(src_x_stride), "+v"(src_ids), "+v"(src_bound), "+v"(src_tokens), "+v"(src_start));
+    if (!is_source) src_tokens = 0;
+    if (!is_source) src_start = 0xFFFFFFFFu;
+    const uint32_t src_entries = src_tokens * K;
+    const uint32_t src_chunks = (src_entries + kSourcesChunk - 1) / kSourcesChunk;
+    const uint32_t src_first_chunk = wave_inclusive_scan(src_chunks, lane) - src_chunks;
+    auto source_of_chunk = [&](uint32_t c) {   // uniform
+        return 63u - (uint32_t)__builtin_clzll(__ballot(src_tokens != 0 && src_first_chunk <= c));
+    };
+
+    // my source: the last one that starts at or before this workgroup (workgroup 0: any)
+    const uint32_t my_g = blockIdx.x == 0 ? 0 : 63u - (uint32_t)__builtin_clzll(__ballot(src_start <= blockIdx.x));
+    const uint32_t first_token = (blockIdx.x - of_lane(src_start, my_g)) * plan.per_group;
+    const uint32_t my_tokens = of_lane(src_tokens, my_g);
+    const uint64_t my_ids = read_lane64(src_ids, my_g);
+    const uint32_t my_first = first_token * K;           // my first entry, counted in its source
+    const uint32_t routes = plan.per_group * K;          // <= kSourcesMaxRoutes
+
+    // lanes of the resolver per route: 8, 4, 2 or 1
+    const uint32_t lpr_log = routes <= 8 ? 3 : routes <= 16 ? 2 : routes <= 32 ? 1 : 0;
+    const uint32_t lpr = 1u << lpr_log;
+    const uint32_t part = lane & (lpr - 1), route = lane >> lpr_log;
+
+    // lane r: the sources that receiver r lays out before mine
+    const uint32_t laid = ws.laid_before[(lane < ws.world ? lane : 0) * G + my_g];
+    auto load_chunk = [&](uint32_t c, uint32_t (&id)[4]) {
+        const uint32_t g = source_of_chunk(c);
+        const uint32_t first = (c - of_lane(src_first_chunk, g)) * kSourcesChunk;
+        const uint32_t last = of_lane(src_entries, g) - 1;
+        const global_t<const uint32_t> *p = global_ptr<const uint32_t>(read_lane64(src_ids, g));
+#pragma unroll
+        for (uint32_t q = 0; q < 4; ++q) {
+            const uint32_t o = first + q * kWave + lane;
+            id[q] = p[o < last ? o : last];
+        }
+    };
+    // (without a condition around any of them: a chunk that is not there asks for the last one and is not counted)
+    auto load_chunks = [&](uint32_t counting, uint32_t (&ids)[NC][4]) {
+#pragma unroll
+        for (uint32_t j = 0; j < NC; ++j) {
+            const uint32_t c = wave + j * counting;
+            load_chunk(c < plan.chunks ? c : plan.chunks - 1, ids[j]);
+        }
+    };
+    // every chunk this wavefront counts: those asked for already, then the rest
+    auto count_chunks = [&](uint32_t counting, const uint32_t (&ids)[NC][4], auto count_chunk) {
+#pragma unroll
+        for (uint32_t j = 0; j < NC; ++j) {
+            const uint32_t c = wave + j * counting;
+            count_chunk(c < plan.chunks ? c : plan.chunks - 1, c < plan.chunks, ids[j]);
+        }
+        for (uint32_t c = wave + NC * counting; c < plan.chunks; c += counting) {
+            uint32_t id[4];
+            load_chunk(c, id);
+            count_chunk(c, true, id);
+        }
+    };
+    uint32_t src_live = src_tokens;
+    auto apply_bounds = [&]() {
+        if (src_bound != 0) {
+            const int32_t bound = *global_ptr<const int32_t>(src_bound);
+            const uint32_t most = bound < 0 ? 0 : (uint32_t)bound;
+            src_live = most < src_tokens ? most : src_tokens;
+        }
+    };
+    auto clear_table = [&](uint32_t words) {
+        for (uint32_t i = tid; i < words; i += nthreads) s_cnt[i] = 0;
+        if (tid == 0) s_counted = 0;
+        lds_barrier();
+    };
+
+    // The three kinds of wavefront each have their whole chain to themselves: where two paths meet, the compiler waits
+    // for what either of them may have asked for.
+    if (blockIdx.x == 0) {
+        // ---- the step's tables, a wavefront per job
+        uint32_t ids[NC][4];
+        load_chunks(waves, ids);
+        // lane i: the i-th source that receiver r lays out
+        auto order_of = [&](uint32_t r) {
+            return ws.order[r * (kMaxWorld / 4) + (lane & (kMaxWorld - 1)) / 4] >> (8 * (lane & 3)) & 0xFFu;
+        };
+        const uint32_t first_order = order_of(wave < ws.world ? wave : 0);
+        apply_bounds();
+        clear_table(G * E);
+        count_chunks(waves, ids, [&](uint32_t c, bool there, const uint32_t (&id)[4]) {
+            const uint32_t g = source_of_chunk(c);
+            const uint32_t first = (c - of_lane(src_first_chunk, g)) * kSourcesChunk;
+            const uint32_t live = there ? of_lane(src_live, g) * K : 0;
+#pragma unroll
+            for (uint32_t q = 0; q < 4; ++q) {
+                const uint32_t x = id[q];
+                if (first + q * kWave + lane < live && x < E) atomicAdd(&s_cnt[g * E + x], 1u);
+            }
+        });
+        lds_barrier();
+        for (uint32_t job = wave; job < ws.world + G; job += waves) {
+            uint32_t upto = 0;
+            if (job < ws.world) {
+                const uint32_t r = job;
+                if (!(fin.recv_mask >> r & 1)) continue;
+                int32_t *const out_tokens = fin.out_num_tokens[r];
+                const uint32_t out_rows = fin.out_rows[r];
+                const uint32_t order = r == wave ? first_order : order_of(r);
+                for (uint32_t l0 = 0; l0 < Le; l0 += kWave) {
+                    const uint32_t l = l0 + lane, e = r * Le + l;
+                    const bool valid = l < Le && e < E;
+                    uint32_t count = 0;
+                    for (uint32_t g = 0; g < G; ++g) count += valid ? s_cnt[g * E + e] : 0;
+                    const uint32_t padded = pad > 1 ? (count + pad - 1) / pad * pad : count;
+                    const uint32_t incl = upto + wave_inclusive_scan(padded, lane);
+                    uint32_t row = incl - padded;
+                    if (valid) {
+                        ws.tokens_per_expert[e] = count;
+                        ws.padded_offset[e] = row;
+                        if (out_tokens != nullptr) out_tokens[l] = (int32_t)count;
+                        if (row + count > out_rows) atomicOr(ws.err, A2A_DEV_RECV_OVERFLOW);
+                    }
+                    for (uint32_t i = 0; i < G; ++i) {   // the sources in the order the receiver lays them out
+                        const uint32_t g = of_lane(order, i);
+                        if (valid) {
+                            ws.slot_base[g * E + e] = row;
+                            row += s_cnt[g * E + e];
+                        }
+                    }
+                    upto = of_lane(incl, kWave - 1);
+                }
+            } else {
+                const uint32_t g = job - ws.world;
+                for (uint32_t e0 = 0; e0 < E; e0 += kWave) {
+                    const uint32_t e = e0 + lane;
+                    const uint32_t count = e < E ? s_cnt[g * E + e] : 0;
+                    const uint32_t incl = upto + wave_inclusive_scan(count, lane);
+                    if (e < E) {
+                        ws.num_routed[g * E + e] = count;
+                        ws.expert_offsets[g * E + e] = incl;
+                    }
+                    upto = of_lane(incl, kWave - 1);
+                }
+            }
+        }
+        return;
+    }
+
+    if (wave != movers) {
+        // ---- counts entries and moves rows
+        uint32_t ids[NC][4];
+        load_chunks(movers, ids);
+        // the units' rows (zeros, without an access, where there is none)
+        u32x4 a[ROUNDS], b[ROUNDS];
+        uint32_t unit_token[ROUNDS], unit_piece[ROUNDS];   // uniform
+        const uint64_t x = read_lane64(src_x, my_g), x_stride = read_lane64(src_x_stride, my_g);
+#pragma unroll
+        for (uint32_t rd = 0; rd < ROUNDS; ++rd) {
+            const uint32_t u = wave + rd * movers;
+            unit_token[rd] = plan.units_magic != 0 ? __umulhi(u, plan.units_magic) : u;
+            unit_piece[rd] = u - unit_token[rd] * plan.units;
+            const uint32_t t = first_token + unit_token[rd];
+            const bool there = unit_token[rd] < plan.per_group && t < my_tokens;
+            const uint64_t row = x + (uint64_t)(there ? t : 0) * x_stride;
+            const uint32_t bytes = there ? num_chunks * (QUANT ? 32 : 16) : 0;
+            const uint32_t offset = (unit_piece[rd] * kWave + lane) * (QUANT ? 32 : 16);
+            a[rd] = load_row_chunk<kNonTemporal>(row, bytes, offset);
+            if constexpr (QUANT) b[rd] = load_row_chunk<kNonTemporal>(row, bytes, offset + 16);
+        }
+        apply_bounds();
+        const uint32_t live_tokens = of_lane(src_live, my_g);
+        clear_table(2 * E);
+
+        count_chunks(movers, ids, [&](uint32_t c, bool there, const uint32_t (&id)[4]) {
+            const uint32_t g = source_of_chunk(c);
+            const uint32_t first = (c - of_lane(src_first_chunk, g)) * kSourcesChunk;
+            const uint32_t live = there ? of_lane(src_live, g) * K : 0;
+            if (g == my_g) {   // uniform
+#pragma unroll
+                for (uint32_t q = 0; q < 4; ++q) {
+                    const uint32_t o = first + q * kWave + lane;
+                    const bool counts = o < live && id[q] < E;
+                    if (counts) atomicAdd(&s_cnt[id[q]], o < my_first ? 0x10001u : 1u);
+                    if (counts && o < my_first) atomicAdd(&s_cnt[E + id[q]], 1u);
+                }
+            } else {
+                // bit r: receiver r lays this source out before mine
+                const uint32_t ahead = (uint32_t)__ballot(lane < ws.world && (laid >> g & 1));
+#pragma unroll
+                for (uint32_t q = 0; q < 4; ++q) {
+                    const uint32_t before = ahead >> (owner_of_expert(ws, id[q]) & (kMaxWorld - 1)) & 1;
+                    if (first + q * kWave + lane < live && id[q] < E) atomicAdd(&s_cnt[id[q]], 1u | before << 16);
+                }
+            }
+        });
+        // this wavefront's entries are in the table before its arrival is counted
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        if (lane == 0) atomicAdd(&s_counted, 1u);
+        if (first_token >= live_tokens) return;   // nothing to send (uniform; the resolver does not wait at the barrier either)
+        const PushSrc &src = args.src[my_g];
+        const bool scaled = QUANT || src.x_scale != nullptr;
+        if constexpr (QUANT) {
+#pragma unroll
+            for (uint32_t rd = 0; rd < ROUNDS; ++rd) {
+                float scale;
+                a[rd] = quantize16(a[rd], b[rd], &scale);
+                const uint32_t piece = unit_piece[rd] * kWave + lane;
+                if (unit_token[rd] < plan.per_group && piece < num_chunks && (lane & 7) == 0) {
+                    s_scale[unit_token[rd]][piece / 8] = scale;
+                }
+            }
+        } else if (scaled) {
+            // the caller's scales of my tokens, a wavefront per token
+            for (uint32_t i = wave; i < plan.per_group; i += movers) {
+                const uint32_t t = first_token + i < my_tokens ? first_token + i : my_tokens - 1;
+                const float *xs = src.x_scale + (size_t)t * src.xs_stride_token;
+                for (uint32_t j = lane; j < Hs; j += kWave) s_scale[i][j] = xs[(size_t)j * src.xs_stride_elem];
+            }
+        }
+        lds_barrier();
+#pragma unroll
+        for (uint32_t rd = 0; rd < ROUNDS; ++rd) {
+            const uint32_t i = unit_token[rd];
+            if (i >= plan.per_group || first_token + i >= live_tokens) continue;   // uniform
+            const uint64_t row_ptr = lane < K ? s_row_ptr[i * K + lane] : 0;
+            store_copies<kDeviceScope>(a[rd], row_ptr, K, num_chunks * 16, (unit_piece[rd] * kWave + lane) * 16);
+        }
+        // each copy's scale row goes out as one contiguous run, a wavefront per copy
+        if (!scaled) return;
+        for (uint32_t p = wave; p < routes; p += movers) {
+            const uint64_t to = s_scale_ptr[p];
+            const uint32_t stride = s_scale_stride[p];
+            if (to == 0) continue;
+            const uint32_t i = K > 1 ? __umulhi(p, args.topk_magic) : p;
+            for (uint32_t j = lane; j < Hs; j += kWave) global_ptr<float>(to)[(size_t)j * stride] = s_scale[i][j];
+        }
+        return;
+    }
+
+    // ---- the resolver
+    // (it shares its SIMD with wavefronts that quantise while the routes are resolved, and the routes are what every
+    // wavefront of the workgroup waits for)
+    __builtin_amdgcn_s_setprio(3);
+    const uint32_t flat = my_first + (route < routes ? route : 0), last_entry = my_tokens * K - 1;
+    const uint32_t id_route = global_ptr<const uint32_t>(my_ids)[flat < last_entry ? flat : last_entry];
+    const PushDst &dst_of_lane = args.dst[lane < ws.world ? lane : 0];
+    const uint64_t my_out_x = (uint64_t)dst_of_lane.out_x, my_out_scale = (uint64_t)dst_of_lane.out_scale;
+    const uint64_t my_out_stride = dst_of_lane.out_stride;
+    const uint32_t my_os_elem = dst_of_lane.os_stride_elem, my_os_token = dst_of_lane.os_stride_token;
+    const uint32_t my_out_rows = dst_of_lane.out_rows;
+    apply_bounds();
+    const uint32_t live_tokens = of_lane(src_live, my_g);
+    clear_table(2 * E);
+    auto group_sum = [&](uint32_t v) {
+        if (lpr_log >= 1) v += dpp_move_u32<0xB1>(v);    // quad_perm [1,0,3,2]
+        if (lpr_log >= 2) v += dpp_move_u32<0x4E>(v);    // quad_perm [2,3,0,1]
+        if (lpr_log >= 3) v += dpp_move_u32<0x141>(v);   // row_half_mirror
+        return v;
+    };
+    const bool in = route < routes && my_first + route < live_tokens * K;
+    const bool route_live = in && id_route < E;
+    const uint32_t e = route_live ? id_route : 0;
+    const uint32_t r = owner_of_expert(ws, e);
+    const uint32_t le = e - r * Le;
+    // copies of my tokens to the same expert at an earlier route of the workgroup
+    if (part == 0 && route < kSourcesMaxRoutes) s_route_expert[route] = in ? id_route : 0xFFFFFFFFu;
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    uint32_t earlier = 0;
+    for (uint32_t qd = part; qd < route && qd < kSourcesMaxRoutes; qd += lpr) earlier += s_route_expert[qd] == id_route ? 1u : 0u;
+    earlier = group_sum(earlier);
+    PushDst dst;
+    dst.out_x = reinterpret_cast<uint8_t *>(__shfl(my_out_x, (int)r));
+    dst.out_scale = reinterpret_cast<float *>(__shfl(my_out_scale, (int)r));
+    dst.out_stride = __shfl(my_out_stride, (int)r);
+    dst.os_stride_elem = __shfl(my_os_elem, (int)r);
+    dst.os_stride_token = __shfl(my_os_token, (int)r);
+    dst.out_rows = __shfl(my_out_rows, (int)r);
+    dst.pad_ = 0;
+
+    // until the counting wavefronts have all said that their entries are in the table (at the lowest
+    // priority: the wavefronts that share this SIMD are among those waited for)
+    __builtin_amdgcn_s_setprio(0);
+    for (uint32_t spins = 0; __hip_atomic_load(&s_counted, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) != movers;) {
+        if (++spins == kQuickSpinLimit) {
+            if (lane == 0) atomicOr(ws.err, A2A_DEV_INTERNAL);
+            break;
+        }
+    }
+    __builtin_amdgcn_s_setprio(3);
+    asm volatile("" ::: "memory");
+    if (first_token >= live_tokens) return;   // nothing to send (uniform)
+
+    // padded rows of the receiver's experts before mine: four terms per lane without a branch (clamped index, masked
+    // value), the rest in a loop
+    const uint32_t mine = s_cnt[e], own = s_cnt[E + e];
+    uint32_t v_rows[4];
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) {
+        const uint32_t n = part + lpr * i;
+        v_rows[i] = s_cnt[r * Le + (n < le ? n : 0)] & 0xFFFFu;
+    }
+    uint32_t base = 0;
+    if (pad > 1) {   // uniform
+#pragma unroll
+        for (uint32_t i = 0; i < 4; ++i) base += part + lpr * i < le ? (v_rows[i] + pad - 1) / pad * pad : 0;
+        for (uint32_t n = 4 * lpr + part; n < le; n += lpr) base += ((s_cnt[r * Le + n] & 0xFFFFu) + pad - 1) / pad * pad;
+    } else {
+#pragma unroll
+        for (uint32_t i = 0; i < 4; ++i) base += part + lpr * i < le ? v_rows[i] : 0;
+        for (uint32_t n = 4 * lpr + part; n < le; n += lpr) base += s_cnt[r * Le + n] & 0xFFFFu;
+    }
+    base = group_sum(base);
+    const uint32_t toff = route_live ? own + earlier : 0;
+    uint64_t to_row, to_scale;
+    uint32_t to_stride;
+    uint32_t slot = resolve_copy(dst, ws, base + (mine >> 16) + earlier, part == 0 && route_live, &to_row, &to_scale, &to_stride);
+    if (!route_live) {
+        slot = kInvalidSlot;
+        to_row = 0;
+        to_scale = 0;
+        to_stride = 0;
+    }
+    if (part == 0 && route < routes) {
+        s_row_ptr[route] = to_row;
+        s_scale_ptr[route] = to_scale;
+        s_scale_stride[route] = to_stride;
+    }
+    lds_barrier();
+    if (part == 0 && in) {
+        if (!route_live) atomicOr(ws.err, A2A_DEV_BAD_EXPERT_ID);
+        ws.route_slot[(size_t)my_g * ws.max_tk + my_first + route] = slot;
+        ws.token_offset[(size_t)my_g * ws.max_tk + my_first + route] = toff;
+    }
+}
+
 // Pack of a large group step, after a routing launch that left, per chunk, the
 // histogram and the rank of every entry inside its chunk, and, for the whole
 // step, the totals per (source, expert) and per expert.  No launch in between
@@ -1926,6 +2355,89 @@ hipError_t launch_dispatch_single(const PushArgs &args, const FinalizeArgs &fin,
         hipExtLaunchKernelGGL(dispatch_single_kernel<false>, dim3(blocks), dim3(threads), lds, stream, timing.start,
                               timing.stop, 0, a, fin, ws, team, per_group);
     }
+    return hipGetLastError();
+}
+
+// Whether a step takes dispatch_sources_kernel, and its shape: tokens of a workgroup as in the kernels of one source
+// (about one workgroup per compute unit); beside the resolver as many wavefronts as there are units to move or chunks
+// to count (8 x 32 tokens of hidden 2048, 2 units and 8 chunks: 6.6 us with 4 wavefronts, 4.6 with 8), in as few rounds
+// as 15 of them need.  The line at 16384 entries: counting costs every workgroup 0.16 us per 1024 of them, where the
+// routing launch it replaces costs 5 to 6 us, and with more than eight tokens of top-8 a workgroup has more routes than
+// its resolver has lanes.  Steps of one source with up to
+// kSingleMaxEntries entries have the two kernels that are made for them (128 tokens 4.54 us against 4.77 here, 1024
+// tokens 15.4 against 16.1).
+bool plan_dispatch_sources(const PushArgs &args, const Workspace &ws, bool quantize, uint32_t total_tokens, SourcesPlan &plan,
+                           uint32_t &groups, uint32_t &threads, uint32_t &rounds) {
+    constexpr uint32_t kComputeUnits = 256;
+    const uint64_t entries = (uint64_t)total_tokens * ws.topk;
+    if (total_tokens == 0 || ws.topk > 8 || entries > kSourcesMaxEntries) return false;
+    if ((uint64_t)ws.num_groups * ws.num_experts > kSourcesMaxTable || args.hidden_dim_scale > kSourcesMaxScales ||
+        (quantize && args.hidden_dim / 128 > kSourcesMaxScales))
+        return false;
+    const uint32_t pieces = quantize ? args.hidden_dim / 16 : args.row_bytes / 16;
+    plan.units = (pieces + kWave - 1) / kWave;
+    plan.units_magic = plan.units > 1 ? 0xFFFFFFFFu / plan.units + 1 : 0;
+    plan.per_group = (total_tokens + kComputeUnits - 1) / kComputeUnits;
+    if (plan.per_group > kSourcesMaxTokens || plan.per_group * ws.topk > kSourcesMaxRoutes) return false;
+    plan.chunks = 0;
+    groups = 0;
+    uint32_t senders = 0;
+    for (uint32_t g = 0; g < ws.num_groups; ++g) {
+        if (args.src[g].num_tokens == 0) continue;
+        if (args.src[g].indices_stride != ws.topk) return false;
+        ++senders;
+        plan.chunks += (args.src[g].num_tokens * ws.topk + kSourcesChunk - 1) / kSourcesChunk;
+        groups += (args.src[g].num_tokens + plan.per_group - 1) / plan.per_group;
+    }
+    if (senders == 1 && entries <= kSingleMaxEntries) return false;
+    const uint32_t units = plan.per_group * plan.units;
+    uint32_t movers = units;
+    if (movers < plan.chunks) movers = plan.chunks;
+    if (movers > 15) movers = 15;
+    rounds = (units + movers - 1) / movers;
+    if (rounds > 1 && movers > (units + rounds - 1) / rounds) movers = (units + rounds - 1) / rounds;
+    threads = (movers + 1) * kWave;
+    return rounds <= 4;
+}
+
+bool dispatch_sources_fits(const PushArgs &args, const Workspace &ws, bool quantize, uint32_t total_tokens) {
+    SourcesPlan plan;
+    uint32_t groups, threads, rounds;
+    return plan_dispatch_sources(args, ws, quantize, total_tokens, plan, groups, threads, rounds);
+}
+
+hipError_t launch_dispatch_sources(const PushArgs &args, const FinalizeArgs &fin, const Workspace &ws, bool quantize,
+                                   uint32_t total_tokens, hipStream_t stream, KernelTiming timing) {
+    SourcesPlan plan;
+    uint32_t groups, threads, rounds;
+    if (!plan_dispatch_sources(args, ws, quantize, total_tokens, plan, groups, threads, rounds)) return hipErrorInvalidValue;
+    PushArgs a = args;
+    uint32_t first = 1;   // behind the workgroup that writes the tables
+    for (uint32_t g = 0; g <= (uint32_t)kMaxWorld; ++g) {
+        a.token_start[g] = first;
+        if (g < ws.num_groups) first += (args.src[g].num_tokens + plan.per_group - 1) / plan.per_group;
+    }
+    const size_t lds = (size_t)(ws.num_groups > 2 ? ws.num_groups : 2) * ws.num_experts * sizeof(uint32_t);
+    const uint32_t counting = threads / kWave - 1;
+    const uint32_t per_wave = (plan.chunks + counting - 1) / counting;
+#define A2A_LAUNCH_SOURCES(NC, R)                                                                                    \
+    do {                                                                                                             \
+        if (quantize)                                                                                                \
+            hipExtLaunchKernelGGL((dispatch_sources_kernel<NC, R, true>), dim3(groups + 1), dim3(threads), lds,      \
+                                  stream, timing.start, timing.stop, 0, a, fin, ws, plan);                           \
+        else                                                                                                         \
+            hipExtLaunchKernelGGL((dispatch_sources_kernel<NC, R, false>), dim3(groups + 1), dim3(threads), lds,     \
+                                  stream, timing.start, timing.stop, 0, a, fin, ws, plan);                           \
+    } while (0)
+    if (rounds == 1) {
+        if (per_wave <= 1) A2A_LAUNCH_SOURCES(1, 1);
+        else A2A_LAUNCH_SOURCES(3, 1);
+    } else if (rounds == 2) {
+        A2A_LAUNCH_SOURCES(3, 2);
+    } else {
+        A2A_LAUNCH_SOURCES(3, 4);
+    }
+#undef A2A_LAUNCH_SOURCES
     return hipGetLastError();
 }
 

@@ -188,6 +188,11 @@ bool dispatch_small_fits(const PushArgs &args, const Workspace &ws, bool quantiz
 hipError_t launch_dispatch_small(const PushArgs &args, const FinalizeArgs &fin, const Workspace &ws,
                                  bool quantize, uint32_t total_tokens, hipStream_t stream,
                                  KernelTiming timing = KernelTiming());
+// One-launch routing + pack for steps of several sources with dense index rows, and for larger steps of one: whether a
+// step takes it, and the launch.
+bool dispatch_sources_fits(const PushArgs &args, const Workspace &ws, bool quantize, uint32_t total_tokens);
+hipError_t launch_dispatch_sources(const PushArgs &args, const FinalizeArgs &fin, const Workspace &ws, bool quantize,
+                                uint32_t total_tokens, hipStream_t stream, KernelTiming timing = KernelTiming());
 // One-launch routing + pack for steps of one source with dense index rows that are too large for
 // the small-step kernel.
 constexpr uint32_t kSingleMaxEntries = 8192;
