@@ -156,11 +156,20 @@ constexpr uint32_t kOneRankMaxTokens = 2048;   // largest step that takes the ON
 // copies that went past it, non-temporal / past: 80 MB 126.0 / 122.1 us, 88 MB 138 / 133, 235 MB 371 / 360).  The ONE_RANK
 // variant's outputs stay non-temporal (15 MB 23.4 us, past 24.0), and so do those of rows that were staged (they are
 // written between the launches of the other ranks' calls).
-// With eight loads a lane, 16 wavefronts a compute unit are enough to keep HBM busy behind such stores, and more of
-// them only have more rows open at a time: 470 MB of output 740 -> 670-700 us.  The launch asks for LDS that nothing
-// uses to bound them.  (Fewer loads a lane need all wavefronts: K = 2 70.5 -> 80.7 us with 18.)
 constexpr uint64_t kStreamedOutput = 84000000;
-constexpr size_t kLds16Waves = 160 * 1024 / 16;   // of a compute unit's 160 KB, which are given out in blocks of 1280 bytes
+
+// With eight loads a lane, 16 wavefronts a compute unit are enough to keep HBM busy, and more of them only have more
+// rows open at a time.  us per combine, all wavefronts / bounded, K = 8: 470 MB of output past the cache 740 / 670-700,
+// 4096 tokens of 14 KB rows 89.3 / 86.2, 8 x 512 tokens 89.9 / 87.9, 6000 tokens 131.1 / 127.2, 2668 tokens of 10 KB rows
+// 43.1 / 42.2, 8 x 128 tokens 23.8 / 23.7.  What counts is the loads in flight, 128 a lane and compute unit: with K = 6
+// (rows of 8 KB) 16 wavefronts make 2048 tokens slower (24.0 / 24.3), 21 do not (24.5 / 24.1; 6000 tokens 66.7 / 64.8, 12 000
+// 132.9 / 127.8), K = 5 59.2 / 58.3; up to four loads a lane need all wavefronts (K = 2: 70.5 / 80.7 with 18).  The launch
+// asks for LDS that nothing uses to bound them.  The ONE_RANK variant is left alone (1024 tokens 23.6 / 23.4-23.7).
+inline size_t lds_to_bound_waves(uint32_t topk) {
+    if (topk <= 4) return 0;
+    constexpr size_t kLds = 160 * 1024;   // of a compute unit, given out in blocks of 1280 bytes
+    return kLds / 128 * (topk < 8 ? topk : 8);
+}
 
 // T: type of the expert_y rows, U: type of out_tokens.  One WAVEFRONT handles
 // one slab of 64 sixteen-byte chunks of one token; wavefronts share nothing, so
@@ -353,14 +362,15 @@ static hipError_t launch_typed(const CombArgs &given, const Workspace &ws, uint3
     const bool plain = args.single_rank != 0 || args.staged_base != nullptr;
     const bool past_cache =
         !plain && (streamed || (uint64_t)total_tokens * args.hidden_dim * Elem<U>::kSize >= kStreamedOutput);
+    const size_t lds = lds_to_bound_waves(ws.topk);
 #define A2A_LAUNCH_GATHER(GROUP, ONE, OUT, LDS)                                                                \
     hipExtLaunchKernelGGL((combine_gather_kernel<T, U, GROUP, ONE, OUT>), grid, dim3(kWave), LDS, stream,      \
                           timing.start, timing.stop, 0, args, ws)
 #define A2A_LAUNCH_GATHER_RANKS(GROUP)                                                                         \
     do {                                                                                                       \
         if (args.single_rank != 0) A2A_LAUNCH_GATHER(GROUP, true, kNonTemporal, 0);                            \
-        else if (past_cache) A2A_LAUNCH_GATHER(GROUP, false, kSystemNonTemporal, GROUP == 8 ? kLds16Waves : 0); \
-        else A2A_LAUNCH_GATHER(GROUP, false, kNonTemporal, 0);                                                 \
+        else if (past_cache) A2A_LAUNCH_GATHER(GROUP, false, kSystemNonTemporal, lds);                         \
+        else A2A_LAUNCH_GATHER(GROUP, false, kNonTemporal, lds);                                               \
     } while (0)
     if (ws.topk > 4) A2A_LAUNCH_GATHER_RANKS(8);
     else if (ws.topk > 2) A2A_LAUNCH_GATHER_RANKS(4);

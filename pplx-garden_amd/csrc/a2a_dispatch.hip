@@ -1624,6 +1624,7 @@ constexpr uint32_t kSourcesMaxTokens = 8;        // of a workgroup
 constexpr uint32_t kSourcesMaxRoutes = 64;
 constexpr uint32_t kSourcesMaxScales = 128;
 constexpr uint32_t kSourcesMaxTable = 12288;     // words of dynamic LDS
+constexpr uint32_t kSourcesMinRow = 2048;        // bytes of a copy from which steps of more than kSingleMaxEntries entries pay
 static_assert(sizeof(PushArgs) + sizeof(FinalizeArgs) + sizeof(Workspace) + sizeof(SourcesPlan) <= 4096, "kernel arguments too large");
 
 template <uint32_t NC, uint32_t ROUNDS, bool QUANT>
@@ -2363,7 +2364,9 @@ hipError_t launch_dispatch_single(const PushArgs &args, const FinalizeArgs &fin,
 // to count (8 x 32 tokens of hidden 2048, 2 units and 8 chunks: 6.6 us with 4 wavefronts, 4.6 with 8), in as few rounds
 // as 15 of them need.  The line at 16384 entries: counting costs every workgroup 0.16 us per 1024 of them, where the
 // routing launch it replaces costs 5 to 6 us, and with more than eight tokens of top-8 a workgroup has more routes than
-// its resolver has lanes.  Steps of one source with up to
+// its resolver has lanes; and above 8192 entries rows of 2 KB, because with smaller ones the counting is what is left
+// (one source of 2048 tokens, hidden 1024: 21.5 us a step against 20.4; hidden 2048 and 1500 tokens: 23.2 against 23.9).
+// Steps of one source with up to
 // kSingleMaxEntries entries have the two kernels that are made for them (128 tokens 4.54 us against 4.77 here, 1024
 // tokens 15.4 against 16.1).
 bool plan_dispatch_sources(const PushArgs &args, const Workspace &ws, bool quantize, uint32_t total_tokens, SourcesPlan &plan,
@@ -2390,6 +2393,7 @@ bool plan_dispatch_sources(const PushArgs &args, const Workspace &ws, bool quant
         groups += (args.src[g].num_tokens + plan.per_group - 1) / plan.per_group;
     }
     if (senders == 1 && entries <= kSingleMaxEntries) return false;
+    if (entries > kSingleMaxEntries && pieces * 16 < kSourcesMinRow) return false;
     const uint32_t units = plan.per_group * plan.units;
     uint32_t movers = units;
     if (movers < plan.chunks) movers = plan.chunks;
