@@ -479,7 +479,6 @@ def split_calls(case, device, routings: int, steps: int, warmup: int, label: str
                 ctx.time_next_kernel(which, pair[0].cuda_event, pair[1].cuda_event)
                 timed.append((key, j, pair))
 
-        own(native.KERNEL_ROUTE, "route")
         own(native.KERNEL_STAGE_SEND, "send")
         send(j)
         for r in range(1, N):
@@ -569,8 +568,7 @@ def split_calls(case, device, routings: int, steps: int, warmup: int, label: str
 
     kernels = {
         "dispatch_send": [
-            kernel("route_hist_kernel", us.get("route", []), lambda j: 0),
-            kernel("stage_send_resolve_kernel", us.get("send", []), lambda j: T * (2 * H + 4 * K) + T * row_d),
+            kernel("stage_send_beside_kernel", us.get("send", []), lambda j: T * (2 * H + 4 * K) + T * row_d),
         ],
         "dispatch_recv": [
             kernel("stage_layout_kernel", us.get("layout", []), lambda j: 0),

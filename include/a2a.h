@@ -321,10 +321,10 @@ int a2a_ctx_read_table(a2a_ctx *ctx, uint32_t rank, uint32_t which,
  *   A2A_KERNEL_ROUTE         the routing launch that precedes the pack of a large
  *                            step (a2a_dispatch) or the staging of a large send
  *                            (a2a_dispatch_send); a step that counts its routing
- *                            inside the pack or the staging launch (a small one,
- *                            or one source alone with up to 8192 copies) or runs
- *                            several routing kernels (A2A_FLAG_SEPARATE_ROUTING)
- *                            has no such launch and leaves those events alone
+ *                            inside the pack or the staging launch (up to 8192 or
+ *                            16384 copies; a send up to 65535) or runs several
+ *                            routing kernels (A2A_FLAG_SEPARATE_ROUTING) has no
+ *                            such launch and leaves those events alone
  *   A2A_KERNEL_GATHER        the gather of the next a2a_combine or a2a_combine_recv
  *   A2A_KERNEL_STAGE_SEND    the staging launch of the next a2a_dispatch_send
  *   A2A_KERNEL_STAGE_RECV    the copy launch of the next a2a_dispatch_recv

@@ -115,6 +115,10 @@ hipError_t launch_stage_send_small(const StageSendArgs &args, const Workspace &w
 bool stage_send_single_fits(const StageSendArgs &args, const Workspace &ws, bool quantize);
 hipError_t launch_stage_send_single(const StageSendArgs &args, const Workspace &ws, const Staging &st,
                                     bool quantize, hipStream_t stream, KernelTiming timing = KernelTiming());
+// One-launch send for larger steps (up to 65535 entries): the routing runs in workgroups beside those that stage the rows.
+bool stage_send_beside_fits(const StageSendArgs &args, const Workspace &ws);
+hipError_t launch_stage_send_beside(const StageSendArgs &args, const Workspace &ws, const Staging &st, bool quantize,
+                                    hipStream_t stream, KernelTiming timing = KernelTiming());
 // The send of a large step after launch_route_accumulate(..., for_send = true).
 hipError_t launch_stage_send_resolve(const StageSendArgs &args, const Workspace &ws, const Staging &st,
                                      bool quantize, hipStream_t stream, KernelTiming timing = KernelTiming());

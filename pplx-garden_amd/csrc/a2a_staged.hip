@@ -846,6 +846,163 @@ __global__ __launch_bounds__(1024) void stage_send_teams_kernel(const StageSendA
     }
 }
 
+// The send of a larger step (up to kSendBesideMaxEntries entries) in ONE launch: where a row is staged does not depend on
+// the routing, so the routing runs beside the rows, in workgroups of its own at the head of the grid.  Such a workgroup
+// has a chunk of as many entries as it has threads.  It counts ALL entries of the sender per expert, with those in front
+// of its chunk in the high half of the word, ranks its own entries among equal ones with ballots (and a scan over the
+// wavefronts), scans the counts over the experts, and then has the position of each of its entries without having
+// waited for anybody.  The counting is redundant, but it runs on compute units that the rows, which are bound by memory,
+// do not fill.  All other workgroups stage rows, a team of wavefronts per token, and nothing else.
+//
+// us per send at the GPU's own pace, two launches (routing, then rows that resolve their own positions) / this one:
+//   fp8 rows of 7168 bytes, K = 8, 1100 tokens   11.5 /  7.3     2048   15.9 / 10.2     4096   20.8 / 14.7     8000   32.7 / 24.5
+//   quantised rows, 2048 tokens                  18.4 / 11.8     4096   26.0 / 19.7
+//   bf16 rows of 14 KB, 2048 tokens              22.4 / 14.4     of 8 KB, K = 4, 4000 tokens   24.8 / 14.5
+//   rows of 2048 bytes, 512 experts, 2000 tokens 10.6 /  7.4     of 1024 bytes, 3000 tokens     9.0 /  7.7
+// (Whole steps of 8 x 2048 tokens through the split calls: 1431 -> 1385.)
+//
+// Dynamic LDS: 2 * E words and, per wavefront, E half words.
+constexpr uint32_t kSendBesideMaxEntries = 65535;   // (the halves of a word)
+constexpr uint32_t kSendBesideAhead = 8;            // entries a thread has on their way while it counts as many
+
+template <bool QUANT>
+__global__ __launch_bounds__(1024) void stage_send_beside_kernel(const StageSendArgs args, const Workspace ws,
+                                                                 const Staging st, const uint32_t team_threads,
+                                                                 const uint32_t chunks) {
+    extern __shared__ uint32_t s_beside[];
+    __shared__ uint32_t scratch[kRouteWaves];
+    __shared__ uint32_t s_carry;
+    A2A_PIN(args.src.x);
+    A2A_PIN(args.src.x_scale);
+    A2A_PIN(args.src.indices);
+    A2A_PIN(args.src.bound_m);
+    A2A_PIN(args.src.x_stride);
+    A2A_PIN(args.src.num_tokens);
+    A2A_PIN(args.rank);
+    A2A_PIN(args.hidden_dim);
+    A2A_PIN(args.row_bytes);
+    A2A_PIN(args.topk_magic);
+    A2A_PIN(ws.num_experts);
+    A2A_PIN(ws.topk);
+    A2A_PIN(ws.dp_size);
+    A2A_PIN(ws.max_tk);
+    A2A_PIN(ws.token_offset);
+    A2A_PIN(ws.err);
+    A2A_PIN(st.send_buf);
+    A2A_PIN(st.pos_token);
+    A2A_PIN(st.disp_stride);
+    A2A_PIN(st.payload_bytes);
+    A2A_PIN(st.max_tokens);
+    const uint32_t tid = threadIdx.x;
+    const uint32_t nthreads = blockDim.x;
+    const uint32_t K = ws.topk;
+    const uint32_t g = args.rank / ws.dp_size;
+    const PushSrc &src = args.src;
+    if (blockIdx.x >= chunks) {
+        // ---- rows
+        const uint32_t teams = nthreads / team_threads, team = tid / team_threads;
+        const uint32_t token = (blockIdx.x - chunks) * teams + team;
+        if (token >= effective_tokens(src.bound_m, src.num_tokens)) return;   // (no barrier below)
+        stage_row<QUANT>(args, st, g, token, team_threads, u32x4{0, 0, 0, 0}, u32x4{0, 0, 0, 0}, team * team_threads);
+        return;
+    }
+
+    // ---- positions
+    const uint32_t lane = tid & (kWave - 1);
+    const uint32_t wave = tid / kWave;
+    const uint32_t waves = nthreads / kWave;
+    const uint32_t E = ws.num_experts;
+    uint32_t *const cnt = s_beside;                                     // [E]
+    uint32_t *const excl = cnt + E;                                     // [E] entries of the experts before e
+    uint16_t *const hist = reinterpret_cast<uint16_t *>(excl + E);      // [waves][E] entries of my chunk
+    const uint32_t entries = src.num_tokens * K;                        // > 0
+    auto id_of = [&](uint32_t f) { return (uint32_t)src.indices[f < entries ? f : entries - 1]; };   // (dense rows)
+    const uint32_t chunk_first = blockIdx.x * nthreads;
+    const uint32_t entry = chunk_first + tid;
+    const uint32_t my_id = id_of(entry);
+    constexpr uint32_t NB = kSendBesideAhead;
+    uint32_t now[NB];
+#pragma unroll
+    for (uint32_t j = 0; j < NB; ++j) now[j] = id_of(j * nthreads + tid);
+    const uint32_t live_entries = effective_tokens(src.bound_m, src.num_tokens) * K;
+    if (blockIdx.x != 0 && chunk_first >= live_entries) return;   // uniform (the first workgroup publishes)
+    for (uint32_t i = tid; i < E; i += nthreads) cnt[i] = 0;
+    for (uint32_t i = tid; i < waves * E; i += nthreads) hist[i] = 0;
+    lds_barrier();
+
+    // my chunk: lanes of this wavefront that hold the same expert id, matched bit by bit
+    const bool in = entry < live_entries;
+    const bool valid = in && my_id < E;
+    uint64_t peers = __ballot(valid);
+    const uint32_t nbits = 32 - __clz((int)(E - 1) | 1);
+    for (uint32_t b = 0; b < nbits; ++b) {
+        const bool bit = (my_id >> b) & 1;
+        const uint64_t set = __ballot(valid && bit);
+        peers &= bit ? set : ~set;
+    }
+    const uint32_t rank_in_wave = __popcll(peers & ((1ull << lane) - 1));
+    if (valid && rank_in_wave == 0) hist[wave * E + my_id] = (uint16_t)__popcll(peers);
+
+    // all entries, the next ones on their way while these are counted
+    for (uint32_t f0 = 0;;) {
+        const uint32_t next = f0 + NB * nthreads;
+        uint32_t then[NB];
+#pragma unroll
+        for (uint32_t j = 0; j < NB; ++j) then[j] = id_of(next + j * nthreads + tid);
+#pragma unroll
+        for (uint32_t j = 0; j < NB; ++j) {
+            const uint32_t f = f0 + j * nthreads + tid;
+            if (f < live_entries && now[j] < E) atomicAdd(&cnt[now[j]], f < chunk_first ? 0x10001u : 1u);
+        }
+        if (next >= live_entries) break;
+        f0 = next;
+#pragma unroll
+        for (uint32_t j = 0; j < NB; ++j) now[j] = then[j];
+    }
+    lds_barrier();
+
+    // per expert: my wavefronts' entries in order, and the scan over the experts (a2a_dispatch_send.cu:236-242)
+    uint32_t carry = 0;
+    for (uint32_t e0 = 0; e0 < E; e0 += nthreads) {
+        const uint32_t e = e0 + tid;
+        uint32_t run = 0;
+        if (e < E) {
+            for (uint32_t w = 0; w < waves; ++w) {
+                const uint32_t c = hist[w * E + e];
+                hist[w * E + e] = (uint16_t)run;
+                run += c;
+            }
+        }
+        const uint32_t c = e < E ? cnt[e] & 0xFFFFu : 0;
+        const uint32_t incl = carry + block_inclusive_scan<true>(c, scratch);
+        if (e < E) {
+            excl[e] = incl - c;
+            if (blockIdx.x == 0) {
+                ws.num_routed[g * E + e] = c;
+                ws.expert_offsets[g * E + e] = incl;
+            }
+        }
+        if (e0 + nthreads < E) {   // uniform: another round follows
+            if (tid == nthreads - 1) s_carry = incl;
+            lds_barrier();
+            carry = s_carry;
+        }
+    }
+    lds_barrier();
+    if (!in) return;
+    uint32_t toff = 0, at = kInvalidSlot;
+    if (valid) {
+        toff = (cnt[my_id] >> 16) + hist[wave * E + my_id] + rank_in_wave;
+        // position of the copy (a2a_dispatch_send.cu:54)
+        at = excl[my_id] + toff;
+        st.pos_token[(size_t)g * ws.max_tk + at] = K > 1 ? __umulhi(entry, args.topk_magic) : entry;
+    } else {
+        atomicOr(ws.err, A2A_DEV_BAD_EXPERT_ID);
+    }
+    ws.token_offset[(size_t)g * ws.max_tk + entry] = toff;
+    ws.route_slot[(size_t)g * ws.max_tk + entry] = at;
+}
+
 // The send of a large step, after a routing launch that left the chunk counts,
 // the in-chunk rank of every entry and the sender's totals per expert and per
 // owning rank.  No launch in between scans anything: wavefront 0 of a token
@@ -1893,6 +2050,29 @@ hipError_t launch_stage_send_single(const StageSendArgs &args, const Workspace &
     } else {
         hipExtLaunchKernelGGL(stage_send_single_kernel<false>, dim3(blocks), dim3(teams * team), lds, stream,
                               timing.start, timing.stop, 0, args, ws, st, team, per_group);
+    }
+    return hipGetLastError();
+}
+
+bool stage_send_beside_fits(const StageSendArgs &args, const Workspace &ws) {
+    return args.src.num_tokens != 0 && args.src.indices_stride == ws.topk &&
+           (uint64_t)args.src.num_tokens * ws.topk <= kSendBesideMaxEntries;
+}
+
+hipError_t launch_stage_send_beside(const StageSendArgs &args, const Workspace &ws, const Staging &st, bool quantize,
+                                    hipStream_t stream, KernelTiming timing) {
+    const uint32_t team = block_for_chunks(quantize ? args.hidden_dim / 16 : args.row_bytes / 16);
+    const uint32_t teams = team < 512 ? 512 / team : 1;
+    const uint32_t threads = teams * team;
+    const uint32_t chunks = (args.src.num_tokens * ws.topk + threads - 1) / threads;
+    const uint32_t blocks = chunks + (args.src.num_tokens + teams - 1) / teams;
+    const size_t lds = (size_t)ws.num_experts * (2 * sizeof(uint32_t) + threads / kWave * sizeof(uint16_t));
+    if (quantize) {
+        hipExtLaunchKernelGGL(stage_send_beside_kernel<true>, dim3(blocks), dim3(threads), lds, stream, timing.start,
+                              timing.stop, 0, args, ws, st, team, chunks);
+    } else {
+        hipExtLaunchKernelGGL(stage_send_beside_kernel<false>, dim3(blocks), dim3(threads), lds, stream, timing.start,
+                              timing.stop, 0, args, ws, st, team, chunks);
     }
     return hipGetLastError();
 }
