@@ -163,12 +163,17 @@ constexpr uint64_t kStreamedOutput = 84000000;
 // 4096 tokens of 14 KB rows 89.3 / 86.2, 8 x 512 tokens 89.9 / 87.9, 6000 tokens 131.1 / 127.2, 2668 tokens of 10 KB rows
 // 43.1 / 42.2, 8 x 128 tokens 23.8 / 23.7.  What counts is the loads in flight, 128 a lane and compute unit: with K = 6
 // (rows of 8 KB) 16 wavefronts make 2048 tokens slower (24.0 / 24.3), 21 do not (24.5 / 24.1; 6000 tokens 66.7 / 64.8, 12 000
-// 132.9 / 127.8), K = 5 59.2 / 58.3; up to four loads a lane need all wavefronts (K = 2: 70.5 / 80.7 with 18).  The launch
+// 132.9 / 127.8), K = 5 59.2 / 58.3; up to four loads a lane need all wavefronts (K = 2: 70.5 / 80.7 with 18).  Behind
+// copies and in front of tokens that go past the cache 96 are enough: whole steps with 16 / 14 / 12 / 11 wavefronts, K = 8,
+// 6000 tokens 216.6 / 214.1 / 212.7 / 214.2, 8 x 4096 tokens 1161 / 1145 / 1139 / 1152, 8 x 2048 tokens of 5 KB fp8 rows 416.1 /
+// 410.2 / 406.7 / 409.3, float rows of 8 KB, 8 x 3000 tokens 663.7 / 657.5 / 655.4 / 656.7; K = 6 with 21 / 18 / 16, 8 x 4096
+// tokens 894.5 / 888.6 / 878.0 (in the cache 14 are 0.9 us better at 4096 tokens and 0.3 worse at 2668, 12 worse).  The launch
 // asks for LDS that nothing uses to bound them.  The ONE_RANK variant is left alone (1024 tokens 23.6 / 23.4-23.7).
-inline size_t lds_to_bound_waves(uint32_t topk) {
+inline size_t lds_to_bound_waves(uint32_t topk, bool past_cache) {
     if (topk <= 4) return 0;
-    constexpr size_t kLds = 160 * 1024;   // of a compute unit, given out in blocks of 1280 bytes
-    return kLds / 128 * (topk < 8 ? topk : 8);
+    constexpr size_t kLds = 160 * 1024, kBlock = 1280;   // of a compute unit, and what it is given out in
+    const size_t waves = (past_cache ? 96 : 128) / (topk < 8 ? topk : 8);
+    return kLds / waves / kBlock * kBlock;
 }
 
 // T: type of the expert_y rows, U: type of out_tokens.  One WAVEFRONT handles
@@ -362,7 +367,7 @@ static hipError_t launch_typed(const CombArgs &given, const Workspace &ws, uint3
     const bool plain = args.single_rank != 0 || args.staged_base != nullptr;
     const bool past_cache =
         !plain && (streamed || (uint64_t)total_tokens * args.hidden_dim * Elem<U>::kSize >= kStreamedOutput);
-    const size_t lds = lds_to_bound_waves(ws.topk);
+    const size_t lds = lds_to_bound_waves(ws.topk, past_cache);
 #define A2A_LAUNCH_GATHER(GROUP, ONE, OUT, LDS)                                                                \
     hipExtLaunchKernelGGL((combine_gather_kernel<T, U, GROUP, ONE, OUT>), grid, dim3(kWave), LDS, stream,      \
                           timing.start, timing.stop, 0, args, ws)
