@@ -54,7 +54,7 @@ struct StageSendArgs {
     uint32_t resolver_wave;   // resolving send: wavefront that resolves the routes (set by the launcher)
 };
 
-// A grid of wavefronts over the pieces (64 sixteen-byte chunks) of a receiver's rows.
+// A grid of wavefronts over the pieces (64 or 128 sixteen-byte chunks) of a receiver's rows.
 struct PieceGrid {
     uint32_t pieces;          // of a row
     uint32_t magic;           // n / pieces = mulhi(n, magic) for the wavefronts of a grid (0 for one piece a row)

@@ -1713,7 +1713,9 @@ __global__ __launch_bounds__(kPieceThreads) void stage_recv_kernel(const StageRe
 // (source, expert), so both sides are fronts through memory.  16384 rows of 14 KB: 105.5 us = 4.45 TB/s
 // with a wavefront per row, 76.5 us = 6.1 TB/s in this order (a plain copy of as many rows in the same
 // order, examples/ceilings.hip: 67.6 us; both sides come from and go to HBM, so loads and stores keep nothing).
+// U: chunks a lane has in flight, one piece being 64 * U chunks (kTwoChunkRows).
 // ---------------------------------------------------------------------------
+template <uint32_t U>
 __global__ __launch_bounds__(kPieceThreads) void combine_send_kernel(const CombineSendArgs args, const Workspace ws,
                                                                      const Staging st) {
     // everything a wavefront takes from the argument block, asked for in one go
@@ -1748,11 +1750,15 @@ __global__ __launch_bounds__(kPieceThreads) void combine_send_kernel(const Combi
     uint32_t total = st.num_recv[2 * r];
     if (total > st.max_recv) total = st.max_recv;
     while (at.row < total) {
-        const uint32_t c = at.piece * kWave + lane;
+        const uint32_t c = at.piece * (U * kWave) + lane;
         const bool fits = row < args.y_rows && pos < ws.max_tk;
-        const bool active = fits && c < num_chunks;
-        u32x4 v = {0, 0, 0, 0};
-        if (active) v = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(args.y + (size_t)row * args.y_stride) + c);
+        const u32x4 *const from = reinterpret_cast<const u32x4 *>(args.y + (size_t)row * args.y_stride) + c;
+        u32x4 v[U];
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) {
+            v[u] = u32x4{0, 0, 0, 0};
+            if (fits && c + u * kWave < num_chunks) v[u] = __builtin_nontemporal_load(from + u * kWave);
+        }
         // the next piece's words travel while this one is copied
         PieceWalk next = at;
         next.advance(args.grid);
@@ -1762,8 +1768,11 @@ __global__ __launch_bounds__(kPieceThreads) void combine_send_kernel(const Combi
         const uint32_t next_pos = source_position[next_probe];
         // every member of the source's dp group reads the same staging rows
         const uint32_t g = ws.dp_size > 1 ? peer / ws.dp_size : peer;
-        if (active)
-            store_copy(v, reinterpret_cast<u32x4 *>(st.comb_buf + ((size_t)g * ws.max_tk + pos) * st.comb_stride) + c);
+        u32x4 *const to = reinterpret_cast<u32x4 *>(st.comb_buf + ((size_t)g * ws.max_tk + pos) * st.comb_stride) + c;
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) {
+            if (fits && c + u * kWave < num_chunks) store_copy(v[u], to + u * kWave);
+        }
         if (!fits && at.piece == 0 && lane == 0) atomicOr(ws.err, A2A_DEV_BAD_SLOT);
         at = next;
         row = next_row;
@@ -1789,15 +1798,21 @@ uint32_t block_for_chunks(uint32_t chunks) {
 //     rows (57344 workgroups' worth of pieces) 88.0 / 86.7 / 82.8 / 78.9 us with 2048 / 4096 / 8192 / 16384 workgroups.
 //     Not more, because the grid is sized for the upper bound and workgroups without rows cost as well:
 //     4096 rows 21.0 / 20.4 / 21.0 / 24.0.
+//     Where a receiver typically gets up to kTwoChunkRows rows, pieces of twice the size and two of them a wavefront: half
+//     the look-ups, and both loads of a piece in flight.  Whole split steps, us, one chunk a lane / two: 8 x 128 tokens 187.8 /
+//     186.0 (rows of 8 KB 147.1 / 144.2, of 2 KB 105.5 / 102.8), 8 x 512 418.6 / 413.8, 8 x 1500 1036.7 / 1030.6, one sender of 4096
+//     367.1 / 361.3; beyond, the tight front is worth more: 8 x 2048 1391 / 1396, 4 x 3000 983 / 993.
 constexpr uint32_t kPieceWorkgroups = 2048;
-constexpr uint32_t kPiecesInOrder = 3;
+constexpr uint32_t kTwoChunkRows = 12288;
 
-uint32_t piece_grid(uint32_t max_rows, uint32_t world, uint32_t chunks, bool in_order, PieceGrid &grid) {
+// `chunks_a_lane`: 16-byte chunks of a row that a lane moves at once.
+uint32_t piece_grid(uint32_t max_rows, uint32_t world, uint32_t chunks, bool in_order, uint32_t chunks_a_lane, PieceGrid &grid) {
     constexpr uint32_t waves = kPieceThreads / kWave;
-    grid.pieces = (chunks + kWave - 1) / kWave;
+    const uint32_t pieces_in_order = chunks_a_lane > 1 ? 2 : 3;
+    grid.pieces = (chunks + chunks_a_lane * kWave - 1) / (chunks_a_lane * kWave);
     const uint64_t most = ((uint64_t)max_rows * grid.pieces + waves - 1) / waves;
     uint64_t blocks = kPieceWorkgroups;
-    if (in_order && most / world / kPiecesInOrder > blocks) blocks = most / world / kPiecesInOrder;
+    if (in_order && most / world / pieces_in_order > blocks) blocks = most / world / pieces_in_order;
     if (blocks > 1u << 16) blocks = 1u << 16;   // (keeps wavefront numbers far below 2^32 / pieces)
     if (blocks > most) blocks = most;
     if (blocks < 1) blocks = 1;
@@ -2128,7 +2143,7 @@ hipError_t launch_stage_recv(const StageRecvArgs &args, const Workspace &ws, con
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
-    const uint32_t blocks = piece_grid(args.max_rows, ws.world, chunks, false, a.grid);
+    const uint32_t blocks = piece_grid(args.max_rows, ws.world, chunks, false, 1, a.grid);
     if (args.streamed) {
         hipExtLaunchKernelGGL(stage_recv_kernel<true>, dim3(blocks), dim3(kPieceThreads), 0, stream, timing.start,
                               timing.stop, 0, a, ws, st);
@@ -2144,9 +2159,15 @@ hipError_t launch_combine_send(const CombineSendArgs &args, const Workspace &ws,
     if (args.max_rows == 0) return hipSuccess;
     const uint32_t chunks = args.row_bytes / 16;
     CombineSendArgs a = args;
-    const uint32_t blocks = piece_grid(args.max_rows, ws.world, chunks, true, a.grid);
-    hipExtLaunchKernelGGL(combine_send_kernel, dim3(blocks), dim3(kPieceThreads), 0, stream, timing.start, timing.stop,
-                          0, a, ws, st);
+    if ((args.max_rows + ws.world - 1) / ws.world <= kTwoChunkRows) {
+        const uint32_t blocks = piece_grid(args.max_rows, ws.world, chunks, true, 2, a.grid);
+        hipExtLaunchKernelGGL(combine_send_kernel<2>, dim3(blocks), dim3(kPieceThreads), 0, stream, timing.start,
+                              timing.stop, 0, a, ws, st);
+    } else {
+        const uint32_t blocks = piece_grid(args.max_rows, ws.world, chunks, true, 1, a.grid);
+        hipExtLaunchKernelGGL(combine_send_kernel<1>, dim3(blocks), dim3(kPieceThreads), 0, stream, timing.start,
+                              timing.stop, 0, a, ws, st);
+    }
     return hipGetLastError();
 }
 
