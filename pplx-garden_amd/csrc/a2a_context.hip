@@ -138,15 +138,15 @@ uint32_t ceil_div_u32(uint64_t n, uint64_t m) { return (uint32_t)((n + m - 1) / 
 bool aligned16(const void *p) { return ((uintptr_t)p & 15) == 0; }
 
 struct DeviceGuard {
-    int prev = -1;
+    int prev = -1, dev;
     bool ok = false;
-    explicit DeviceGuard(int dev) {
+    explicit DeviceGuard(int device) : dev(device) {
         if (hipGetDevice(&prev) == hipSuccess) {
             ok = prev == dev || hipSetDevice(dev) == hipSuccess;
         }
     }
     ~DeviceGuard() {
-        if (ok && prev >= 0) (void)hipSetDevice(prev);
+        if (ok && prev >= 0 && prev != dev) (void)hipSetDevice(prev);
     }
 };
 

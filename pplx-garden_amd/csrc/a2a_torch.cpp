@@ -3,7 +3,8 @@
 // A step of eight ranks is sixteen operator calls (thirty-two through the split calls), and each has to
 // look at six to eight tensors (shape, strides, type, address: some forty attributes) before one of them
 // launches anything.  In Python that was 5.8 us a call, so that a decode step of 12 us on the GPU took 93;
-// here a call that launches nothing is 0.4 us, most of it the interpreter's own way in and out.
+// here a call that launches nothing is 0.2-0.3 us, most of it the interpreter's own way in and out (through a
+// Python function in front of it 0.1 us more: Method below; 8 ranks x 1 token 11.3 -> 10.6 us a step).
 //
 // Plays the part of the reference's pyo3 classes (python-ext/src/py_p2p_all_to_all.rs:17-205) one level
 // higher: it takes the tensors themselves and makes the checks of the reference's operator
@@ -383,10 +384,73 @@ struct Taken {
 
 void *current_stream(const Operator *op) { return c10::hip::getCurrentHIPStream(op->device).stream(); }
 
-// dispatch(out_expert_num_tokens, out_expert_x, out_expert_x_scale, dp_x, dp_x_scale, indices, weights, bound_m,
-//          do_send, do_recv)
-PyObject *dispatch(Operator *op, PyObject *const *a, Py_ssize_t n) {
-    if (n != 10) return PyErr_Format(PyExc_TypeError, "dispatch takes 10 arguments");
+// The arguments of a call by position and by name, as a Python function with these parameters would take them: `a` comes
+// in with the defaults (null where there is none) and goes out complete.
+constexpr int kMostParameters = 10;
+
+struct Parameters {
+    const char *call;
+    int count;
+    const char *name[kMostParameters];
+    PyObject *interned[kMostParameters];   // (names in a call are interned strings: found by address)
+};
+
+Parameters dispatch_parameters = {"dispatch", 10,
+                                  {"out_expert_num_tokens", "out_expert_x", "out_expert_x_scale", "dp_x", "dp_x_scale",
+                                   "indices", "weights", "bound_m", "do_send", "do_recv"}, {}};
+Parameters combine_parameters = {"combine", 8,
+                                 {"out_tokens", "indices", "weights", "expert_y", "bound_m", "do_send", "do_recv",
+                                  "accumulate"}, {}};
+
+bool intern_names(Parameters &p) {
+    for (int i = 0; i < p.count; ++i) {
+        p.interned[i] = PyUnicode_InternFromString(p.name[i]);
+        if (p.interned[i] == nullptr) return false;
+    }
+    return true;
+}
+
+bool take_arguments(const Parameters &p, PyObject *const *args, Py_ssize_t n, PyObject *keywords, PyObject **a) {
+    if (n > p.count) {
+        PyErr_Format(PyExc_TypeError, "%s() takes %d arguments but %zd were given", p.call, p.count, n);
+        return false;
+    }
+    for (Py_ssize_t i = 0; i < n; ++i) a[i] = args[i];
+    uint32_t given = (1u << n) - 1;
+    const Py_ssize_t named = keywords != nullptr ? PyTuple_GET_SIZE(keywords) : 0;
+    for (Py_ssize_t i = 0; i < named; ++i) {
+        PyObject *const key = PyTuple_GET_ITEM(keywords, i);
+        int at = 0;
+        while (at < p.count && p.interned[at] != key) ++at;
+        if (at == p.count) {
+            for (at = 0; at < p.count && PyUnicode_Compare(p.interned[at], key) != 0; ++at) {
+            }
+        }
+        if (at == p.count) {
+            PyErr_Format(PyExc_TypeError, "%s() got an unexpected keyword argument '%U'", p.call, key);
+            return false;
+        }
+        if (given >> at & 1) {
+            PyErr_Format(PyExc_TypeError, "%s() got multiple values for argument '%s'", p.call, p.name[at]);
+            return false;
+        }
+        given |= 1u << at;
+        a[at] = args[n + i];
+    }
+    for (int i = 0; i < p.count; ++i) {
+        if (a[i] == nullptr) {
+            PyErr_Format(PyExc_TypeError, "%s() missing required argument: '%s'", p.call, p.name[i]);
+            return false;
+        }
+    }
+    return true;
+}
+
+// dispatch(out_expert_num_tokens, out_expert_x, out_expert_x_scale, dp_x, dp_x_scale, indices, weights, bound_m=None,
+//          do_send=True, do_recv=True)
+PyObject *dispatch(Operator *op, PyObject *const *args, Py_ssize_t n, PyObject *keywords) {
+    PyObject *a[kMostParameters] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, Py_None, Py_True, Py_True};
+    if (!take_arguments(dispatch_parameters, args, n, keywords, a)) return nullptr;
     const int do_send = PyObject_IsTrue(a[8]), do_recv = PyObject_IsTrue(a[9]);
     if (do_send < 0 || do_recv < 0) return nullptr;
     A2A_REQUIRE(do_send || do_recv);
@@ -517,9 +581,10 @@ PyObject *dispatch(Operator *op, PyObject *const *a, Py_ssize_t n) {
     Py_RETURN_NONE;
 }
 
-// combine(out_tokens, indices, weights, expert_y, bound_m, do_send, do_recv, accumulate)
-PyObject *combine(Operator *op, PyObject *const *a, Py_ssize_t n) {
-    if (n != 8) return PyErr_Format(PyExc_TypeError, "combine takes 8 arguments");
+// combine(out_tokens, indices, weights, expert_y, bound_m=None, do_send=True, do_recv=True, accumulate=False)
+PyObject *combine(Operator *op, PyObject *const *args, Py_ssize_t n, PyObject *keywords) {
+    PyObject *a[kMostParameters] = {nullptr, nullptr, nullptr, nullptr, Py_None, Py_True, Py_True, Py_False};
+    if (!take_arguments(combine_parameters, args, n, keywords, a)) return nullptr;
     const int do_send = PyObject_IsTrue(a[5]), do_recv = PyObject_IsTrue(a[6]), accumulate = PyObject_IsTrue(a[7]);
     if (do_send < 0 || do_recv < 0 || accumulate < 0) return nullptr;
     A2A_REQUIRE(do_send || do_recv);
@@ -619,10 +684,10 @@ PyObject *combine(Operator *op, PyObject *const *a, Py_ssize_t n) {
 }
 
 // A torch call (data_ptr of a tensor without storage, say) may throw: no C++ exception enters the interpreter.
-template <PyObject *(*CALL)(Operator *, PyObject *const *, Py_ssize_t)>
-PyObject *guarded(PyObject *self, PyObject *const *args, Py_ssize_t n) {
+template <PyObject *(*CALL)(Operator *, PyObject *const *, Py_ssize_t, PyObject *)>
+PyObject *guarded(PyObject *self, PyObject *const *args, Py_ssize_t n, PyObject *keywords) {
     try {
-        return CALL(reinterpret_cast<Operator *>(self), args, n);
+        return CALL(reinterpret_cast<Operator *>(self), args, n, keywords);
     } catch (python_error &e) {
         e.restore();
     } catch (const std::exception &e) {
@@ -632,12 +697,66 @@ PyObject *guarded(PyObject *self, PyObject *const *args, Py_ssize_t n) {
 }
 
 PyMethodDef operator_methods[] = {
-    {"dispatch", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(guarded<dispatch>)), METH_FASTCALL, nullptr},
-    {"combine", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(guarded<combine>)), METH_FASTCALL, nullptr},
+    {"dispatch", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(guarded<dispatch>)), METH_FASTCALL | METH_KEYWORDS,
+     nullptr},
+    {"combine", reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(guarded<combine>)), METH_FASTCALL | METH_KEYWORDS,
+     nullptr},
     {nullptr, nullptr, 0, nullptr},
 };
 
 PyTypeObject OperatorType = {PyVarObject_HEAD_INIT(nullptr, 0)};
+
+// ---------------------------------------------------------------------------
+// Method: stands in a Python class in the place of a function `f(self, ...)` that hands its arguments to the method of the
+// same name of `self._operator`.  Looked up on an object whose `_operator` is one it gives that method itself, so that a
+// call does not pass through a Python frame; otherwise, and looked up on the class, the function.
+// ---------------------------------------------------------------------------
+struct Method {
+    PyObject_HEAD
+    PyObject *name, *function;
+};
+
+PyObject *operator_attribute;   // "_operator"
+
+PyObject *method_new(PyTypeObject *type, PyObject *args, PyObject *) {
+    PyObject *name, *function;
+    if (!PyArg_ParseTuple(args, "UO", &name, &function)) return nullptr;
+    Method *m = reinterpret_cast<Method *>(type->tp_alloc(type, 0));
+    if (m == nullptr) return nullptr;
+    Py_INCREF(name);
+    PyUnicode_InternInPlace(&name);
+    m->name = name;
+    Py_INCREF(function);
+    m->function = function;
+    return reinterpret_cast<PyObject *>(m);
+}
+
+void method_dealloc(PyObject *self) {
+    Py_XDECREF(reinterpret_cast<Method *>(self)->name);
+    Py_XDECREF(reinterpret_cast<Method *>(self)->function);
+    Py_TYPE(self)->tp_free(self);
+}
+
+PyObject *method_get(PyObject *self, PyObject *object, PyObject *) {
+    Method *m = reinterpret_cast<Method *>(self);
+    if (object == nullptr || object == Py_None) {
+        Py_INCREF(m->function);
+        return m->function;
+    }
+    PyObject *const op = PyObject_GetAttr(object, operator_attribute);
+    if (op == nullptr) {
+        if (!PyErr_ExceptionMatches(PyExc_AttributeError)) return nullptr;
+        PyErr_Clear();
+    } else if (Py_TYPE(op) == &OperatorType) {
+        PyObject *const bound = PyObject_GetAttr(op, m->name);
+        Py_DECREF(op);
+        return bound;
+    }
+    Py_XDECREF(op);
+    return PyMethod_New(m->function, object);
+}
+
+PyTypeObject MethodType = {PyVarObject_HEAD_INIT(nullptr, 0)};
 
 PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_a2a_torch", nullptr, -1, nullptr, nullptr, nullptr, nullptr, nullptr};
 
@@ -659,7 +778,14 @@ bool add_type(PyObject *module, PyTypeObject &type, const char *name, const char
 PyMODINIT_FUNC PyInit__a2a_torch(void) {
     PyObject *m = PyModule_Create(&module_def);
     if (m == nullptr) return nullptr;
-    if (!add_type(m, ContextType, "_a2a_torch.Context", "Context", sizeof(Context), context_new, context_dealloc,
+    operator_attribute = PyUnicode_InternFromString("_operator");
+    if (operator_attribute == nullptr || !intern_names(dispatch_parameters) || !intern_names(combine_parameters)) {
+        Py_DECREF(m);
+        return nullptr;
+    }
+    MethodType.tp_descr_get = method_get;
+    if (!add_type(m, MethodType, "_a2a_torch.Method", "Method", sizeof(Method), method_new, method_dealloc, nullptr) ||
+        !add_type(m, ContextType, "_a2a_torch.Context", "Context", sizeof(Context), context_new, context_dealloc,
                   context_methods) ||
         !add_type(m, OperatorType, "_a2a_torch.Operator", "Operator", sizeof(Operator), operator_new, operator_dealloc,
                   operator_methods)) {

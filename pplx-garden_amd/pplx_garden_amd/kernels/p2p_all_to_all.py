@@ -120,7 +120,9 @@ class P2PAllToAll(AllToAllKernel):
 
         self._all_to_all = global_group.world.acquire_context(self._key, make_context)
         # dispatch() and combine() themselves: checks and calls in native code (a2a_torch.cpp)
-        self._operator = load_extension().Operator(
+        extension = load_extension()
+        _call_without_a_frame(extension)
+        self._operator = extension.Operator(
             self._all_to_all.shared, rank, self._dp_size, hidden_dim,
             -1 if hidden_dim_scale is None else hidden_dim_scale, self._num_local_experts, num_experts_per_token,
             in_dtype, out_dtype, scale_dtype is not None, -1 if self._device.index is None else self._device.index)
@@ -193,3 +195,15 @@ class P2PAllToAll(AllToAllKernel):
             self._all_to_all = None
             self._operator = None
             self._global_group.world.release_context(self._key)
+
+
+_DEFINED = {name: P2PAllToAll.__dict__[name] for name in ("dispatch", "combine")}
+
+
+def _call_without_a_frame(extension) -> None:
+    """From the first operator on, `op.dispatch` and `op.combine` are the native operator's methods (same names, defaults and
+    checks); looked up on the class, and after `destroy()`, they are the functions above.  What somebody else has put in their
+    place in the class stays."""
+    for name, function in _DEFINED.items():
+        if P2PAllToAll.__dict__.get(name) is function:
+            setattr(P2PAllToAll, name, extension.Method(name, function))
