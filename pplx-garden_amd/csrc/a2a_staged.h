@@ -33,7 +33,9 @@ struct Staging {
     uint32_t *source_position = nullptr; // [N][max_recv]
     uint32_t *source_dispatch_offset = nullptr;  // [N][max_recv]  a2a_worker.rs:636-656
     uint32_t *combine_send_offset = nullptr;     // [N][max_recv]  a2a_worker.rs:659-667
-    uint32_t *source_row = nullptr;      // [N][max_recv]: staged row a received row is copied from (sender * max_tokens + token)
+    uint4 *moves = nullptr;              // [N][max_recv]: what the copies need of a received row, side by side: its row in the
+                                         // receiver's buffer, the staged row it comes from (sender * max_tokens + token), its
+                                         // source and its position there
     uint32_t *num_recv = nullptr;        // [N][2]: received rows, rows from other nodes
     size_t disp_stride = 0;
     size_t comb_stride = 0;
@@ -54,7 +56,7 @@ struct StageSendArgs {
     uint32_t resolver_wave;   // resolving send: wavefront that resolves the routes (set by the launcher)
 };
 
-// A grid of wavefronts over the pieces (64 or 128 sixteen-byte chunks) of a receiver's rows.
+// A grid of wavefronts over the pieces (128 sixteen-byte chunks) of a receiver's rows.
 struct PieceGrid {
     uint32_t pieces;          // of a row
     uint32_t magic;           // n / pieces = mulhi(n, magic) for the wavefronts of a grid (0 for one piece a row)

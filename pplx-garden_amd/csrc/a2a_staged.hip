@@ -1108,6 +1108,8 @@ __global__ __launch_bounds__(1024) void stage_send_resolve_kernel(const StageSen
 }
 
 constexpr uint32_t kPieceThreads = 256;   // threads of a workgroup of the kernels that copy rows in pieces
+constexpr uint32_t kPieceLoads = 2;       // sixteen-byte chunks of a piece that a lane moves, both in flight
+constexpr uint32_t kPieceChunks = kPieceLoads * kWave;
 
 // A team of `team` threads (one or more whole wavefronts) copies a staged row of `num_chunks` 16-byte pieces:
 // eight loads per thread in flight.  Ordinary loads, because the recvs of the other ranks its token was routed to read
@@ -1493,7 +1495,7 @@ __device__ __forceinline__ void lay_out_rows(const StageRecvArgs &args, const Wo
         // the token behind the position: asked for first, used last
         const uint32_t token = m.pos < ws.max_tk ? st.pos_token[(size_t)m.g * ws.max_tk + m.pos] : 0;
         write_row_tables(t, ws, st, r, row, m, args.max_private);
-        st.source_row[(size_t)r * st.max_recv + row] = m.g * st.max_tokens + token;
+        st.moves[(size_t)r * st.max_recv + row] = uint4{m.dst_row, m.g * st.max_tokens + token, m.g, m.pos};
     }
 }
 
@@ -1557,7 +1559,7 @@ __global__ __launch_bounds__(1024) void stage_recv_first_few_kernel(const StageR
         const uint32_t token = st.pos_token[(size_t)m.g * ws.max_tk + m.pos];
         if (tid == 0) {
             write_row_tables(t, ws, st, r, row, m, args.max_private);
-            st.source_row[(size_t)r * st.max_recv + row] = m.g * st.max_tokens + token;
+            st.moves[(size_t)r * st.max_recv + row] = uint4{m.dst_row, m.g * st.max_tokens + token, m.g, m.pos};
         }
         if (dst.out_x != nullptr) {
             if (m.dst_row >= dst.out_rows) {
@@ -1594,7 +1596,7 @@ __global__ __launch_bounds__(1024) void stage_layout_kernel(const StageRecvArgs 
     lay_out_rows(args, ws, st, r, blockIdx.x - r * args.slices, s_recv, s_order);
 }
 
-// Rows cut into pieces of 64 sixteen-byte chunks, a wavefront each: wavefront w of the grid takes the
+// Rows cut into pieces of kPieceChunks sixteen-byte chunks, a wavefront each: wavefront w of the grid takes the
 // pieces w, w + wavefronts, ... of all rows counted through.
 struct PieceWalk {
     uint32_t row, piece;
@@ -1616,7 +1618,7 @@ struct PieceWalk {
 // A recv that did not lay the receivers out.  It only moves rows, and what bounds it is the write side of
 // HBM while the reads can come from the Infinity Cache: every staged row is read by the recvs of all the
 // ranks its token was routed to.  Hence
-//  - the rows are walked in the order of arrival by a grid of wavefronts, one 16-byte chunk a lane, so that
+//  - the rows are walked in the order of arrival by a grid of wavefronts, two 16-byte chunks a lane, so that
 //    reads and writes each advance as ONE front through memory.  A wavefront per row with eight chunks a
 //    lane in flight kept 4096 rows half open at a time: rows of 7392 bytes, 16384 a launch (8 ranks x 2048
 //    tokens), 52.1 us = 4.65 TB/s of reads and writes then, 42.1 us in this order;
@@ -1644,8 +1646,7 @@ __global__ __launch_bounds__(kPieceThreads) void stage_recv_kernel(const StageRe
     A2A_PIN(args.grid.step_rows);
     A2A_PIN(args.grid.step_pieces);
     A2A_PIN(st.send_buf);
-    A2A_PIN(st.padded_index);
-    A2A_PIN(st.source_row);
+    A2A_PIN(st.moves);
     A2A_PIN(st.num_recv);
     A2A_PIN(st.disp_stride);
     A2A_PIN(st.payload_bytes);
@@ -1655,15 +1656,13 @@ __global__ __launch_bounds__(kPieceThreads) void stage_recv_kernel(const StageRe
     const uint32_t lane = tid & (kWave - 1);
     const PushDst &dst = args.dst;
     const uint32_t num_chunks = args.row_bytes / 16;
-    const uint32_t *padded_index = st.padded_index + (size_t)r * st.max_recv;
-    const uint32_t *source_row = st.source_row + (size_t)r * st.max_recv;
-    // The first piece's two table words are asked for together with the number of rows received
+    const uint4 *moves = st.moves + (size_t)r * st.max_recv;
+    // The first piece's table entry is asked for together with the number of rows received
     // (a row index the tables do not hold reads entry 0 and is dropped by the loop's bound).
     PieceWalk at;
     at.start(args.grid, __builtin_amdgcn_readfirstlane(blockIdx.x * (kPieceThreads / kWave) + tid / kWave));
     const uint32_t probe = at.row < st.max_recv ? at.row : 0;
-    uint32_t dst_row = padded_index[probe];
-    uint32_t from = source_row[probe];
+    uint4 move = moves[probe];
     uint32_t total = st.num_recv[2 * r];
     if (total > st.max_recv) total = st.max_recv;   // flagged by the layout: more rows than the region was sized for
 
@@ -1671,24 +1670,29 @@ __global__ __launch_bounds__(kPieceThreads) void stage_recv_kernel(const StageRe
     if (dst.out_x == nullptr) return;
 
     while (at.row < total) {
-        const uint8_t *src = st.send_buf + (size_t)from * st.disp_stride;
-        const uint32_t c = at.piece * kWave + lane;
+        const uint32_t dst_row = move.x;
+        const uint8_t *src = st.send_buf + (size_t)move.y * st.disp_stride;
+        const uint32_t chunk = at.piece * kPieceChunks + lane, c = at.piece * kWave + lane;   // c: of the scales
         const bool fits = dst_row < dst.out_rows;
-        const bool active = fits && c < num_chunks;
         const bool scaled = fits && dst.out_scale != nullptr && c < args.hidden_dim_scale;
-        u32x4 v = {0, 0, 0, 0};
+        u32x4 v[kPieceLoads];
         float scale = 0.0f;
-        if (active) v = reinterpret_cast<const u32x4 *>(src)[c];
+#pragma unroll
+        for (uint32_t u = 0; u < kPieceLoads; ++u) {
+            v[u] = u32x4{0, 0, 0, 0};
+            if (fits && chunk + u * kWave < num_chunks) v[u] = reinterpret_cast<const u32x4 *>(src)[chunk + u * kWave];
+        }
         if (scaled) scale = reinterpret_cast<const float *>(src + st.payload_bytes)[c];
-        // the next piece's words travel while this one is copied
+        // the next piece's entry travels while this one is copied
         PieceWalk next = at;
         next.advance(args.grid);
         const uint32_t next_probe = next.row < total ? next.row : at.row;
-        const uint32_t next_dst = padded_index[next_probe];
-        const uint32_t next_from = source_row[next_probe];
-        if (active) {
-            u32x4 *const to = reinterpret_cast<u32x4 *>(dst.out_x + (size_t)dst_row * dst.out_stride) + c;
-            if constexpr (STREAM) __builtin_nontemporal_store(v, to); else store_copy(v, to);
+        const uint4 next_move = moves[next_probe];
+        u32x4 *const to = reinterpret_cast<u32x4 *>(dst.out_x + (size_t)dst_row * dst.out_stride) + chunk;
+#pragma unroll
+        for (uint32_t u = 0; u < kPieceLoads; ++u) {
+            if (!fits || chunk + u * kWave >= num_chunks) continue;
+            if constexpr (STREAM) __builtin_nontemporal_store(v[u], to + u * kWave); else store_copy(v[u], to + u * kWave);
         }
         if (scaled) dst.out_scale[(size_t)dst_row * dst.os_stride_token + (size_t)c * dst.os_stride_elem] = scale;
         if (fits && dst.out_scale != nullptr) {
@@ -1700,8 +1704,7 @@ __global__ __launch_bounds__(kPieceThreads) void stage_recv_kernel(const StageRe
         }
         if (!fits && at.piece == 0 && lane == 0) atomicOr(ws.err, A2A_DEV_RECV_OVERFLOW);
         at = next;
-        dst_row = next_dst;
-        from = next_from;
+        move = next_move;
     }
 }
 
@@ -1711,11 +1714,9 @@ __global__ __launch_bounds__(kPieceThreads) void stage_recv_kernel(const StageRe
 // (a2a_combine_send.cu:124-136,196-205).  Walked in pieces as stage_recv_kernel is, and for the same
 // reason: in the order of arrival the rows written are consecutive per source and the rows read per
 // (source, expert), so both sides are fronts through memory.  16384 rows of 14 KB: 105.5 us = 4.45 TB/s
-// with a wavefront per row, 76.5 us = 6.1 TB/s in this order (a plain copy of as many rows in the same
-// order, examples/ceilings.hip: 67.6 us; both sides come from and go to HBM, so loads and stores keep nothing).
-// U: chunks a lane has in flight, one piece being 64 * U chunks (kTwoChunkRows).
+// with a wavefront per row, 76.5 us = 6.1 TB/s in this order with one chunk a lane (a plain copy of as many rows in the
+// same order, examples/ceilings.hip: 67.6 us; both sides come from and go to HBM, so loads and stores keep nothing).
 // ---------------------------------------------------------------------------
-template <uint32_t U>
 __global__ __launch_bounds__(kPieceThreads) void combine_send_kernel(const CombineSendArgs args, const Workspace ws,
                                                                      const Staging st) {
     // everything a wavefront takes from the argument block, asked for in one go
@@ -1727,57 +1728,45 @@ __global__ __launch_bounds__(kPieceThreads) void combine_send_kernel(const Combi
     A2A_PIN(args.grid.magic);
     A2A_PIN(args.grid.step_rows);
     A2A_PIN(args.grid.step_pieces);
-    A2A_PIN(ws.dp_size);
     A2A_PIN(ws.max_tk);
     A2A_PIN(st.comb_buf);
-    A2A_PIN(st.padded_index);
-    A2A_PIN(st.source_rank);
-    A2A_PIN(st.source_position);
+    A2A_PIN(st.moves);
     A2A_PIN(st.comb_stride);
     A2A_PIN(st.max_recv);
     const uint32_t r = args.rank;
     const uint32_t lane = threadIdx.x & (kWave - 1);
     const uint32_t num_chunks = args.row_bytes / 16;
-    const uint32_t *padded_index = st.padded_index + (size_t)r * st.max_recv;
-    const uint32_t *source_rank = st.source_rank + (size_t)r * st.max_recv;
-    const uint32_t *source_position = st.source_position + (size_t)r * st.max_recv;
+    const uint4 *moves = st.moves + (size_t)r * st.max_recv;
     PieceWalk at;
     at.start(args.grid, __builtin_amdgcn_readfirstlane(blockIdx.x * (kPieceThreads / kWave) + threadIdx.x / kWave));
     const uint32_t probe = at.row < st.max_recv ? at.row : 0;
-    uint32_t row = padded_index[probe];
-    uint32_t peer = source_rank[probe];
-    uint32_t pos = source_position[probe];
+    uint4 move = moves[probe];
     uint32_t total = st.num_recv[2 * r];
     if (total > st.max_recv) total = st.max_recv;
     while (at.row < total) {
-        const uint32_t c = at.piece * (U * kWave) + lane;
+        const uint32_t c = at.piece * kPieceChunks + lane;
+        const uint32_t row = move.x, g = move.z, pos = move.w;   // (every member of a dp group reads the same staging rows)
         const bool fits = row < args.y_rows && pos < ws.max_tk;
         const u32x4 *const from = reinterpret_cast<const u32x4 *>(args.y + (size_t)row * args.y_stride) + c;
-        u32x4 v[U];
+        u32x4 v[kPieceLoads];
 #pragma unroll
-        for (uint32_t u = 0; u < U; ++u) {
+        for (uint32_t u = 0; u < kPieceLoads; ++u) {
             v[u] = u32x4{0, 0, 0, 0};
             if (fits && c + u * kWave < num_chunks) v[u] = __builtin_nontemporal_load(from + u * kWave);
         }
-        // the next piece's words travel while this one is copied
+        // the next piece's entry travels while this one is copied
         PieceWalk next = at;
         next.advance(args.grid);
         const uint32_t next_probe = next.row < total ? next.row : at.row;
-        const uint32_t next_row = padded_index[next_probe];
-        const uint32_t next_peer = source_rank[next_probe];
-        const uint32_t next_pos = source_position[next_probe];
-        // every member of the source's dp group reads the same staging rows
-        const uint32_t g = ws.dp_size > 1 ? peer / ws.dp_size : peer;
+        const uint4 next_move = moves[next_probe];
         u32x4 *const to = reinterpret_cast<u32x4 *>(st.comb_buf + ((size_t)g * ws.max_tk + pos) * st.comb_stride) + c;
 #pragma unroll
-        for (uint32_t u = 0; u < U; ++u) {
+        for (uint32_t u = 0; u < kPieceLoads; ++u) {
             if (fits && c + u * kWave < num_chunks) store_copy(v[u], to + u * kWave);
         }
         if (!fits && at.piece == 0 && lane == 0) atomicOr(ws.err, A2A_DEV_BAD_SLOT);
         at = next;
-        row = next_row;
-        peer = next_peer;
-        pos = next_pos;
+        move = next_move;
     }
 }
 
@@ -1791,28 +1780,25 @@ uint32_t block_for_chunks(uint32_t chunks) {
 // The rows of a receiver are copied in pieces by a grid of wavefronts that walks all pieces of all rows in
 // order.  The host knows an upper bound of the rows (every copy of every sender); a receiver typically gets
 // 1/N of it.
-//   - recv: at most 2048 workgroups, the wavefronts that fit the GPU at once (4096 and 8192 workgroups: 43.7 and
-//     43.9 us against 42.1 at 16384 rows of 7 KB).
-//   - combine-send (`in_order`): more workgroups than fit, so that a wavefront of the typical receiver has three
-//     pieces and the hardware, which starts workgroups in order, keeps the front of its 14 KB rows tight: 16384
-//     rows (57344 workgroups' worth of pieces) 88.0 / 86.7 / 82.8 / 78.9 us with 2048 / 4096 / 8192 / 16384 workgroups.
-//     Not more, because the grid is sized for the upper bound and workgroups without rows cost as well:
-//     4096 rows 21.0 / 20.4 / 21.0 / 24.0.
-//     Where a receiver typically gets up to kTwoChunkRows rows, pieces of twice the size and two of them a wavefront: half
-//     the look-ups, and both loads of a piece in flight.  Whole split steps, us, one chunk a lane / two: 8 x 128 tokens 187.8 /
-//     186.0 (rows of 8 KB 147.1 / 144.2, of 2 KB 105.5 / 102.8), 8 x 512 418.6 / 413.8, 8 x 1500 1036.7 / 1030.6, one sender of 4096
-//     367.1 / 361.3; beyond, the tight front is worth more: 8 x 2048 1391 / 1396, 4 x 3000 983 / 993.
+//   - combine-send, and recvs of receivers that typically get kInOrderRows rows (`in_order`): a wavefront per piece of the
+//     typical receiver (more loop), so that the hardware, which starts workgroups in order, keeps the front of reads and
+//     writes tight, but not fewer than the wavefronts that fit the GPU at once.
+//   - other recvs: 2048 workgroups, those that fit (4096 and 8192: 43.7 and 43.9 us against 42.1 at 16384 rows of 7 KB, one
+//     chunk a lane).
+// Two chunks a lane instead of one, one table entry instead of three words, whole split steps, us: 8 x 128 tokens of 14 KB
+// bf16 rows 187.8 -> 184.1 (of 8 KB 147 -> 143, of 2 KB 105.5 -> 100.4), 8 x 512 of 7 KB 418.6 -> 407.4, one sender of 4096
+// 367.1 -> 352.0, 8 x 2048 1391 -> 1362, 4 x 3000 983 -> 962.  In order or not (recv): 8 x 512 409.4 / 407.4, one sender of 4096
+// (4096 rows a receiver) 353.7 / 352.0, 8 x 2048 (16384) 1362 / 1372, 4 x 3000 (24000) 962 / 969.  Four chunks a lane in
+// the combine-send: 8 x 2048 1402 against 1380, the others level.
 constexpr uint32_t kPieceWorkgroups = 2048;
-constexpr uint32_t kTwoChunkRows = 12288;
+constexpr uint32_t kInOrderRows = 8192;
 
-// `chunks_a_lane`: 16-byte chunks of a row that a lane moves at once.
-uint32_t piece_grid(uint32_t max_rows, uint32_t world, uint32_t chunks, bool in_order, uint32_t chunks_a_lane, PieceGrid &grid) {
+uint32_t piece_grid(uint32_t max_rows, uint32_t world, uint32_t chunks, bool in_order, PieceGrid &grid) {
     constexpr uint32_t waves = kPieceThreads / kWave;
-    const uint32_t pieces_in_order = chunks_a_lane > 1 ? 2 : 3;
-    grid.pieces = (chunks + chunks_a_lane * kWave - 1) / (chunks_a_lane * kWave);
+    grid.pieces = (chunks + kPieceChunks - 1) / kPieceChunks;
     const uint64_t most = ((uint64_t)max_rows * grid.pieces + waves - 1) / waves;
     uint64_t blocks = kPieceWorkgroups;
-    if (in_order && most / world / pieces_in_order > blocks) blocks = most / world / pieces_in_order;
+    if (in_order && most / world > blocks) blocks = most / world;
     if (blocks > 1u << 16) blocks = 1u << 16;   // (keeps wavefront numbers far below 2^32 / pieces)
     if (blocks > most) blocks = most;
     if (blocks < 1) blocks = 1;
@@ -1869,7 +1855,7 @@ int staging_allocate(Staging &st, const a2a_config &cfg, std::string *error) {
     const size_t o_spos = carve(N * max_recv * sizeof(uint32_t));
     const size_t o_sdo = carve(N * max_recv * sizeof(uint32_t));
     const size_t o_cso = carve(N * max_recv * sizeof(uint32_t));
-    const size_t o_srow = carve(N * max_recv * sizeof(uint32_t));
+    const size_t o_moves = carve(N * max_recv * sizeof(uint4));
     const size_t o_nrecv = carve(N * 2 * sizeof(uint32_t));
     hipError_t e = hipMalloc(&st.arena, off);
     if (e != hipSuccess) {
@@ -1888,7 +1874,7 @@ int staging_allocate(Staging &st, const a2a_config &cfg, std::string *error) {
     st.source_position = reinterpret_cast<uint32_t *>(base + o_spos);
     st.source_dispatch_offset = reinterpret_cast<uint32_t *>(base + o_sdo);
     st.combine_send_offset = reinterpret_cast<uint32_t *>(base + o_cso);
-    st.source_row = reinterpret_cast<uint32_t *>(base + o_srow);
+    st.moves = reinterpret_cast<uint4 *>(base + o_moves);
     st.num_recv = reinterpret_cast<uint32_t *>(base + o_nrecv);
     // Tables are read before they are written only through misuse; start from zero.
     e = hipMemset(base + o_pos, 0, o_comb - o_pos);
@@ -2143,7 +2129,7 @@ hipError_t launch_stage_recv(const StageRecvArgs &args, const Workspace &ws, con
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
-    const uint32_t blocks = piece_grid(args.max_rows, ws.world, chunks, false, 1, a.grid);
+    const uint32_t blocks = piece_grid(args.max_rows, ws.world, chunks, typical >= kInOrderRows, a.grid);
     if (args.streamed) {
         hipExtLaunchKernelGGL(stage_recv_kernel<true>, dim3(blocks), dim3(kPieceThreads), 0, stream, timing.start,
                               timing.stop, 0, a, ws, st);
@@ -2159,15 +2145,9 @@ hipError_t launch_combine_send(const CombineSendArgs &args, const Workspace &ws,
     if (args.max_rows == 0) return hipSuccess;
     const uint32_t chunks = args.row_bytes / 16;
     CombineSendArgs a = args;
-    if ((args.max_rows + ws.world - 1) / ws.world <= kTwoChunkRows) {
-        const uint32_t blocks = piece_grid(args.max_rows, ws.world, chunks, true, 2, a.grid);
-        hipExtLaunchKernelGGL(combine_send_kernel<2>, dim3(blocks), dim3(kPieceThreads), 0, stream, timing.start,
-                              timing.stop, 0, a, ws, st);
-    } else {
-        const uint32_t blocks = piece_grid(args.max_rows, ws.world, chunks, true, 1, a.grid);
-        hipExtLaunchKernelGGL(combine_send_kernel<1>, dim3(blocks), dim3(kPieceThreads), 0, stream, timing.start,
-                              timing.stop, 0, a, ws, st);
-    }
+    const uint32_t blocks = piece_grid(args.max_rows, ws.world, chunks, true, a.grid);
+    hipExtLaunchKernelGGL(combine_send_kernel, dim3(blocks), dim3(kPieceThreads), 0, stream, timing.start, timing.stop,
+                          0, a, ws, st);
     return hipGetLastError();
 }
 
