@@ -47,6 +47,31 @@ __device__ __forceinline__ void store_copies(u32x4 v, uint64_t row_ptr, uint32_t
     }
 }
 
+// One scale of a copy.  Rows of scales share their first and last cache lines with the rows before and after, which
+// other compute units write: kept in a compute unit's L2 in the hope of the rest they cost the rows their place in it.
+// Stored non-temporally the pack of 4096 tokens (rows of 7168 bytes, 56 scales) takes 69.0 us for 70.7 and that of
+// 8 sources of 512 tokens (5120 bytes, 40 scales) 52.3 for 54.0, with and without a reader behind it; rows of 16 scales are
+// level and rows of 8, four to a line, lose (18.9 us for 18.5).  Scales stored by COLUMN are single words of lines that
+// have to meet somewhere (non-temporal: 68 us for 36), and copies that are stored past the Infinity Cache leave it to
+// the scales (non-temporal: 485 us for 454).
+constexpr uint32_t kScalesPastL2 = 32;   // a cache line of them
+
+template <int POLICY>
+__device__ __forceinline__ void store_scale(float scale, float *row, uint32_t j, uint32_t stride, uint32_t num_scales) {
+    if ((POLICY & kNonTemporal) == 0 && stride == 1 && num_scales >= kScalesPastL2) {
+        __builtin_nontemporal_store(scale, row + j);
+    } else {
+        row[(size_t)j * stride] = scale;
+        asm volatile("");   // keeps the two stores apart: merged into one they lose the policy
+    }
+}
+
+// Rows up to this size have the caller's scales asked for before the row: behind the row's stores their trip would begin
+// only when those have been acknowledged (memory operations of a wavefront complete in order).  2684 tokens of 5120 bytes,
+// scales by row: 34.6 -> 33.2 us, by column 38.9 -> 36.4; 8001 tokens 90.5 -> 85.4.  With four workgroups of 7168 bytes on
+// a compute unit that wait is what holds the stores in flight back, and without it 4096 tokens took 68.6 us for 66.0.
+constexpr uint32_t kScalesAheadBytes = 6144;
+
 // Moves the row of `token` to its copies.  Lanes 0..K-1 of EVERY wavefront hold
 // the row pointer, scale pointer and scale stride of route k (0 = no copy).
 // The row is loaded here, AFTER the routes are known, unless the caller passes
@@ -103,22 +128,27 @@ __device__ __forceinline__ void push_rows(const PushArgs &args, const PushSrc &s
             const uint32_t k = i / Hl;
             const uint32_t j = i - k * Hl;
             const uint64_t sp = s_scale_ptr[k];
-            if (sp != 0) reinterpret_cast<float *>(sp)[(size_t)j * s_scale_stride[k]] = s_scale[j];
+            if (sp != 0) store_scale<POLICY>(s_scale[j], reinterpret_cast<float *>(sp), j, s_scale_stride[k], Hs);
         }
     } else {
         const uint32_t num_chunks = live ? args.row_bytes / 16 : 0;
+        const bool scaled = src.x_scale != nullptr && live;
+        const float *const xs = src.x_scale + (size_t)token * src.xs_stride_token;
+        const bool ahead = args.row_bytes <= kScalesAheadBytes;
+        float first_scale = 0.0f;
+        if (scaled && ahead && tid < args.hidden_dim_scale) first_scale = xs[(size_t)tid * src.xs_stride_elem];
         for (uint32_t c = tid; c < num_chunks; c += team_threads) {
             const u32x4 v = PRE && c == tid ? pre_a : __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(x_row) + c);
             store_copies<POLICY>(v, row_ptr, K, num_chunks * 16, c * 16);
         }
-        if (src.x_scale != nullptr && live) {
-            const float *xs = src.x_scale + (size_t)token * src.xs_stride_token;
+        if (scaled) {
             for (uint32_t j = tid; j < args.hidden_dim_scale; j += team_threads) {
-                const float s = xs[(size_t)j * src.xs_stride_elem];
+                float s = first_scale;
+                if (!ahead || j != tid) s = xs[(size_t)j * src.xs_stride_elem];
                 for (uint32_t k = 0; k < K; ++k) {
                     const uint64_t sp = read_lane64(scale_ptr, k);
                     const uint32_t ss = __builtin_amdgcn_readlane((int)scale_stride, (int)k);
-                    if (sp != 0) reinterpret_cast<float *>(sp)[(size_t)j * ss] = s;
+                    if (sp != 0) store_scale<POLICY>(s, reinterpret_cast<float *>(sp), j, ss, args.hidden_dim_scale);
                 }
             }
         }
