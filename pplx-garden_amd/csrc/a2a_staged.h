@@ -73,6 +73,7 @@ struct StageRecvArgs {
     uint32_t max_rows;        // upper bound of received rows known to the host
     bool streamed;            // the copies are written past the Infinity Cache (received_past_cache)
     PieceGrid grid;           // set by the launcher
+    uint32_t scale_blocks;    // workgroups in front of the grid that move scales by column (launcher)
     // the first recv of a step only: it lays out every receiver
     uint32_t valid_mask;      // sources that sent tokens in this step (the others count as empty)
     uint32_t max_private;     // rows per source in the private part of a receive region (a2a_worker.rs:646-656)

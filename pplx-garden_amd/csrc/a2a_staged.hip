@@ -1627,8 +1627,48 @@ struct PieceWalk {
 //    non-temporally, which keeps THEM out of it: 37.0 us = 6.5 TB/s (rows of 14 KB, 235 MB staged: 84.3 -> 69.3 us;
 //    470 MB staged, more than the cache holds: 172 -> 143 us with non-temporal loads as the other side).
 // A row's scales travel with its first pieces; they are 3 us of the 42 (rows of scales are not whole cache
-// lines: their ends are written by two wavefronts at different times).
-template <bool STREAM>
+// lines: their ends are written by two wavefronts at different times).  Scales that the caller wants by COLUMN would be a
+// cache line a word that way, written by as many wavefronts as it has words: COLUMNS moves them in workgroups of their own in
+// front of the grid, a wavefront for kScaleColumns columns of 64 rows in the order of arrival, whose rows lie side by side run
+// by run (an expert's rows of one source).  Step of 8 x 2048 tokens of 7168 bytes 1422 -> 1382 us, of 8 x 400 353 -> 347, one
+// sender of 4096 367 -> 356.  Their chain (entries, staged words, stores) is longer than a piece's, so with few words to
+// move (kColumnWords, of a typical receiver) the pieces carry them: 1600 rows of 56 (90 thousand) 222 us against 225,
+// 4800 of 16 (77) 212 against 217, 8192 of 8 (66) 202 against 211; on the other side 2400 of 56 (134) 291 against 288, 2048 of
+// 56 (115) 210 against 208.6, 9600 of 16 (154) 332.5 against 329.7.
+constexpr uint32_t kScaleColumns = 8;
+constexpr uint64_t kColumnWords = 112 * 1024;
+
+// Whether scales of these strides are columns: the next row's word is nearer than the row's next word.
+__host__ __device__ __forceinline__ bool scales_by_column(const PushDst &dst) {
+    return dst.out_scale != nullptr && dst.os_stride_token < dst.os_stride_elem;
+}
+
+// The scales of the received rows, by column.  `unit`, `units`: of the wavefronts that do this.
+__device__ __forceinline__ void receive_scale_columns(const StageRecvArgs &args, const Workspace &ws, const Staging &st,
+                                                      const uint4 *moves, uint32_t total, uint32_t unit, uint32_t units) {
+    const uint32_t lane = threadIdx.x & (kWave - 1);
+    const uint32_t num_scales = args.hidden_dim_scale;
+    const uint32_t slices = (num_scales + kScaleColumns - 1) / kScaleColumns;
+    for (; unit / slices * kWave < total; unit += units) {
+        const uint32_t row = unit / slices * kWave + lane;
+        const uint32_t first = unit % slices * kScaleColumns;
+        const uint4 move = moves[row < total ? row : total - 1];
+        if (row >= total || move.x >= args.dst.out_rows) continue;   // (rows that do not fit are flagged where they are copied)
+        const u32x4 *from = reinterpret_cast<const u32x4 *>(st.send_buf + (size_t)move.y * st.disp_stride + st.payload_bytes) +
+                            first / 4;
+        float *to = args.dst.out_scale + (size_t)move.x * args.dst.os_stride_token + (size_t)first * args.dst.os_stride_elem;
+        // (a staged row has 16 spare bytes behind its scales)
+        u32x4 v[kScaleColumns / 4];
+#pragma unroll
+        for (uint32_t i = 0; i < kScaleColumns / 4; ++i) v[i] = first + 4 * i < num_scales ? from[i] : u32x4{0, 0, 0, 0};
+#pragma unroll
+        for (uint32_t j = 0; j < kScaleColumns; ++j) {
+            if (first + j < num_scales) to[(size_t)j * args.dst.os_stride_elem] = __uint_as_float(v[j / 4][j % 4]);
+        }
+    }
+}
+
+template <bool STREAM, bool COLUMNS>
 __global__ __launch_bounds__(kPieceThreads) void stage_recv_kernel(const StageRecvArgs args, const Workspace ws,
                                                                    const Staging st) {
     // everything a wavefront takes from the argument block, asked for in one go
@@ -1645,6 +1685,7 @@ __global__ __launch_bounds__(kPieceThreads) void stage_recv_kernel(const StageRe
     A2A_PIN(args.grid.magic);
     A2A_PIN(args.grid.step_rows);
     A2A_PIN(args.grid.step_pieces);
+    if constexpr (COLUMNS) A2A_PIN(args.scale_blocks);
     A2A_PIN(st.send_buf);
     A2A_PIN(st.moves);
     A2A_PIN(st.num_recv);
@@ -1660,13 +1701,21 @@ __global__ __launch_bounds__(kPieceThreads) void stage_recv_kernel(const StageRe
     // The first piece's table entry is asked for together with the number of rows received
     // (a row index the tables do not hold reads entry 0 and is dropped by the loop's bound).
     PieceWalk at;
-    at.start(args.grid, __builtin_amdgcn_readfirstlane(blockIdx.x * (kPieceThreads / kWave) + tid / kWave));
+    const uint32_t scale_blocks = COLUMNS ? args.scale_blocks : 0;
+    const uint32_t block = blockIdx.x - scale_blocks;   // (wraps around for the workgroups in front: they move scales)
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    at.start(args.grid, COLUMNS && blockIdx.x < scale_blocks ? 0 : block * (kPieceThreads / kWave) + wave);
     const uint32_t probe = at.row < st.max_recv ? at.row : 0;
     uint4 move = moves[probe];
     uint32_t total = st.num_recv[2 * r];
     if (total > st.max_recv) total = st.max_recv;   // flagged by the layout: more rows than the region was sized for
 
-    if (blockIdx.x == 0) hand_over_counts(args, ws, dst.out_rows);
+    if (COLUMNS && blockIdx.x < scale_blocks) {
+        receive_scale_columns(args, ws, st, moves, total, blockIdx.x * (kPieceThreads / kWave) + wave,
+                              scale_blocks * (kPieceThreads / kWave));
+        return;
+    }
+    if (block == 0) hand_over_counts(args, ws, dst.out_rows);
     if (dst.out_x == nullptr) return;
 
     while (at.row < total) {
@@ -1674,7 +1723,7 @@ __global__ __launch_bounds__(kPieceThreads) void stage_recv_kernel(const StageRe
         const uint8_t *src = st.send_buf + (size_t)move.y * st.disp_stride;
         const uint32_t chunk = at.piece * kPieceChunks + lane, c = at.piece * kWave + lane;   // c: of the scales
         const bool fits = dst_row < dst.out_rows;
-        const bool scaled = fits && dst.out_scale != nullptr && c < args.hidden_dim_scale;
+        const bool scaled = !COLUMNS && fits && dst.out_scale != nullptr && c < args.hidden_dim_scale;
         u32x4 v[kPieceLoads];
         float scale = 0.0f;
 #pragma unroll
@@ -1695,7 +1744,7 @@ __global__ __launch_bounds__(kPieceThreads) void stage_recv_kernel(const StageRe
             if constexpr (STREAM) __builtin_nontemporal_store(v[u], to + u * kWave); else store_copy(v[u], to + u * kWave);
         }
         if (scaled) dst.out_scale[(size_t)dst_row * dst.os_stride_token + (size_t)c * dst.os_stride_elem] = scale;
-        if (fits && dst.out_scale != nullptr) {
+        if (!COLUMNS && fits && dst.out_scale != nullptr) {
             // rows with more scales than pieces have lanes
             for (uint32_t q = c + args.grid.pieces * kWave; q < args.hidden_dim_scale; q += args.grid.pieces * kWave) {
                 dst.out_scale[(size_t)dst_row * dst.os_stride_token + (size_t)q * dst.os_stride_elem] =
@@ -2130,13 +2179,25 @@ hipError_t launch_stage_recv(const StageRecvArgs &args, const Workspace &ws, con
         if (e != hipSuccess) return e;
     }
     const uint32_t blocks = piece_grid(args.max_rows, ws.world, chunks, typical >= kInOrderRows, a.grid);
-    if (args.streamed) {
-        hipExtLaunchKernelGGL(stage_recv_kernel<true>, dim3(blocks), dim3(kPieceThreads), 0, stream, timing.start,
-                              timing.stop, 0, a, ws, st);
-    } else {
-        hipExtLaunchKernelGGL(stage_recv_kernel<false>, dim3(blocks), dim3(kPieceThreads), 0, stream, timing.start,
-                              timing.stop, 0, a, ws, st);
+    // Scales by column: a wavefront for every kScaleColumns columns of 64 rows that the receiver typically gets.
+    const bool columns = args.dst.out_x != nullptr && scales_by_column(args.dst) &&
+                         (uint64_t)typical * args.hidden_dim_scale >= kColumnWords;
+    a.scale_blocks = 0;
+    if (columns) {
+        const uint64_t units = ((uint64_t)typical + kWave - 1) / kWave *
+                               ((args.hidden_dim_scale + kScaleColumns - 1) / kScaleColumns);
+        const uint64_t blocks_of_units = (units + kPieceThreads / kWave - 1) / (kPieceThreads / kWave);
+        a.scale_blocks = blocks_of_units < 1 ? 1 : blocks_of_units < kPieceWorkgroups ? (uint32_t)blocks_of_units : kPieceWorkgroups;
     }
+#define A2A_LAUNCH_RECV(STREAM, COLUMNS)                                                                            \
+    hipExtLaunchKernelGGL((stage_recv_kernel<STREAM, COLUMNS>), dim3(blocks + a.scale_blocks), dim3(kPieceThreads), 0, \
+                          stream, timing.start, timing.stop, 0, a, ws, st)
+    if (args.streamed) {
+        if (columns) A2A_LAUNCH_RECV(true, true); else A2A_LAUNCH_RECV(true, false);
+    } else {
+        if (columns) A2A_LAUNCH_RECV(false, true); else A2A_LAUNCH_RECV(false, false);
+    }
+#undef A2A_LAUNCH_RECV
     return hipGetLastError();
 }
 

@@ -1,5 +1,6 @@
-"""Scales of the steps that are routed in a launch of their own (more than 16384 entries): the caller's, by row and by column,
-and those of quantised rows, at the sizes where their stores and loads change, against the oracle bit for bit."""
+"""Scales of the steps that are routed in a launch of their own (more than 16384 entries), the caller's, by row and by column,
+and those of quantised rows, and of the recvs that copy by pieces of rows: at the sizes where their stores and loads change,
+against the oracle bit for bit."""
 
 from dataclasses import replace
 
@@ -39,3 +40,22 @@ def test_quantised_rows(hidden):
     case = replace(scaled(C1, 1), hidden_dim=hidden, name="scales", num_tokens=2100, seed=77 + hidden)
     print(f"hidden={hidden}", flush=True)
     run_and_check(case, [2100, 0, 1, 0, 50, 0, 0, 3])
+
+
+# tokens, experts, top-k, hidden, scales
+RECEIVED = [
+    ([300, 0], 64, 8, 2560, 20),              # few words: they travel with the rows
+    ([3584, 3584], 16, 8, 512, 4),            # the smallest step whose columns have workgroups of their own
+    ([3583, 3584], 16, 8, 512, 4),            # a word below it
+    ([701, 3, 2650], 9, 8, 3968, 31),         # a last slice of seven columns, a last block of some rows
+    ([1, 900, 900, 0], 4, 4, 4352, 136),      # one expert a rank
+]
+
+
+@pytest.mark.parametrize("tokens,experts,topk,hidden,scales", RECEIVED, ids=[f"{s[0]}_h{s[3]}_s{s[4]}" for s in RECEIVED])
+def test_received_columns(tokens, experts, topk, hidden, scales):
+    print(f"tokens={tokens} hidden={hidden} scales={scales}", flush=True)
+    cfg = RefConfig("columns", len(tokens), 1, max(tokens), experts, hidden, scales, topk, FP8, BF16, F32, expert_padding=4)
+    world = [make_ref_rank(cfg, r, t) for r, t in enumerate(tokens)]
+    rows = rows_for(cfg, world)
+    check(cfg, world, rows, run_gpu(cfg, world, rows, DEV, split=True, scale_layout="col"))
