@@ -85,7 +85,8 @@ constexpr uint32_t kScalesAheadBytes = 6144;
 // passes `live` false.
 // PRE: the thread's first piece of the row was asked for earlier (first_piece) and is passed in.
 // POLICY: cache policy of the copies' stores.
-template <bool QUANT, bool PRE = false, int POLICY = QUANT ? kDeviceScope : kOrdinary>
+// SCALES: whether the caller's scales are moved too (quantised rows always have theirs).
+template <bool QUANT, bool PRE = false, int POLICY = QUANT ? kDeviceScope : kOrdinary, bool SCALES = true>
 __device__ __forceinline__ void push_rows(const PushArgs &args, const PushSrc &src, uint32_t token, uint32_t K,
                                           uint64_t row_ptr, uint64_t scale_ptr, uint32_t scale_stride,
                                           float *s_scale, uint64_t *s_scale_ptr, uint32_t *s_scale_stride,
@@ -132,7 +133,7 @@ __device__ __forceinline__ void push_rows(const PushArgs &args, const PushSrc &s
         }
     } else {
         const uint32_t num_chunks = live ? args.row_bytes / 16 : 0;
-        const bool scaled = src.x_scale != nullptr && live;
+        const bool scaled = SCALES && src.x_scale != nullptr && live;
         const float *const xs = src.x_scale + (size_t)token * src.xs_stride_token;
         const bool ahead = args.row_bytes <= kScalesAheadBytes;
         float first_scale = 0.0f;
@@ -2038,6 +2039,160 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8))) void 
     }
 }
 
+// Scales by column (the next row's word is nearer than the row's next word).  Word by word beside the rows each of them is a
+// cache line touched by a workgroup of its own, on any of eight L2s.  The resolving pack moves the caller's in workgroups of
+// their own instead, in front of those of the tokens: each takes kSpanChunks chunks of a source's entries, sorts them by
+// expert in LDS, so that the rows of an expert lie side by side, and moves kScaleColumns columns of them.
+// What bounds them is their chain of trips to a saturated memory, so there are four: the bound, everything the rows'
+// places are made of, all the scales (a 16-byte load an entry), all the stores.
+// (With a trip or more for each round of entries: 39 us for the 2684 tokens below.)  Beside the rows / in workgroups of their own,
+// whole steps: 2684 tokens of 5120 bytes 79.2 / 75.8 us, 8 x 512 of 7168 166.4 / 161.9, of 2048 tokens and two
+// experts each 252 / 224, one sender of 3000 with 4096 bytes 72.6 / 68.7.  Eight or sixteen columns a workgroup: 78.3 and 84.5 of
+// the first, level from 4096 tokens on.  Copies that are stored past the Infinity Cache keep their scales: 1165 us
+// against 1122 for 8 x 4096 tokens, whose column words then meet in no cache.
+constexpr uint32_t kScaleColumns = 4;                         // one 16-byte load
+constexpr uint32_t kSpanChunks = 2;
+constexpr uint32_t kSpan = kSpanChunks * kRouteBlock;
+constexpr uint32_t kColumnThreads = 256;                      // at least (rows from 4 KB on): an entry per thread and round are all
+constexpr uint32_t kColumnRounds = kSpan / kColumnThreads;
+
+struct ScaleColumns {
+    uint32_t blocks;   // workgroups that move scales by column
+    uint32_t slices;   // of kScaleColumns columns
+};
+
+// Workgroup `unit` of those.  Dynamic LDS: kSpan + 3 * E words.
+__device__ __forceinline__ void push_scale_columns(const PushArgs &args, const Workspace &ws, const ScaleColumns &columns,
+                                                   uint32_t unit, const uint32_t *per_source, const uint32_t *per_expert,
+                                                   uint32_t *lds, uint32_t *scratch) {
+    __shared__ uint64_t s_to[kMaxWorld];        // per receiver: where its first scale is (0: none wanted),
+    __shared__ uint32_t s_stride[kMaxWorld];    // the stride of its rows
+    __shared__ uint32_t s_elem[kMaxWorld];      // and of its columns,
+    __shared__ uint32_t s_rows[kMaxWorld];      // how many rows it has
+    __shared__ uint32_t s_rank[kMaxWorld];      // and the padded rows of the receivers before it, negated
+    __shared__ uint32_t s_carry[2];
+    const uint32_t tid = threadIdx.x, nthreads = blockDim.x;
+    const uint32_t G = ws.num_groups, E = ws.num_experts, K = ws.topk, Le = ws.experts_per_rank;
+    uint32_t *const s_list = lds;               // [kSpan]: place of the entry in the span | expert << 16
+    uint32_t *const s_first = lds + kSpan;      // [2][E]: where the entries of a chunk begin in the list
+    uint32_t *const s_base = s_first + 2 * E;   // [E]
+    uint32_t span = unit / columns.slices;
+    const uint32_t first_column = (unit - span * columns.slices) * kScaleColumns;
+    uint32_t g = 0;
+    for (; g + 1 < G; ++g) {
+        const uint32_t spans = ((args.token_start[g + 1] - args.token_start[g]) * K + kSpan - 1) / kSpan;
+        if (span < spans) break;
+        span -= spans;
+    }
+    const PushSrc &src = args.src[g];
+    const uint32_t entries = effective_tokens(src.bound_m, src.num_tokens) * K;
+    const uint32_t first = span * kSpan;
+    if (src.x_scale == nullptr || first >= entries) return;
+    const uint32_t here = entries - first < kSpan ? entries - first : kSpan;
+    const uint32_t chunk0 = span * kSpanChunks;
+    const bool two = here > kRouteBlock;        // the second chunk has entries
+    const uint32_t *counts = ws.chunk_counts + (size_t)g * E * ws.nb_max;   // [E][nb_max]
+    const uint32_t pad = ws.expert_padding;
+    const bool alone = args.single_source != 0;
+
+    // The entries travel together with the tables.
+    uint32_t id[kColumnRounds], place[kColumnRounds];
+#pragma unroll
+    for (uint32_t q = 0; q < kColumnRounds; ++q) {
+        const uint32_t i = q * nthreads + tid;
+        const uint32_t entry = first + (i < here ? i : 0), token = entry / K;
+        id[q] = (uint32_t)src.indices[(size_t)token * src.indices_stride + (entry - token * K)];
+        place[q] = ws.local_rank[(size_t)g * ws.max_tk + entry];
+    }
+    if (tid < ws.world) {
+        const PushDst &dst = args.dst[tid];
+        s_to[tid] = dst.out_x != nullptr ? (uint64_t)dst.out_scale : 0;
+        s_stride[tid] = dst.os_stride_token;
+        s_elem[tid] = dst.os_stride_elem;
+        s_rows[tid] = dst.out_rows;
+    }
+    // Per expert: where its entries begin in the list, and the row of an entry as the sum of its place in the
+    // list, s_base and s_rank (modulo 2^32); the terms are those of the resolving wavefronts below.
+    uint32_t rows_before = 0, listed = 0;
+    for (uint32_t e0 = 0; e0 < E; e0 += nthreads) {
+        const bool valid = e0 + tid < E;
+        const uint32_t e = valid ? e0 + tid : 0;
+        const uint32_t r = owner_of_expert(ws, e);
+        const uint32_t *mine = counts + (size_t)e * ws.nb_max;
+        const uint32_t before = alone ? 0 : ws.laid_before[r * G + g];
+        uint32_t rows = per_expert[e];
+        uint32_t in_first = mine[chunk0], in_second = mine[two ? chunk0 + 1 : chunk0];
+        uint32_t v_chunk[8], v_source[8];
+#pragma unroll
+        for (uint32_t n = 0; n < 8; ++n) {
+            v_chunk[n] = mine[n < chunk0 ? n : 0];
+            v_source[n] = alone ? 0 : per_source[e * G + (n < G ? n : 0)];
+        }
+        uint32_t base = 0;
+#pragma unroll
+        for (uint32_t n = 0; n < 8; ++n) {
+            base += n < chunk0 ? v_chunk[n] : 0;
+            base += n < G && (before >> n & 1) ? v_source[n] : 0;
+        }
+        // longer sums
+        for (uint32_t n0 = 8; n0 < chunk0; n0 += 8) {
+#pragma unroll
+            for (uint32_t n = 0; n < 8; ++n) v_chunk[n] = mine[n0 + n < chunk0 ? n0 + n : 0];
+#pragma unroll
+            for (uint32_t n = 0; n < 8; ++n) base += n0 + n < chunk0 ? v_chunk[n] : 0;
+        }
+        for (uint32_t n = 8; n < G && !alone; ++n) base += before >> n & 1 ? per_source[e * G + n] : 0;
+        if (pad > 1) rows = (rows + pad - 1) / pad * pad;
+        if (!valid) rows = in_first = 0;
+        if (!valid || !two) in_second = 0;
+        const uint32_t to_rows = rows_before + block_inclusive_scan(rows, scratch);
+        const uint32_t to_list = listed + block_inclusive_scan(in_first + in_second, scratch);
+        const uint32_t begins = to_list - in_first - in_second;
+        if (valid) {
+            s_first[e] = begins;
+            s_first[E + e] = begins + in_first;
+            s_base[e] = base + (to_rows - rows) - begins;
+            if (e == r * Le) s_rank[r] = 0u - (to_rows - rows);
+        }
+        if (tid == nthreads - 1) {
+            s_carry[0] = to_rows;
+            s_carry[1] = to_list;
+        }
+        __syncthreads();
+        rows_before = s_carry[0];
+        listed = s_carry[1];
+    }
+#pragma unroll
+    for (uint32_t q = 0; q < kColumnRounds; ++q) {
+        const uint32_t i = q * nthreads + tid;
+        if (i < here && id[q] < E) s_list[s_first[(i < kRouteBlock ? 0 : E) + id[q]] + place[q]] = i | id[q] << 16;
+    }
+    __syncthreads();
+    if (listed == 0) return;
+
+    const float *from = src.x_scale + first_column;
+    u32x4 v[kColumnRounds];
+#pragma unroll
+    for (uint32_t q = 0; q < kColumnRounds; ++q) {
+        const uint32_t i = q * nthreads + tid;
+        const uint32_t token = (first + (s_list[i < listed ? i : 0] & 0xFFFFu)) / K;
+        v[q] = *reinterpret_cast<const u32x4 *>(from + (size_t)token * src.xs_stride_token);
+    }
+#pragma unroll
+    for (uint32_t q = 0; q < kColumnRounds; ++q) {
+        const uint32_t i = q * nthreads + tid;
+        if (i >= listed) break;
+        const uint32_t e = s_list[i] >> 16;
+        const uint32_t r = owner_of_expert(ws, e);
+        const uint32_t slot = i + s_base[e] + s_rank[r];
+        if (s_to[r] == 0 || slot >= s_rows[r]) continue;   // (a row that does not fit is flagged beside it)
+        const size_t elem = s_elem[r];
+        global_t<float> *to = global_ptr<float>(s_to[r]) + (size_t)slot * s_stride[r] + first_column * elem;
+#pragma unroll
+        for (uint32_t j = 0; j < kScaleColumns; ++j) to[j * elem] = __uint_as_float(v[q][j]);
+    }
+}
+
 // Pack of a large group step, after a routing launch that left, per chunk, the
 // histogram and the rank of every entry inside its chunk, and, for the whole
 // step, the totals per (source, expert) and per expert.  No launch in between
@@ -2052,9 +2207,10 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8))) void 
 // the grid holds one workgroup per receiver (expert counts for the caller,
 // layout tables) and one per source (its totals and their scan); the last of
 // them hands the totals over to the next step.
-template <bool QUANT, int POLICY>
-__global__ __launch_bounds__(1024) void dispatch_resolve_kernel(const PushArgs args, const FinalizeArgs fin,
-                                                                const Workspace ws) {
+// COLUMNS: the caller's scales go out by column (push_scale_columns, whose dynamic LDS it has).
+template <bool QUANT, int POLICY, bool COLUMNS = false>
+__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(COLUMNS ? 8 : 4))) void dispatch_resolve_kernel(const PushArgs args, const FinalizeArgs fin,
+                                                                const Workspace ws, const ScaleColumns columns) {
     __shared__ float s_scale[QUANT ? kMaxLdsScales : 1];
     __shared__ uint64_t s_scale_ptr[A2A_MAX_EXPERTS_PER_TOKEN];
     __shared__ uint32_t s_scale_stride[A2A_MAX_EXPERTS_PER_TOKEN];
@@ -2064,6 +2220,7 @@ __global__ __launch_bounds__(1024) void dispatch_resolve_kernel(const PushArgs a
     __shared__ uint32_t tot[A2A_MAX_EXPERTS + kMaxWorld];
     __shared__ uint32_t scratch[kRouteWaves];
     __shared__ uint32_t s_carry;
+    extern __shared__ uint32_t s_columns[];
 
     const uint32_t tid = threadIdx.x;
     const uint32_t lane = tid & (kWave - 1);
@@ -2078,7 +2235,14 @@ __global__ __launch_bounds__(1024) void dispatch_resolve_kernel(const PushArgs a
 
     // The receiver and source workgroups come first in the grid, so that they run
     // beside the token workgroups instead of after them.
-    const uint32_t extras = ws.world + G;
+    uint32_t extras = ws.world + G;
+    if constexpr (COLUMNS) {
+        extras += columns.blocks;
+        if (blockIdx.x >= ws.world + G && blockIdx.x < extras) {
+            push_scale_columns(args, ws, columns, blockIdx.x - (ws.world + G), per_source, per_expert, s_columns, scratch);
+            return;
+        }
+    }
     if (blockIdx.x < extras) {
         const uint32_t extra = blockIdx.x;
         if (extra < ws.world) {
@@ -2205,8 +2369,8 @@ __global__ __launch_bounds__(1024) void dispatch_resolve_kernel(const PushArgs a
         scale_ptr = s_route_scale_ptr[lane];
         scale_stride = s_route_scale_stride[lane];
     }
-    push_rows<QUANT, false, POLICY>(args, src, token, K, row_ptr, scale_ptr, scale_stride, s_scale, s_scale_ptr,
-                                    s_scale_stride, threadIdx.x, blockDim.x, true);
+    push_rows<QUANT, false, POLICY, !COLUMNS>(args, src, token, K, row_ptr, scale_ptr, scale_stride, s_scale, s_scale_ptr,
+                                              s_scale_stride, threadIdx.x, blockDim.x, true);
 }
 
 hipError_t launch_dispatch_push(const PushArgs &args, const Workspace &ws, bool quantize,
@@ -2475,6 +2639,25 @@ hipError_t launch_dispatch_sources(const PushArgs &args, const FinalizeArgs &fin
     return hipGetLastError();
 }
 
+// The workgroups that move the caller's scales by column: none for quantised rows, whose scales come about beside the rows,
+// none when a receiver wants them by row or a source's are not 16-byte pieces of four columns.
+static ScaleColumns plan_scale_columns(const PushArgs &args, const Workspace &ws, bool quantize, uint32_t threads) {
+    ScaleColumns columns = {0, args.hidden_dim_scale / kScaleColumns};
+    if (quantize || columns.slices == 0 || args.hidden_dim_scale % kScaleColumns != 0 || threads < kColumnThreads) return columns;
+    for (uint32_t r = 0; r < ws.world; ++r) {
+        if (args.dst[r].out_x != nullptr && args.dst[r].out_scale != nullptr && !scales_by_column(args.dst[r])) return columns;
+    }
+    uint64_t spans = 0;
+    for (uint32_t g = 0; g < ws.num_groups; ++g) {
+        const PushSrc &src = args.src[g];
+        if (src.num_tokens == 0) continue;
+        if (src.xs_stride_elem != 1 || src.xs_stride_token % 4 != 0 || (uintptr_t)src.x_scale % 16 != 0) return columns;
+        spans += ((uint64_t)src.num_tokens * ws.topk + kSpan - 1) / kSpan;
+    }
+    columns.blocks = (uint32_t)(spans * columns.slices);
+    return columns;
+}
+
 // How the copies are written: past the Infinity Cache (`streamed`), otherwise quantised rows at device scope and others
 // with ordinary stores (device scope: 1 us less of 24 for 8 KB rows, but 3-5 us more of 33 for rows of 5120 bytes).
 hipError_t launch_dispatch_resolve(const PushArgs &args, const FinalizeArgs &fin, const Workspace &ws, bool quantize,
@@ -2494,11 +2677,16 @@ hipError_t launch_dispatch_resolve(const PushArgs &args, const FinalizeArgs &fin
     }
     if (senders != 1) a.single_source = 0;    // here only "one source has tokens": the rows may be strided
     if (a.single_source != 0) a.single = args.src[a.single_source - 1];
-#define A2A_LAUNCH_RESOLVE(Q, P)                                                                                   \
-    hipExtLaunchKernelGGL((dispatch_resolve_kernel<Q, P>), dim3(blocks), dim3(threads), 0, stream, timing.start,  \
-                          timing.stop, 0, a, fin, ws)
+    ScaleColumns columns = {0, 0};
+    if (!streamed) columns = plan_scale_columns(args, ws, quantize, threads);
+    const size_t lds = columns.blocks != 0 ? (kSpan + 3 * (size_t)ws.num_experts) * sizeof(uint32_t) : 0;
+#define A2A_LAUNCH_RESOLVE(...)                                                                                    \
+    hipExtLaunchKernelGGL((dispatch_resolve_kernel<__VA_ARGS__>), dim3(blocks + columns.blocks), dim3(threads),    \
+                          lds, stream, timing.start, timing.stop, 0, a, fin, ws, columns)
     if (quantize) {
         if (streamed) A2A_LAUNCH_RESOLVE(true, kDeviceNonTemporal); else A2A_LAUNCH_RESOLVE(true, kDeviceScope);
+    } else if (columns.blocks != 0) {
+        A2A_LAUNCH_RESOLVE(false, kOrdinary, true);
     } else {
         if (streamed) A2A_LAUNCH_RESOLVE(false, kDeviceNonTemporal); else A2A_LAUNCH_RESOLVE(false, kOrdinary);
     }

@@ -100,6 +100,11 @@ struct PushDst {
     uint32_t pad_;
 };
 
+// Whether a receiver's scales are stored by column: the next row's word is nearer than the row's next word.
+inline bool scales_by_column(const PushDst &dst) {
+    return dst.out_scale != nullptr && dst.os_stride_token < dst.os_stride_elem;
+}
+
 struct PushArgs {
     PushSrc src[kMaxWorld];
     PushDst dst[kMaxWorld];

@@ -1638,11 +1638,6 @@ struct PieceWalk {
 constexpr uint32_t kScaleColumns = 8;
 constexpr uint64_t kColumnWords = 112 * 1024;
 
-// Whether scales of these strides are columns: the next row's word is nearer than the row's next word.
-__host__ __device__ __forceinline__ bool scales_by_column(const PushDst &dst) {
-    return dst.out_scale != nullptr && dst.os_stride_token < dst.os_stride_elem;
-}
-
 // The scales of the received rows, by column.  `unit`, `units`: of the wavefronts that do this.
 __device__ __forceinline__ void receive_scale_columns(const StageRecvArgs &args, const Workspace &ws, const Staging &st,
                                                       const uint4 *moves, uint32_t total, uint32_t unit, uint32_t units) {

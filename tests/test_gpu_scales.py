@@ -4,11 +4,13 @@ against the oracle bit for bit."""
 
 from dataclasses import replace
 
+import numpy as np
 import pytest
 import torch
 
+import a2a_oracle as oracle
 from a2a_cases import C1, scaled
-from a2a_transport import RefConfig, check, make_ref_rank, rows_for, run_gpu
+from a2a_transport import RefConfig, _bytes, check, make_ops, make_ref_rank, rows_for, run_gpu
 from test_gpu_sources import run_and_check
 
 pytestmark = pytest.mark.gpu
@@ -22,6 +24,8 @@ GIVEN = [
     ([1500, 0, 700, 33], 128, 8, 6144, 48),   # the widest row whose scales are asked for ahead of it
     ([2100, 17], 33, 8, 6160, 55),            # the next wider one; an expert a receiver has not got
     ([1300, 1400], 24, 7, 256, 128),          # more scales than the row has threads
+    ([1300, 2500, 1], 1024, 6, 4096, 32),     # more experts than threads; a span that ends in its first chunk of entries
+    ([16384, 16385, 3], 6, 1, 4096, 4),       # whole spans, and one entry more; a single slice of columns
 ]
 
 
@@ -59,3 +63,55 @@ def test_received_columns(tokens, experts, topk, hidden, scales):
     world = [make_ref_rank(cfg, r, t) for r, t in enumerate(tokens)]
     rows = rows_for(cfg, world)
     check(cfg, world, rows, run_gpu(cfg, world, rows, DEV, split=True, scale_layout="col"))
+
+
+@pytest.mark.parametrize("how", ["bounds", "repeats", "too_few_rows", "unaligned", "by_column_too", "one_by_row"])
+def test_columns_of_unusual_steps(how):
+    """Scales by column of a step with `bounds` on the device, with experts that repeat inside a token, with a receive buffer
+    that the last rows do not fit, with source scales that are not 16-byte pieces, with source scales that are columns
+    themselves, and with one receiver that takes rows."""
+    print(how, flush=True)
+    tokens, bounds = [1400, 900, 0, 64], [None] * 4
+    cfg = RefConfig("unusual", 4, 1, 1400, 40, 4096, 32, 8, FP8, BF16, F32, expert_padding=8)
+    world = [make_ref_rank(cfg, r, t) for r, t in enumerate(tokens)]
+    if how == "bounds":
+        bounds = [1290, 1, None, 0]
+    if how == "repeats":
+        for rd in world:
+            rd.indices[::3, 7] = rd.indices[::3, 0]
+    rows = rows_for(cfg, world) - (70 if how == "too_few_rows" else 0)
+    inputs = [oracle.RankInput(x=_bytes(rd.dp_x), indices=rd.indices.numpy(), x_scale=rd.dp_x_scale.numpy(), bound_m=b)
+              for rd, b in zip(world, bounds)]
+    fits = rows_for(cfg, world)
+    want = oracle.dispatch_world(inputs, num_experts=40, world_size=4, node_size=4, expert_padding=8, out_rows=fits,
+                                 quantize=False, hidden_dim_scale=32)
+    ops = make_ops(cfg, DEV)
+    try:
+        outs = []
+        for r, rd in enumerate(world):
+            xs = rd.dp_x_scale.to(DEV)
+            if how == "unaligned":
+                wide = torch.zeros((xs.shape[0], 36), device=DEV)
+                wide[:, 1:33] = xs
+                xs = wide[:, 1:33]
+            if how == "by_column_too":
+                xs = xs.t().contiguous().t()
+            x = torch.full((rows, 4096), 0xA5, dtype=torch.uint8, device=DEV)
+            s = torch.full((rows, 32) if how == "one_by_row" and r == 1 else (32, rows), -7.0, device=DEV)
+            if s.shape[0] != rows:
+                s = s.t()
+            outs.append((x, s))
+            ops[r].dispatch(out_expert_num_tokens=torch.zeros(10, dtype=torch.int32, device=DEV),
+                            out_expert_x=x.view(FP8), out_expert_x_scale=s, dp_x=rd.dp_x.to(DEV), dp_x_scale=xs,
+                            indices=rd.indices.view(torch.uint32).to(DEV), weights=rd.weights.to(DEV),
+                            bound_m=None if bounds[r] is None else torch.tensor([bounds[r]], dtype=torch.int32, device=DEV))
+        torch.cuda.synchronize(DEV)
+        assert bool(ops[0].context.status()) == (how == "too_few_rows")
+        for (x, s), w in zip(outs, want):
+            wr = w.written[:rows]
+            np.testing.assert_array_equal(x.cpu().numpy()[wr], w.x[:rows][wr])
+            np.testing.assert_array_equal(s.cpu().numpy()[wr].view(np.uint32), w.x_scale[:rows][wr].view(np.uint32))
+            assert (x.cpu().numpy()[~wr] == 0xA5).all() and (s.cpu().numpy()[~wr] == -7.0).all()
+    finally:
+        for op in ops:
+            op.destroy()
