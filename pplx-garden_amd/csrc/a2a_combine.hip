@@ -168,7 +168,11 @@ constexpr uint64_t kStreamedOutput = 84000000;
 // 6000 tokens 216.6 / 214.1 / 212.7 / 214.2, 8 x 4096 tokens 1161 / 1145 / 1139 / 1152, 8 x 2048 tokens of 5 KB fp8 rows 416.1 /
 // 410.2 / 406.7 / 409.3, float rows of 8 KB, 8 x 3000 tokens 663.7 / 657.5 / 655.4 / 656.7; K = 6 with 21 / 18 / 16, 8 x 4096
 // tokens 894.5 / 888.6 / 878.0 (in the cache 14 are 0.9 us better at 4096 tokens and 0.3 worse at 2668, 12 worse).  The launch
-// asks for LDS that nothing uses to bound them.  The ONE_RANK variant is left alone (1024 tokens 23.6 / 23.4-23.7).
+// asks for LDS that nothing uses to bound them.  The ONE_RANK variant is left alone (1024 tokens 23.6 / 23.4-23.7), and so are
+// steps whose wavefronts fit the GPU all at once (kAllAtOnce): bounded to 16 they take a second, half empty round (rows of
+// 14 KB: 8 x 40 tokens 9.08 / 8.68 us unbounded, 8 x 64 13.14 / 12.53; level where 16 hold them all and at 8064 wavefronts).
+constexpr uint64_t kAllAtOnce = 32 * 256;
+
 inline size_t lds_to_bound_waves(uint32_t topk, bool past_cache) {
     if (topk <= 4) return 0;
     constexpr size_t kLds = 160 * 1024, kBlock = 1280;   // of a compute unit, and what it is given out in
@@ -367,7 +371,7 @@ static hipError_t launch_typed(const CombArgs &given, const Workspace &ws, uint3
     const bool plain = args.single_rank != 0 || args.staged_base != nullptr;
     const bool past_cache =
         !plain && (streamed || (uint64_t)total_tokens * args.hidden_dim * Elem<U>::kSize >= kStreamedOutput);
-    const size_t lds = lds_to_bound_waves(ws.topk, past_cache);
+    const size_t lds = (uint64_t)slabs * total_tokens <= kAllAtOnce ? 0 : lds_to_bound_waves(ws.topk, past_cache);
 #define A2A_LAUNCH_GATHER(GROUP, ONE, OUT, LDS)                                                                \
     hipExtLaunchKernelGGL((combine_gather_kernel<T, U, GROUP, ONE, OUT>), grid, dim3(kWave), LDS, stream,      \
                           timing.start, timing.stop, 0, args, ws)
