@@ -480,8 +480,9 @@ int plan_dispatch_group(a2a_ctx *ctx, const a2a_config &c, const a2a_dispatch_ar
 }
 
 // Second half: the launches of an accepted plan on the tables of `ws`.
-// `streamed`: whether the pack wrote its copies past the Infinity Cache.  The one-launch packs of small steps never do (at
-// most 8192 entries: the line is rows of 39 KB away), nor does the push behind separate routing launches.
+// `streamed`: whether the pack wrote its copies past the Infinity Cache.  The one-launch packs never do: that of several
+// sources (up to 16384 entries) is not taken by steps that would, the others have at most 8192 entries (the line is rows of
+// 39 KB away); nor does the push behind separate routing launches.
 int launch_dispatch_group(a2a_ctx *ctx, const a2a_config &c, const Workspace &ws, const GroupPlan &plan,
                           uint32_t quantize, hipStream_t s, KernelTiming pack_timing, KernelTiming route_timing,
                           bool &streamed) {
