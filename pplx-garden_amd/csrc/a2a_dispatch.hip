@@ -47,22 +47,26 @@ __device__ __forceinline__ void store_copies(u32x4 v, uint64_t row_ptr, uint32_t
     }
 }
 
-// One scale of a copy.  Rows of scales share their first and last cache lines with the rows before and after, which
-// other compute units write: kept in a compute unit's L2 in the hope of the rest they cost the rows their place in it.
-// Stored non-temporally the pack of 4096 tokens (rows of 7168 bytes, 56 scales) takes 69.0 us for 70.7 and that of
-// 8 sources of 512 tokens (5120 bytes, 40 scales) 52.3 for 54.0, with and without a reader behind it; rows of 16 scales are
-// level and rows of 8, four to a line, lose (18.9 us for 18.5).  Scales stored by COLUMN are single words of lines that
-// have to meet somewhere (non-temporal: 68 us for 36), and copies that are stored past the Infinity Cache leave it to
-// the scales (non-temporal: 485 us for 454).
-constexpr uint32_t kScalesPastL2 = 32;   // a cache line of them
+// How a pack moves scales: word by word beside the rows, that with non-temporal stores, or not at all (by column in
+// workgroups of their own, push_scale_columns).
+constexpr int kScalesPlain = 0, kScalesPastL2 = 1, kScalesApart = 2;
 
-template <int POLICY>
-__device__ __forceinline__ void store_scale(float scale, float *row, uint32_t j, uint32_t stride, uint32_t num_scales) {
-    if ((POLICY & kNonTemporal) == 0 && stride == 1 && num_scales >= kScalesPastL2) {
-        __builtin_nontemporal_store(scale, row + j);
+// Rows of scales share their first and last cache lines with the rows before and after, which other compute units write: kept
+// in a compute unit's L2 in the hope of the rest they cost the rows their place in it.  Stored non-temporally the pack of
+// 4096 tokens (top-8, rows of 7168 bytes, 56 scales) takes 69.0 us for 70.7 and that of 8 sources of 512 tokens (5120 bytes,
+// 40 scales) 52.3 for 54.0, with and without a reader behind it.  Not so with few copies to a token (2636 tokens of 5120
+// bytes, K = 1 / 2 / 4 / 6 / 8: 20.0 / 22.2 / 25.3 / 28.1 / 32.6 us plain, 20.2 / 22.5 / 25.6 / 28.3 / 32.0), with fewer
+// scales than a cache line has (16: level; 8: 18.9 us for 18.5), by COLUMN, single words of lines that have to meet
+// somewhere (68 us for 36), and beside copies that are stored past the Infinity Cache, which leave it to the scales (485 us
+// for 454).
+constexpr uint32_t kLineOfScales = 32;
+
+template <int SCALES>
+__device__ __forceinline__ void store_scale(float scale, float *row, uint32_t j, uint32_t stride) {
+    if constexpr (SCALES == kScalesPastL2) {
+        __builtin_nontemporal_store(scale, row + j);   // (a row of scales: stride 1)
     } else {
         row[(size_t)j * stride] = scale;
-        asm volatile("");   // keeps the two stores apart: merged into one they lose the policy
     }
 }
 
@@ -85,8 +89,8 @@ constexpr uint32_t kScalesAheadBytes = 6144;
 // passes `live` false.
 // PRE: the thread's first piece of the row was asked for earlier (first_piece) and is passed in.
 // POLICY: cache policy of the copies' stores.
-// SCALES: whether the caller's scales are moved too (quantised rows always have theirs).
-template <bool QUANT, bool PRE = false, int POLICY = QUANT ? kDeviceScope : kOrdinary, bool SCALES = true>
+// SCALES: kScales... above (quantised rows always have theirs).
+template <bool QUANT, bool PRE = false, int POLICY = QUANT ? kDeviceScope : kOrdinary, int SCALES = kScalesPlain>
 __device__ __forceinline__ void push_rows(const PushArgs &args, const PushSrc &src, uint32_t token, uint32_t K,
                                           uint64_t row_ptr, uint64_t scale_ptr, uint32_t scale_stride,
                                           float *s_scale, uint64_t *s_scale_ptr, uint32_t *s_scale_stride,
@@ -129,11 +133,11 @@ __device__ __forceinline__ void push_rows(const PushArgs &args, const PushSrc &s
             const uint32_t k = i / Hl;
             const uint32_t j = i - k * Hl;
             const uint64_t sp = s_scale_ptr[k];
-            if (sp != 0) store_scale<POLICY>(s_scale[j], reinterpret_cast<float *>(sp), j, s_scale_stride[k], Hs);
+            if (sp != 0) store_scale<SCALES>(s_scale[j], reinterpret_cast<float *>(sp), j, s_scale_stride[k]);
         }
     } else {
         const uint32_t num_chunks = live ? args.row_bytes / 16 : 0;
-        const bool scaled = SCALES && src.x_scale != nullptr && live;
+        const bool scaled = SCALES != kScalesApart && src.x_scale != nullptr && live;
         const float *const xs = src.x_scale + (size_t)token * src.xs_stride_token;
         const bool ahead = args.row_bytes <= kScalesAheadBytes;
         float first_scale = 0.0f;
@@ -149,7 +153,7 @@ __device__ __forceinline__ void push_rows(const PushArgs &args, const PushSrc &s
                 for (uint32_t k = 0; k < K; ++k) {
                     const uint64_t sp = read_lane64(scale_ptr, k);
                     const uint32_t ss = __builtin_amdgcn_readlane((int)scale_stride, (int)k);
-                    if (sp != 0) store_scale<POLICY>(s, reinterpret_cast<float *>(sp), j, ss, args.hidden_dim_scale);
+                    if (sp != 0) store_scale<SCALES>(s, reinterpret_cast<float *>(sp), j, ss);
                 }
             }
         }
@@ -2207,9 +2211,9 @@ __device__ __forceinline__ void push_scale_columns(const PushArgs &args, const W
 // the grid holds one workgroup per receiver (expert counts for the caller,
 // layout tables) and one per source (its totals and their scan); the last of
 // them hands the totals over to the next step.
-// COLUMNS: the caller's scales go out by column (push_scale_columns, whose dynamic LDS it has).
-template <bool QUANT, int POLICY, bool COLUMNS = false>
-__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(COLUMNS ? 8 : 4))) void dispatch_resolve_kernel(const PushArgs args, const FinalizeArgs fin,
+// SCALES: kScales...; where they are moved apart, push_scale_columns' dynamic LDS is there.
+template <bool QUANT, int POLICY, int SCALES>
+__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(SCALES == kScalesApart ? 8 : 4))) void dispatch_resolve_kernel(const PushArgs args, const FinalizeArgs fin,
                                                                 const Workspace ws, const ScaleColumns columns) {
     __shared__ float s_scale[QUANT ? kMaxLdsScales : 1];
     __shared__ uint64_t s_scale_ptr[A2A_MAX_EXPERTS_PER_TOKEN];
@@ -2236,7 +2240,7 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(COLUMNS ? 
     // The receiver and source workgroups come first in the grid, so that they run
     // beside the token workgroups instead of after them.
     uint32_t extras = ws.world + G;
-    if constexpr (COLUMNS) {
+    if constexpr (SCALES == kScalesApart) {
         extras += columns.blocks;
         if (blockIdx.x >= ws.world + G && blockIdx.x < extras) {
             push_scale_columns(args, ws, columns, blockIdx.x - (ws.world + G), per_source, per_expert, s_columns, scratch);
@@ -2369,8 +2373,8 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(COLUMNS ? 
         scale_ptr = s_route_scale_ptr[lane];
         scale_stride = s_route_scale_stride[lane];
     }
-    push_rows<QUANT, false, POLICY, !COLUMNS>(args, src, token, K, row_ptr, scale_ptr, scale_stride, s_scale, s_scale_ptr,
-                                              s_scale_stride, threadIdx.x, blockDim.x, true);
+    push_rows<QUANT, false, POLICY, SCALES>(args, src, token, K, row_ptr, scale_ptr, scale_stride, s_scale, s_scale_ptr,
+                                            s_scale_stride, threadIdx.x, blockDim.x, true);
 }
 
 hipError_t launch_dispatch_push(const PushArgs &args, const Workspace &ws, bool quantize,
@@ -2658,6 +2662,15 @@ static ScaleColumns plan_scale_columns(const PushArgs &args, const Workspace &ws
     return columns;
 }
 
+// Whether the pack of a step whose copies stay in the Infinity Cache stores its scales non-temporally (kScalesPastL2).
+static bool scales_past_l2(const PushArgs &args, const Workspace &ws) {
+    if (ws.topk < 8 || args.hidden_dim_scale < kLineOfScales) return false;
+    for (uint32_t r = 0; r < ws.world; ++r) {
+        if (args.dst[r].out_x != nullptr && args.dst[r].out_scale != nullptr && args.dst[r].os_stride_elem != 1) return false;
+    }
+    return true;
+}
+
 // How the copies are written: past the Infinity Cache (`streamed`), otherwise quantised rows at device scope and others
 // with ordinary stores (device scope: 1 us less of 24 for 8 KB rows, but 3-5 us more of 33 for rows of 5120 bytes).
 hipError_t launch_dispatch_resolve(const PushArgs &args, const FinalizeArgs &fin, const Workspace &ws, bool quantize,
@@ -2683,12 +2696,18 @@ hipError_t launch_dispatch_resolve(const PushArgs &args, const FinalizeArgs &fin
 #define A2A_LAUNCH_RESOLVE(...)                                                                                    \
     hipExtLaunchKernelGGL((dispatch_resolve_kernel<__VA_ARGS__>), dim3(blocks + columns.blocks), dim3(threads),    \
                           lds, stream, timing.start, timing.stop, 0, a, fin, ws, columns)
-    if (quantize) {
-        if (streamed) A2A_LAUNCH_RESOLVE(true, kDeviceNonTemporal); else A2A_LAUNCH_RESOLVE(true, kDeviceScope);
+    const bool past_l2 = scales_past_l2(args, ws);
+    if (streamed) {
+        if (quantize) A2A_LAUNCH_RESOLVE(true, kDeviceNonTemporal, kScalesPlain);
+        else A2A_LAUNCH_RESOLVE(false, kDeviceNonTemporal, kScalesPlain);
+    } else if (quantize) {
+        if (past_l2) A2A_LAUNCH_RESOLVE(true, kDeviceScope, kScalesPastL2);
+        else A2A_LAUNCH_RESOLVE(true, kDeviceScope, kScalesPlain);
     } else if (columns.blocks != 0) {
-        A2A_LAUNCH_RESOLVE(false, kOrdinary, true);
+        A2A_LAUNCH_RESOLVE(false, kOrdinary, kScalesApart);
     } else {
-        if (streamed) A2A_LAUNCH_RESOLVE(false, kDeviceNonTemporal); else A2A_LAUNCH_RESOLVE(false, kOrdinary);
+        if (past_l2) A2A_LAUNCH_RESOLVE(false, kOrdinary, kScalesPastL2);
+        else A2A_LAUNCH_RESOLVE(false, kOrdinary, kScalesPlain);
     }
 #undef A2A_LAUNCH_RESOLVE
     return hipGetLastError();
