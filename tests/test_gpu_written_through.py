@@ -1,0 +1,32 @@
+"""Large steps of long rows without scales, whose copies are written through the L2s, and their neighbours on the other side of
+each line of that rule: rows and combined tokens against the oracle."""
+
+import pytest
+import torch
+
+from a2a_transport import RefConfig, check, make_ref_rank, rows_for, run_gpu
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda:0")
+BF16, F32 = torch.bfloat16, torch.float32
+
+# tokens, experts, top-k, hidden, type: copies of 120 MB are the line
+STEPS = [
+    ([2441, 1], 16, 6, 4096, BF16),        # 120.03 MB: written through
+    ([2440, 1], 16, 6, 4096, BF16),        # 119.98 MB: not
+    ([2000, 500], 17, 6, 4096, BF16),      # an expert a receiver has not got
+    ([4300, 0, 10], 24, 7, 2048, BF16),    # the shortest rows
+    ([2500, 10], 24, 6, 4088, BF16),       # rows that are not multiples of 2 KB: not
+    ([1500, 1], 12, 5, 8192, BF16),        # five copies a token: not
+    ([620, 625], 32, 6, 4096, F32),        # 122 MB of 16 KB rows
+    ([560, 3], 64, 8, 7168, F32),          # rows longer than a workgroup has threads for
+]
+
+
+@pytest.mark.parametrize("tokens,experts,topk,hidden,dtype", STEPS, ids=[f"{s[0]}_k{s[2]}_h{s[3]}" for s in STEPS])
+def test_large_steps_of_long_rows(tokens, experts, topk, hidden, dtype):
+    print(f"tokens={tokens} topk={topk} hidden={hidden} {dtype}", flush=True)
+    cfg = RefConfig("through", len(tokens), 1, max(tokens), experts, hidden, None, topk, dtype, dtype, None, expert_padding=2)
+    world = [make_ref_rank(cfg, r, t) for r, t in enumerate(tokens)]
+    rows = rows_for(cfg, world)
+    check(cfg, world, rows, run_gpu(cfg, world, rows, DEV, split=False))
