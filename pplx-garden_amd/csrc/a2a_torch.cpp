@@ -4,7 +4,7 @@
 // look at six to eight tensors (shape, strides, type, address: some forty attributes) before one of them
 // launches anything.  In Python that was 5.8 us a call, so that a decode step of 12 us on the GPU took 93;
 // here a call that launches nothing is 0.2-0.3 us, most of it the interpreter's own way in and out (through a
-// Python function in front of it 0.1 us more: Method below; 8 ranks x 1 token 11.3 -> 10.6 us a step).
+// Python function in front of it 0.1 us more: call_without_a_frame below; 8 ranks x 1 token 11.3 -> 10.6 us a step).
 //
 // Plays the part of the reference's pyo3 classes (python-ext/src/py_p2p_all_to_all.rs:17-205) one level
 // higher: it takes the tensors themselves and makes the checks of the reference's operator
@@ -707,58 +707,73 @@ PyMethodDef operator_methods[] = {
 PyTypeObject OperatorType = {PyVarObject_HEAD_INIT(nullptr, 0)};
 
 // ---------------------------------------------------------------------------
-// Method: stands in a Python class in the place of a function `f(self, ...)` that hands its arguments to the method of the
-// same name of `self._operator`.  Looked up on an object whose `_operator` is one it gives that method itself, so that a
-// call does not pass through a Python frame; otherwise, and looked up on the class, the function.
+// call_without_a_frame(function): calls of the Python function `f(self, ...)`, which hands its arguments to the method of the
+// same name of `self._operator`, run that method without a Python frame in between.  The function stays the object it is, and
+// with it whatever is looked up, bound, inspected or kept; only the way the interpreter enters it changes.  What is called
+// is decided at the call: without a native operator in `_operator` (after `destroy()`, say) the function itself runs, and so
+// it does under a profiler or debugger and once somebody has given it other code or defaults.
 // ---------------------------------------------------------------------------
-struct Method {
-    PyObject_HEAD
-    PyObject *name, *function;
-};
-
 PyObject *operator_attribute;   // "_operator"
 
-PyObject *method_new(PyTypeObject *type, PyObject *args, PyObject *) {
-    PyObject *name, *function;
-    if (!PyArg_ParseTuple(args, "UO", &name, &function)) return nullptr;
-    Method *m = reinterpret_cast<Method *>(type->tp_alloc(type, 0));
-    if (m == nullptr) return nullptr;
-    Py_INCREF(name);
-    PyUnicode_InternInPlace(&name);
-    m->name = name;
-    Py_INCREF(function);
-    m->function = function;
-    return reinterpret_cast<PyObject *>(m);
-}
+struct Frameless {
+    const Parameters &parameters;
+    PyObject *(*call)(PyObject *, PyObject *const *, Py_ssize_t, PyObject *);
+    vectorcallfunc enter;           // how the interpreter enters the function itself
+    PyObject *code, *defaults;      // the function's, when it was given the other entry
+};
 
-void method_dealloc(PyObject *self) {
-    Py_XDECREF(reinterpret_cast<Method *>(self)->name);
-    Py_XDECREF(reinterpret_cast<Method *>(self)->function);
-    Py_TYPE(self)->tp_free(self);
-}
+Frameless frameless_dispatch = {dispatch_parameters, guarded<dispatch>, nullptr, nullptr, nullptr};
+Frameless frameless_combine = {combine_parameters, guarded<combine>, nullptr, nullptr, nullptr};
 
-PyObject *method_get(PyObject *self, PyObject *object, PyObject *) {
-    Method *m = reinterpret_cast<Method *>(self);
-    if (object == nullptr || object == Py_None) {
-        Py_INCREF(m->function);
-        return m->function;
+template <Frameless &F>
+PyObject *enter_operator(PyObject *function, PyObject *const *args, size_t n, PyObject *keywords) {
+    const PyThreadState *const thread = PyThreadState_Get();
+    if (PyVectorcall_NARGS(n) > 0 && thread->c_tracefunc == nullptr && thread->c_profilefunc == nullptr &&
+        PyFunction_GET_CODE(function) == F.code && PyFunction_GET_DEFAULTS(function) == F.defaults) {
+        PyObject *const op = PyObject_GetAttr(args[0], operator_attribute);
+        if (op == nullptr) {
+            if (!PyErr_ExceptionMatches(PyExc_AttributeError)) return nullptr;
+            PyErr_Clear();
+        } else if (Py_TYPE(op) == &OperatorType) {
+            PyObject *const result = F.call(op, args + 1, PyVectorcall_NARGS(n) - 1, keywords);
+            Py_DECREF(op);
+            return result;
+        }
+        Py_XDECREF(op);
     }
-    PyObject *const op = PyObject_GetAttr(object, operator_attribute);
-    if (op == nullptr) {
-        if (!PyErr_ExceptionMatches(PyExc_AttributeError)) return nullptr;
-        PyErr_Clear();
-    } else if (Py_TYPE(op) == &OperatorType) {
-        PyObject *const bound = PyObject_GetAttr(op, m->name);
-        Py_DECREF(op);
-        return bound;
-    }
-    Py_XDECREF(op);
-    return PyMethod_New(m->function, object);
+    return F.enter(function, args, n, keywords);
 }
 
-PyTypeObject MethodType = {PyVarObject_HEAD_INIT(nullptr, 0)};
+template <Frameless &F>
+void set_entry(PyFunctionObject *f) {
+    if (f->vectorcall == enter_operator<F>) return;
+    F.enter = f->vectorcall;
+    Py_XINCREF(f->func_code);
+    Py_XINCREF(f->func_defaults);
+    Py_XSETREF(F.code, f->func_code);
+    Py_XSETREF(F.defaults, f->func_defaults);
+    f->vectorcall = enter_operator<F>;
+}
 
-PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_a2a_torch", nullptr, -1, nullptr, nullptr, nullptr, nullptr, nullptr};
+PyObject *call_without_a_frame(PyObject *, PyObject *function) {
+    if (!PyFunction_Check(function)) return PyErr_Format(PyExc_TypeError, "a Python function is expected");
+    PyFunctionObject *const f = reinterpret_cast<PyFunctionObject *>(function);
+    if (PyUnicode_CompareWithASCIIString(f->func_name, frameless_dispatch.parameters.call) == 0) {
+        set_entry<frameless_dispatch>(f);
+    } else if (PyUnicode_CompareWithASCIIString(f->func_name, frameless_combine.parameters.call) == 0) {
+        set_entry<frameless_combine>(f);
+    } else {
+        return PyErr_Format(PyExc_ValueError, "no call of the operator has the name %U", f->func_name);
+    }
+    Py_RETURN_NONE;
+}
+
+PyMethodDef module_methods[] = {
+    {"call_without_a_frame", call_without_a_frame, METH_O, nullptr},
+    {nullptr, nullptr, 0, nullptr},
+};
+
+PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_a2a_torch", nullptr, -1, module_methods, nullptr, nullptr, nullptr, nullptr};
 
 bool add_type(PyObject *module, PyTypeObject &type, const char *name, const char *short_name, size_t size, newfunc make,
               destructor drop, PyMethodDef *methods) {
@@ -783,9 +798,7 @@ PyMODINIT_FUNC PyInit__a2a_torch(void) {
         Py_DECREF(m);
         return nullptr;
     }
-    MethodType.tp_descr_get = method_get;
-    if (!add_type(m, MethodType, "_a2a_torch.Method", "Method", sizeof(Method), method_new, method_dealloc, nullptr) ||
-        !add_type(m, ContextType, "_a2a_torch.Context", "Context", sizeof(Context), context_new, context_dealloc,
+    if (!add_type(m, ContextType, "_a2a_torch.Context", "Context", sizeof(Context), context_new, context_dealloc,
                   context_methods) ||
         !add_type(m, OperatorType, "_a2a_torch.Operator", "Operator", sizeof(Operator), operator_new, operator_dealloc,
                   operator_methods)) {

@@ -197,13 +197,11 @@ class P2PAllToAll(AllToAllKernel):
             self._global_group.world.release_context(self._key)
 
 
-_DEFINED = {name: P2PAllToAll.__dict__[name] for name in ("dispatch", "combine")}
+_DEFINED = (P2PAllToAll.dispatch, P2PAllToAll.combine)
 
 
 def _call_without_a_frame(extension) -> None:
-    """From the first operator on, `op.dispatch` and `op.combine` are the native operator's methods (same names, defaults and
-    checks); looked up on the class, and after `destroy()`, they are the functions above.  What somebody else has put in their
-    place in the class stays."""
-    for name, function in _DEFINED.items():
-        if P2PAllToAll.__dict__.get(name) is function:
-            setattr(P2PAllToAll, name, extension.Method(name, function))
+    """From the first operator on, calls of these two functions on an operator that is not destroyed run the native operator's
+    methods (same names, defaults and checks) without a Python frame; the functions stay the objects they are."""
+    for function in _DEFINED:
+        extension.call_without_a_frame(function)

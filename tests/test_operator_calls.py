@@ -1,8 +1,11 @@
 """Calls of the operator that reach the native code without a Python frame take their arguments as the functions they stand for
-do (by position and by name, with the defaults), and give way to whatever a user puts in their place."""
+do (by position and by name, with the defaults), are bound, inspected and kept as those are, and give way to whatever a user puts
+in their place."""
 
 import inspect
+import sys
 import types
+import weakref
 
 import pytest
 import torch
@@ -38,7 +41,6 @@ def test_arguments_by_name_by_position_and_by_default(world):
                          ((), dict(reversed(list(d.items())), do_recv=True, bound_m=None)),
                          ((), {"".join(list(k)): v for k, v in d.items()})]:      # (names that are not interned)
         op = make(P2PAllToAll, 0)
-        assert isinstance(op.dispatch, types.BuiltinFunctionType)
         assert op.dispatch(*args, **kwargs) is None and context.pending("dispatch") == 1
         with pytest.raises(RuntimeError, match="destroyed"):
             make(P2PAllToAll, 1).dispatch(**d)
@@ -51,6 +53,48 @@ def test_arguments_by_name_by_position_and_by_default(world):
         op.dispatch(**d, do_send=True, do_recv=False)
     with pytest.raises(AssertionError):
         op.dispatch(**d, do_send=False, do_recv=False)
+
+
+@pytest.mark.parametrize("halves", [{}, dict(do_recv=False), dict(do_send=False)])
+@pytest.mark.parametrize("name", ["dispatch", "combine"])
+def test_a_method_taken_before_destroy_refuses_calls_after_it(world, name, halves):
+    context, make, d, c = world
+    op = make(P2PAllToAll, 0)
+    held = getattr(op, name)
+    op._operator = None     # as destroy() leaves it
+    with pytest.raises(AssertionError):
+        held(**(d if name == "dispatch" else c), **halves)
+    assert context.pending(name) == 0
+
+
+@pytest.mark.parametrize("name", ["dispatch", "combine"])
+def test_a_method_is_the_functions_bound_to_the_operator(world, name):
+    _, make, _, _ = world
+    op = make(P2PAllToAll, 0)
+    method, function = getattr(op, name), getattr(P2PAllToAll, name)
+    assert isinstance(method, types.MethodType) and method.__self__ is op and method.__func__ is function
+    assert list(inspect.signature(method).parameters) == list(inspect.signature(function).parameters)[1:]
+    assert inspect.signature(method).parameters["do_recv"].default is True
+    assert method.__annotations__["weights"] and weakref.WeakMethod(method)() == method
+    alive = weakref.ref(op)
+    del op
+    assert alive() is not None      # kept by the bound method
+
+
+def test_profilers_see_the_function_and_other_code_of_it_runs(world, monkeypatch):
+    context, make, d, c = world
+    seen = []
+    sys.setprofile(lambda frame, event, arg: seen.append(frame.f_code) if event == "call" else None)
+    try:
+        make(P2PAllToAll, 0).dispatch(**d)
+    finally:
+        sys.setprofile(None)
+    assert P2PAllToAll.dispatch.__code__ in seen and context.pending("dispatch") == 1
+    monkeypatch.setattr(P2PAllToAll.combine, "__defaults__", (None, False, False, False))
+    with pytest.raises(AssertionError, match="do_send || do_recv"):
+        make(P2PAllToAll, 0).combine(**c)
+    monkeypatch.undo()
+    assert make(P2PAllToAll, 0).combine(**c) is None and context.pending("combine") == 1
 
 
 @pytest.mark.parametrize("args,kwargs,match", [
