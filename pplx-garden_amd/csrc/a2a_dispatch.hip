@@ -18,6 +18,7 @@
 // copies are written depends on how much of the Infinity Cache they fill (see
 // copies_past_cache in a2a_rules.h).
 #include "a2a_device.h"
+#include "a2a_rules.h"
 #include "a2a_scan.h"
 
 namespace a2a {
@@ -2671,24 +2672,8 @@ static bool scales_past_l2(const PushArgs &args, const Workspace &ws) {
     return true;
 }
 
-// Whether copies that are not quantised are stored at device scope.  Ordinary stores leave them dirty in eight L2s, which write
-// them back in an order of their own; written through, the copies of large steps of long rows without scales reach
-// memory as the rows are worked off.  us per step, ordinary / written through (per dispatch in brackets), K = 6: 6000 tokens
-// of 8 KB 143.6 / 137.9 (78.8 / 73.2), 3200 81.8 / 79.1, 3600 of 12 KB 129.9 / 125.5, 2700 of 14 KB (K = 8) 137.2 / 132.7, 1500
-// 80.5 / 78.6, 10 000 of 4 KB 123.0 / 117.8, 1600 of 28 KB 134.7 / 130.6; with a reader of the copies in between level to
-// 1.6 % better.  It loses with few copies a token (K = 2: 173.0 / 177.0; K = 4 148.2 / 146.1, behind a reader 245.6 / 247.4),
-// with rows of 2 KB (131.7 / 134.1) or of 5888 bytes (106.5 / 107.7), with rows that bring scales (fp8 rows of 5120 bytes 75.3 /
-// 77.5, of 4096 behind a reader 300 / 308), and below kWrittenThrough bytes of copies (4 KB rows, 79 MB: dispatch 24.0 /
-// 24.9; 108 MB level).
-constexpr uint64_t kWrittenThrough = 120000000;
-
-static bool written_through(const PushArgs &args, const Workspace &ws, uint32_t total_tokens) {
-    return args.hidden_dim_scale == 0 && ws.topk >= 6 && args.row_bytes >= 4096 && args.row_bytes % 2048 == 0 &&
-           (uint64_t)total_tokens * ws.topk * args.row_bytes >= kWrittenThrough;
-}
-
 // How the copies are written: past the Infinity Cache (`streamed`), otherwise quantised rows at device scope and others
-// with ordinary stores, except long rows without scales in large steps.
+// with ordinary stores, except long rows without scales in large steps (copies_written_through in a2a_rules.h).
 hipError_t launch_dispatch_resolve(const PushArgs &args, const FinalizeArgs &fin, const Workspace &ws, bool quantize,
                                    uint32_t total_tokens, bool streamed, hipStream_t stream, KernelTiming timing) {
     uint32_t threads = push_threads(args, quantize);
@@ -2721,7 +2706,8 @@ hipError_t launch_dispatch_resolve(const PushArgs &args, const FinalizeArgs &fin
         else A2A_LAUNCH_RESOLVE(true, kDeviceScope, kScalesPlain);
     } else if (columns.blocks != 0) {
         A2A_LAUNCH_RESOLVE(false, kOrdinary, kScalesApart);
-    } else if (written_through(args, ws, total_tokens)) {
+    } else if (args.hidden_dim_scale == 0 &&
+               copies_written_through((uint64_t)total_tokens * ws.topk * args.row_bytes, args.row_bytes, ws.topk)) {
         A2A_LAUNCH_RESOLVE(false, kDeviceScope, kScalesPlain);
     } else {
         if (past_l2) A2A_LAUNCH_RESOLVE(false, kOrdinary, kScalesPastL2);

@@ -54,7 +54,41 @@ inline bool copies_past_cache(uint64_t copies, bool quantize, uint32_t topk) {
     return copies >= kStreamCopies && (quantize || topk > 2);
 }
 
-// The same for the recvs of the split calls, from kStreamReceived bytes of copies in all of a step's recvs on.  What this
+// Whether copies that stay in the Infinity Cache, are not quantised and bring no scales are stored at device scope.  Ordinary
+// stores leave them dirty in eight L2s, which write them back in an order of their own; written through, they reach memory as
+// the rows are worked off, but every store is held until it is there.  What decides is how much of its last 4 KB a row fills
+// (an L2's 16 channels of 256 bytes repeat after 4 KB: the fuller the rows, the more evenly the stores of a workgroup lie on
+// them) and how many copies a load feeds.  us per step whose buffers are not those of the step before, ordinary / written
+// through, with nothing between dispatch and combine | with a sweep that reads the received rows | with one that reads them
+// and writes expert_y:
+//                        K = 6, 280 MB                                K = 8, 280 MB
+//    4608 bytes  131.9 / 136.5 | 236.1 / 240.1 | 263.6 / 266.0  122.4 / 124.4 | 228.5 / 231.2 | 260.1 / 262.2
+//    6144        125.5 / 127.4 | 231.2 / 234.2 | 259.4 / 262.2  124.7 / 119.3 | 226.0 / 228.3 | 254.6 / 256.9
+//    7168        127.9 / 124.8 | 230.9 / 232.5 | 258.8 / 260.6  125.9 / 120.9 | 226.2 / 226.9 | 257.6 / 258.7
+//    8192        130.6 / 125.8 | 228.7 / 229.0 | 258.2 / 255.8  126.5 / 122.3 | 229.0 / 227.0 | 259.8 / 257.1
+//    9216        125.1 / 126.1 | 235.8 / 236.5 | 263.6 / 264.9  124.7 / 119.7 | 230.9 / 231.8 | 265.3 / 265.1
+//   10240        125.1 / 124.8 | 234.2 / 235.5 | 263.7 / 265.1  125.6 / 120.3 | 230.9 / 231.2 | 264.0 / 264.3
+//   12288        129.9 / 123.9 | 231.1 / 231.0 | 261.4 / 260.7  125.7 / 121.3 | 231.5 / 230.4 | 263.9 / 262.5
+//   12800        126.6 / 126.6 | 240.8 / 241.4 | 273.9 / 274.4  122.8 / 119.5 | 235.0 / 235.4 | 271.8 / 270.4
+//   28672        129.7 / 125.7 | 249.3 / 245.5 | 281.9 / 279.7  123.9 / 122.1 | 249.9 / 248.9 | 285.8 / 284.7
+// Of 23 lengths between 4096 and 28672 bytes, K = 6 to 8, nothing between, every one with topk * (share of whole 4 KB filled)
+// of at least 5 is level or gains, up to 5 %, and every one below is level or loses, up to 3.4 %; K = 7 turns at 5888 bytes
+// (0.719).  Behind a sweep the rows that are less than three quarters full lose 1 to 1.7 % also with K = 8 (5120: 224.1 /
+// 228.0), those above lie between -1 and +2 %.  Steps over the same buffers again and again, as no user's are, gain less or
+// lose: 280 MB of 8 KB 110.8 / 110.6, of 4 KB 112.8 / 116.0.
+// It loses with few copies a token (K = 4 behind a reader 245.6 / 247.4), with rows of 2 KB (131.7 / 134.1), with rows that
+// bring scales (fp8 rows of 5120 bytes 75.3 / 77.5, of 4096 behind a reader 300 / 308), and below kWrittenThrough bytes of copies
+// (4 KB rows, 79 MB: dispatch 24.0 / 24.9; 108 MB level).
+constexpr uint64_t kWrittenThrough = 120000000;
+
+inline bool copies_written_through(uint64_t copies, uint32_t row_bytes, uint32_t topk) {
+    constexpr uint64_t kPeriod = 4096;
+    const uint64_t whole = (row_bytes + kPeriod - 1) / kPeriod * kPeriod;
+    return copies >= kWrittenThrough && topk >= 6 && row_bytes >= kPeriod && 4ull * row_bytes >= 3 * whole &&
+           (uint64_t)topk * row_bytes >= 5 * whole;
+}
+
+// copies_past_cache for the recvs of the split calls, from kStreamReceived bytes of copies in all of a step's recvs on.  What this
 // keeps in the cache are the STAGED rows, which the recvs of all the ranks a token was routed to read, and the copies of the
 // first recvs are gone anyway by the time the last one has run.  Whole steps, us, copies kept / past the cache, with a
 // sweep that reads the received rows, and with one that reads them and writes expert_y:

@@ -10,21 +10,26 @@ pytestmark = pytest.mark.gpu
 DEV = torch.device("cuda:0")
 BF16, F32 = torch.bfloat16, torch.float32
 
-# tokens, experts, top-k, hidden, type: copies of 120 MB are the line
+# tokens, experts, top-k, hidden, type, whether they are written through: copies of 120 MB are the line
 STEPS = [
-    ([2441, 1], 16, 6, 4096, BF16),        # 120.03 MB: written through
-    ([2440, 1], 16, 6, 4096, BF16),        # 119.98 MB: not
-    ([2000, 500], 17, 6, 4096, BF16),      # an expert a receiver has not got
-    ([4300, 0, 10], 24, 7, 2048, BF16),    # the shortest rows
-    ([2500, 10], 24, 6, 4088, BF16),       # rows that are not multiples of 2 KB: not
-    ([1500, 1], 12, 5, 8192, BF16),        # five copies a token: not
-    ([620, 625], 32, 6, 4096, F32),        # 122 MB of 16 KB rows
-    ([560, 3], 64, 8, 7168, F32),          # rows longer than a workgroup has threads for
+    ([2441, 1], 16, 6, 4096, BF16, True),         # 120.03 MB
+    ([2440, 1], 16, 6, 4096, BF16, False),        # 119.98 MB
+    ([2000, 500], 17, 6, 4096, BF16, True),       # an expert a receiver has not got
+    ([4300, 0, 10], 24, 7, 2048, BF16, True),     # the shortest rows
+    ([2500, 10], 24, 6, 4088, BF16, True),        # rows that are not multiples of 2 KB: the last 4 KB nearly full
+    ([1500, 1], 12, 5, 8192, BF16, False),        # five copies a token
+    ([620, 625], 32, 6, 4096, F32, True),         # 122 MB of 16 KB rows
+    ([560, 3], 64, 8, 7168, F32, True),           # rows longer than a workgroup has threads for
+    ([2000, 1], 16, 6, 5120, BF16, True),         # six copies of rows whose last 4 KB are half full: just enough
+    ([2000, 1], 16, 6, 5112, BF16, False),        # and one piece less
+    ([2900, 1], 16, 7, 3072, BF16, True),         # rows that are three quarters full: seven copies are enough
+    ([3300, 1], 16, 6, 3072, BF16, False),        # six are not
+    ([2900, 1], 18, 8, 3064, BF16, False),        # nor are eight of shorter ones
 ]
 
 
-@pytest.mark.parametrize("tokens,experts,topk,hidden,dtype", STEPS, ids=[f"{s[0]}_k{s[2]}_h{s[3]}" for s in STEPS])
-def test_large_steps_of_long_rows(tokens, experts, topk, hidden, dtype):
+@pytest.mark.parametrize("tokens,experts,topk,hidden,dtype,through", STEPS, ids=[f"{s[0]}_k{s[2]}_h{s[3]}" for s in STEPS])
+def test_large_steps_of_long_rows(tokens, experts, topk, hidden, dtype, through):
     print(f"tokens={tokens} topk={topk} hidden={hidden} {dtype}", flush=True)
     cfg = RefConfig("through", len(tokens), 1, max(tokens), experts, hidden, None, topk, dtype, dtype, None, expert_padding=2)
     world = [make_ref_rank(cfg, r, t) for r, t in enumerate(tokens)]

@@ -9,6 +9,7 @@ import pytest
 
 from test_gpu_shapes import STREAMED, copies_of
 from test_gpu_split import PIECES
+from test_gpu_written_through import STEPS
 
 CSRC = Path(__file__).resolve().parent.parent / "pplx-garden_amd" / "csrc"
 
@@ -19,6 +20,9 @@ uint32_t layers(uint32_t tokens) { return a2a::token_layers(tokens).layers; }
 uint32_t layer_rows(uint32_t tokens) { return a2a::token_layers(tokens).rows; }
 int past_cache(uint64_t copies, int quantize, uint32_t k) { return a2a::copies_past_cache(copies, quantize != 0, k); }
 int received_past_cache(uint64_t copies) { return a2a::received_past_cache(copies); }
+int written_through(uint64_t copies, uint32_t row_bytes, uint32_t k) {
+    return a2a::copies_written_through(copies, row_bytes, k);
+}
 int one_launch(uint32_t rows, uint32_t row_bytes, uint32_t items, uint32_t threads) {
     return a2a::first_recv_in_one_launch(rows, row_bytes, items, threads);
 }
@@ -38,6 +42,7 @@ def rules(tmp_path_factory):
     lib = ctypes.CDLL(str(folder / "rules.so"))
     lib.past_cache.argtypes = [ctypes.c_uint64, ctypes.c_int, ctypes.c_uint32]
     lib.received_past_cache.argtypes = [ctypes.c_uint64]
+    lib.written_through.argtypes = [ctypes.c_uint64, ctypes.c_uint32, ctypes.c_uint32]
     return lib
 
 
@@ -61,6 +66,23 @@ def test_copies_that_the_infinity_cache_can_hold_stay_there_for_their_reader(rul
 @pytest.mark.parametrize("row,hidden,scales,k,tokens,streamed", STREAMED)
 def test_the_gpu_tests_of_streamed_steps_lie_on_the_side_they_are_meant_for(rules, row, hidden, scales, k, tokens, streamed):
     assert bool(rules.past_cache(copies_of(row, hidden, k, tokens), 0, k)) == streamed
+
+
+def test_rows_that_leave_much_of_their_last_4_kb_empty_are_not_written_through(rules):
+    size = 200000000
+    assert all(rules.written_through(size, row, k) for row in (4096, 7168, 8192, 12288, 14336, 16384, 28672) for k in (6, 7, 8))
+    assert not any(rules.written_through(size, row, 6) for row in (2048, 4080, 4112, 4608, 5120, 5888, 6144, 6656, 8704, 9216))
+    assert rules.written_through(size, 6144, 7) and rules.written_through(size, 9216, 8) and rules.written_through(size, 12800, 7)
+    assert not any(rules.written_through(size, row, k) for row in (4352, 5888, 6128, 8704) for k in (7, 8, 64))
+    assert not any(rules.written_through(size, 8192, k) for k in (1, 4, 5)) and not rules.written_through(119999999, 8192, 8)
+    assert rules.written_through(size, 0xFFFFF000, 64)
+
+
+@pytest.mark.parametrize("tokens,experts,topk,hidden,dtype,through", STEPS)
+def test_the_gpu_tests_of_written_through_steps_lie_on_the_side_they_are_meant_for(rules, tokens, experts, topk, hidden, dtype,
+                                                                                   through):
+    row = hidden * dtype.itemsize
+    assert bool(rules.written_through(sum(tokens) * topk * row, row, topk)) == through
 
 
 def test_received_rows_that_the_cache_can_keep_stay_there(rules):
