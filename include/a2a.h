@@ -321,8 +321,9 @@ int a2a_ctx_read_table(a2a_ctx *ctx, uint32_t rank, uint32_t which,
  *   A2A_KERNEL_ROUTE         the routing launch that precedes the pack of a large
  *                            step (a2a_dispatch) or the staging of a large send
  *                            (a2a_dispatch_send); a step that counts its routing
- *                            inside the pack or the staging launch (up to 8192 or
- *                            16384 copies; a send up to 65535) or runs several
+ *                            inside the pack or the staging launch (with dense index
+ *                            rows up to 8192 or 16384 copies, a send up to 65535;
+ *                            fewer with a gap behind the rows) or runs several
  *                            routing kernels (A2A_FLAG_SEPARATE_ROUTING) has no
  *                            such launch and leaves those events alone
  *   A2A_KERNEL_GATHER        the gather of the next a2a_combine or a2a_combine_recv

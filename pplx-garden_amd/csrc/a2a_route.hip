@@ -443,7 +443,8 @@ hipError_t launch_route_accumulate(const RouteArgs &args, const Workspace &ws, u
     // one workgroup per chunk and one more that hands over the totals between steps
     const dim3 grid(total_blocks + 1);
     if (for_send) {
-        hipLaunchKernelGGL(route_hist_kernel<2>, grid, dim3(kRouteBlock), 0, stream, args, ws);
+        hipExtLaunchKernelGGL(route_hist_kernel<2>, grid, dim3(kRouteBlock), 0, stream, timing.start, timing.stop,
+                              0, args, ws);
     } else {
         hipExtLaunchKernelGGL(route_hist_kernel<1>, grid, dim3(kRouteBlock), 0, stream, timing.start, timing.stop,
                               0, args, ws);

@@ -22,6 +22,63 @@ class WorldResult:
     out_tokens: List[np.ndarray]      # per rank [T, H] bf16 codes (uint16)
 
 
+class RouteWatch:
+    """Whether the next call on `ctx` that routes its tokens does so in a launch of its own, in front of the one that moves the
+    rows (KERNEL_ROUTE's events are left alone by calls that route and move in one launch)."""
+
+    def __init__(self, ctx):
+        from pplx_garden_amd.native.p2p_all_to_all import KERNEL_ROUTE
+
+        self._events = [torch.cuda.Event(enable_timing=True) for _ in range(3)]
+        for e in self._events:
+            e.record()
+        torch.cuda.synchronize()
+        self._before = self._events[2].elapsed_time(self._events[0])
+        ctx.time_next_kernel(KERNEL_ROUTE, self._events[0].cuda_event, self._events[1].cuda_event)
+
+    def launched(self) -> bool:
+        torch.cuda.synchronize()
+        return self._events[2].elapsed_time(self._events[0]) != self._before
+
+
+def with_gap(indices: torch.Tensor, gap: int = 3) -> torch.Tensor:
+    """The same index rows with `gap` words behind each of them, which are ids of no expert."""
+    if indices.shape[0] == 0:
+        return indices
+    wide = torch.full((indices.shape[0], indices.shape[1] + gap), -2, dtype=torch.int32, device=indices.device)
+    wide[:, :indices.shape[1]] = indices.view(torch.int32)
+    return wide.view(indices.dtype)[:, :indices.shape[1]]
+
+
+def dispatch_world_with_strays(inputs, *, num_experts: int, world_size: int, expert_padding: int, out_rows: int, quantize: bool,
+                               hidden_dim_scale: int = 0):
+    """The oracle's dispatch of one node where ids of `num_experts` and above name no expert and their copies go nowhere: to the
+    experts of one rank more, which has no tokens and so leaves the others' layout as it is.  Returns (outs, routes): of each
+    source its counts, offsets per expert, offsets of the entries (0 for those that go nowhere) and slots (-1 for those)."""
+    Le = num_experts // world_size
+    assert Le * world_size == num_experts
+    strays = [np.asarray(i.indices).astype(np.int64) >= num_experts for i in inputs]
+    moved = [oracle.RankInput(x=i.x, indices=np.where(s, num_experts, np.asarray(i.indices).astype(np.int64)), x_scale=i.x_scale,
+                              bound_m=i.bound_m) for i, s in zip(inputs, strays)]
+    nobody = oracle.RankInput(x=inputs[0].x[:0], indices=moved[0].indices[:0],
+                              x_scale=None if inputs[0].x_scale is None else inputs[0].x_scale[:0])
+    outs = oracle.dispatch_world(moved + [nobody], num_experts=num_experts + Le, world_size=world_size + 1,
+                                 node_size=world_size + 1, expert_padding=expert_padding,
+                                 out_rows=out_rows + sum(int(s.sum()) for s in strays) + Le * expert_padding, quantize=quantize,
+                                 hidden_dim_scale=hidden_dim_scale)
+    for o in outs[:world_size]:
+        assert not o.written[out_rows:].any()
+        o.x, o.written = o.x[:out_rows], o.written[:out_rows]
+        o.x_scale = None if o.x_scale is None else o.x_scale[:out_rows]
+    routes = []
+    for g, (i, s) in enumerate(zip(moved, strays)):
+        n = i.indices.shape[0] if i.bound_m is None else i.bound_m
+        count, toff, eoff = oracle.route(i.indices[:n], num_experts + Le)
+        routes.append((count[:num_experts], eoff[:num_experts], np.where(s[:n].reshape(-1), 0, toff),
+                       np.where(s, -1, outs[0].slots[g])))
+    return outs[:world_size], routes
+
+
 def act_numpy(q: np.ndarray, scale: np.ndarray) -> np.ndarray:
     """The 'expert' of the reference's test: 2 * dequantised row, as bf16 codes
     (tests/p2p_all_to_all/test_p2p_all_to_all.py:44-50 with the block layout of
@@ -74,20 +131,22 @@ def make_ops(case: Case, device: torch.device, max_num_tokens: Optional[int] = N
 
 def run_gpu(case: Case, world_data: Sequence[RankData], rows: int, device: torch.device,
             split: bool = False, expert_y_override=None, context_flags: int = 0, ops=None,
-            order: Optional[Sequence[int]] = None) -> WorldResult:
+            order: Optional[Sequence[int]] = None, strided: bool = False, routes: Optional[list] = None) -> WorldResult:
     """dispatch -> 2*dequant -> combine on the GPU through the operator API.
 
     split=False: every rank calls dispatch()/combine() with do_send and do_recv
     (the group calls of the library); split=True: all sends, then all recvs (the
     four split calls).  With `ops` the given operators are used (and kept): several
-    steps on one context.  `order`: in which the ranks make the group calls."""
+    steps on one context.  `order`: in which the ranks make the group calls.  `strided`: index rows with a gap behind
+    them.  `routes` gets, for the group call or for every send that has tokens, whether it routed in a launch of its own."""
     N, H, Hs, Le = case.world_size, case.hidden_dim, case.hidden_dim_scale, case.experts_per_rank
     own_ops = ops is None
     if own_ops:
         _, ops = make_ops(case, device, context_flags=context_flags)
     try:
         dev = [
-            dict(x=rd.x.to(device), idx=rd.indices_u32.to(device), w=rd.weights.to(device))
+            dict(x=rd.x.to(device), idx=with_gap(rd.indices_u32.to(device)) if strided else rd.indices_u32.to(device),
+                 w=rd.weights.to(device))
             for rd in world_data
         ]
         outs = []
@@ -103,15 +162,26 @@ def run_gpu(case: Case, world_data: Sequence[RankData], rows: int, device: torch
                             out_expert_x_scale=outs[r]["s"], dp_x=dev[r]["x"], dp_x_scale=None,
                             indices=dev[r]["idx"], weights=dev[r]["w"], **kw)
 
+        watches = []
+
+        def watch():
+            if routes is not None:
+                watches.append(RouteWatch(ops[0].context))
+
         if split:
             for r in range(N):
+                if world_data[r].indices.shape[0]:
+                    watch()
                 dispatch(r, do_send=True, do_recv=False)
             for r in range(N):
                 dispatch(r, do_send=False, do_recv=True)
         else:
+            watch()
             for r in order or range(N):
                 dispatch(r)
         torch.cuda.synchronize(device)
+        if routes is not None:
+            routes.extend(w.launched() for w in watches)
         flags = ops[0].context.status()
         assert flags == 0, f"device error flags {flags}"
 

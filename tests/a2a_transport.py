@@ -11,6 +11,7 @@ import numpy as np
 import torch
 
 import a2a_oracle as oracle
+from a2a_harness import RouteWatch
 
 SENTINEL = 0xA5
 _NP_OUT = {torch.bfloat16: "bf16", torch.float16: "f16", torch.float32: "f32"}
@@ -134,9 +135,10 @@ def to_f32(a: np.ndarray, dtype: torch.dtype) -> np.ndarray:
 
 
 def run_gpu(cfg: RefConfig, world: List[RefRank], rows: int, device: torch.device, split: bool,
-            scale_layout: str = "row"):
+            scale_layout: str = "row", routes: Optional[list] = None):
     """dispatch -> act -> combine through the operator; returns per-rank dicts of numpy results.
-    scale_layout "col": the output scale tensor is the transpose of a [Hs, rows] buffer (strided)."""
+    scale_layout "col": the output scale tensor is the transpose of a [Hs, rows] buffer (strided).
+    `routes` gets, for the group call or for every send that has tokens, whether it routed in a launch of its own."""
     N, H, Hs = cfg.world_size, cfg.hidden_dim, cfg.hidden_dim_scale
     Le = -(-cfg.num_experts // N)
     ops = make_ops(cfg, device)
@@ -161,15 +163,26 @@ def run_gpu(cfg: RefConfig, world: List[RefRank], rows: int, device: torch.devic
                             out_expert_x_scale=outs[r]["s"], dp_x=dev[r]["x"], dp_x_scale=dev[r]["xs"],
                             indices=dev[r]["idx"], weights=dev[r]["w"], bound_m=None, **kw)
 
+        watches = []
+
+        def watch():
+            if routes is not None:
+                watches.append(RouteWatch(ops[0].context))
+
         if split:
             for r in range(N):
+                if world[r].dp_x.shape[0]:
+                    watch()
                 dispatch(r, do_send=True, do_recv=False)
             for r in range(N):
                 dispatch(r, do_send=False, do_recv=True)
         else:
+            watch()
             for r in range(N):
                 dispatch(r)
         torch.cuda.synchronize(device)
+        if routes is not None:
+            routes.extend(w.launched() for w in watches)
         assert ops[0].context.status() == 0
 
         ys = [act(outs[r]["x"], outs[r]["s"]).to(cfg.out_dtype) for r in range(N)]
