@@ -1,5 +1,6 @@
 """The one-launch dispatch of steps of several sources (and of larger steps of one) against the oracle, bit for bit: rows,
-scales, counts and every routing table of every source, at the sizes where its divisions of the work can go wrong."""
+scales, counts and every routing table of every source, at the sizes where its divisions of the work can go wrong; and steps
+beyond its limits, which have a routing launch of their own."""
 
 from dataclasses import replace
 
@@ -9,7 +10,7 @@ import torch
 
 import a2a_oracle as oracle
 from a2a_cases import C1, bf16_codes, make_rank, scaled
-from a2a_harness import SENTINEL, make_ops, rows_needed
+from a2a_harness import SENTINEL, RouteWatch, dispatch_world_with_strays, make_ops, rows_needed, with_gap
 from a2a_transport import RefConfig, check, make_ref_rank, rows_for, run_gpu
 from pplx_garden_amd.native import p2p_all_to_all as native
 
@@ -17,10 +18,11 @@ pytestmark = pytest.mark.gpu
 DEV = torch.device("cuda:0")
 
 
-def run_and_check(case, tokens, bounds=None, repeats=False, strided=False, stray=False):
+def run_and_check(case, tokens, bounds=None, repeats=False, strided=False, stray=False, two_launches=False):
     """One dispatch of `tokens[r]` tokens of every rank; `repeats`: every third token names its first expert twice;
-    `strided`: index rows with a gap behind them (another kernel's step, the same result); `stray`: the first token of
-    every source names an expert that does not exist (flagged, its other copies are sent)."""
+    `strided`: index rows with a gap behind them (another kernel's step, the same result); `stray`: some tokens of every
+    source, its first and whole wavefronts of the larger ones among them, name experts that do not exist (flagged, all other
+    copies are sent as if those were not there); `two_launches`: the step has a routing launch of its own."""
     N, Le, H, Hs, K, E = (case.world_size, case.experts_per_rank, case.hidden_dim, case.hidden_dim_scale, case.topk,
                           case.num_experts)
     bounds = bounds or [None] * N
@@ -29,35 +31,41 @@ def run_and_check(case, tokens, bounds=None, repeats=False, strided=False, stray
         for rd in world:
             rd.indices[::3, K - 1] = rd.indices[::3, 0]
     rows = rows_needed(case, world)
-    inputs = [oracle.RankInput(x=bf16_codes(rd.x), indices=rd.indices.numpy(), bound_m=b) for rd, b in zip(world, bounds)]
-    want = oracle.dispatch_world(inputs, num_experts=E, world_size=N, node_size=case.node_size or N,
-                                 expert_padding=case.expert_padding, out_rows=rows, quantize=True)
+    if stray:
+        for rd in world:
+            rd.indices[::5, K - 1] = E + 3
+            rd.indices[1::7, 0] = -1          # (0xFFFFFFFF)
+            rd.indices[20:40] = E             # whole wavefronts of them
+    inputs = [oracle.RankInput(x=bf16_codes(rd.x), indices=rd.indices.numpy().view(np.uint32), bound_m=b)
+              for rd, b in zip(world, bounds)]
+    if stray:
+        want, routes = dispatch_world_with_strays(inputs, num_experts=E, world_size=N, expert_padding=case.expert_padding,
+                                                  out_rows=rows, quantize=True)
+    else:
+        want = oracle.dispatch_world(inputs, num_experts=E, world_size=N, node_size=case.node_size or N,
+                                     expert_padding=case.expert_padding, out_rows=rows, quantize=True)
+        routes = []
+        for r, rd in enumerate(world):
+            n_eff = tokens[r] if bounds[r] is None else bounds[r]
+            count, toff, eoff = oracle.route(rd.indices.numpy()[:n_eff], E)
+            routes.append((count, eoff, toff, want[0].slots[r][:n_eff].reshape(-1)))
     _, ops = make_ops(case, DEV, max_num_tokens=max(tokens))
     try:
         t = []
         for r, rd in enumerate(world):
-            idx = rd.indices.clone()
-            if stray and idx.shape[0]:
-                idx[0, K - 1] = E + 3
-            idx = idx.view(torch.uint32).to(DEV)
-            if strided and idx.shape[0]:
-                wide = torch.zeros((idx.shape[0], K + 3), dtype=torch.uint32, device=DEV)
-                wide[:, :K] = idx
-                idx = wide[:, :K]
-            t.append(dict(x=rd.x.to(DEV), idx=idx, w=rd.weights.to(DEV),
+            idx = rd.indices_u32.to(DEV)
+            t.append(dict(x=rd.x.to(DEV), idx=with_gap(idx) if strided else idx, w=rd.weights.to(DEV),
                           b=None if bounds[r] is None else torch.tensor([bounds[r]], dtype=torch.int32, device=DEV),
                           n=torch.full((Le,), -1, dtype=torch.int32, device=DEV),
                           ox=torch.full((rows, H), SENTINEL, dtype=torch.uint8, device=DEV).view(torch.float8_e4m3fn),
                           os=torch.full((rows, Hs), -7.0, dtype=torch.float32, device=DEV)))
+        ctx = ops[0].context
+        watch = RouteWatch(ctx)
         for r in range(N):
             ops[r].dispatch(out_expert_num_tokens=t[r]["n"], out_expert_x=t[r]["ox"], out_expert_x_scale=t[r]["os"],
                             dp_x=t[r]["x"], dp_x_scale=None, indices=t[r]["idx"], weights=t[r]["w"], bound_m=t[r]["b"])
-        torch.cuda.synchronize(DEV)
-        ctx = ops[0].context
-        if stray:
-            assert ctx.status() & 1     # A2A_DEV_BAD_EXPERT_ID
-            return
-        assert ctx.status() == 0
+        assert watch.launched() == two_launches
+        assert ctx.status() == (native.DEV_BAD_EXPERT_ID if stray else 0)
         for r in range(N):
             n_local = max(0, min(Le, E - r * Le))
             np.testing.assert_array_equal(t[r]["n"].cpu().numpy()[:n_local], want[r].num_tokens[:n_local])
@@ -67,14 +75,13 @@ def run_and_check(case, tokens, bounds=None, repeats=False, strided=False, stray
             np.testing.assert_array_equal(got_x[wr], want[r].x[wr])
             np.testing.assert_array_equal(got_s[wr].view(np.uint32), want[r].x_scale[wr].view(np.uint32))
             assert (got_x[~wr] == SENTINEL).all() and (got_s[~wr] == -7.0).all()
-            n_eff = tokens[r] if bounds[r] is None else bounds[r]
-            count, toff, eoff = oracle.route(world[r].indices.numpy()[:n_eff], E)
+            count, eoff, toff, slots = routes[r]
             np.testing.assert_array_equal(ctx.read_table(r, native.TABLE_NUM_ROUTED, E).numpy(), count)
             np.testing.assert_array_equal(ctx.read_table(r, native.TABLE_EXPERT_OFFSETS, E).numpy(), eoff)
-            if n_eff:
-                np.testing.assert_array_equal(ctx.read_table(r, native.TABLE_TOKEN_OFFSET, n_eff * K).numpy(), toff)
-                np.testing.assert_array_equal(ctx.read_table(r, native.TABLE_SLOT, n_eff * K).numpy(),
-                                              want[0].slots[r][:n_eff].reshape(-1))
+            if toff.size:
+                np.testing.assert_array_equal(ctx.read_table(r, native.TABLE_TOKEN_OFFSET, toff.size).numpy(), toff)
+                np.testing.assert_array_equal(ctx.read_table(r, native.TABLE_SLOT, toff.size).numpy().astype(np.uint32),
+                                              slots.reshape(-1).astype(np.uint32))     # (-1: nowhere)
     finally:
         for op in ops:
             op.destroy()
@@ -95,16 +102,21 @@ STEPS = {
     "top3_bounds": (replace(BASE, topk=3), [70, 40, 0, 9, 70, 1, 2, 55], dict(bounds=[None, 0, None, 5, 69, None, 1, 55])),
     "1024_tokens": (replace(BASE, hidden_dim=7168, num_experts=256), [128] * 8, {}),
     "2048_tokens_eight_a_workgroup": (replace(BASE, hidden_dim=7168, expert_padding=128), [250, 256, 262, 256, 256, 255, 257, 256], {}),
-    "2049_tokens_the_two_launches": (BASE, [257] + [256] * 7, {}),
-    "2048_tokens_of_one": (replace(BASE, hidden_dim=1024), [0, 0, 0, 2048, 0, 0, 0, 0], dict(repeats=True)),
+    "2049_tokens_the_two_launches": (BASE, [257] + [256] * 7, dict(two_launches=True)),
+    "2048_tokens_of_one": (BASE, [0, 0, 0, 2048, 0, 0, 0, 0], dict(repeats=True)),
+    "2048_short_rows_of_one_the_two_launches": (replace(BASE, hidden_dim=1024), [0, 0, 0, 2048, 0, 0, 0, 0],
+                                                dict(repeats=True, two_launches=True)),
     "1025_tokens_of_one_bound_513": (BASE, [1025] + [0] * 7, dict(bounds=[513] + [None] * 7)),
     "16_ranks_384_experts": (replace(BASE, world_size=16, num_experts=384, hidden_dim=384), [40, 0, 7, 64] * 4, {}),
     "32_ranks_all_tables": (replace(BASE, world_size=32, num_experts=384, hidden_dim=256), [1 + 3 * (r % 5) for r in range(32)], {}),
-    "32_ranks_tables_too_large": (replace(BASE, world_size=32, num_experts=512, hidden_dim=256), [9] * 32, {}),
+    "32_ranks_tables_too_large": (replace(BASE, world_size=32, num_experts=512, hidden_dim=256), [9] * 32, dict(two_launches=True)),
     "two_ranks_many_experts_each": (replace(BASE, world_size=2, num_experts=300), [90, 61], {}),
     "hidden_14336_two_nodes": (replace(BASE, world_size=4, num_experts=64, hidden_dim=14336, node_size=2), [3, 20, 0, 300], {}),
     "strided_the_general_kernel": (BASE, [20] * 8, dict(strided=True)),
-    "expert_that_is_none": (BASE, [5, 0, 9, 1, 30, 2, 2, 2], dict(stray=True)),
+    "experts_that_are_none": (BASE, [5, 0, 9, 1, 30, 2, 2, 2], dict(stray=True)),
+    "experts_that_are_none_eight_a_workgroup": (replace(BASE, expert_padding=4), [250, 256, 3, 255, 256, 0, 257, 700],
+                                                dict(stray=True, repeats=True)),
+    "experts_that_are_none_the_two_launches": (BASE, [257] + [256] * 7, dict(stray=True, two_launches=True)),
 }
 
 
@@ -116,19 +128,24 @@ def test_steps_of_several_sources(name):
 
 
 BF16, F16, F32, FP8 = torch.bfloat16, torch.float16, torch.float32, torch.float8_e4m3fn
+# configuration, tokens, layout of the scales, whether there is a routing launch of its own
 TRANSPORT = {
-    "fp8_row": (RefConfig("fp8_row", 8, 1, 128, 64, 5120, 40, 8, FP8, BF16, F32), [128, 0, 42, 1, 128, 0, 42, 1], "row"),
-    "fp8_col_pad16": (RefConfig("fp8_col", 8, 1, 250, 64, 1024, 8, 8, FP8, BF16, F32, expert_padding=16), [250] * 8, "col"),
-    "bf16_no_scales": (RefConfig("bf16", 4, 1, 300, 32, 4096, None, 6, BF16, BF16, None), [300, 1, 0, 299], "row"),
-    "f32_rows_of_16_kb": (RefConfig("f32", 2, 1, 40, 16, 4096, None, 2, F32, F32, None, node_size=1), [40, 3], "row"),
-    "f16_one_chunk": (RefConfig("f16", 3, 1, 33, 9, 8, None, 3, F16, F16, None), [33, 0, 32], "row"),
+    "fp8_row": (RefConfig("fp8_row", 8, 1, 128, 64, 5120, 40, 8, FP8, BF16, F32), [128, 0, 42, 1, 128, 0, 42, 1], "row", False),
+    "fp8_col_pad16": (RefConfig("fp8_col", 8, 1, 250, 64, 2048, 16, 8, FP8, BF16, F32, expert_padding=16), [250] * 8, "col", False),
+    "fp8_col_pad16_short_rows": (RefConfig("fp8_col", 8, 1, 250, 64, 1024, 8, 8, FP8, BF16, F32, expert_padding=16), [250] * 8,
+                                 "col", True),
+    "bf16_no_scales": (RefConfig("bf16", 4, 1, 300, 32, 4096, None, 6, BF16, BF16, None), [300, 1, 0, 299], "row", False),
+    "f32_rows_of_16_kb": (RefConfig("f32", 2, 1, 40, 16, 4096, None, 2, F32, F32, None, node_size=1), [40, 3], "row", False),
+    "f16_one_chunk": (RefConfig("f16", 3, 1, 33, 9, 8, None, 3, F16, F16, None), [33, 0, 32], "row", False),
 }
 
 
 @pytest.mark.parametrize("name", TRANSPORT)
 def test_rows_moved_as_they_are(name):
-    cfg, tokens, layout = TRANSPORT[name]
+    cfg, tokens, layout, two_launches = TRANSPORT[name]
     print(f"{name} tokens={tokens}", flush=True)
     world = [make_ref_rank(cfg, r, t) for r, t in enumerate(tokens)]
     rows = rows_for(cfg, world)
-    check(cfg, world, rows, run_gpu(cfg, world, rows, DEV, split=False, scale_layout=layout))
+    routes = []
+    check(cfg, world, rows, run_gpu(cfg, world, rows, DEV, split=False, scale_layout=layout, routes=routes))
+    assert routes == [two_launches]
