@@ -8,8 +8,8 @@ import torch
 
 import a2a_oracle as oracle
 from a2a_cases import C0, C1, C2, bf16_codes, make_world, scaled
-from a2a_harness import (SENTINEL, WorldResult, assert_combine_close, assert_dispatch_equal, make_ops, rows_needed,
-                         run_gpu, run_oracle)
+from a2a_harness import (SENTINEL, RouteWatch, WorldResult, assert_combine_close, assert_dispatch_equal, make_ops, rows_needed,
+                         run_gpu, run_oracle, with_gap)
 from a2a_transport import RefConfig, make_ref_rank, oracle_combine, oracle_dispatch, rows_for
 from a2a_transport import make_ops as make_transport_ops
 from pplx_garden_amd.native import p2p_all_to_all as native
@@ -58,12 +58,14 @@ def test_quantiser_on_every_bf16_value_and_many_scales():
 
 
 @pytest.mark.parametrize("split", [False, True], ids=["group", "split"])
-@pytest.mark.parametrize("repeat", [1, 110, 450], ids=["one_launch_small", "one_launch_single", "two_launch"])
-def test_quantiser_on_nan_infinity_and_the_largest_bf16_value(repeat, split):
+@pytest.mark.parametrize("repeat,gap", [(1, False), (110, False), (450, False), (450, True)],
+                         ids=["one_launch_small", "one_launch_single", "two_launch_dispatch", "two_launches"])
+def test_quantiser_on_nan_infinity_and_the_largest_bf16_value(repeat, gap, split):
     """A NaN poisons its group of 128 (scale NaN, every code the NaN code), an infinity makes the
     scale infinite: bit for bit what the oracle says (which the CPU tests pin against a hand-written
-    expectation and torch's operations), in every dispatch kernel that quantises (10, 1100 and 4500
-    tokens take the three paths of the group call and of the split send)."""
+    expectation and torch's operations), in the dispatch kernels that quantise: 10, 1100 and 4500
+    tokens take a launch, a launch and two launches as a group call, and one launch each as a split send;
+    with a gap behind the index rows 4500 tokens are two launches either way."""
     from a2a_nonfinite import bad_rows, expected_special_groups
 
     bits, kinds = bad_rows()
@@ -87,12 +89,14 @@ def test_quantiser_on_nan_infinity_and_the_largest_bf16_value(repeat, split):
                      x=torch.full((2 * T, H), SENTINEL, dtype=torch.uint8, device=DEV).view(torch.float8_e4m3fn),
                      s=torch.full((2 * T, H // 128), -7.0, dtype=torch.float32, device=DEV)) for _ in range(2)]
         phases = [dict(do_send=True, do_recv=False), dict(do_send=False, do_recv=True)] if split else [dict()]
+        watch = RouteWatch(ops[0].context)
         for kw in phases:
             for r in range(2):
+                ids = ins[r]["idx"].view(torch.uint32).to(DEV)
                 ops[r].dispatch(out_expert_num_tokens=outs[r]["n"], out_expert_x=outs[r]["x"],
                                 out_expert_x_scale=outs[r]["s"], dp_x=ins[r]["x"].to(DEV), dp_x_scale=None,
-                                indices=ins[r]["idx"].view(torch.uint32).to(DEV), weights=ins[r]["w"].to(DEV), **kw)
-        torch.cuda.synchronize(DEV)
+                                indices=with_gap(ids) if gap else ids, weights=ins[r]["w"].to(DEV), **kw)
+        assert watch.launched() == (gap or (repeat == 450 and not split))
         assert ops[0].context.status() == 0
         for r in range(2):
             wr = want[r].written
@@ -114,7 +118,8 @@ def test_quantiser_on_nan_infinity_and_the_largest_bf16_value(repeat, split):
 
 
 @pytest.mark.parametrize("split", [False, True], ids=["group", "split"])
-@pytest.mark.parametrize("case", [C0, scaled(C0, 700), scaled(C0, 1200)], ids=["one_launch", "one_launch_mid_size", "two_launch"])
+@pytest.mark.parametrize("case", [C0, scaled(C0, 700), scaled(C0, 1200)],
+                         ids=["one_launch", "one_launch_mid_size", "two_launch_dispatch"])
 def test_bound_m_limits_the_tokens(case, split):
     world = make_world(case, "all")
     bounds = [case.num_tokens, 0, 17, 1]
@@ -337,12 +342,13 @@ def test_errors_are_reported_not_faulted():
             op.destroy()
 
 
+@pytest.mark.parametrize("tokens,gap", [(1500, False), (4200, True)], ids=["one_launch", "two_launches"])
 @pytest.mark.parametrize("split", [False, True], ids=["group", "split"])
-def test_device_errors_in_the_two_launch_paths(split):
+def test_device_errors_of_larger_steps(split, tokens, gap):
     """The same two device-side errors (an expert id out of range, receive buffers that are too small)
-    on a step large enough for the two-launch dispatch and send: flagged, not faulted, and the context
-    keeps working afterwards."""
-    case = scaled(C0, 1500)
+    on a larger step in one launch, and on one with a gap behind the index rows that takes the two-launch
+    dispatch and send: flagged, not faulted, and the context keeps working afterwards."""
+    case = scaled(C0, tokens)
     world = make_world(case, "one")
     N, Le, H, Hs = case.world_size, case.experts_per_rank, case.hidden_dim, case.hidden_dim_scale
     _, ops = make_ops(case, DEV)
@@ -358,12 +364,16 @@ def test_device_errors_in_the_two_launch_paths(split):
                       ox=torch.full((rows, H), SENTINEL, dtype=torch.uint8, device=DEV).view(torch.float8_e4m3fn),
                       os=torch.zeros((rows, Hs), dtype=torch.float32, device=DEV)) for _ in range(N)]
             x, w = rd.x.to(DEV), rd.weights.to(DEV)
+            ids = indices.view(torch.uint32).to(DEV)
+            if gap:
+                ids = with_gap(ids)
+            watch = RouteWatch(ctx)
             for ph in phases:
                 for r in range(N):
                     ops[r].dispatch(out_expert_num_tokens=t[r]["n"], out_expert_x=t[r]["ox"],
                                     out_expert_x_scale=t[r]["os"], dp_x=x if r == 0 else x[:0], dp_x_scale=None,
-                                    indices=(indices if r == 0 else indices[:0]).view(torch.uint32).to(DEV),
-                                    weights=w if r == 0 else w[:0], **ph)
+                                    indices=ids if r == 0 else ids[:0], weights=w if r == 0 else w[:0], **ph)
+            assert watch.launched() == gap
             return t
 
         run(bad, 16)
@@ -413,19 +423,21 @@ def test_operator_asserts_like_the_reference():
 
 
 @pytest.mark.parametrize("split", [False, True], ids=["group", "split"])
-@pytest.mark.parametrize("case,sources", [(C1, "all"), (scaled(C1, 1200), "one"), (scaled(C1, 300), "all"),
-                                          (scaled(C1, 40), "ragged"), (scaled(C1, 900), "one")],
-                         ids=["one_launch_dispatch", "two_launch_dispatch_one_source", "two_launch_dispatch", "ragged",
-                              "one_launch_dispatch_larger_source"])
-def test_calls_can_be_captured_in_a_hip_graph(case, sources, split):
+@pytest.mark.parametrize("case,sources,gap", [(C1, "all", False), (scaled(C1, 1200), "one", False),
+                                              (scaled(C1, 300), "all", False), (scaled(C1, 40), "ragged", False),
+                                              (scaled(C1, 900), "one", False), (scaled(C1, 2100), "one", True)],
+                         ids=["one_launch_dispatch", "one_launch_dispatch_large_source", "two_launch_dispatch", "ragged",
+                              "one_launch_dispatch_larger_source", "two_launches"])
+def test_calls_can_be_captured_in_a_hip_graph(case, sources, gap, split):
     """The calls only enqueue kernels whose arguments travel by value (no allocation, copy or
     synchronisation inside), so a dispatch + combine can be captured once and replayed
     (docs/fabric-lib.md:15 lists graph capture as a feature of the reference): the two group calls
     of every rank, or the four split calls of every rank (all sends, all recvs, all combine-sends,
     all combine-recvs) on a context whose staging was allocated at create.  Every replay, with eager
     work in between, must reproduce what the ORACLE says, bit for bit for the dispatch and within the
-    combine's tolerance.  The larger cases take the two-launch dispatch, whose step totals alternate
-    between two copies in device memory: the replays land on either copy."""
+    combine's tolerance.  300 tokens of every rank take the two-launch dispatch, and 2100 of one rank with a
+    gap behind the index rows that and the two-launch send: their totals alternate between two copies in
+    device memory, and the replays land on either copy."""
     world = make_world(case, sources)
     rows = rows_needed(case, world)
     N, Le, H, Hs = case.world_size, case.experts_per_rank, case.hidden_dim, case.hidden_dim_scale
@@ -439,7 +451,8 @@ def test_calls_can_be_captured_in_a_hip_graph(case, sources, split):
     try:
         t = []
         for r, rd in enumerate(world):
-            t.append(dict(x=rd.x.to(DEV), idx=rd.indices_u32.to(DEV), w=rd.weights.to(DEV),
+            ids = rd.indices_u32.to(DEV)
+            t.append(dict(x=rd.x.to(DEV), idx=with_gap(ids) if gap else ids, w=rd.weights.to(DEV),
                           n=torch.zeros(Le, dtype=torch.int32, device=DEV),
                           ox=torch.zeros((rows, H), dtype=torch.uint8, device=DEV).view(torch.float8_e4m3fn),
                           os=torch.zeros((rows, Hs), dtype=torch.float32, device=DEV),
@@ -479,8 +492,10 @@ def test_calls_can_be_captured_in_a_hip_graph(case, sources, split):
             for a in t:
                 a["n"].zero_(); a["ox"].view(torch.uint8).zero_(); a["os"].zero_(); a["o"].zero_()
 
+        watch = RouteWatch(ops[0].context)
         step()
         check("eager")
+        assert watch.launched() == (gap or (case.num_tokens == 300 and not split))
         assert ops[0].context.status() == 0
         graph = torch.cuda.CUDAGraph()
         side = torch.cuda.Stream(device=DEV)
