@@ -168,7 +168,11 @@ constexpr uint64_t kStreamedOutput = 84000000;
 // 6000 tokens 216.6 / 214.1 / 212.7 / 214.2, 8 x 4096 tokens 1161 / 1145 / 1139 / 1152, 8 x 2048 tokens of 5 KB fp8 rows 416.1 /
 // 410.2 / 406.7 / 409.3, float rows of 8 KB, 8 x 3000 tokens 663.7 / 657.5 / 655.4 / 656.7; K = 6 with 21 / 18 / 16, 8 x 4096
 // tokens 894.5 / 888.6 / 878.0 (in the cache 14 are 0.9 us better at 4096 tokens and 0.3 worse at 2668, 12 worse).  The launch
-// asks for LDS that nothing uses to bound them.  The ONE_RANK variant is left alone (1024 tokens 23.6 / 23.4-23.7), and so are
+// asks for LDS that nothing uses to bound them; with all of a compute unit's LDS given out, a kernel of another stream that
+// wants some waits for wavefronts to end, as it does without the bound, where they take all the wave slots.  Eight combines
+// beside bf16 matrix products on another stream, us for both, all wavefronts / bounded: 4096 tokens and eight products of
+// 4096 x 2048 x 7168 1370 / 1350, of 4096 x 7168 x 7168 2974 / 2917, 32 of 512 x 7168 x 2048 1393 / 1380; 8 x 512 tokens 1374 / 1365,
+// 2963 / 2933, 1403 / 1402.  The ONE_RANK variant is left alone (1024 tokens 23.6 / 23.4-23.7), and so are
 // steps whose wavefronts fit the GPU all at once (kAllAtOnce): bounded to 16 they take a second, half empty round (rows of
 // 14 KB: 8 x 40 tokens 9.08 / 8.68 us unbounded, 8 x 64 13.14 / 12.53; level where 16 hold them all and at 8064 wavefronts).
 constexpr uint64_t kAllAtOnce = 32 * 256;
