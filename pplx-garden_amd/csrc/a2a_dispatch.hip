@@ -2055,6 +2055,10 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8))) void 
 // experts each 252 / 224, one sender of 3000 with 4096 bytes 72.6 / 68.7.  Eight or sixteen columns a workgroup: 78.3 and 84.5 of
 // the first, level from 4096 tokens on.  Copies that are stored past the Infinity Cache keep their scales: 1165 us
 // against 1122 for 8 x 4096 tokens, whose column words then meet in no cache.
+// The token workgroups of that pack pay for these: one kernel is one register budget, and held to 64 vector registers
+// (eight wavefronts a SIMD) it spills 5 of them and 118 scalar ones (24 bytes of scratch a lane), where the packs without
+// column workgroups have 56, seven wavefronts and no spills.  2668 tokens of 5120 bytes: 27.6 us and 135.0 MB of traffic,
+// with scales by row 26.7 us and 128.3 MB, of 126.9 MB that the dispatch cannot do without.
 constexpr uint32_t kScaleColumns = 4;                         // one 16-byte load
 constexpr uint32_t kSpanChunks = 2;
 constexpr uint32_t kSpan = kSpanChunks * kRouteBlock;
@@ -2561,13 +2565,13 @@ hipError_t launch_dispatch_single(const PushArgs &args, const FinalizeArgs &fin,
 // Whether a step takes dispatch_sources_kernel, and its shape: tokens of a workgroup as in the kernels of one source
 // (about one workgroup per compute unit); beside the resolver as many wavefronts as there are units to move or chunks
 // to count (8 x 32 tokens of hidden 2048, 2 units and 8 chunks: 6.6 us with 4 wavefronts, 4.6 with 8), in as few rounds
-// as 15 of them need.  The line at 16384 entries: counting costs every workgroup 0.16 us per 1024 of them, where the
-// routing launch it replaces costs 5 to 6 us, and with more than eight tokens of top-8 a workgroup has more routes than
-// its resolver has lanes; and above 8192 entries rows of 2 KB, because with smaller ones the counting is what is left
-// (one source of 2048 tokens, hidden 1024: 21.5 us a step against 20.4; hidden 2048 and 1500 tokens: 23.2 against 23.9).
-// Steps of one source with up to
-// kSingleMaxEntries entries have the two kernels that are made for them (128 tokens 4.54 us against 4.77 here, 1024
-// tokens 15.4 against 16.1).
+// as 15 of them need.  The line at 16384 entries is the resolver's: with more than eight tokens of top-8 a workgroup has
+// more routes than its one resolving wavefront has lanes.  It is not the counting's, which costs every workgroup 0.16 us
+// per 1024 entries where the routing launch it replaces costs 5 to 6 us: level near 32 000 by these figures.  Larger steps
+// with two resolving wavefronts have not been measured.  Above 8192 entries rows of 2 KB, because with smaller ones the
+// counting is what is left (one source of 2048 tokens, hidden 1024: 21.5 us a step against 20.4; hidden 2048 and 1500
+// tokens: 23.2 against 23.9).  Steps of one source with up to kSingleMaxEntries entries have the two kernels that are made
+// for them (128 tokens 4.54 us against 4.77 here, 1024 tokens 15.4 against 16.1).
 bool plan_dispatch_sources(const PushArgs &args, const Workspace &ws, bool quantize, uint32_t total_tokens, SourcesPlan &plan,
                            uint32_t &groups, uint32_t &threads, uint32_t &rounds) {
     constexpr uint32_t kComputeUnits = 256;
