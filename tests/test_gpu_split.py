@@ -41,7 +41,7 @@ def test_split_parity(case, sources, device):
 
 F32, BF16, FP8 = torch.float32, torch.bfloat16, torch.float8_e4m3fn
 PIECES = [
-    # the recv's and the combine-send's rows are cut into pieces of 64 chunks of 16 bytes
+    # the recv's and the combine-send's rows are cut into pieces of 128 chunks of 16 bytes
     RefConfig("last-piece-not-full", 2, 1, 300, 16, 2944, 23, 4, FP8, BF16, F32),
     RefConfig("one-chunk-rows", 4, 1, 500, 16, 8, None, 4, BF16, BF16, None),
     RefConfig("more-scales-than-lanes", 2, 1, 400, 8, 512, 128, 2, FP8, BF16, F32),
