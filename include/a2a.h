@@ -101,9 +101,9 @@ typedef struct a2a_config {
  * on their first use. */
 #define A2A_FLAG_PREALLOC_STAGING 1u
 /* Never take the one-launch paths (routing counted inside the dispatch or send
- * kernel: small steps, and group steps of one source up to 8192 copies); always
- * run the routing kernels, then the pack.  Results are identical either way;
- * the flag exists to compare the two. */
+ * kernel: small steps, with dense index rows group steps of up to 16384 copies
+ * and sends of up to 65535); always run the routing kernels, then the pack.
+ * Results are identical either way; the flag exists to compare the two. */
 #define A2A_FLAG_SEPARATE_ROUTING 2u
 
 /* replaces AllToAllContext::new, a2a_context.rs:124-259 */
