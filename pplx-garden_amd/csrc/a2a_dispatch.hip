@@ -91,7 +91,9 @@ constexpr uint32_t kScalesAheadBytes = 6144;
 // PRE: the thread's first piece of the row was asked for earlier (first_piece) and is passed in.
 // POLICY: cache policy of the copies' stores.
 // SCALES: kScales... above (quantised rows always have theirs).
-template <bool QUANT, bool PRE = false, int POLICY = QUANT ? kDeviceScope : kOrdinary, int SCALES = kScalesPlain>
+// PIECES: 16-byte pieces of a copy that a thread moves together (pieces_per_lane in a2a_rules.h), all asked for before the
+// first is stored.
+template <bool QUANT, bool PRE = false, int POLICY = QUANT ? kDeviceScope : kOrdinary, int SCALES = kScalesPlain, int PIECES = 1>
 __device__ __forceinline__ void push_rows(const PushArgs &args, const PushSrc &src, uint32_t token, uint32_t K,
                                           uint64_t row_ptr, uint64_t scale_ptr, uint32_t scale_stride,
                                           float *s_scale, uint64_t *s_scale_ptr, uint32_t *s_scale_stride,
@@ -105,7 +107,28 @@ __device__ __forceinline__ void push_rows(const PushArgs &args, const PushSrc &s
     if constexpr (QUANT) {
         const uint32_t num_chunks = live ? args.hidden_dim / 16 : 0;  // 16 bf16 in, 16 fp8 out per lane
         const uint32_t Hs = args.hidden_dim_scale;
-        for (uint32_t base = wave * kWave; base < num_chunks; base += team_threads) {
+        for (uint32_t base = wave * kWave; PIECES > 1 && base < num_chunks; base += PIECES * team_threads) {
+            u32x4 a[PIECES], b[PIECES];
+#pragma unroll
+            for (uint32_t u = 0; u < PIECES; ++u) {
+                const uint32_t c = base + u * team_threads + lane;
+                a[u] = b[u] = u32x4{0, 0, 0, 0};
+                if (c >= num_chunks) continue;
+                const u32x4 *p = reinterpret_cast<const u32x4 *>(x_row + (size_t)c * 32);
+                a[u] = __builtin_nontemporal_load(p);
+                b[u] = __builtin_nontemporal_load(p + 1);
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < PIECES; ++u) {
+                if (base + u * team_threads >= num_chunks) break;   // uniform
+                const uint32_t c = base + u * team_threads + lane;
+                float scale;
+                const u32x4 q = quantize16(a[u], b[u], &scale);
+                store_copies<POLICY>(q, row_ptr, K, num_chunks * 16, c * 16);
+                if (c < num_chunks && (lane & 7) == 0 && c / 8 < kMaxLdsScales) s_scale[c / 8] = scale;
+            }
+        }
+        for (uint32_t base = wave * kWave; PIECES == 1 && base < num_chunks; base += team_threads) {
             const uint32_t c = base + lane;
             const bool active = c < num_chunks;
             u32x4 a = {0, 0, 0, 0}, b = {0, 0, 0, 0};
@@ -143,7 +166,21 @@ __device__ __forceinline__ void push_rows(const PushArgs &args, const PushSrc &s
         const bool ahead = args.row_bytes <= kScalesAheadBytes;
         float first_scale = 0.0f;
         if (scaled && ahead && tid < args.hidden_dim_scale) first_scale = xs[(size_t)tid * src.xs_stride_elem];
-        for (uint32_t c = tid; c < num_chunks; c += team_threads) {
+        for (uint32_t c = tid; PIECES > 1 && c < num_chunks; c += PIECES * team_threads) {
+            u32x4 v[PIECES];
+#pragma unroll
+            for (uint32_t u = 0; u < PIECES; ++u) {
+                v[u] = u32x4{0, 0, 0, 0};
+                if (c + u * team_threads < num_chunks)
+                    v[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(x_row) + c + u * team_threads);
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < PIECES; ++u) {
+                if (c + u * team_threads < num_chunks)
+                    store_copies<POLICY>(v[u], row_ptr, K, num_chunks * 16, (c + u * team_threads) * 16);
+            }
+        }
+        for (uint32_t c = tid; PIECES == 1 && c < num_chunks; c += team_threads) {
             const u32x4 v = PRE && c == tid ? pre_a : __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(x_row) + c);
             store_copies<POLICY>(v, row_ptr, K, num_chunks * 16, c * 16);
         }
@@ -208,9 +245,9 @@ __device__ __forceinline__ uint32_t resolve_copy(const PushDst &dst, const Works
     return wanted && !fits ? kInvalidSlot : slot;
 }
 
-uint32_t push_threads(const PushArgs &args, bool quantize) {
+uint32_t push_threads(const PushArgs &args, bool quantize, uint32_t pieces = 1) {
     const uint32_t chunks = quantize ? args.hidden_dim / 16 : args.row_bytes / 16;
-    uint32_t threads = (chunks + kWave - 1) / kWave * kWave;
+    uint32_t threads = (chunks + pieces * kWave - 1) / (pieces * kWave) * kWave;
     if (threads < (uint32_t)kWave) threads = kWave;
     if (threads > 1024) threads = 1024;
     return threads;
@@ -2217,7 +2254,10 @@ __device__ __forceinline__ void push_scale_columns(const PushArgs &args, const W
 // layout tables) and one per source (its totals and their scan); the last of
 // them hands the totals over to the next step.
 // SCALES: kScales...; where they are moved apart, push_scale_columns' dynamic LDS is there.
-template <bool QUANT, int POLICY, int SCALES>
+// PIECES: pieces of a copy that a thread moves (pieces_per_lane in a2a_rules.h): with few copies a token what bounds this
+// kernel is how many tokens are in flight, and fewer wavefronts each are more of them.  12 000 tokens of 5888 bytes with two
+// copies 70 -> 46 us (212 MB; a push of these rows whose places are known beforehand: 39 to 43).
+template <bool QUANT, int POLICY, int SCALES, int PIECES>
 __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(SCALES == kScalesApart ? 8 : 4))) void dispatch_resolve_kernel(const PushArgs args, const FinalizeArgs fin,
                                                                 const Workspace ws, const ScaleColumns columns) {
     __shared__ float s_scale[QUANT ? kMaxLdsScales : 1];
@@ -2378,8 +2418,8 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(SCALES == 
         scale_ptr = s_route_scale_ptr[lane];
         scale_stride = s_route_scale_stride[lane];
     }
-    push_rows<QUANT, false, POLICY, SCALES>(args, src, token, K, row_ptr, scale_ptr, scale_stride, s_scale, s_scale_ptr,
-                                            s_scale_stride, threadIdx.x, blockDim.x, true);
+    push_rows<QUANT, false, POLICY, SCALES, PIECES>(args, src, token, K, row_ptr, scale_ptr, scale_stride, s_scale,
+                                                    s_scale_ptr, s_scale_stride, threadIdx.x, blockDim.x, true);
 }
 
 hipError_t launch_dispatch_push(const PushArgs &args, const Workspace &ws, bool quantize,
@@ -2677,10 +2717,14 @@ static bool scales_past_l2(const PushArgs &args, const Workspace &ws) {
 }
 
 // How the copies are written: past the Infinity Cache (`streamed`), otherwise quantised rows at device scope and others
-// with ordinary stores, except long rows without scales in large steps (copies_written_through in a2a_rules.h).
+// with ordinary stores, except long rows without scales in large steps (copies_written_through in a2a_rules.h) and
+// rows of which a thread moves several pieces (pieces_per_lane there).
 hipError_t launch_dispatch_resolve(const PushArgs &args, const FinalizeArgs &fin, const Workspace &ws, bool quantize,
                                    uint32_t total_tokens, bool streamed, hipStream_t stream, KernelTiming timing) {
-    uint32_t threads = push_threads(args, quantize);
+    bool by_column = false;
+    for (uint32_t r = 0; r < ws.world; ++r) by_column |= args.dst[r].out_x != nullptr && scales_by_column(args.dst[r]);
+    const uint32_t pieces = pieces_per_lane(ws.topk, quantize ? args.hidden_dim / 16 : args.row_bytes / 16, quantize, by_column);
+    uint32_t threads = push_threads(args, quantize, pieces);
     if (threads < ws.experts_per_rank) {   // a receiver workgroup has one thread per local expert
         threads = (ws.experts_per_rank + kWave - 1) / kWave * kWave;
     }
@@ -2696,28 +2740,35 @@ hipError_t launch_dispatch_resolve(const PushArgs &args, const FinalizeArgs &fin
     if (senders != 1) a.single_source = 0;    // here only "one source has tokens": the rows may be strided
     if (a.single_source != 0) a.single = args.src[a.single_source - 1];
     ScaleColumns columns = {0, 0};
-    if (!streamed) columns = plan_scale_columns(args, ws, quantize, threads);
+    if (!streamed && pieces == 1) columns = plan_scale_columns(args, ws, quantize, threads);
     const size_t lds = columns.blocks != 0 ? (kSpan + 3 * (size_t)ws.num_experts) * sizeof(uint32_t) : 0;
+#define A2A_LAUNCH_RESOLVE_PIECES(PIECES, ...)                                                                     \
+    hipExtLaunchKernelGGL((dispatch_resolve_kernel<__VA_ARGS__, PIECES>), dim3(blocks + columns.blocks),           \
+                          dim3(threads), lds, stream, timing.start, timing.stop, 0, a, fin, ws, columns)
 #define A2A_LAUNCH_RESOLVE(...)                                                                                    \
-    hipExtLaunchKernelGGL((dispatch_resolve_kernel<__VA_ARGS__>), dim3(blocks + columns.blocks), dim3(threads),    \
-                          lds, stream, timing.start, timing.stop, 0, a, fin, ws, columns)
-    const bool past_l2 = scales_past_l2(args, ws);
+    do {                                                                                                           \
+        if (pieces == 4) A2A_LAUNCH_RESOLVE_PIECES(4, __VA_ARGS__);                                                \
+        else if (pieces == 2) A2A_LAUNCH_RESOLVE_PIECES(2, __VA_ARGS__);                                           \
+        else A2A_LAUNCH_RESOLVE_PIECES(1, __VA_ARGS__);                                                            \
+    } while (0)
+    const bool past_l2 = scales_past_l2(args, ws);   // (only with eight copies a token and more: one piece a lane)
     if (streamed) {
         if (quantize) A2A_LAUNCH_RESOLVE(true, kDeviceNonTemporal, kScalesPlain);
         else A2A_LAUNCH_RESOLVE(false, kDeviceNonTemporal, kScalesPlain);
     } else if (quantize) {
-        if (past_l2) A2A_LAUNCH_RESOLVE(true, kDeviceScope, kScalesPastL2);
+        if (past_l2) A2A_LAUNCH_RESOLVE_PIECES(1, true, kDeviceScope, kScalesPastL2);
         else A2A_LAUNCH_RESOLVE(true, kDeviceScope, kScalesPlain);
     } else if (columns.blocks != 0) {
-        A2A_LAUNCH_RESOLVE(false, kOrdinary, kScalesApart);
-    } else if (args.hidden_dim_scale == 0 &&
-               copies_written_through((uint64_t)total_tokens * ws.topk * args.row_bytes, args.row_bytes, ws.topk)) {
+        A2A_LAUNCH_RESOLVE_PIECES(1, false, kOrdinary, kScalesApart);
+    } else if (pieces > 1 || (args.hidden_dim_scale == 0 &&
+                              copies_written_through((uint64_t)total_tokens * ws.topk * args.row_bytes, args.row_bytes, ws.topk))) {
         A2A_LAUNCH_RESOLVE(false, kDeviceScope, kScalesPlain);
     } else {
-        if (past_l2) A2A_LAUNCH_RESOLVE(false, kOrdinary, kScalesPastL2);
-        else A2A_LAUNCH_RESOLVE(false, kOrdinary, kScalesPlain);
+        if (past_l2) A2A_LAUNCH_RESOLVE_PIECES(1, false, kOrdinary, kScalesPastL2);
+        else A2A_LAUNCH_RESOLVE_PIECES(1, false, kOrdinary, kScalesPlain);
     }
 #undef A2A_LAUNCH_RESOLVE
+#undef A2A_LAUNCH_RESOLVE_PIECES
     return hipGetLastError();
 }
 

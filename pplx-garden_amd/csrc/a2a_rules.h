@@ -76,7 +76,9 @@ inline bool copies_past_cache(uint64_t copies, bool quantize, uint32_t topk) {
 // (0.719).  Behind a sweep the rows that are less than three quarters full lose 1 to 1.7 % also with K = 8 (5120: 224.1 /
 // 228.0), those above lie between -1 and +2 %.  Steps over the same buffers again and again, as no user's are, gain less or
 // lose: 280 MB of 8 KB 110.8 / 110.6, of 4 KB 112.8 / 116.0.
-// It loses with few copies a token (K = 4 behind a reader 245.6 / 247.4), with rows of 2 KB (131.7 / 134.1), with rows that
+// It loses with few copies a token (K = 4 behind a reader 245.6 / 247.4; not where a thread moves several pieces,
+// pieces_per_lane, which are written through at every size: fp8 rows of 5 KB, K = 4 73.9 / 73.5, bf16 of 14 KB, K = 1 275 / 267,
+// behind a reader 391 / 384), with rows of 2 KB (131.7 / 134.1), with rows that
 // bring scales (fp8 rows of 5120 bytes 75.3 / 77.5, of 4096 behind a reader 300 / 308), and below kWrittenThrough bytes of copies
 // (4 KB rows, 79 MB: dispatch 24.0 / 24.9; 108 MB level).
 constexpr uint64_t kWrittenThrough = 120000000;
@@ -86,6 +88,39 @@ inline bool copies_written_through(uint64_t copies, uint32_t row_bytes, uint32_t
     const uint64_t whole = (row_bytes + kPeriod - 1) / kPeriod * kPeriod;
     return copies >= kWrittenThrough && topk >= 6 && row_bytes >= kPeriod && 4ull * row_bytes >= 3 * whole &&
            (uint64_t)topk * row_bytes >= 5 * whole;
+}
+
+// Sixteen-byte pieces of a copy that a thread of the resolving pack moves, and with it the wavefronts of a token's workgroup.
+// All of a workgroup's wavefronts are held through the chain of look-ups that ends in the rows' places, and a token with few
+// copies brings few bytes for it: with a piece a thread and one or two copies the pack ran at 3.0 to 3.8 TB/s where a push of
+// the same rows without any look-ups does 5.4.  Fewer wavefronts a token are more tokens in flight.  With many copies it is
+// the rows held open at a time that cost.  us per step, ordinary rows with one piece (what there was before) / 1, 2 and 4
+// pieces, all at device scope:
+//                     K = 1                     K = 2                     K = 4                     K = 6
+//    bf16  2 KB   80.7 /  81  68  68       94.4 /  98  85  85       94.1 /  96  92  92       88.3 /  89  87  87
+//    bf16  4 KB  142.5 / 147 120 116      116.9 / 121 106 108       91.3 /  92  92  93       84.5 /  84  87  87
+//    bf16  5.9 KB 233.0 / 236 165 157     139.6 / 139 107 108       99.6 / 101  91  92       86.9 /  88  87  87
+//    bf16 14 KB  301.7 / 299 216 196      197.1 / 192 152 155      138.4 / 138 131 133      147.6 / 147 156 158
+//    f32  28 KB  458.9 / 469 440 381      320.7 / 320 297 300      289.3 / 289 299 304      292.5 / 293 300 304
+//    fp8   5 KB  273.3 / 283 219 205      188.4 / 197 158 156      140.2 / 146 132 132      126.6 / 132 127 126
+//    fp8   7 KB  297.4 / 296 235 222      186.6 / 188 156 157      140.6 / 142 131 132      129.5 / 129 126 126
+//    quantised 4 KB 217 / 217 195 195     175.8 / 176 169 170      135.7 / 136 137 139      126.1 / 126 128 129
+//    quantised 5 KB 302 / 297 236 232     202.8 / 200 172 173      144.8 / 145 140 141      130.5 / 130 131 132
+//    quantised 7 KB 312 / 307 257 253     191.1 / 189 170 173      141.6 / 140 138 141      128.4 / 129 131 132
+// and with a sweep between dispatch and combine that reads the received rows, before / as it is: K = 1, bf16 rows of 14 KB
+// 535 / 385, quantised of 7 KB 372 / 316; K = 2, bf16 of 5.9 KB 169 / 144, fp8 of 7 KB 243 / 215; K = 4, fp8 of 5 KB
+// 125.5 / 120.7, bf16 of 14 KB 253 / 236.  (K = 2 with rows of 28 KB: two pieces 461, four 438.)
+// Four copies a token: two pieces where a piece a thread makes workgroups that do not fill a compute unit's 32 places for
+// wavefronts (3, 5, 6, 7, 14 of them, not 1, 4, 8 or 16), and for the shortest unquantised rows; not where scales go out by
+// column, which workgroups of fewer than 256 threads leave to the rows (fp8 rows of 2944 bytes 116.6 / 121.5, of 5120 level;
+// with K = 1 and 2 the pieces gain more than that: 158 / 136 and 150 / 138).
+inline uint32_t pieces_per_lane(uint32_t topk, uint32_t chunks, bool quantize, bool by_column) {
+    if (topk == 1) return 4;
+    if (topk <= 3) return chunks > 1024 ? 4 : 2;
+    if (topk > 4 || by_column) return 1;
+    const uint32_t waves = (chunks + 63) / 64;
+    const bool fills = waves > 16 || (waves & (waves - 1)) == 0;
+    return !fills || (!quantize && waves == 2) ? 2 : 1;
 }
 
 // copies_past_cache for the recvs of the split calls, from kStreamReceived bytes of copies in all of a step's recvs on.  What this

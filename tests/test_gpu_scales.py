@@ -27,7 +27,8 @@ GIVEN = [
     ([2100, 17], 33, 8, 6160, 55),            # the next wider one; an expert a receiver has not got
     ([1300, 1400], 24, 7, 256, 128),          # more scales than the row has threads
     ([1300, 2500, 1], 1024, 6, 4096, 32),     # more experts than threads; a span that ends in its first chunk of entries
-    ([16384, 16385, 3], 6, 1, 4096, 4),       # whole spans, and one entry more; a single slice of columns
+    ([16384, 16385, 3], 6, 1, 4096, 4),       # a copy a token: by column beside the rows
+    ([2048, 2049, 3], 16, 8, 4096, 4),        # whole spans, and a token more; a single slice of columns
 ]
 
 

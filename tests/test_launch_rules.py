@@ -7,6 +7,7 @@ from pathlib import Path
 
 import pytest
 
+from test_gpu_pieces import MOVED, QUANTISED
 from test_gpu_shapes import STREAMED, copies_of
 from test_gpu_split import PIECES
 from test_gpu_written_through import STEPS
@@ -22,6 +23,9 @@ int past_cache(uint64_t copies, int quantize, uint32_t k) { return a2a::copies_p
 int received_past_cache(uint64_t copies) { return a2a::received_past_cache(copies); }
 int written_through(uint64_t copies, uint32_t row_bytes, uint32_t k) {
     return a2a::copies_written_through(copies, row_bytes, k);
+}
+uint32_t pieces(uint32_t k, uint32_t chunks, int quantize, int by_column) {
+    return a2a::pieces_per_lane(k, chunks, quantize != 0, by_column != 0);
 }
 int one_launch(uint32_t rows, uint32_t row_bytes, uint32_t items, uint32_t threads) {
     return a2a::first_recv_in_one_launch(rows, row_bytes, items, threads);
@@ -83,6 +87,19 @@ def test_the_gpu_tests_of_written_through_steps_lie_on_the_side_they_are_meant_f
                                                                                    through):
     row = hidden * dtype.itemsize
     assert bool(rules.written_through(sum(tokens) * topk * row, row, topk)) == through
+
+
+def test_pieces_of_a_thread(rules):
+    # the fewer copies a token has, the more of its row a thread moves; never with five copies and more
+    assert [rules.pieces(k, 320, 0, 0) for k in (1, 2, 3, 4, 5, 8, 64)] == [4, 2, 2, 2, 1, 1, 1]
+    # four copies: where a piece a thread makes workgroups of 3, 5, 6, 7 or 14 wavefronts (and 2, unquantised)
+    waves = [w for w in range(1, 40) if rules.pieces(4, 64 * w, 1, 0) == 2]
+    assert waves == [3, 5, 6, 7, 9, 10, 11, 12, 13, 14, 15]
+    assert rules.pieces(4, 128, 0, 0) == 2 and rules.pieces(4, 128, 1, 0) == 1 and rules.pieces(4, 320, 0, 1) == 1
+    for k, hidden, dtype, scales, layout, pieces in MOVED:
+        assert rules.pieces(k, hidden * dtype.itemsize // 16, 0, layout == "col") == pieces, (k, hidden)
+    for k, hidden, pieces in QUANTISED:
+        assert rules.pieces(k, hidden // 16, 1, 0) == pieces, (k, hidden)
 
 
 def test_received_rows_that_the_cache_can_keep_stay_there(rules):
