@@ -184,6 +184,48 @@ inline size_t lds_to_bound_waves(uint32_t topk, bool past_cache) {
     return kLds / waves / kBlock * kBlock;
 }
 
+// One slab of a token's output row: the rows that lanes 0..K-1 hold (address 0: not there), weighted and added up.
+template <typename T, typename U, int GROUP, int LOAD, int OUT>
+__device__ __forceinline__ void gather_slab(uint64_t row_ptr, float weight, uint32_t K, uint32_t num_chunks, uint32_t slab,
+                                            uint32_t lane, uint8_t *out_row, bool accumulate) {
+    constexpr int V = vec_elems<T>();
+    const uint32_t chunk = slab * kWave + lane;
+    const bool active = chunk < num_chunks;
+    float acc[V];
+#pragma unroll
+    for (int j = 0; j < V; ++j) acc[j] = 0.0f;
+    if (accumulate && active) load_elems<U, V>(out_row + (size_t)chunk * V * Elem<U>::kSize, acc);
+
+    // GROUP routes at a time, all their loads asked for before the first is used.  A row is read through
+    // a buffer descriptor of its own: uniform base, one offset register for all rows, and the descriptor's
+    // bound takes the place of every condition (lanes past the row's end and rows that are not there read
+    // zeros without touching memory).
+    const uint64_t there = __ballot(row_ptr != 0);
+    const uint32_t row_bytes = num_chunks * 16;
+    for (uint32_t k0 = 0; k0 < K; k0 += GROUP) {
+        u32x4 raw[GROUP];
+        float w[GROUP];
+#pragma unroll
+        for (int k = 0; k < GROUP; ++k) {
+            const uint64_t row = read_lane64(row_ptr, k0 + k);
+            w[k] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(weight), (int)(k0 + k)));
+            raw[k] = load_row_chunk<LOAD>(row, row_bytes, chunk * 16);
+        }
+        const uint32_t have = (uint32_t)(there >> k0) & ((1u << GROUP) - 1);
+        if (have == (1u << GROUP) - 1) {
+#pragma unroll
+            for (int k = 0; k < GROUP; ++k) fma_chunk<T, V>(raw[k], w[k], acc);
+        } else {
+            // (a row that is not there adds nothing, also with a weight that is not finite)
+#pragma unroll
+            for (int k = 0; k < GROUP; ++k) {
+                if (have >> k & 1) fma_chunk<T, V>(raw[k], w[k], acc);
+            }
+        }
+    }
+    store_elems<U, V, OUT>((uint64_t)out_row, num_chunks * V * Elem<U>::kSize, chunk, acc);
+}
+
 // T: type of the expert_y rows, U: type of out_tokens.  One WAVEFRONT handles
 // one slab of 64 sixteen-byte chunks of one token; wavefronts share nothing, so
 // a compute unit keeps many of them in flight and the latency of resolving a
@@ -197,7 +239,6 @@ inline size_t lds_to_bound_waves(uint32_t topk, bool past_cache) {
 // 4096-token step hides them and is 0.3 us faster without the variant).
 template <typename T, typename U, int GROUP, bool ONE_RANK, int OUT>
 __global__ __launch_bounds__(kWave) void combine_gather_kernel(const CombArgs args, const Workspace ws) {
-    constexpr int V = vec_elems<T>();
     constexpr int LOAD = OUT == kNonTemporal ? kNonTemporal : kDeviceNonTemporal;
     if constexpr (ONE_RANK) {
         // everything the head of a wavefront needs from the argument block, asked for in one go
@@ -205,7 +246,6 @@ __global__ __launch_bounds__(kWave) void combine_gather_kernel(const CombArgs ar
         A2A_PIN(args.single_rank);
         A2A_PIN(args.hidden_dim);
         A2A_PIN(args.accumulate);
-        A2A_PIN(args.staged_base);
         A2A_PIN(args.single.out);
         A2A_PIN(args.single.indices);
         A2A_PIN(args.single.weights);
@@ -231,7 +271,6 @@ __global__ __launch_bounds__(kWave) void combine_gather_kernel(const CombArgs ar
         A2A_PIN(args.layer_rows);
         A2A_PIN(args.hidden_dim);
         A2A_PIN(args.accumulate);
-        A2A_PIN(args.staged_base);
         A2A_PIN(ws.world);
         A2A_PIN(ws.dp_size);
         A2A_PIN(ws.num_experts);
@@ -244,7 +283,7 @@ __global__ __launch_bounds__(kWave) void combine_gather_kernel(const CombArgs ar
     const uint32_t lane = threadIdx.x;
     const uint32_t E = ws.num_experts;
     const uint32_t K = ws.topk;
-    const uint32_t num_chunks = args.hidden_dim / V;
+    const uint32_t num_chunks = args.hidden_dim / vec_elems<T>();
     // the grid: slabs of a token side by side, then its tokens (no division stands in front of the loads)
     const uint32_t token_global = ONE_RANK ? blockIdx.y : blockIdx.z * args.layer_rows + blockIdx.y;
     const uint32_t slab = blockIdx.x;
@@ -279,7 +318,7 @@ __global__ __launch_bounds__(kWave) void combine_gather_kernel(const CombArgs ar
     // each and pick their receiver's descriptor with a lane shuffle.
     uint64_t y_base = 0, y_stride = 0;
     uint32_t y_rows = 0;
-    if (lane < ws.world && args.staged_base == nullptr) {
+    if (lane < ws.world) {
         y_base = (uint64_t)args.src[lane].y;
         y_stride = args.src[lane].y_stride;
         y_rows = args.src[lane].y_rows;
@@ -289,10 +328,6 @@ __global__ __launch_bounds__(kWave) void combine_gather_kernel(const CombArgs ar
     if (lane < K) {
         expert = (uint32_t)dst.indices[(size_t)token * dst.indices_stride + lane];
         weight = dst.weights[(size_t)token * dst.weights_stride + lane];
-        // (after a group dispatch: the copy's row in its receiver's buffer; after the sends of the split
-        // calls: its position in the sender's expert-sorted order, a2a_combine_recv.cu:67-73 = exclusive
-        // offset of the expert + token offset, which the send wrote here so that no second, dependent
-        // look-up stands in front of the rows: 0.5 us of a 128-token combine-recv)
         slot = ws.route_slot[(size_t)group * ws.max_tk + token * K + lane];
     }
     const bool expert_ok = expert < E;
@@ -303,54 +338,59 @@ __global__ __launch_bounds__(kWave) void combine_gather_kernel(const CombArgs ar
     uint64_t row_ptr = 0;
     if (lane < K) {
         bool ok = false;
-        if (args.staged_base != nullptr) {
-            if (expert_ok && slot < ws.max_tk) {
-                row_ptr = (uint64_t)(args.staged_base + ((size_t)group * ws.max_tk + slot) * args.staged_stride);
-                ok = true;
-            }
-        } else if (expert_ok && r_base != 0 && slot < r_rows) {
+        if (expert_ok && r_base != 0 && slot < r_rows) {
             row_ptr = r_base + (uint64_t)slot * r_stride;
             ok = true;
         }
         if (!ok && slab == 0) atomicOr(ws.err, A2A_DEV_BAD_SLOT);
     }
 
-    const uint32_t chunk = slab * kWave + lane;
-    const bool active = chunk < num_chunks;
-    uint8_t *const out_row = dst.out + (size_t)token * dst.out_stride;
-    float acc[V];
-#pragma unroll
-    for (int j = 0; j < V; ++j) acc[j] = 0.0f;
-    if (args.accumulate && active) load_elems<U, V>(out_row + (size_t)chunk * V * Elem<U>::kSize, acc);
+    gather_slab<T, U, GROUP, LOAD, OUT>(row_ptr, weight, K, num_chunks, slab, lane, dst.out + (size_t)token * dst.out_stride,
+                                        args.accumulate != 0);
+}
 
-    // GROUP routes at a time, all their loads asked for before the first is used.  A row is read through
-    // a buffer descriptor of its own: uniform base, one offset register for all rows, and the descriptor's
-    // bound takes the place of every condition (lanes past the row's end and rows that are not there read
-    // zeros without touching memory).
-    const uint64_t there = __ballot(row_ptr != 0);
-    const uint32_t row_bytes = num_chunks * 16;
-    for (uint32_t k0 = 0; k0 < K; k0 += GROUP) {
-        u32x4 raw[GROUP];
-        float w[GROUP];
-#pragma unroll
-        for (int k = 0; k < GROUP; ++k) {
-            const uint64_t row = read_lane64(row_ptr, k0 + k);
-            w[k] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(weight), (int)(k0 + k)));
-            raw[k] = load_row_chunk<LOAD>(row, row_bytes, chunk * 16);
-        }
-        const uint32_t have = (uint32_t)(there >> k0) & ((1u << GROUP) - 1);
-        if (have == (1u << GROUP) - 1) {
-#pragma unroll
-            for (int k = 0; k < GROUP; ++k) fma_chunk<T, V>(raw[k], w[k], acc);
-        } else {
-            // (a row that is not there adds nothing, also with a weight that is not finite)
-#pragma unroll
-            for (int k = 0; k < GROUP; ++k) {
-                if (have >> k & 1) fma_chunk<T, V>(raw[k], w[k], acc);
-            }
+// The combine's recv of the split calls: the rows are the staged ones of ONE sender, at the positions its send recorded
+// per copy (a2a_combine_recv.cu:67-73 = exclusive offset of the expert + token offset), so that there is no receiver to
+// look up and no second, dependent load in front of the rows.  What it needs is passed as the few words that they are
+// (kShortArguments); otherwise as combine_gather_kernel.
+template <typename T, typename U, int GROUP>
+__global__ __launch_bounds__(kWave) void combine_staged_kernel(const CombineStagedArgs args) {
+    A2A_PIN(args.out);
+    A2A_PIN(args.indices);
+    A2A_PIN(args.weights);
+    A2A_PIN(args.bound_m);
+    A2A_PIN(args.route_slot);
+    A2A_PIN(args.staged);
+    A2A_PIN(args.out_stride);
+    A2A_PIN(args.staged_stride);
+    A2A_PIN(args.indices_stride);
+    A2A_PIN(args.weights_stride);
+    A2A_PIN(args.num_tokens);
+    A2A_PIN(args.layer_rows);
+    A2A_PIN(args.max_tk);
+    A2A_PIN(args.hidden_dim);
+    A2A_PIN(args.num_experts);
+    A2A_PIN(args.topk);
+    A2A_PIN(args.accumulate);
+    const uint32_t lane = threadIdx.x;
+    const uint32_t K = args.topk;
+    const uint32_t slab = blockIdx.x;
+    const uint32_t token = blockIdx.z * args.layer_rows + blockIdx.y;
+    if (token >= effective_tokens(args.bound_m, args.num_tokens)) return;
+    float weight = 0.0f;
+    uint64_t row_ptr = 0;
+    if (lane < K) {
+        const uint32_t expert = (uint32_t)args.indices[(size_t)token * args.indices_stride + lane];
+        weight = args.weights[(size_t)token * args.weights_stride + lane];
+        const uint32_t slot = args.route_slot[token * K + lane];
+        if (expert < args.num_experts && slot < args.max_tk) {
+            row_ptr = (uint64_t)(args.staged + (size_t)slot * args.staged_stride);
+        } else if (slab == 0) {
+            atomicOr(args.err, A2A_DEV_BAD_SLOT);
         }
     }
-    store_elems<U, V, OUT>((uint64_t)out_row, num_chunks * V * Elem<U>::kSize, chunk, acc);
+    gather_slab<T, U, GROUP, kNonTemporal, kNonTemporal>(row_ptr, weight, K, args.hidden_dim / vec_elems<T>(), slab, lane,
+                                                         args.out + (size_t)token * args.out_stride, args.accumulate != 0);
 }
 
 template <typename T, typename U>
@@ -372,9 +412,8 @@ static hipError_t launch_typed(const CombArgs &given, const Workspace &ws, uint3
     const TokenLayers layers = token_layers(total_tokens);
     args.layer_rows = layers.rows;
     const dim3 grid(slabs, layers.rows, layers.layers);
-    const bool plain = args.single_rank != 0 || args.staged_base != nullptr;
     const bool past_cache =
-        !plain && (streamed || (uint64_t)total_tokens * args.hidden_dim * Elem<U>::kSize >= kStreamedOutput);
+        args.single_rank == 0 && (streamed || (uint64_t)total_tokens * args.hidden_dim * Elem<U>::kSize >= kStreamedOutput);
     const size_t lds = (uint64_t)slabs * total_tokens <= kAllAtOnce ? 0 : lds_to_bound_waves(ws.topk, past_cache);
 #define A2A_LAUNCH_GATHER(GROUP, ONE, OUT, LDS)                                                                \
     hipExtLaunchKernelGGL((combine_gather_kernel<T, U, GROUP, ONE, OUT>), grid, dim3(kWave), LDS, stream,      \
@@ -411,6 +450,41 @@ hipError_t launch_combine_gather(const CombArgs &args, const Workspace &ws, uint
     A2A_COMBINE_CASE(A2A_F32, F32, A2A_BF16, Bf16)
     A2A_COMBINE_CASE(A2A_F32, F32, A2A_F16, F16)
 #undef A2A_COMBINE_CASE
+    return hipErrorInvalidValue;
+}
+
+template <typename T, typename U>
+static hipError_t launch_staged_typed(const CombineStagedArgs &given, hipStream_t stream, KernelTiming timing) {
+    CombineStagedArgs args = given;
+    const uint32_t slabs = (args.hidden_dim / vec_elems<T>() + kWave - 1) / kWave;
+    const TokenLayers layers = token_layers(args.num_tokens);
+    args.layer_rows = layers.rows;
+    const dim3 grid(slabs, layers.rows, layers.layers);
+    const bool bounded = args.num_tokens > kOneRankMaxTokens && (uint64_t)slabs * args.num_tokens > kAllAtOnce;
+    const size_t lds = bounded ? lds_to_bound_waves(args.topk, false) : 0;
+#define A2A_LAUNCH_STAGED(GROUP)                                                                              \
+    hipExtLaunchKernelGGL((combine_staged_kernel<T, U, GROUP>), grid, dim3(kWave), lds, stream, timing.start, \
+                          timing.stop, 0, args)
+    if (args.topk > 4) A2A_LAUNCH_STAGED(8);
+    else if (args.topk > 2) A2A_LAUNCH_STAGED(4);
+    else if (args.topk > 1) A2A_LAUNCH_STAGED(2);
+    else A2A_LAUNCH_STAGED(1);
+#undef A2A_LAUNCH_STAGED
+    return hipGetLastError();
+}
+
+hipError_t launch_combine_staged(const CombineStagedArgs &args, uint32_t in_dtype, uint32_t out_dtype, hipStream_t stream,
+                                 KernelTiming timing) {
+    if (args.num_tokens == 0) return hipSuccess;
+    // (staged rows have elements as wide as those of the output)
+#define A2A_STAGED_CASE(IN_TAG, IN_T, OUT_TAG, OUT_T) \
+    if (in_dtype == IN_TAG && out_dtype == OUT_TAG) return launch_staged_typed<IN_T, OUT_T>(args, stream, timing);
+    A2A_STAGED_CASE(A2A_BF16, Bf16, A2A_BF16, Bf16)
+    A2A_STAGED_CASE(A2A_BF16, Bf16, A2A_F16, F16)
+    A2A_STAGED_CASE(A2A_F16, F16, A2A_F16, F16)
+    A2A_STAGED_CASE(A2A_F16, F16, A2A_BF16, Bf16)
+    A2A_STAGED_CASE(A2A_F32, F32, A2A_F32, F32)
+#undef A2A_STAGED_CASE
     return hipErrorInvalidValue;
 }
 

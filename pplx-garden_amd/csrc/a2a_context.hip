@@ -352,11 +352,12 @@ size_t carve_workspace(const a2a_config &c, uint32_t max_tokens, uint8_t *base, 
     const size_t o_routed = carve((size_t)N * E * sizeof(uint32_t));
     const size_t o_offsets = carve((size_t)N * E * sizeof(uint32_t));
     const size_t o_base = carve((size_t)N * E * sizeof(uint32_t));
+    // (the flags lie behind the senders' tables and in front of the receivers': some kernels find them by their distance)
+    const size_t o_err = carve(sizeof(uint32_t));
     const size_t o_tpe = carve((size_t)E * sizeof(uint32_t));
     const size_t o_poff = carve((size_t)E * sizeof(uint32_t));
     const size_t o_slot = carve((size_t)N * ws.max_tk * sizeof(uint32_t));
     const size_t o_toff = carve((size_t)N * ws.max_tk * sizeof(uint32_t));
-    const size_t o_err = carve(sizeof(uint32_t));
     const size_t o_order = carve((size_t)N * kMaxWorld);
     const size_t o_before = carve((size_t)N * ws.num_groups * sizeof(uint32_t));
     const size_t o_chunk_counts = carve((size_t)N * ws.nb_max * E * sizeof(uint32_t));
@@ -1113,15 +1114,13 @@ int a2a_combine_send(a2a_ctx *ctx, uint32_t rank, const void *expert_y, size_t e
     DeviceGuard guard(c.device);
     CombineSendArgs cs;
     memset(&cs, 0, sizeof cs);
-    cs.rank = rank;
     cs.y = static_cast<const uint8_t *>(expert_y);
     cs.y_stride = expert_y_stride;
     cs.y_rows = (uint32_t)(expert_y_rows > 0xFFFFFFFFull ? 0xFFFFFFFFull : expert_y_rows);
     cs.row_bytes = (uint32_t)((size_t)c.hidden_dim * c.out_elemsize);
-    cs.max_rows = rows_upper_bound(ctx);
     const KernelTiming timing = ctx->timing[A2A_KERNEL_COMBINE_SEND];
     ctx->timing[A2A_KERNEL_COMBINE_SEND] = KernelTiming();
-    hipError_t e = launch_combine_send(cs, ctx->ws, ctx->staging, static_cast<hipStream_t>(stream), timing);
+    hipError_t e = launch_combine_send(cs, rank, rows_upper_bound(ctx), ctx->ws, ctx->staging, static_cast<hipStream_t>(stream), timing);
     if (e != hipSuccess) return hip_fail(ctx, e, "launch combine_send");
     ctx->staging.combine_sent_mask |= 1u << rank;
     return A2A_OK;

@@ -147,17 +147,44 @@ struct CombArgs {
     uint32_t token_start[kMaxWorld + 1];
     uint32_t hidden_dim;
     uint32_t accumulate;
-    // Split calls: rows are read from a staging buffer at the sender's own
-    // positions (exclusive expert offset + token offset) instead of from the
-    // receivers' expert_y at route_slot.  Null for the group call.
-    const uint8_t *staged_base;
-    uint64_t staged_stride;
     // r + 1 when rank r alone has tokens to combine (0 otherwise), and a copy of dst[r] at a fixed place
     // (set by the launcher; see PushArgs::single).
     uint32_t single_rank;
     uint32_t layer_rows;   // tokens of one layer of the grid (set by the launcher)
     CombDst single;
 };
+
+// A launch whose arguments take at most this many bytes costs the host 2.7 us, one with 8 bytes more 3.4 to 3.8 and
+// one with 3.8 KB 4.0 to 4.3 (empty kernels enqueued behind a running one).  The small steps of the split calls are four
+// launches a rank that the host enqueues as fast as it can, and with long arguments a launch took it 7 us while the GPU kept
+// up with it.  So their kernels get the few words that they use instead of the blocks around this, and no hidden arguments
+// (blockDim, gridDim), and do not load what they do not use.  us per step, long / short: 16 ranks, 17 tokens of 11.8 KB, K = 1
+// 271.0 / 203.5, 17 of 2.9 KB, K = 8 252.4 / 198.4, 8 ranks with up to 745 tokens 112.6 / 87.7; at the GPU's own pace 8 x 128
+// tokens of 14 KB 174.7 / 166.8, 16 x 17 195 / 176.
+constexpr size_t kShortArguments = 112;
+
+// Combine's recv of the split calls; tables and staged rows are those of the sender's dp group.
+struct CombineStagedArgs {
+    uint8_t *out;
+    const int32_t *indices;
+    const float *weights;
+    const int32_t *bound_m;
+    const uint32_t *route_slot;
+    const uint8_t *staged;
+    uint32_t *err;
+    uint64_t out_stride;      // bytes
+    uint64_t staged_stride;
+    uint32_t indices_stride;
+    uint32_t weights_stride;
+    uint32_t num_tokens;
+    uint32_t layer_rows;      // tokens of one layer of the grid (set by the launcher)
+    uint32_t max_tk;
+    uint32_t hidden_dim;
+    uint32_t num_experts;
+    uint32_t topk;
+    uint32_t accumulate;
+};
+static_assert(sizeof(CombineStagedArgs) <= kShortArguments, "");
 
 // Events a caller wants recorded when a kernel itself begins and ends (both
 // null: an ordinary launch).
@@ -208,6 +235,9 @@ hipError_t launch_dispatch_single(const PushArgs &args, const FinalizeArgs &fin,
 // `streamed`: the step's copies went past the Infinity Cache (copies_past_cache).
 hipError_t launch_combine_gather(const CombArgs &args, const Workspace &ws, uint32_t in_dtype,
                                  uint32_t out_dtype, uint32_t total_tokens, bool streamed, hipStream_t stream,
+                                 KernelTiming timing = KernelTiming());
+
+hipError_t launch_combine_staged(const CombineStagedArgs &args, uint32_t in_dtype, uint32_t out_dtype, hipStream_t stream,
                                  KernelTiming timing = KernelTiming());
 
 // Makes a value from the argument block count as used where this stands, so that the scalar loads of

@@ -56,6 +56,35 @@ struct StageSendArgs {
     uint32_t resolver_wave;   // resolving send: wavefront that resolves the routes (set by the launcher)
 };
 
+constexpr uint32_t kTableUnit = 64;   // words: the workspace's tables begin at multiples of it
+
+// What stage_send_quick_kernel needs (kShortArguments); buffers and tables are those of the sender's dp group.
+struct SendQuickArgs {
+    const uint8_t *x;
+    const float *x_scale;
+    const int32_t *indices;
+    const int32_t *bound_m;
+    uint64_t x_stride;        // bytes
+    uint8_t *staged;
+    uint32_t *pos_token;
+    uint32_t *num_routed;
+    uint32_t *token_offset;
+    uint32_t *route_slot;
+    uint32_t xs_stride_elem;  // elements
+    uint32_t xs_stride_token;
+    uint32_t num_tokens;
+    uint32_t num_scales;
+    uint32_t sizes;           // from bit 0: sixteen-byte pieces of a row (10), experts (11), routes per token (7)
+    uint32_t distances;       // from num_routed on: to expert_offsets in kTableUnit (10), to the context's flags in words (22)
+
+    __device__ __forceinline__ uint32_t pieces() const { return sizes & 0x3FF; }
+    __device__ __forceinline__ uint32_t num_experts() const { return sizes >> 10 & 0x7FF; }
+    __device__ __forceinline__ uint32_t topk() const { return sizes >> 21; }
+    __device__ __forceinline__ uint32_t *expert_offsets() const { return num_routed + kTableUnit * (distances & 0x3FF); }
+    __device__ __forceinline__ uint32_t *flags() const { return num_routed + (distances >> 10); }
+};
+static_assert(sizeof(SendQuickArgs) <= kShortArguments, "");
+
 // A grid of wavefronts over the pieces (128 sixteen-byte chunks) of a receiver's rows.
 struct PieceGrid {
     uint32_t pieces;          // of a row
@@ -64,7 +93,13 @@ struct PieceGrid {
     uint32_t step_pieces;
 };
 
-struct StageRecvArgs {
+// The staged row's stride: the reference's format (payload, scales, spare bytes; rows are whole 16-byte chunks) rounded up
+// to whole cache lines.
+__host__ __device__ inline size_t staged_row_stride(size_t row_bytes, size_t num_scales) {
+    return (row_bytes + (num_scales * 4 + 15) / 16 * 16 + 16 + 255) / 256 * 256;
+}
+
+struct StageRecvArgs {   // of a recv as the host has it, and of the kernels that lay receivers out
     PushDst dst;
     int32_t *out_num_tokens;  // rows per local expert for the caller, may be null
     uint32_t rank;
@@ -72,8 +107,6 @@ struct StageRecvArgs {
     uint32_t hidden_dim_scale;
     uint32_t max_rows;        // upper bound of received rows known to the host
     bool streamed;            // the copies are written past the Infinity Cache (received_past_cache)
-    PieceGrid grid;           // set by the launcher
-    uint32_t scale_blocks;    // workgroups in front of the grid that move scales by column (launcher)
     // the first recv of a step only: it lays out every receiver
     uint32_t valid_mask;      // sources that sent tokens in this step (the others count as empty)
     uint32_t max_private;     // rows per source in the private part of a receive region (a2a_worker.rs:646-656)
@@ -81,15 +114,47 @@ struct StageRecvArgs {
     uint32_t slices;          // workgroups per receiver that is laid out for later recvs (launcher)
 };
 
+// What the kernel needs that copies a receiver's rows (kShortArguments).
+struct RecvRowsArgs {
+    uint8_t *out_x;
+    float *out_scale;
+    int32_t *out_num_tokens;  // may be null
+    const uint8_t *staged;
+    const uint4 *moves;       // the receiver's
+    const uint32_t *num_recv; // the receiver's
+    uint32_t *counts;         // rows of its experts
+    uint64_t out_stride;      // bytes
+    uint32_t os_stride_elem;  // elements
+    uint32_t os_stride_token;
+    uint32_t out_rows;
+    uint32_t row_bytes;
+    uint32_t num_scales;
+    uint32_t max_recv;
+    uint32_t pieces, magic, step_rows, step_pieces;   // PieceGrid
+    uint32_t scale_blocks;    // workgroups in front of the grid that move scales by column
+    // experts of the receiver, from their counts on to their first rows (in kTableUnit), and back to the context's flags (words)
+    uint32_t num_local : 11, to_first_rows : 5, to_flags : 16;
+
+    __device__ __forceinline__ uint32_t *flags() const { return counts - to_flags; }
+};
+static_assert(sizeof(RecvRowsArgs) <= kShortArguments, "");
+
 struct CombineSendArgs {
     const uint8_t *y;
     uint64_t y_stride;
     uint32_t y_rows;
-    uint32_t rank;
     uint32_t row_bytes;
-    uint32_t max_rows;
-    PieceGrid grid;           // set by the launcher
+    // the launcher's
+    uint8_t *staged;
+    uint64_t staged_stride;
+    const uint4 *moves;       // the receiver's
+    const uint32_t *num_recv; // the receiver's
+    uint32_t *err;
+    uint32_t max_recv;
+    uint32_t max_tk;
+    PieceGrid grid;
 };
+static_assert(sizeof(CombineSendArgs) <= kShortArguments, "");
 
 struct CombineRecvArgs {
     CombDst dst;
@@ -130,8 +195,9 @@ hipError_t launch_stage_send_resolve(const StageSendArgs &args, const Workspace 
 hipError_t launch_stage_recv(const StageRecvArgs &args, const Workspace &ws, const Staging &st, bool first_of_step,
                              hipStream_t stream, KernelTiming timing = KernelTiming(),
                              KernelTiming layout_timing = KernelTiming());
-hipError_t launch_combine_send(const CombineSendArgs &args, const Workspace &ws, const Staging &st,
-                               hipStream_t stream, KernelTiming timing = KernelTiming());
+// `max_rows`: upper bound of the receiver's rows known to the host.
+hipError_t launch_combine_send(const CombineSendArgs &args, uint32_t rank, uint32_t max_rows, const Workspace &ws,
+                               const Staging &st, hipStream_t stream, KernelTiming timing = KernelTiming());
 hipError_t launch_combine_recv(const CombineRecvArgs &args, const Workspace &ws, const Staging &st,
                                uint32_t in_dtype, uint32_t out_dtype, hipStream_t stream,
                                KernelTiming timing = KernelTiming());

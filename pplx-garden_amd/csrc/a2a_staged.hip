@@ -2,6 +2,7 @@
 #include "a2a_rules.h"
 #include "a2a_staged.h"
 
+#include <algorithm>
 #include <cstring>
 
 #include "a2a_device.h"
@@ -325,49 +326,38 @@ __device__ __forceinline__ void scan_counts_for_routes(const uint32_t *s_cnt, ui
 constexpr uint32_t kSendQuickSpinLimit = 1u << 22;   // (a resolver that gives up flags A2A_DEV_INTERNAL; never seen)
 
 template <uint32_t NB, bool QUANT>
-__global__ __launch_bounds__(1024) void stage_send_quick_kernel(const StageSendArgs args, const Workspace ws,
-                                                                const Staging st) {
+__global__ __launch_bounds__(1024) void stage_send_quick_kernel(const SendQuickArgs args) {
     extern __shared__ uint32_t s_cnt[];
     __shared__ uint32_t s_counted;   // counting wavefronts whose entries are in the table
     // everything the head of a workgroup takes from the argument block, asked for in one go
-    A2A_PIN(args.src.x);
-    A2A_PIN(args.src.x_scale);
-    A2A_PIN(args.src.indices);
-    A2A_PIN(args.src.bound_m);
-    A2A_PIN(args.src.x_stride);
-    A2A_PIN(args.src.num_tokens);
-    A2A_PIN(args.rank);
-    A2A_PIN(args.hidden_dim);
-    A2A_PIN(args.row_bytes);
-    A2A_PIN(ws.num_experts);
-    A2A_PIN(ws.topk);
-    A2A_PIN(ws.dp_size);
-    A2A_PIN(ws.max_tk);
-    A2A_PIN(ws.num_routed);
-    A2A_PIN(ws.expert_offsets);
-    A2A_PIN(ws.token_offset);
-    A2A_PIN(ws.err);
-    A2A_PIN(st.send_buf);
-    A2A_PIN(st.pos_token);
-    A2A_PIN(st.disp_stride);
-    A2A_PIN(st.payload_bytes);
-    A2A_PIN(st.max_tokens);
+    A2A_PIN(args.x);
+    A2A_PIN(args.x_scale);
+    A2A_PIN(args.indices);
+    A2A_PIN(args.bound_m);
+    A2A_PIN(args.x_stride);
+    A2A_PIN(args.staged);
+    A2A_PIN(args.pos_token);
+    A2A_PIN(args.num_routed);
+    A2A_PIN(args.token_offset);
+    A2A_PIN(args.route_slot);
+    A2A_PIN(args.num_tokens);
+    A2A_PIN(args.num_scales);
+    A2A_PIN(args.sizes);
+    A2A_PIN(args.distances);
     const uint32_t tid = threadIdx.x;
-    const uint32_t nthreads = blockDim.x;
+    const uint32_t num_chunks = args.pieces();   // pieces of a row, one per thread
+    const uint32_t counters = (num_chunks + kWave - 1) / kWave * kWave;   // threads that count entries and move the row
+    const uint32_t nthreads = counters + kWave;
     const uint32_t lane = tid & (kWave - 1);
     const uint32_t wave = tid / kWave;
     const uint32_t waves = nthreads / kWave;
     const bool resolver = wave == waves - 1;
-    const uint32_t counters = nthreads - kWave;   // threads that count entries and move the row
-    const uint32_t E = ws.num_experts;
-    const uint32_t K = ws.topk;
-    const uint32_t g = args.rank / ws.dp_size;
+    const uint32_t E = args.num_experts();
+    const uint32_t K = args.topk();
     const uint32_t token = blockIdx.x;
-    const PushSrc &src = args.src;
-    const uint32_t tokens = src.num_tokens;   // the grid: one workgroup per token
+    const uint32_t tokens = args.num_tokens;  // the grid: one workgroup per token
     const uint32_t entries = tokens * K;      // > 0
     const uint32_t my_first = token * K;
-    const uint32_t num_chunks = QUANT ? args.hidden_dim / 16 : args.row_bytes / 16;   // pieces of a row, one per thread
     const bool has_piece = tid < num_chunks;
 
     // What each kind of wavefront takes from memory, asked for before anything else is done: the
@@ -381,9 +371,9 @@ __global__ __launch_bounds__(1024) void stage_send_quick_kernel(const StageSendA
 #pragma unroll
         for (uint32_t j = 0; j < NB; ++j) {
             const uint32_t f = j * counters + tid;
-            early[j] = (uint32_t)src.indices[f < entries ? f : entries - 1];
+            early[j] = (uint32_t)args.indices[f < entries ? f : entries - 1];
         }
-        const uint8_t *x_row = src.x + (size_t)token * src.x_stride;
+        const uint8_t *x_row = args.x + (size_t)token * args.x_stride;
         if (has_piece) {
             if constexpr (QUANT) {
                 const u32x4 *piece = reinterpret_cast<const u32x4 *>(x_row + (size_t)tid * 32);
@@ -394,16 +384,16 @@ __global__ __launch_bounds__(1024) void stage_send_quick_kernel(const StageSendA
             }
         }
         if constexpr (!QUANT) {
-            if (src.x_scale != nullptr && tid < args.hidden_dim_scale) {
-                first_scale = src.x_scale[(size_t)token * src.xs_stride_token + (size_t)tid * src.xs_stride_elem];
+            if (args.x_scale != nullptr && tid < args.num_scales) {
+                first_scale = args.x_scale[(size_t)token * args.xs_stride_token + (size_t)tid * args.xs_stride_elem];
             }
         }
     } else {
         // (the resolver shares its SIMD with wavefronts that quantise while the positions are resolved)
         __builtin_amdgcn_s_setprio(3);
-        my_id = (uint32_t)src.indices[my_first + (lane < K ? lane : 0)];
+        my_id = (uint32_t)args.indices[my_first + (lane < K ? lane : 0)];
     }
-    const uint32_t eff = effective_tokens(src.bound_m, tokens);
+    const uint32_t eff = effective_tokens(args.bound_m, tokens);
     const uint32_t flat_entries = eff * K;
     const bool live = token < eff;   // uniform
 
@@ -425,7 +415,7 @@ __global__ __launch_bounds__(1024) void stage_send_quick_kernel(const StageSendA
 #pragma unroll
             for (uint32_t j = 0; j < NB; ++j) {
                 const uint32_t f = f0 + j * counters + tid;
-                x[j] = f < flat_entries ? (uint32_t)src.indices[f] : 0xFFFFFFFFu;
+                x[j] = f < flat_entries ? (uint32_t)args.indices[f] : 0xFFFFFFFFu;
             }
 #pragma unroll
             for (uint32_t j = 0; j < NB; ++j) {
@@ -438,8 +428,8 @@ __global__ __launch_bounds__(1024) void stage_send_quick_kernel(const StageSendA
         if (lane == 0) atomicAdd(&s_counted, 1u);
         if (!live) return;   // past bound_m: nothing to stage (uniform)
 
-        uint8_t *row = st.send_buf + ((size_t)g * st.max_tokens + token) * st.disp_stride;
-        float *row_scale = reinterpret_cast<float *>(row + st.payload_bytes);
+        uint8_t *row = args.staged + (size_t)token * staged_row_stride(num_chunks * 16, args.num_scales);
+        float *row_scale = reinterpret_cast<float *>(row + num_chunks * 16);
         if constexpr (QUANT) {
             float scale;
             const u32x4 q = quantize16(pre_a, pre_b, &scale);
@@ -449,11 +439,11 @@ __global__ __launch_bounds__(1024) void stage_send_quick_kernel(const StageSendA
             }
         } else {
             if (has_piece) reinterpret_cast<u32x4 *>(row)[tid] = pre_a;
-            if (src.x_scale != nullptr) {
-                if (tid < args.hidden_dim_scale) row_scale[tid] = first_scale;
-                const float *xs = src.x_scale + (size_t)token * src.xs_stride_token;
-                for (uint32_t j = tid + counters; j < args.hidden_dim_scale; j += counters) {
-                    row_scale[j] = xs[(size_t)j * src.xs_stride_elem];
+            if (args.x_scale != nullptr) {
+                if (tid < args.num_scales) row_scale[tid] = first_scale;
+                const float *xs = args.x_scale + (size_t)token * args.xs_stride_token;
+                for (uint32_t j = tid + counters; j < args.num_scales; j += counters) {
+                    row_scale[j] = xs[(size_t)j * args.xs_stride_elem];
                 }
             }
         }
@@ -472,7 +462,7 @@ __global__ __launch_bounds__(1024) void stage_send_quick_kernel(const StageSendA
     __builtin_amdgcn_s_setprio(0);
     for (uint32_t spins = 0; __hip_atomic_load(&s_counted, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) != waves - 1;) {
         if (++spins == kSendQuickSpinLimit) {
-            if (lane == 0) atomicOr(ws.err, A2A_DEV_INTERNAL);
+            if (lane == 0) atomicOr(args.flags(), A2A_DEV_INTERNAL);
             break;
         }
     }
@@ -482,8 +472,7 @@ __global__ __launch_bounds__(1024) void stage_send_quick_kernel(const StageSendA
     // Scan over the experts; a route takes its expert's word and the entries of the experts before it.
     // Token 0 publishes.
     uint32_t my_word, my_excl;
-    scan_counts_for_routes(s_cnt, E, lane, my_id, token == 0, ws.num_routed + g * E, ws.expert_offsets + g * E, my_word,
-                           my_excl);
+    scan_counts_for_routes(s_cnt, E, lane, my_id, token == 0, args.num_routed, args.expert_offsets(), my_word, my_excl);
     if (!live) return;   // past bound_m: no positions to write (uniform)
     if (lane < K) {
         uint32_t toff = 0, at = kInvalidSlot;
@@ -491,12 +480,12 @@ __global__ __launch_bounds__(1024) void stage_send_quick_kernel(const StageSendA
             toff = (my_word >> 16) + repeats;
             // position of the copy (a2a_dispatch_send.cu:54)
             at = my_excl + toff;
-            st.pos_token[(size_t)g * ws.max_tk + at] = token;
+            args.pos_token[at] = token;
         } else {
-            atomicOr(ws.err, A2A_DEV_BAD_EXPERT_ID);
+            atomicOr(args.flags(), A2A_DEV_BAD_EXPERT_ID);
         }
-        ws.token_offset[(size_t)g * ws.max_tk + my_first + lane] = toff;
-        ws.route_slot[(size_t)g * ws.max_tk + my_first + lane] = at;
+        args.token_offset[my_first + lane] = toff;
+        args.route_slot[my_first + lane] = at;
     }
 }
 
@@ -1574,14 +1563,12 @@ __global__ __launch_bounds__(1024) void stage_recv_first_few_kernel(const StageR
 
 // The receiver's counts for the caller (a2a_dispatch_recv.cu:220-224).  One workgroup of a recv that did
 // not lay the receiver out itself.
-__device__ __forceinline__ void hand_over_counts(const StageRecvArgs &args, const Workspace &ws, uint32_t out_rows) {
-    const uint32_t E = ws.num_experts, Le = ws.experts_per_rank;
-    const uint32_t first = args.rank * Le;
-    const uint32_t n_local = first >= E ? 0 : (E - first < Le ? E - first : Le);
-    for (uint32_t le = threadIdx.x; le < n_local; le += blockDim.x) {
-        const uint32_t tpe = ws.tokens_per_expert[first + le];
+__device__ __forceinline__ void hand_over_counts(const RecvRowsArgs &args) {
+    for (uint32_t le = threadIdx.x; le < args.num_local; le += kPieceThreads) {
+        const uint32_t tpe = args.counts[le];
         if (args.out_num_tokens != nullptr) args.out_num_tokens[le] = (int32_t)tpe;
-        if (ws.padded_offset[first + le] + tpe > out_rows) atomicOr(ws.err, A2A_DEV_RECV_OVERFLOW);
+        if (args.counts[kTableUnit * args.to_first_rows + le] + tpe > args.out_rows)
+            atomicOr(args.flags(), A2A_DEV_RECV_OVERFLOW);
     }
 }
 
@@ -1639,86 +1626,82 @@ constexpr uint32_t kScaleColumns = 8;
 constexpr uint64_t kColumnWords = 112 * 1024;
 
 // The scales of the received rows, by column.  `unit`, `units`: of the wavefronts that do this.
-__device__ __forceinline__ void receive_scale_columns(const StageRecvArgs &args, const Workspace &ws, const Staging &st,
-                                                      const uint4 *moves, uint32_t total, uint32_t unit, uint32_t units) {
+__device__ __forceinline__ void receive_scale_columns(const RecvRowsArgs &args, uint32_t total, uint32_t unit, uint32_t units) {
     const uint32_t lane = threadIdx.x & (kWave - 1);
-    const uint32_t num_scales = args.hidden_dim_scale;
+    const uint32_t num_scales = args.num_scales;
+    const size_t staged_stride = staged_row_stride(args.row_bytes, num_scales);
     const uint32_t slices = (num_scales + kScaleColumns - 1) / kScaleColumns;
     for (; unit / slices * kWave < total; unit += units) {
         const uint32_t row = unit / slices * kWave + lane;
         const uint32_t first = unit % slices * kScaleColumns;
-        const uint4 move = moves[row < total ? row : total - 1];
-        if (row >= total || move.x >= args.dst.out_rows) continue;   // (rows that do not fit are flagged where they are copied)
-        const u32x4 *from = reinterpret_cast<const u32x4 *>(st.send_buf + (size_t)move.y * st.disp_stride + st.payload_bytes) +
+        const uint4 move = args.moves[row < total ? row : total - 1];
+        if (row >= total || move.x >= args.out_rows) continue;   // (rows that do not fit are flagged where they are copied)
+        const u32x4 *from = reinterpret_cast<const u32x4 *>(args.staged + (size_t)move.y * staged_stride + args.row_bytes) +
                             first / 4;
-        float *to = args.dst.out_scale + (size_t)move.x * args.dst.os_stride_token + (size_t)first * args.dst.os_stride_elem;
+        float *to = args.out_scale + (size_t)move.x * args.os_stride_token + (size_t)first * args.os_stride_elem;
         // (a staged row has 16 spare bytes behind its scales)
         u32x4 v[kScaleColumns / 4];
 #pragma unroll
         for (uint32_t i = 0; i < kScaleColumns / 4; ++i) v[i] = first + 4 * i < num_scales ? from[i] : u32x4{0, 0, 0, 0};
 #pragma unroll
         for (uint32_t j = 0; j < kScaleColumns; ++j) {
-            if (first + j < num_scales) to[(size_t)j * args.dst.os_stride_elem] = __uint_as_float(v[j / 4][j % 4]);
+            if (first + j < num_scales) to[(size_t)j * args.os_stride_elem] = __uint_as_float(v[j / 4][j % 4]);
         }
     }
 }
 
 template <bool STREAM, bool COLUMNS>
-__global__ __launch_bounds__(kPieceThreads) void stage_recv_kernel(const StageRecvArgs args, const Workspace ws,
-                                                                   const Staging st) {
+__global__ __launch_bounds__(kPieceThreads) void stage_recv_kernel(const RecvRowsArgs args) {
     // everything a wavefront takes from the argument block, asked for in one go
-    A2A_PIN(args.dst.out_x);
-    A2A_PIN(args.dst.out_scale);
-    A2A_PIN(args.dst.out_stride);
-    A2A_PIN(args.dst.os_stride_elem);
-    A2A_PIN(args.dst.os_stride_token);
-    A2A_PIN(args.dst.out_rows);
-    A2A_PIN(args.rank);
+    A2A_PIN(args.out_x);
+    A2A_PIN(args.out_scale);
+    A2A_PIN(args.out_stride);
+    A2A_PIN(args.os_stride_elem);
+    A2A_PIN(args.os_stride_token);
+    A2A_PIN(args.out_rows);
     A2A_PIN(args.row_bytes);
-    A2A_PIN(args.hidden_dim_scale);
-    A2A_PIN(args.grid.pieces);
-    A2A_PIN(args.grid.magic);
-    A2A_PIN(args.grid.step_rows);
-    A2A_PIN(args.grid.step_pieces);
+    A2A_PIN(args.num_scales);
+    A2A_PIN(args.pieces);
+    A2A_PIN(args.magic);
+    A2A_PIN(args.step_rows);
+    A2A_PIN(args.step_pieces);
     if constexpr (COLUMNS) A2A_PIN(args.scale_blocks);
-    A2A_PIN(st.send_buf);
-    A2A_PIN(st.moves);
-    A2A_PIN(st.num_recv);
-    A2A_PIN(st.disp_stride);
-    A2A_PIN(st.payload_bytes);
-    A2A_PIN(st.max_recv);
-    const uint32_t r = args.rank;
+    A2A_PIN(args.staged);
+    A2A_PIN(args.moves);
+    A2A_PIN(args.num_recv);
+    A2A_PIN(args.max_recv);
     const uint32_t tid = threadIdx.x;
     const uint32_t lane = tid & (kWave - 1);
-    const PushDst &dst = args.dst;
     const uint32_t num_chunks = args.row_bytes / 16;
-    const uint4 *moves = st.moves + (size_t)r * st.max_recv;
+    const uint4 *const moves = args.moves;
+    const PieceGrid grid = {args.pieces, args.magic, args.step_rows, args.step_pieces};
     // The first piece's table entry is asked for together with the number of rows received
     // (a row index the tables do not hold reads entry 0 and is dropped by the loop's bound).
+    const size_t staged_stride = staged_row_stride(args.row_bytes, args.num_scales);
     PieceWalk at;
     const uint32_t scale_blocks = COLUMNS ? args.scale_blocks : 0;
     const uint32_t block = blockIdx.x - scale_blocks;   // (wraps around for the workgroups in front: they move scales)
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid / kWave);
-    at.start(args.grid, COLUMNS && blockIdx.x < scale_blocks ? 0 : block * (kPieceThreads / kWave) + wave);
-    const uint32_t probe = at.row < st.max_recv ? at.row : 0;
+    at.start(grid, COLUMNS && blockIdx.x < scale_blocks ? 0 : block * (kPieceThreads / kWave) + wave);
+    const uint32_t probe = at.row < args.max_recv ? at.row : 0;
     uint4 move = moves[probe];
-    uint32_t total = st.num_recv[2 * r];
-    if (total > st.max_recv) total = st.max_recv;   // flagged by the layout: more rows than the region was sized for
+    uint32_t total = *args.num_recv;
+    if (total > args.max_recv) total = args.max_recv;   // flagged by the layout: more rows than the region was sized for
 
     if (COLUMNS && blockIdx.x < scale_blocks) {
-        receive_scale_columns(args, ws, st, moves, total, blockIdx.x * (kPieceThreads / kWave) + wave,
+        receive_scale_columns(args, total, blockIdx.x * (kPieceThreads / kWave) + wave,
                               scale_blocks * (kPieceThreads / kWave));
         return;
     }
-    if (block == 0) hand_over_counts(args, ws, dst.out_rows);
-    if (dst.out_x == nullptr) return;
+    if (block == 0) hand_over_counts(args);
+    if (args.out_x == nullptr) return;
 
     while (at.row < total) {
         const uint32_t dst_row = move.x;
-        const uint8_t *src = st.send_buf + (size_t)move.y * st.disp_stride;
+        const uint8_t *src = args.staged + (size_t)move.y * staged_stride;
         const uint32_t chunk = at.piece * kPieceChunks + lane, c = at.piece * kWave + lane;   // c: of the scales
-        const bool fits = dst_row < dst.out_rows;
-        const bool scaled = !COLUMNS && fits && dst.out_scale != nullptr && c < args.hidden_dim_scale;
+        const bool fits = dst_row < args.out_rows;
+        const bool scaled = !COLUMNS && fits && args.out_scale != nullptr && c < args.num_scales;
         u32x4 v[kPieceLoads];
         float scale = 0.0f;
 #pragma unroll
@@ -1726,27 +1709,27 @@ __global__ __launch_bounds__(kPieceThreads) void stage_recv_kernel(const StageRe
             v[u] = u32x4{0, 0, 0, 0};
             if (fits && chunk + u * kWave < num_chunks) v[u] = reinterpret_cast<const u32x4 *>(src)[chunk + u * kWave];
         }
-        if (scaled) scale = reinterpret_cast<const float *>(src + st.payload_bytes)[c];
+        if (scaled) scale = reinterpret_cast<const float *>(src + args.row_bytes)[c];
         // the next piece's entry travels while this one is copied
         PieceWalk next = at;
-        next.advance(args.grid);
+        next.advance(grid);
         const uint32_t next_probe = next.row < total ? next.row : at.row;
         const uint4 next_move = moves[next_probe];
-        u32x4 *const to = reinterpret_cast<u32x4 *>(dst.out_x + (size_t)dst_row * dst.out_stride) + chunk;
+        u32x4 *const to = reinterpret_cast<u32x4 *>(args.out_x + (size_t)dst_row * args.out_stride) + chunk;
 #pragma unroll
         for (uint32_t u = 0; u < kPieceLoads; ++u) {
             if (!fits || chunk + u * kWave >= num_chunks) continue;
             if constexpr (STREAM) __builtin_nontemporal_store(v[u], to + u * kWave); else store_copy(v[u], to + u * kWave);
         }
-        if (scaled) dst.out_scale[(size_t)dst_row * dst.os_stride_token + (size_t)c * dst.os_stride_elem] = scale;
-        if (!COLUMNS && fits && dst.out_scale != nullptr) {
+        if (scaled) args.out_scale[(size_t)dst_row * args.os_stride_token + (size_t)c * args.os_stride_elem] = scale;
+        if (!COLUMNS && fits && args.out_scale != nullptr) {
             // rows with more scales than pieces have lanes
-            for (uint32_t q = c + args.grid.pieces * kWave; q < args.hidden_dim_scale; q += args.grid.pieces * kWave) {
-                dst.out_scale[(size_t)dst_row * dst.os_stride_token + (size_t)q * dst.os_stride_elem] =
-                    reinterpret_cast<const float *>(src + st.payload_bytes)[q];
+            for (uint32_t q = c + grid.pieces * kWave; q < args.num_scales; q += grid.pieces * kWave) {
+                args.out_scale[(size_t)dst_row * args.os_stride_token + (size_t)q * args.os_stride_elem] =
+                    reinterpret_cast<const float *>(src + args.row_bytes)[q];
             }
         }
-        if (!fits && at.piece == 0 && lane == 0) atomicOr(ws.err, A2A_DEV_RECV_OVERFLOW);
+        if (!fits && at.piece == 0 && lane == 0) atomicOr(args.flags(), A2A_DEV_RECV_OVERFLOW);
         at = next;
         move = next_move;
     }
@@ -1761,8 +1744,7 @@ __global__ __launch_bounds__(kPieceThreads) void stage_recv_kernel(const StageRe
 // with a wavefront per row, 76.5 us = 6.1 TB/s in this order with one chunk a lane (a plain copy of as many rows in the
 // same order, examples/ceilings.hip: 67.6 us; both sides come from and go to HBM, so loads and stores keep nothing).
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(kPieceThreads) void combine_send_kernel(const CombineSendArgs args, const Workspace ws,
-                                                                     const Staging st) {
+__global__ __launch_bounds__(kPieceThreads) void combine_send_kernel(const CombineSendArgs args) {
     // everything a wavefront takes from the argument block, asked for in one go
     A2A_PIN(args.y);
     A2A_PIN(args.y_stride);
@@ -1772,25 +1754,25 @@ __global__ __launch_bounds__(kPieceThreads) void combine_send_kernel(const Combi
     A2A_PIN(args.grid.magic);
     A2A_PIN(args.grid.step_rows);
     A2A_PIN(args.grid.step_pieces);
-    A2A_PIN(ws.max_tk);
-    A2A_PIN(st.comb_buf);
-    A2A_PIN(st.moves);
-    A2A_PIN(st.comb_stride);
-    A2A_PIN(st.max_recv);
-    const uint32_t r = args.rank;
+    A2A_PIN(args.max_tk);
+    A2A_PIN(args.staged);
+    A2A_PIN(args.moves);
+    A2A_PIN(args.num_recv);
+    A2A_PIN(args.staged_stride);
+    A2A_PIN(args.max_recv);
     const uint32_t lane = threadIdx.x & (kWave - 1);
     const uint32_t num_chunks = args.row_bytes / 16;
-    const uint4 *moves = st.moves + (size_t)r * st.max_recv;
+    const uint4 *const moves = args.moves;
     PieceWalk at;
     at.start(args.grid, __builtin_amdgcn_readfirstlane(blockIdx.x * (kPieceThreads / kWave) + threadIdx.x / kWave));
-    const uint32_t probe = at.row < st.max_recv ? at.row : 0;
+    const uint32_t probe = at.row < args.max_recv ? at.row : 0;
     uint4 move = moves[probe];
-    uint32_t total = st.num_recv[2 * r];
-    if (total > st.max_recv) total = st.max_recv;
+    uint32_t total = *args.num_recv;
+    if (total > args.max_recv) total = args.max_recv;
     while (at.row < total) {
         const uint32_t c = at.piece * kPieceChunks + lane;
         const uint32_t row = move.x, g = move.z, pos = move.w;   // (every member of a dp group reads the same staging rows)
-        const bool fits = row < args.y_rows && pos < ws.max_tk;
+        const bool fits = row < args.y_rows && pos < args.max_tk;
         const u32x4 *const from = reinterpret_cast<const u32x4 *>(args.y + (size_t)row * args.y_stride) + c;
         u32x4 v[kPieceLoads];
 #pragma unroll
@@ -1803,12 +1785,12 @@ __global__ __launch_bounds__(kPieceThreads) void combine_send_kernel(const Combi
         next.advance(args.grid);
         const uint32_t next_probe = next.row < total ? next.row : at.row;
         const uint4 next_move = moves[next_probe];
-        u32x4 *const to = reinterpret_cast<u32x4 *>(st.comb_buf + ((size_t)g * ws.max_tk + pos) * st.comb_stride) + c;
+        u32x4 *const to = reinterpret_cast<u32x4 *>(args.staged + ((size_t)g * args.max_tk + pos) * args.staged_stride) + c;
 #pragma unroll
         for (uint32_t u = 0; u < kPieceLoads; ++u) {
             if (fits && c + u * kWave < num_chunks) store_copy(v[u], to + u * kWave);
         }
-        if (!fits && at.piece == 0 && lane == 0) atomicOr(ws.err, A2A_DEV_BAD_SLOT);
+        if (!fits && at.piece == 0 && lane == 0) atomicOr(args.err, A2A_DEV_BAD_SLOT);
         at = next;
         move = next_move;
     }
@@ -1866,7 +1848,7 @@ int staging_allocate(Staging &st, const a2a_config &cfg, std::string *error) {
     // at a stride rounded up to whole cache lines: the buffer is the library's own, and rows that begin in
     // the middle of a line cost every recv that reads them (4096 tokens: 120.7 -> 115.4 us for the recvs of
     // eight ranks).
-    st.disp_stride = align_up_sz(a2a_dispatch_token_stride(&cfg), 256);
+    st.disp_stride = staged_row_stride((size_t)cfg.hidden_dim * cfg.in_elemsize, cfg.hidden_dim_scale);
     st.comb_stride = a2a_combine_token_stride(&cfg);
     st.payload_bytes = (uint32_t)align_up_sz((size_t)cfg.hidden_dim * cfg.in_elemsize, 16);
     st.max_tokens = cfg.max_num_tokens;
@@ -1992,20 +1974,35 @@ hipError_t launch_stage_send_small(const StageSendArgs &args, const Workspace &w
     // The quick form: dense index rows, a piece of the row per thread and a wavefront beside them.
     const uint32_t pieces = quantize ? args.hidden_dim / 16 : args.row_bytes / 16;
     if (args.src.indices_stride == ws.topk && pieces + kWave <= 1024) {
-        const uint32_t quick_threads = (pieces + kWave - 1) / kWave * kWave + kWave;
-        const uint32_t counters = quick_threads - kWave;
+        const uint32_t counters = (pieces + kWave - 1) / kWave * kWave;
         const uint32_t per_thread = (args.src.num_tokens * ws.topk + counters - 1) / counters;
         const size_t quick_lds = (size_t)ws.num_experts * sizeof(uint32_t);
+        const size_t g = args.rank / ws.dp_size;
+        SendQuickArgs q;
+        q.x = args.src.x;
+        q.x_scale = args.src.x_scale;
+        q.indices = args.src.indices;
+        q.bound_m = args.src.bound_m;
+        q.x_stride = args.src.x_stride;
+        q.staged = st.send_buf + g * st.max_tokens * st.disp_stride;
+        q.pos_token = st.pos_token + g * ws.max_tk;
+        q.num_routed = ws.num_routed + g * ws.num_experts;
+        q.token_offset = ws.token_offset + g * ws.max_tk;
+        q.route_slot = ws.route_slot + g * ws.max_tk;
+        q.xs_stride_elem = args.src.xs_stride_elem;
+        q.xs_stride_token = args.src.xs_stride_token;
+        q.num_tokens = args.src.num_tokens;
+        q.num_scales = args.hidden_dim_scale;
+        q.sizes = pieces | ws.num_experts << 10 | ws.topk << 21;
+        q.distances = (uint32_t)(ws.expert_offsets - ws.num_routed) / kTableUnit | (uint32_t)(ws.err - q.num_routed) << 10;
 #define A2A_LAUNCH_SEND_QUICK(NB)                                                                                    \
     do {                                                                                                             \
         if (quantize)                                                                                                \
             hipExtLaunchKernelGGL((stage_send_quick_kernel<NB, true>), dim3(args.src.num_tokens),                    \
-                                  dim3(quick_threads), quick_lds, stream, timing.start, timing.stop, 0, args, ws,    \
-                                  st);                                                                               \
+                                  dim3(counters + kWave), quick_lds, stream, timing.start, timing.stop, 0, q);       \
         else                                                                                                         \
             hipExtLaunchKernelGGL((stage_send_quick_kernel<NB, false>), dim3(args.src.num_tokens),                   \
-                                  dim3(quick_threads), quick_lds, stream, timing.start, timing.stop, 0, args, ws,    \
-                                  st);                                                                               \
+                                  dim3(counters + kWave), quick_lds, stream, timing.start, timing.stop, 0, q);       \
     } while (0)
         if (per_thread <= 1) A2A_LAUNCH_SEND_QUICK(1);
         else if (per_thread <= 2) A2A_LAUNCH_SEND_QUICK(2);
@@ -2173,20 +2170,44 @@ hipError_t launch_stage_recv(const StageRecvArgs &args, const Workspace &ws, con
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
-    const uint32_t blocks = piece_grid(args.max_rows, ws.world, chunks, typical >= kInOrderRows, a.grid);
+    PieceGrid grid;
+    const uint32_t blocks = piece_grid(args.max_rows, ws.world, chunks, typical >= kInOrderRows, grid);
+    const uint32_t first = args.rank * ws.experts_per_rank;
+    RecvRowsArgs m;
+    m.out_x = args.dst.out_x;
+    m.out_scale = args.dst.out_scale;
+    m.out_num_tokens = args.out_num_tokens;
+    m.staged = st.send_buf;
+    m.moves = st.moves + (size_t)args.rank * st.max_recv;
+    m.num_recv = st.num_recv + 2 * args.rank;
+    m.counts = ws.tokens_per_expert + first;
+    m.out_stride = args.dst.out_stride;
+    m.os_stride_elem = args.dst.os_stride_elem;
+    m.os_stride_token = args.dst.os_stride_token;
+    m.out_rows = args.dst.out_rows;
+    m.row_bytes = args.row_bytes;
+    m.num_scales = args.hidden_dim_scale;
+    m.max_recv = st.max_recv;
+    m.pieces = grid.pieces;
+    m.magic = grid.magic;
+    m.step_rows = grid.step_rows;
+    m.step_pieces = grid.step_pieces;
+    m.num_local = first >= ws.num_experts ? 0 : std::min(ws.num_experts - first, ws.experts_per_rank);
+    m.to_first_rows = (uint32_t)(ws.padded_offset - ws.tokens_per_expert) / kTableUnit;
+    m.to_flags = (uint32_t)(m.counts - ws.err);
     // Scales by column: a wavefront for every kScaleColumns columns of 64 rows that the receiver typically gets.
     const bool columns = args.dst.out_x != nullptr && scales_by_column(args.dst) &&
                          (uint64_t)typical * args.hidden_dim_scale >= kColumnWords;
-    a.scale_blocks = 0;
+    m.scale_blocks = 0;
     if (columns) {
         const uint64_t units = ((uint64_t)typical + kWave - 1) / kWave *
                                ((args.hidden_dim_scale + kScaleColumns - 1) / kScaleColumns);
         const uint64_t blocks_of_units = (units + kPieceThreads / kWave - 1) / (kPieceThreads / kWave);
-        a.scale_blocks = blocks_of_units < 1 ? 1 : blocks_of_units < kPieceWorkgroups ? (uint32_t)blocks_of_units : kPieceWorkgroups;
+        m.scale_blocks = blocks_of_units < 1 ? 1 : blocks_of_units < kPieceWorkgroups ? (uint32_t)blocks_of_units : kPieceWorkgroups;
     }
 #define A2A_LAUNCH_RECV(STREAM, COLUMNS)                                                                            \
-    hipExtLaunchKernelGGL((stage_recv_kernel<STREAM, COLUMNS>), dim3(blocks + a.scale_blocks), dim3(kPieceThreads), 0, \
-                          stream, timing.start, timing.stop, 0, a, ws, st)
+    hipExtLaunchKernelGGL((stage_recv_kernel<STREAM, COLUMNS>), dim3(blocks + m.scale_blocks), dim3(kPieceThreads), 0, \
+                          stream, timing.start, timing.stop, 0, m)
     if (args.streamed) {
         if (columns) A2A_LAUNCH_RECV(true, true); else A2A_LAUNCH_RECV(true, false);
     } else {
@@ -2196,30 +2217,47 @@ hipError_t launch_stage_recv(const StageRecvArgs &args, const Workspace &ws, con
     return hipGetLastError();
 }
 
-hipError_t launch_combine_send(const CombineSendArgs &args, const Workspace &ws, const Staging &st,
-                               hipStream_t stream, KernelTiming timing) {
-    if (args.max_rows == 0) return hipSuccess;
+hipError_t launch_combine_send(const CombineSendArgs &args, uint32_t rank, uint32_t max_rows, const Workspace &ws,
+                               const Staging &st, hipStream_t stream, KernelTiming timing) {
+    if (max_rows == 0) return hipSuccess;
     const uint32_t chunks = args.row_bytes / 16;
     CombineSendArgs a = args;
-    const uint32_t blocks = piece_grid(args.max_rows, ws.world, chunks, true, a.grid);
+    a.staged = st.comb_buf;
+    a.staged_stride = st.comb_stride;
+    a.moves = st.moves + (size_t)rank * st.max_recv;
+    a.num_recv = st.num_recv + 2 * rank;
+    a.err = ws.err;
+    a.max_recv = st.max_recv;
+    a.max_tk = ws.max_tk;
+    const uint32_t blocks = piece_grid(max_rows, ws.world, chunks, true, a.grid);
     hipExtLaunchKernelGGL(combine_send_kernel, dim3(blocks), dim3(kPieceThreads), 0, stream, timing.start, timing.stop,
-                          0, a, ws, st);
+                          0, a);
     return hipGetLastError();
 }
 
 hipError_t launch_combine_recv(const CombineRecvArgs &args, const Workspace &ws, const Staging &st,
                                uint32_t in_dtype, uint32_t out_dtype, hipStream_t stream, KernelTiming timing) {
-    CombArgs ca;
-    std::memset(&ca, 0, sizeof ca);
-    ca.dst[args.rank] = args.dst;
-    for (uint32_t r = 0; r <= (uint32_t)kMaxWorld; ++r) {
-        ca.token_start[r] = r <= args.rank ? 0 : args.dst.num_tokens;
-    }
-    ca.hidden_dim = args.hidden_dim;
-    ca.accumulate = args.accumulate;
-    ca.staged_base = st.comb_buf;
-    ca.staged_stride = st.comb_stride;
-    return launch_combine_gather(ca, ws, in_dtype, out_dtype, args.dst.num_tokens, false, stream, timing);
+    const size_t g = args.rank / ws.dp_size;
+    CombineStagedArgs a;
+    a.out = args.dst.out;
+    a.indices = args.dst.indices;
+    a.weights = args.dst.weights;
+    a.bound_m = args.dst.bound_m;
+    a.route_slot = ws.route_slot + g * ws.max_tk;
+    a.staged = st.comb_buf + g * ws.max_tk * st.comb_stride;
+    a.err = ws.err;
+    a.out_stride = args.dst.out_stride;
+    a.staged_stride = st.comb_stride;
+    a.indices_stride = args.dst.indices_stride;
+    a.weights_stride = args.dst.weights_stride;
+    a.num_tokens = args.dst.num_tokens;
+    a.layer_rows = 0;
+    a.max_tk = ws.max_tk;
+    a.hidden_dim = args.hidden_dim;
+    a.num_experts = ws.num_experts;
+    a.topk = ws.topk;
+    a.accumulate = args.accumulate;
+    return launch_combine_staged(a, in_dtype, out_dtype, stream, timing);
 }
 
 }  // namespace a2a
