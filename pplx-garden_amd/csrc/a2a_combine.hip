@@ -184,17 +184,21 @@ inline size_t lds_to_bound_waves(uint32_t topk, bool past_cache) {
     return kLds / waves / kBlock * kBlock;
 }
 
-// One slab of a token's output row: the rows that lanes 0..K-1 hold (address 0: not there), weighted and added up.
-template <typename T, typename U, int GROUP, int LOAD, int OUT>
-__device__ __forceinline__ void gather_slab(uint64_t row_ptr, float weight, uint32_t K, uint32_t num_chunks, uint32_t slab,
-                                            uint32_t lane, uint8_t *out_row, bool accumulate) {
+// PIECES slabs of a token's output row, from piece `slab` * PIECES on: the rows that lanes 0..K-1 hold (address 0: not there),
+// weighted and added up.
+template <typename T, typename U, int GROUP, int PIECES, int LOAD, int OUT>
+__device__ __forceinline__ void gather_slabs(uint64_t row_ptr, float weight, uint32_t K, uint32_t num_chunks, uint32_t slab,
+                                             uint32_t lane, uint8_t *out_row, bool accumulate) {
     constexpr int V = vec_elems<T>();
-    const uint32_t chunk = slab * kWave + lane;
-    const bool active = chunk < num_chunks;
-    float acc[V];
+    const uint32_t first = slab * PIECES * kWave + lane;
+    float acc[PIECES][V];
 #pragma unroll
-    for (int j = 0; j < V; ++j) acc[j] = 0.0f;
-    if (accumulate && active) load_elems<U, V>(out_row + (size_t)chunk * V * Elem<U>::kSize, acc);
+    for (int p = 0; p < PIECES; ++p) {
+        const uint32_t chunk = first + p * kWave;
+#pragma unroll
+        for (int j = 0; j < V; ++j) acc[p][j] = 0.0f;
+        if (accumulate && chunk < num_chunks) load_elems<U, V>(out_row + (size_t)chunk * V * Elem<U>::kSize, acc[p]);
+    }
 
     // GROUP routes at a time, all their loads asked for before the first is used.  A row is read through
     // a buffer descriptor of its own: uniform base, one offset register for all rows, and the descriptor's
@@ -203,41 +207,50 @@ __device__ __forceinline__ void gather_slab(uint64_t row_ptr, float weight, uint
     const uint64_t there = __ballot(row_ptr != 0);
     const uint32_t row_bytes = num_chunks * 16;
     for (uint32_t k0 = 0; k0 < K; k0 += GROUP) {
-        u32x4 raw[GROUP];
+        u32x4 raw[GROUP][PIECES];
         float w[GROUP];
 #pragma unroll
         for (int k = 0; k < GROUP; ++k) {
             const uint64_t row = read_lane64(row_ptr, k0 + k);
             w[k] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(weight), (int)(k0 + k)));
-            raw[k] = load_row_chunk<LOAD>(row, row_bytes, chunk * 16);
+#pragma unroll
+            for (int p = 0; p < PIECES; ++p) raw[k][p] = load_row_chunk<LOAD>(row, row_bytes, (first + p * kWave) * 16);
         }
         const uint32_t have = (uint32_t)(there >> k0) & ((1u << GROUP) - 1);
         if (have == (1u << GROUP) - 1) {
 #pragma unroll
-            for (int k = 0; k < GROUP; ++k) fma_chunk<T, V>(raw[k], w[k], acc);
+            for (int k = 0; k < GROUP; ++k) {
+#pragma unroll
+                for (int p = 0; p < PIECES; ++p) fma_chunk<T, V>(raw[k][p], w[k], acc[p]);
+            }
         } else {
             // (a row that is not there adds nothing, also with a weight that is not finite)
 #pragma unroll
             for (int k = 0; k < GROUP; ++k) {
-                if (have >> k & 1) fma_chunk<T, V>(raw[k], w[k], acc);
+                if (!(have >> k & 1)) continue;
+#pragma unroll
+                for (int p = 0; p < PIECES; ++p) fma_chunk<T, V>(raw[k][p], w[k], acc[p]);
             }
         }
     }
-    store_elems<U, V, OUT>((uint64_t)out_row, num_chunks * V * Elem<U>::kSize, chunk, acc);
+#pragma unroll
+    for (int p = 0; p < PIECES; ++p)
+        store_elems<U, V, OUT>((uint64_t)out_row, num_chunks * V * Elem<U>::kSize, first + p * kWave, acc[p]);
 }
 
 // T: type of the expert_y rows, U: type of out_tokens.  One WAVEFRONT handles
-// one slab of 64 sixteen-byte chunks of one token; wavefronts share nothing, so
+// one slab (PIECES of them) of 64 sixteen-byte chunks of one token; wavefronts share nothing, so
 // a compute unit keeps many of them in flight and the latency of resolving a
 // token's routes is hidden by the loads of its neighbours.  GROUP routes are
 // loaded before the first is used: the smallest of 1, 2, 4, 8 that holds K, or
 // groups of 8 (a load that fills a group up costs its issue only, but at K = 1
-// three of them were 10 %: 96.7 -> 106.4 us for 16000 tokens).  ONE_RANK: one rank
+// three of them were 10 %: 96.7 -> 106.4 us for 16000 tokens).  PIECES: slabs a wavefront moves (two_pieces_a_lane in
+// a2a_rules.h).  ONE_RANK: one rank
 // alone has tokens and the step is small; its descriptor is read from a fixed
 // place in the argument block, which takes two dependent scalar loads out of
 // the head of every wavefront (0.1-0.4 us of a step of 128 to 1024 tokens; a
 // 4096-token step hides them and is 0.3 us faster without the variant).
-template <typename T, typename U, int GROUP, bool ONE_RANK, int OUT>
+template <typename T, typename U, int GROUP, int PIECES, bool ONE_RANK, int OUT>
 __global__ __launch_bounds__(kWave) void combine_gather_kernel(const CombArgs args, const Workspace ws) {
     constexpr int LOAD = OUT == kNonTemporal ? kNonTemporal : kDeviceNonTemporal;
     if constexpr (ONE_RANK) {
@@ -345,7 +358,7 @@ __global__ __launch_bounds__(kWave) void combine_gather_kernel(const CombArgs ar
         if (!ok && slab == 0) atomicOr(ws.err, A2A_DEV_BAD_SLOT);
     }
 
-    gather_slab<T, U, GROUP, LOAD, OUT>(row_ptr, weight, K, num_chunks, slab, lane, dst.out + (size_t)token * dst.out_stride,
+    gather_slabs<T, U, GROUP, PIECES, LOAD, OUT>(row_ptr, weight, K, num_chunks, slab, lane, dst.out + (size_t)token * dst.out_stride,
                                         args.accumulate != 0);
 }
 
@@ -353,7 +366,7 @@ __global__ __launch_bounds__(kWave) void combine_gather_kernel(const CombArgs ar
 // per copy (a2a_combine_recv.cu:67-73 = exclusive offset of the expert + token offset), so that there is no receiver to
 // look up and no second, dependent load in front of the rows.  What it needs is passed as the few words that they are
 // (kShortArguments); otherwise as combine_gather_kernel.
-template <typename T, typename U, int GROUP>
+template <typename T, typename U, int GROUP, int PIECES>
 __global__ __launch_bounds__(kWave) void combine_staged_kernel(const CombineStagedArgs args) {
     A2A_PIN(args.out);
     A2A_PIN(args.indices);
@@ -389,7 +402,7 @@ __global__ __launch_bounds__(kWave) void combine_staged_kernel(const CombineStag
             atomicOr(args.err, A2A_DEV_BAD_SLOT);
         }
     }
-    gather_slab<T, U, GROUP, kNonTemporal, kNonTemporal>(row_ptr, weight, K, args.hidden_dim / vec_elems<T>(), slab, lane,
+    gather_slabs<T, U, GROUP, PIECES, kNonTemporal, kNonTemporal>(row_ptr, weight, K, args.hidden_dim / vec_elems<T>(), slab, lane,
                                                          args.out + (size_t)token * args.out_stride, args.accumulate != 0);
 }
 
@@ -408,26 +421,30 @@ static hipError_t launch_typed(const CombArgs &given, const Workspace &ws, uint3
     if (ranks_with_tokens != 1 || total_tokens > kOneRankMaxTokens || streamed) args.single_rank = 0;
     if (args.single_rank != 0) args.single = given.dst[args.single_rank - 1];
     const uint32_t chunks = args.hidden_dim / V;
-    const uint32_t slabs = (chunks + kWave - 1) / kWave;
+    const bool two = two_pieces_a_lane(ws.topk, (uint64_t)((chunks + kWave - 1) / kWave) * total_tokens);
+    const uint32_t width = two ? 2 * kWave : kWave;
+    const uint32_t slabs = (chunks + width - 1) / width;
     const TokenLayers layers = token_layers(total_tokens);
     args.layer_rows = layers.rows;
     const dim3 grid(slabs, layers.rows, layers.layers);
     const bool past_cache =
         args.single_rank == 0 && (streamed || (uint64_t)total_tokens * args.hidden_dim * Elem<U>::kSize >= kStreamedOutput);
     const size_t lds = (uint64_t)slabs * total_tokens <= kAllAtOnce ? 0 : lds_to_bound_waves(ws.topk, past_cache);
-#define A2A_LAUNCH_GATHER(GROUP, ONE, OUT, LDS)                                                                \
-    hipExtLaunchKernelGGL((combine_gather_kernel<T, U, GROUP, ONE, OUT>), grid, dim3(kWave), LDS, stream,      \
-                          timing.start, timing.stop, 0, args, ws)
-#define A2A_LAUNCH_GATHER_RANKS(GROUP)                                                                         \
+#define A2A_LAUNCH_GATHER(GROUP, PIECES, ONE, OUT, LDS)                                                        \
+    hipExtLaunchKernelGGL((combine_gather_kernel<T, U, GROUP, PIECES, ONE, OUT>), grid, dim3(kWave), LDS,      \
+                          stream, timing.start, timing.stop, 0, args, ws)
+#define A2A_LAUNCH_GATHER_RANKS(GROUP, PIECES)                                                                 \
     do {                                                                                                       \
-        if (args.single_rank != 0) A2A_LAUNCH_GATHER(GROUP, true, kNonTemporal, 0);                            \
-        else if (past_cache) A2A_LAUNCH_GATHER(GROUP, false, kSystemNonTemporal, lds);                         \
-        else A2A_LAUNCH_GATHER(GROUP, false, kNonTemporal, lds);                                               \
+        if (args.single_rank != 0) A2A_LAUNCH_GATHER(GROUP, PIECES, true, kNonTemporal, 0);                    \
+        else if (past_cache) A2A_LAUNCH_GATHER(GROUP, PIECES, false, kSystemNonTemporal, lds);                 \
+        else A2A_LAUNCH_GATHER(GROUP, PIECES, false, kNonTemporal, lds);                                       \
     } while (0)
-    if (ws.topk > 4) A2A_LAUNCH_GATHER_RANKS(8);
-    else if (ws.topk > 2) A2A_LAUNCH_GATHER_RANKS(4);
-    else if (ws.topk > 1) A2A_LAUNCH_GATHER_RANKS(2);
-    else A2A_LAUNCH_GATHER_RANKS(1);
+    if (ws.topk > 4) A2A_LAUNCH_GATHER_RANKS(8, 1);
+    else if (ws.topk > 2) A2A_LAUNCH_GATHER_RANKS(4, 1);
+    else if (ws.topk > 1 && two) A2A_LAUNCH_GATHER_RANKS(2, 2);
+    else if (ws.topk > 1) A2A_LAUNCH_GATHER_RANKS(2, 1);
+    else if (two) A2A_LAUNCH_GATHER_RANKS(1, 2);
+    else A2A_LAUNCH_GATHER_RANKS(1, 1);
 #undef A2A_LAUNCH_GATHER_RANKS
 #undef A2A_LAUNCH_GATHER
     return hipGetLastError();
@@ -456,19 +473,24 @@ hipError_t launch_combine_gather(const CombArgs &args, const Workspace &ws, uint
 template <typename T, typename U>
 static hipError_t launch_staged_typed(const CombineStagedArgs &given, hipStream_t stream, KernelTiming timing) {
     CombineStagedArgs args = given;
-    const uint32_t slabs = (args.hidden_dim / vec_elems<T>() + kWave - 1) / kWave;
+    const uint32_t chunks = args.hidden_dim / vec_elems<T>();
+    const bool two = two_pieces_a_lane(args.topk, (uint64_t)((chunks + kWave - 1) / kWave) * args.num_tokens);
+    const uint32_t width = two ? 2 * kWave : kWave;
+    const uint32_t slabs = (chunks + width - 1) / width;
     const TokenLayers layers = token_layers(args.num_tokens);
     args.layer_rows = layers.rows;
     const dim3 grid(slabs, layers.rows, layers.layers);
     const bool bounded = args.num_tokens > kOneRankMaxTokens && (uint64_t)slabs * args.num_tokens > kAllAtOnce;
     const size_t lds = bounded ? lds_to_bound_waves(args.topk, false) : 0;
-#define A2A_LAUNCH_STAGED(GROUP)                                                                              \
-    hipExtLaunchKernelGGL((combine_staged_kernel<T, U, GROUP>), grid, dim3(kWave), lds, stream, timing.start, \
-                          timing.stop, 0, args)
-    if (args.topk > 4) A2A_LAUNCH_STAGED(8);
-    else if (args.topk > 2) A2A_LAUNCH_STAGED(4);
-    else if (args.topk > 1) A2A_LAUNCH_STAGED(2);
-    else A2A_LAUNCH_STAGED(1);
+#define A2A_LAUNCH_STAGED(GROUP, PIECES)                                                                      \
+    hipExtLaunchKernelGGL((combine_staged_kernel<T, U, GROUP, PIECES>), grid, dim3(kWave), lds, stream,       \
+                          timing.start, timing.stop, 0, args)
+    if (args.topk > 4) A2A_LAUNCH_STAGED(8, 1);
+    else if (args.topk > 2) A2A_LAUNCH_STAGED(4, 1);
+    else if (args.topk > 1 && two) A2A_LAUNCH_STAGED(2, 2);
+    else if (args.topk > 1) A2A_LAUNCH_STAGED(2, 1);
+    else if (two) A2A_LAUNCH_STAGED(1, 2);
+    else A2A_LAUNCH_STAGED(1, 1);
 #undef A2A_LAUNCH_STAGED
     return hipGetLastError();
 }

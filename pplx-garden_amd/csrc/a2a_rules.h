@@ -23,6 +23,25 @@ inline TokenLayers token_layers(uint32_t tokens) {
     return t;
 }
 
+// Whether a wavefront of the gather moves two slabs of a token's row instead of one.  With one or two copies a token a slab is
+// one or two loads a lane behind a chain of arguments, ids and places: all the wavefronts that fit have too few of them in flight,
+// and the dispatcher starts no more than some 4300 a us.  us per combine, bf16 rows unless said otherwise, one slab / two / four:
+//                          K = 1                    K = 2                    K = 4
+//    8 x 3000 of 2 KB    24.9 /  19.8 /  20.4     28.8 /  28.0 /  29.6     42.8 /  43.3 /  43.5
+//             of 5.9 KB  67.1 /  48.6 /  55.0     74.6 /  70.7 /  76.2    115.5 / 118.7 / 125.3
+//             of 8 KB    88.4 /  66.7 /  68.5     99.9 /  97.8 /  99.8    163.3 / 166.9 / 168.1
+//             of 14 KB  137.2 / 114.7 / 121.4    174.1 / 169.6 / 174.2
+//    8 x 800  of 8 KB    26.3 /  21.0 /  21.4     30.4 /  29.5 /  29.3     45.4 /  45.9 /  46.1
+//        float of 28 KB  72.9 /  63.1 /  63.7     93.3 /  91.1 /  93.0    149.0 / 152.7 / 157.7
+//    8 x 200  of 5.9 KB   7.9 /   6.7 /   6.8      8.4 /   8.0 /   8.4     11.1 /  10.9 /  11.6
+//    8 x 40   of 8 KB     4.4 /   3.8 /   3.9      4.6 /   4.1 /   4.2      5.1 /   4.8 /   5.0
+//             of 4 KB     3.45 /  3.47 /  3.63     3.5 /   3.7 /   3.9      (1280 wavefronts)
+//    8 x 4    of 14 KB    3.2 /   3.35 /  3.45     3.3 /   3.3 /   3.6      (448)
+// Eight copies lose 1 to 6 % with two.  Steps of few wavefronts end with the chain, which is shorter with one slab.
+constexpr uint64_t kFewSlabs = 1536;
+
+inline bool two_pieces_a_lane(uint32_t topk, uint64_t slabs) { return topk <= 2 && slabs > kFewSlabs; }
+
 // Cache policy of a large step's copies and of its combined tokens.  From kStreamCopies bytes of copies on the pack
 // sends them past the 256 MB Infinity Cache (device scope and non-temporal) and the combine sends its tokens past it
 // too: such a step cannot stay there until it is read, and lines that are not left dirty need not be written back

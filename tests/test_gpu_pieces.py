@@ -1,5 +1,5 @@
-"""Large steps with few copies a token, of whose rows a thread of the pack moves one, two or four pieces of 16 bytes: rows that
-end at the edges of a wavefront's, a workgroup's and a round's pieces, against the oracle."""
+"""Steps with few copies a token, of whose rows a thread of the pack moves one, two or four pieces of 16 bytes and a lane of the
+gather one or two: rows that end at the edges of a wavefront's, a workgroup's and a round's pieces, against the oracle."""
 
 from dataclasses import replace
 
@@ -7,12 +7,12 @@ import pytest
 import torch
 
 from a2a_cases import C1, scaled
-from a2a_transport import RefConfig, check, make_ref_rank, rows_for, run_gpu
+from a2a_transport import RefConfig, check, make_ops, make_ref_rank, rows_for, run_gpu
 from test_gpu_sources import run_and_check
 
 pytestmark = pytest.mark.gpu
 DEV = torch.device("cuda:0")
-BF16, F32, FP8 = torch.bfloat16, torch.float32, torch.float8_e4m3fn
+BF16, F16, F32, FP8 = torch.bfloat16, torch.float16, torch.float32, torch.float8_e4m3fn
 
 # top-k, elements of a row, type, scales, layout of the scales, pieces a thread moves
 MOVED = [
@@ -61,3 +61,58 @@ def test_quantised_rows(topk, hidden, pieces):
     case = replace(scaled(C1, 1), world_size=3, num_experts=18, topk=topk, hidden_dim=hidden, name="pieces", num_tokens=max(tokens),
                    seed=91 + hidden)
     run_and_check(case, tokens, two_launches=True, stray=topk == 2)
+
+
+# Combines of which a wavefront moves one or two slabs of 64 pieces of a token's row: ranks, tokens, top-k, elements, type, two
+GATHERS = [
+    (2, 768, 1, 512, BF16, False),        # 1536 slabs: the largest step of one each
+    (1, 1537, 1, 512, BF16, True),        # one more; rows that end with the first of a wavefront's two
+    (3, 300, 1, 1032, BF16, True),        # three slabs, the last with one piece
+    (3, 300, 2, 1528, F16, True),         # three, the last but for one piece full
+    (2, 400, 2, 1024, BF16, True),        # two whole ones
+    (2, 2100, 2, 516, F32, True),         # float rows, a slab and five pieces; more tokens than the sole sender's variant takes
+    (2, 1100, 3, 1024, BF16, False),
+]
+
+
+@pytest.mark.parametrize("split", [False, True])
+@pytest.mark.parametrize("ranks,tokens,topk,hidden,dtype,two", GATHERS, ids=[f"t{g[1]}_k{g[2]}_h{g[3]}" for g in GATHERS])
+def test_combined_tokens(ranks, tokens, topk, hidden, dtype, two, split):
+    print(f"ranks={ranks} tokens={tokens} topk={topk} hidden={hidden} {dtype} split={split}", flush=True)
+    cfg = RefConfig("gather", ranks, 1, tokens, 7, hidden, None, topk, dtype, dtype, None)
+    world = [make_ref_rank(cfg, r, tokens) for r in range(ranks)]
+    rows = rows_for(cfg, world)
+    check(cfg, world, rows, run_gpu(cfg, world, rows, DEV, split=split))
+
+
+@pytest.mark.parametrize("topk", [1, 2])
+@pytest.mark.parametrize("in_dtype,out_dtype", [(BF16, F32), (F32, BF16), (torch.float16, BF16)])
+def test_combined_types_accumulated(topk, in_dtype, out_dtype):
+    """Two slabs a wavefront onto what is there, of every width of rows and tokens; a token without copies keeps what it has."""
+    ranks, tokens, hidden = 2, 900, 1048
+    g = torch.Generator().manual_seed(topk)
+    cfg = RefConfig("gather", ranks, 1, tokens, 6, hidden, None, topk, in_dtype, out_dtype, None)
+    world = [make_ref_rank(cfg, r, tokens) for r in range(ranks)]
+    rows = rows_for(cfg, world)
+    ops = make_ops(cfg, DEV)
+    try:
+        x = [rd.dp_x.to(DEV) for rd in world]
+        idx = [rd.indices.view(torch.uint32).to(DEV) for rd in world]
+        w = [rd.weights.to(DEV) for rd in world]
+        got_x = [torch.zeros((rows, hidden), dtype=in_dtype, device=DEV) for _ in world]
+        before = [torch.randn((tokens, hidden), generator=g).to(out_dtype) for _ in world]
+        out = [b.to(DEV) for b in before]
+        for r in range(ranks):
+            ops[r].dispatch(torch.zeros(3, dtype=torch.int32, device=DEV), got_x[r], None, x[r], None, idx[r], w[r])
+        for r in range(ranks):   # (the rows come back as they went: a token's weights add up to one)
+            ops[r].combine(out[r], idx[r], w[r], got_x[r], accumulate=True)
+        torch.cuda.synchronize(DEV)
+        assert ops[0].context.status() == 0
+        ulp = 2.0 ** -8 if out_dtype == BF16 else 2.0 ** -22   # one rounding of the sum to its type
+        for r in range(ranks):
+            want = before[r].double() + world[r].dp_x.double()
+            size = before[r].double().abs() + world[r].dp_x.double().abs()
+            assert ((out[r].cpu().double() - want).abs() <= ulp * size + 1e-30).all()
+    finally:
+        for op in ops:
+            op.destroy()

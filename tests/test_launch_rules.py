@@ -7,7 +7,7 @@ from pathlib import Path
 
 import pytest
 
-from test_gpu_pieces import MOVED, QUANTISED
+from test_gpu_pieces import GATHERS, MOVED, QUANTISED
 from test_gpu_shapes import STREAMED, copies_of
 from test_gpu_split import PIECES
 from test_gpu_written_through import STEPS
@@ -27,6 +27,7 @@ int written_through(uint64_t copies, uint32_t row_bytes, uint32_t k) {
 uint32_t pieces(uint32_t k, uint32_t chunks, int quantize, int by_column) {
     return a2a::pieces_per_lane(k, chunks, quantize != 0, by_column != 0);
 }
+int two_pieces(uint32_t k, uint64_t slabs) { return a2a::two_pieces_a_lane(k, slabs); }
 int one_launch(uint32_t rows, uint32_t row_bytes, uint32_t items, uint32_t threads) {
     return a2a::first_recv_in_one_launch(rows, row_bytes, items, threads);
 }
@@ -100,6 +101,12 @@ def test_pieces_of_a_thread(rules):
         assert rules.pieces(k, hidden * dtype.itemsize // 16, 0, layout == "col") == pieces, (k, hidden)
     for k, hidden, pieces in QUANTISED:
         assert rules.pieces(k, hidden // 16, 1, 0) == pieces, (k, hidden)
+
+
+def test_pieces_of_the_gather(rules):
+    for ranks, tokens, topk, hidden, dtype, two in GATHERS:
+        slabs = -(-hidden * dtype.itemsize // 1024) * ranks * tokens
+        assert bool(rules.two_pieces(topk, slabs)) == two, (tokens, topk)
 
 
 def test_received_rows_that_the_cache_can_keep_stay_there(rules):
