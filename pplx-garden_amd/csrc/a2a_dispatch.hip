@@ -17,6 +17,8 @@
 // scalars.  Token rows are loaded non-temporally (each is read once).  How the
 // copies are written depends on how much of the Infinity Cache they fill (see
 // copies_past_cache in a2a_rules.h).
+#include <algorithm>
+
 #include "a2a_device.h"
 #include "a2a_rules.h"
 #include "a2a_scan.h"
@@ -1695,6 +1697,8 @@ constexpr uint32_t kSourcesMaxEntries = 16384;
 constexpr uint32_t kSourcesChunk = 4 * kWave;    // entries that a wavefront asks for with four loads
 constexpr uint32_t kSourcesMaxTokens = 8;        // of a workgroup
 constexpr uint32_t kSourcesMaxRoutes = 64;
+constexpr uint32_t kSourcesMaxUnits = 60;        // of a workgroup
+constexpr uint64_t kSourcesMaxVisits = 20000000; // entries x workgroups of steps with more than a workgroup's worth per compute unit
 constexpr uint32_t kSourcesMaxScales = 128;
 constexpr uint32_t kSourcesMaxTable = 12288;     // words of dynamic LDS
 constexpr uint32_t kSourcesMinRow = 2048;        // bytes of a copy from which steps of more than kSingleMaxEntries entries pay
@@ -2603,7 +2607,9 @@ hipError_t launch_dispatch_single(const PushArgs &args, const FinalizeArgs &fin,
 }
 
 // Whether a step takes dispatch_sources_kernel, and its shape: tokens of a workgroup as in the kernels of one source
-// (about one workgroup per compute unit); beside the resolver as many wavefronts as there are units to move or chunks
+// (about one workgroup per compute unit) as long as a workgroup can hold them, and otherwise, with about two workgroups per
+// compute unit (the tables' one among them: with 513 the last one starts when another has ended), or as many as there are
+// when each holds what it can; beside the resolver as many wavefronts as there are units to move or chunks
 // to count (8 x 32 tokens of hidden 2048, 2 units and 8 chunks: 6.6 us with 4 wavefronts, 4.6 with 8), in as few rounds
 // as 15 of them need.  The line at 16384 entries is the resolver's: with more than eight tokens of top-8 a workgroup has
 // more routes than its one resolving wavefront has lanes.  It is not the counting's, which costs every workgroup 0.16 us
@@ -2611,7 +2617,26 @@ hipError_t launch_dispatch_single(const PushArgs &args, const FinalizeArgs &fin,
 // with two resolving wavefronts have not been measured.  Above 8192 entries rows of 2 KB, because with smaller ones the
 // counting is what is left (one source of 2048 tokens, hidden 1024: 21.5 us a step against 20.4; hidden 2048 and 1500
 // tokens: 23.2 against 23.9).  Steps of one source with up to kSingleMaxEntries entries have the two kernels that are made
-// for them (128 tokens 4.54 us against 4.77 here, 1024 tokens 15.4 against 16.1).
+// for them (128 tokens 4.54 us against 4.77 here, 1024 tokens 15.4 against 16.1) unless a row's pieces leave these no
+// wavefront beside them: float rows of 16 KB and more, K = 8, us per step before / here: 4 tokens 9.6 / 8.5, 128 14.2 / 11.3, 400
+// 27.9 / 23.8; of 28 KB 10.8 / 10.0, 20.7 / 15.7, 48.5 / 41.0.
+// Steps of more tokens than 256 workgroups hold, us per step in two launches (or, below 3 * 2^19 visits, with the general
+// kernel) / here:
+//                      K = 1               K = 2               K = 4               K = 8
+//   bf16 2 KB  8 x 300   16.3 /  12.4        17.0 /  13.7        21.1 /  16.1
+//        8 KB  8 x 240   23.1 /  16.7        29.7 /  20.4        39.9 /  30.3        62.0 /  56.0
+//              8 x 600   40.9 /  36.9        53.8 /  45.2
+//       14 KB  8 x 160   24.9 /  20.1        31.8 /  26.0        42.5 /  34.7        69.8 /  63.4
+//              8 x 400   44.8 /  41.0        62.6 /  57.5        94.0 /  90.9
+//   f32 16 KB  8 x 109   38.2 /  16.2        43.1 /  19.1        39.6 /  27.8        58.7 /  49.9
+//              8 x 240   36.2 /  28.6        44.4 /  36.7        71.0 /  60.9       112.1 / 107.5
+//       28 KB  8 x 109   46.4 /  24.0        54.0 /  32.2        60.2 /  44.2        94.3 /  82.9
+//   fp8  7 KB  8 x 400   37.6 /  30.3        49.5 /  40.7        69.8 /  62.6
+//   quantised  8 x 300   34.7 /  31.4        43.5 /  39.0        59.3 /  52.1
+// What ends it is the counting, every entry by every workgroup: 1143 workgroups x 16 000 entries (bf16 8 KB, K = 2) 81.3 / 79.6,
+// 2000 x 16 000 (14 KB) 133.2 / 134.8, 1800 x 14 400 (fp8, K = 1) 116.4 / 119.3, 2057 x 14 400 (2 KB) 36.0 / 42.4.  Quantised rows
+// do not gain beyond two workgroups a compute unit (600: 54.8 / 57.5, K = 2 71.3 / 73.8).  Where 256 workgroups do hold a step, two a
+// compute unit lose up to 12 % or gain up to 10, by how the rows divide among the wavefronts.
 bool plan_dispatch_sources(const PushArgs &args, const Workspace &ws, bool quantize, uint32_t total_tokens, SourcesPlan &plan,
                            uint32_t &groups, uint32_t &threads, uint32_t &rounds) {
     constexpr uint32_t kComputeUnits = 256;
@@ -2623,28 +2648,43 @@ bool plan_dispatch_sources(const PushArgs &args, const Workspace &ws, bool quant
     const uint32_t pieces = quantize ? args.hidden_dim / 16 : args.row_bytes / 16;
     plan.units = (pieces + kWave - 1) / kWave;
     plan.units_magic = plan.units > 1 ? 0xFFFFFFFFu / plan.units + 1 : 0;
+    auto groups_of = [&](uint32_t per_group) {
+        uint32_t n = 0;
+        for (uint32_t g = 0; g < ws.num_groups; ++g) n += (args.src[g].num_tokens + per_group - 1) / per_group;
+        return n;
+    };
+    // what a workgroup can hold: tokens, a lane of the resolver per route, four rounds of fifteen wavefronts
+    const uint32_t most = std::min({kSourcesMaxTokens, kSourcesMaxRoutes / ws.topk, kSourcesMaxUnits / plan.units});
+    if (most == 0) return false;
     plan.per_group = (total_tokens + kComputeUnits - 1) / kComputeUnits;
-    if (plan.per_group > kSourcesMaxTokens || plan.per_group * ws.topk > kSourcesMaxRoutes) return false;
+    const bool spread = plan.per_group > most;
+    if (spread) {
+        plan.per_group = most;
+        if (ws.topk * plan.units >= 8) {
+            plan.per_group = std::min(most, (total_tokens + 2 * kComputeUnits - 1) / (2 * kComputeUnits));
+            while (plan.per_group < most && groups_of(plan.per_group) >= 2 * kComputeUnits) ++plan.per_group;
+        }
+    }
     plan.chunks = 0;
-    groups = 0;
+    groups = groups_of(plan.per_group);
     uint32_t senders = 0;
     for (uint32_t g = 0; g < ws.num_groups; ++g) {
         if (args.src[g].num_tokens == 0) continue;
         if (args.src[g].indices_stride != ws.topk) return false;
         ++senders;
         plan.chunks += (args.src[g].num_tokens * ws.topk + kSourcesChunk - 1) / kSourcesChunk;
-        groups += (args.src[g].num_tokens + plan.per_group - 1) / plan.per_group;
     }
-    if (senders == 1 && entries <= kSingleMaxEntries) return false;
+    if (senders == 1 && entries <= kSingleMaxEntries && pieces + kWave <= 1024) return false;
+    if (spread && (quantize ? groups >= 2 * kComputeUnits : entries * groups > kSourcesMaxVisits)) return false;
     if (entries > kSingleMaxEntries && pieces * 16 < kSourcesMinRow) return false;
     const uint32_t units = plan.per_group * plan.units;
     uint32_t movers = units;
     if (movers < plan.chunks) movers = plan.chunks;
     if (movers > 15) movers = 15;
-    rounds = (units + movers - 1) / movers;
+    rounds = (units + movers - 1) / movers;   // <= 4
     if (rounds > 1 && movers > (units + rounds - 1) / rounds) movers = (units + rounds - 1) / rounds;
     threads = (movers + 1) * kWave;
-    return rounds <= 4;
+    return true;
 }
 
 bool dispatch_sources_fits(const PushArgs &args, const Workspace &ws, bool quantize, uint32_t total_tokens) {

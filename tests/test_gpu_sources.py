@@ -149,3 +149,47 @@ def test_rows_moved_as_they_are(name):
     routes = []
     check(cfg, world, rows, run_gpu(cfg, world, rows, DEV, split=False, scale_layout=layout, routes=routes))
     assert routes == [two_launches]
+
+
+# Steps of more tokens than a workgroup per compute unit holds, and of one source whose rows leave no wavefront beside their
+# pieces: ranks' tokens, experts, top-k, elements, type, scales, layout of the scales, whether there is a routing launch
+SPREAD = {
+    "f32_16_kb_two_a_workgroup": ([300, 0, 301, 270], 30, 2, 4096, F32, None, "row", False),
+    "f32_28_kb_of_one": ([0, 900, 0], 24, 8, 7168, F32, None, "row", False),
+    "f32_16_kb_of_one": ([130, 0], 16, 8, 4096, F32, None, "row", False),
+    "f32_16_kb_one_token": ([0, 0, 1], 9, 1, 4096, F32, None, "row", False),
+    "bf16_2_kb_eight_a_workgroup": ([700, 0, 1, 1400], 17, 1, 1024, BF16, None, "row", False),
+    "bf16_14_kb_one_copy": ([1601, 31], 10, 1, 7168, BF16, None, "row", False),
+    "fp8_scales_by_column": ([1201, 1198, 2], 12, 2, 7168, FP8, 56, "col", False),
+    "fp8_scales_by_row_pad": ([1300, 3, 1300], 33, 3, 2944, FP8, 23, "row", False),
+    "f16_1500_workgroups": ([6001, 5999], 6, 1, 1024, F16, None, "row", False),
+    "f16_2000_workgroups_the_two_launches": ([8001, 7999], 6, 1, 1024, F16, None, "row", True),
+}
+
+
+@pytest.mark.parametrize("name", SPREAD)
+def test_more_workgroups_than_compute_units(name):
+    tokens, experts, topk, hidden, dtype, scales, layout, two_launches = SPREAD[name]
+    print(f"{name} tokens={tokens}", flush=True)
+    cfg = RefConfig(name, len(tokens), 1, max(tokens), experts, hidden, scales, topk, dtype, BF16 if dtype == FP8 else dtype,
+                    F32 if scales else None, expert_padding=5 if "pad" in name else 1)
+    world = [make_ref_rank(cfg, r, t) for r, t in enumerate(tokens)]
+    rows = rows_for(cfg, world)
+    routes = []
+    check(cfg, world, rows, run_gpu(cfg, world, rows, DEV, split=False, scale_layout=layout, routes=routes))
+    assert routes == [two_launches]
+
+
+SPREAD_QUANTISED = {
+    "512_workgroups_and_the_tables": (replace(BASE, topk=4, hidden_dim=2048), [320] * 8, dict(repeats=True)),
+    "two_short_copies": (replace(BASE, topk=2, hidden_dim=1024, expert_padding=16), [2049, 0, 0, 1, 300, 0, 0, 17], dict(stray=True)),
+    "bounds": (replace(BASE, topk=3, hidden_dim=4096), [700, 800, 0, 5, 701, 0, 0, 9], dict(bounds=[699, 0, None, 5, None, None, None, 1])),
+    "beyond_two_a_compute_unit": (replace(BASE, topk=2, hidden_dim=1024), [4080, 0, 0, 1, 0, 0, 0, 17], dict(two_launches=True)),
+}
+
+
+@pytest.mark.parametrize("name", SPREAD_QUANTISED)
+def test_more_workgroups_than_compute_units_quantised(name):
+    case, tokens, how = SPREAD_QUANTISED[name]
+    print(f"{name} tokens={tokens}", flush=True)
+    run_and_check(replace(case, name=name, num_tokens=max(tokens), seed=47_000), tokens, **how)
