@@ -186,6 +186,32 @@ struct CombineStagedArgs {
 };
 static_assert(sizeof(CombineStagedArgs) <= kShortArguments, "");
 
+// The group's combine of a small step in which one rank alone has tokens, with dense index and weight rows and receivers whose
+// rows are alike (sole_args in a2a_combine.hip).
+constexpr uint32_t kSoleReceivers = 10;
+
+struct CombineSoleArgs {
+    const uint8_t *y;         // rows of receiver 0
+    uint8_t *out;
+    const int32_t *indices;
+    const float *weights;
+    const uint32_t *route_slot;
+    uint32_t *err;
+    uint32_t y_stride;        // in 16 bytes
+    uint32_t y_rows;
+    uint32_t out_stride;      // in 8 bytes
+    uint32_t hidden_dim;
+    uint32_t le_magic;
+    uint32_t sizes;           // from bit 0: experts (11), routes per token (7), experts per rank (11), accumulate (1)
+    int32_t y_offset[kSoleReceivers];   // receivers' rows from y on, in 16 bytes
+
+    __device__ __forceinline__ uint32_t num_experts() const { return sizes & 0x7FF; }
+    __device__ __forceinline__ uint32_t topk() const { return sizes >> 11 & 0x7F; }
+    __device__ __forceinline__ uint32_t experts_per_rank() const { return sizes >> 18 & 0x7FF; }
+    __device__ __forceinline__ bool accumulate() const { return sizes >> 29 != 0; }
+};
+static_assert(sizeof(CombineSoleArgs) <= kShortArguments, "");
+
 // Events a caller wants recorded when a kernel itself begins and ends (both
 // null: an ordinary launch).
 struct KernelTiming {

@@ -47,7 +47,7 @@ def test_stores_in_inline_assembly_carry_the_wait_states_the_compiler_inserts(tm
 def test_kernels_of_short_arguments_take_no_hidden_ones():
     # blockDim and gridDim are arguments too, which the compiler adds: the launch would be a long one
     text = "\n".join((ROOT / "csrc" / name).read_text() for name in ("a2a_staged.hip", "a2a_combine.hip"))
-    short = {"SendQuickArgs", "RecvRowsArgs", "CombineSendArgs", "CombineStagedArgs"}
+    short = {"SendQuickArgs", "RecvRowsArgs", "CombineSendArgs", "CombineStagedArgs", "CombineSoleArgs"}
     found = set()
     for kind, body in re.findall(r"\((?:const )?(\w+)(?: &| )args[^)]*\) \{\n(.*?)^\}", text, re.M | re.S):
         if kind in short:
