@@ -2607,9 +2607,9 @@ hipError_t launch_dispatch_single(const PushArgs &args, const FinalizeArgs &fin,
 }
 
 // Whether a step takes dispatch_sources_kernel, and its shape: tokens of a workgroup as in the kernels of one source
-// (about one workgroup per compute unit) as long as a workgroup can hold them, and otherwise, with about two workgroups per
-// compute unit (the tables' one among them: with 513 the last one starts when another has ended), or as many as there are
-// when each holds what it can; beside the resolver as many wavefronts as there are units to move or chunks
+// (about one workgroup per compute unit) as long as a workgroup can hold them, and otherwise, or where that is better, with about
+// two workgroups per compute unit (the tables' one among them: with 513 the last one starts when another has ended), or as
+// many as there are when each holds what it can; beside the resolver as many wavefronts as there are units to move or chunks
 // to count (8 x 32 tokens of hidden 2048, 2 units and 8 chunks: 6.6 us with 4 wavefronts, 4.6 with 8), in as few rounds
 // as 15 of them need.  The line at 16384 entries is the resolver's: with more than eight tokens of top-8 a workgroup has
 // more routes than its one resolving wavefront has lanes.  It is not the counting's, which costs every workgroup 0.16 us
@@ -2635,8 +2635,13 @@ hipError_t launch_dispatch_single(const PushArgs &args, const FinalizeArgs &fin,
 //   quantised  8 x 300   34.7 /  31.4        43.5 /  39.0        59.3 /  52.1
 // What ends it is the counting, every entry by every workgroup: 1143 workgroups x 16 000 entries (bf16 8 KB, K = 2) 81.3 / 79.6,
 // 2000 x 16 000 (14 KB) 133.2 / 134.8, 1800 x 14 400 (fp8, K = 1) 116.4 / 119.3, 2057 x 14 400 (2 KB) 36.0 / 42.4.  Quantised rows
-// do not gain beyond two workgroups a compute unit (600: 54.8 / 57.5, K = 2 71.3 / 73.8).  Where 256 workgroups do hold a step, two a
-// compute unit lose up to 12 % or gain up to 10, by how the rows divide among the wavefronts.
+// are two registers' loads a piece: beyond two workgroups a compute unit they are moved in two rounds instead of four, and up to
+// three workgroups a compute unit (K = 1, hidden 2048, 8 x 640 28.7 / 21.6; 4096, 731 workgroups 41.2 / 36.7; K = 2 49.0 / 46.7; 914
+// workgroups 57.3 / 58.9; 5120, 694 workgroups 39.7 / 37.2, 853 45.3 / 46.3).  Where 256 workgroups do hold a step, two a compute unit
+// lose up to 12 % or gain up to 10, by how the rows divide among the wavefronts; with eight copies of more than 1024 tokens they
+// gain (one a compute unit / two: bf16 of 8 KB, 8 x 160 38.8 / 35.6, 8 x 208 4.8 %, one source of 1100 34.9 / 31.3, of 1500 42.6 / 40.3;
+// fp8 of 7 KB, 8 x 160 49.0 / 46.3, 8 x 240 1.7 %; quantised of 7 KB, 8 x 160 50.3 / 47.9, but with four tokens a workgroup 8 x 192
+// 57.4 / 60.0, 8 x 256 2.1 % slower).
 bool plan_dispatch_sources(const PushArgs &args, const Workspace &ws, bool quantize, uint32_t total_tokens, SourcesPlan &plan,
                            uint32_t &groups, uint32_t &threads, uint32_t &rounds) {
     constexpr uint32_t kComputeUnits = 256;
@@ -2658,12 +2663,15 @@ bool plan_dispatch_sources(const PushArgs &args, const Workspace &ws, bool quant
     if (most == 0) return false;
     plan.per_group = (total_tokens + kComputeUnits - 1) / kComputeUnits;
     const bool spread = plan.per_group > most;
+    // tokens of a workgroup when there are two per compute unit, the tables' one among them
+    uint32_t of_two = std::min(most, (total_tokens + 2 * kComputeUnits - 1) / (2 * kComputeUnits));
+    while (of_two < most && groups_of(of_two) >= 2 * kComputeUnits) ++of_two;
     if (spread) {
-        plan.per_group = most;
-        if (ws.topk * plan.units >= 8) {
-            plan.per_group = std::min(most, (total_tokens + 2 * kComputeUnits - 1) / (2 * kComputeUnits));
-            while (plan.per_group < most && groups_of(plan.per_group) >= 2 * kComputeUnits) ++plan.per_group;
-        }
+        plan.per_group = ws.topk * plan.units >= 8 ? of_two : most;
+        if (quantize && groups_of(plan.per_group) >= 2 * kComputeUnits)
+            plan.per_group = std::max(1u, std::min(most, kSourcesMaxUnits / 2 / plan.units));
+    } else if (ws.topk == 8 && plan.per_group > 4 && (!quantize || of_two <= 3)) {
+        plan.per_group = of_two;
     }
     plan.chunks = 0;
     groups = groups_of(plan.per_group);
@@ -2675,7 +2683,7 @@ bool plan_dispatch_sources(const PushArgs &args, const Workspace &ws, bool quant
         plan.chunks += (args.src[g].num_tokens * ws.topk + kSourcesChunk - 1) / kSourcesChunk;
     }
     if (senders == 1 && entries <= kSingleMaxEntries && pieces + kWave <= 1024) return false;
-    if (spread && (quantize ? groups >= 2 * kComputeUnits : entries * groups > kSourcesMaxVisits)) return false;
+    if (spread && (quantize ? groups >= 3 * kComputeUnits : entries * groups > kSourcesMaxVisits)) return false;
     if (entries > kSingleMaxEntries && pieces * 16 < kSourcesMinRow) return false;
     const uint32_t units = plan.per_group * plan.units;
     uint32_t movers = units;

@@ -162,6 +162,7 @@ SPREAD = {
     "bf16_14_kb_one_copy": ([1601, 31], 10, 1, 7168, BF16, None, "row", False),
     "fp8_scales_by_column": ([1201, 1198, 2], 12, 2, 7168, FP8, 56, "col", False),
     "fp8_scales_by_row_pad": ([1300, 3, 1300], 33, 3, 2944, FP8, 23, "row", False),
+    "bf16_eight_copies_of_one": ([1025, 0], 20, 8, 4096, BF16, None, "row", False),
     "f16_1500_workgroups": ([6001, 5999], 6, 1, 1024, F16, None, "row", False),
     "f16_2000_workgroups_the_two_launches": ([8001, 7999], 6, 1, 1024, F16, None, "row", True),
 }
@@ -184,7 +185,10 @@ SPREAD_QUANTISED = {
     "512_workgroups_and_the_tables": (replace(BASE, topk=4, hidden_dim=2048), [320] * 8, dict(repeats=True)),
     "two_short_copies": (replace(BASE, topk=2, hidden_dim=1024, expert_padding=16), [2049, 0, 0, 1, 300, 0, 0, 17], dict(stray=True)),
     "bounds": (replace(BASE, topk=3, hidden_dim=4096), [700, 800, 0, 5, 701, 0, 0, 9], dict(bounds=[699, 0, None, 5, None, None, None, 1])),
-    "beyond_two_a_compute_unit": (replace(BASE, topk=2, hidden_dim=1024), [4080, 0, 0, 1, 0, 0, 0, 17], dict(two_launches=True)),
+    "beyond_two_a_compute_unit": (replace(BASE, topk=2, hidden_dim=2048), [4080, 0, 0, 1, 0, 0, 0, 17], dict(stray=True)),
+    "beyond_three_a_compute_unit": (replace(BASE, topk=2, hidden_dim=2048), [6130, 0, 0, 1, 0, 0, 0, 17], dict(two_launches=True)),
+    "beyond_two_a_compute_unit_two_rounds": (replace(BASE, topk=3, hidden_dim=5120), [4000, 0, 0, 1, 90, 0, 0, 17], dict(repeats=True)),
+    "eight_copies_three_a_workgroup": (BASE, [1025, 0, 1, 0, 40, 0, 0, 434], dict(repeats=True)),
 }
 
 
