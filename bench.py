@@ -577,7 +577,7 @@ def split_calls(case, device, routings: int, steps: int, warmup: int, label: str
             seq_kernel("stage_recv_kernel", later, later_seq),
         ],
         "combine_send": [seq_kernel("combine_send_kernel", csend, csend_seq)],
-        "combine_recv": [kernel("combine_gather_kernel", us.get("combine_recv", []), lambda j: c_bytes)],
+        "combine_recv": [kernel("combine_staged_kernel", us.get("combine_recv", []), lambda j: c_bytes)],
     }
     one_rank_kernels = sum(k["avg_us"] for k in (kernels["dispatch_send"] + kernels["dispatch_recv"][:2]
                                                  + kernels["combine_send"] + kernels["combine_recv"]) if k)
