@@ -25,6 +25,14 @@ STEPS = [
     ([2900, 1], 16, 7, 3072, BF16, True),         # rows that are three quarters full: seven copies are enough
     ([3300, 1], 16, 6, 3072, BF16, False),        # six are not
     ([2900, 1], 18, 8, 3064, BF16, False),        # nor are eight of shorter ones
+    # steps of more than 16384 copies, which no single launch takes
+    ([2402, 1], 16, 7, 3568, BF16, True),         # 120.03 MB
+    ([2401, 1], 16, 7, 3568, BF16, False),        # 119.98 MB
+    ([1400, 1340], 32, 6, 4096, F32, True),       # 269 MB of 16 KB rows
+    ([1300, 1440], 32, 6, 4352, F32, True),       # rows longer than a workgroup has threads for
+    ([2799, 1], 16, 6, 5120, BF16, True),         # just enough
+    ([2799, 1], 16, 6, 5112, BF16, False),        # and one piece less
+    ([3300, 1], 12, 5, 8192, BF16, False),        # five copies a token
 ]
 
 
