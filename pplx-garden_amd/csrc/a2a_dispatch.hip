@@ -2771,7 +2771,8 @@ hipError_t launch_dispatch_resolve(const PushArgs &args, const FinalizeArgs &fin
                                    uint32_t total_tokens, bool streamed, hipStream_t stream, KernelTiming timing) {
     bool by_column = false;
     for (uint32_t r = 0; r < ws.world; ++r) by_column |= args.dst[r].out_x != nullptr && scales_by_column(args.dst[r]);
-    const uint32_t pieces = pieces_per_lane(ws.topk, quantize ? args.hidden_dim / 16 : args.row_bytes / 16, quantize, by_column);
+    const uint32_t pieces = pieces_per_lane(ws.topk, quantize ? args.hidden_dim / 16 : args.row_bytes / 16, quantize, by_column,
+                                            ws.experts_per_rank);
     uint32_t threads = push_threads(args, quantize, pieces);
     if (threads < ws.experts_per_rank) {   // a receiver workgroup has one thread per local expert
         threads = (ws.experts_per_rank + kWave - 1) / kWave * kWave;

@@ -133,7 +133,21 @@ inline bool copies_written_through(uint64_t copies, uint32_t row_bytes, uint32_t
 // wavefronts (3, 5, 6, 7, 14 of them, not 1, 4, 8 or 16), and for the shortest unquantised rows; not where scales go out by
 // column, which workgroups of fewer than 256 threads leave to the rows (fp8 rows of 2944 bytes 116.6 / 121.5, of 5120 level;
 // with K = 1 and 2 the pieces gain more than that: 158 / 136 and 150 / 138).
-inline uint32_t pieces_per_lane(uint32_t topk, uint32_t chunks, bool quantize, bool by_column) {
+// A workgroup has a thread per local expert in any case.  Where these are as many as pieces, several pieces a thread make no
+// wavefront fewer and the stores at device scope cost 1 to 4 %.  us per dispatch of 2 x 12 000 tokens, several pieces / one: 128
+// local experts, bf16 of 2 KB, K = 1, 2, 4 47.1 / 46.1, 57.0 / 55.4, 74.8 / 72.8; 256, bf16 of 1.3 KB 79.8 / 77.6, 92.7 / 89.6,
+// 111.1 / 107.0, fp8 of 4 KB, K = 1, 2 98.0 / 94.5, 119.7 / 118.5; 512, fp8 of 5 KB 217.6 / 210.5, 262.1 / 257.2, 309.6 / 315.5,
+// float of 8 KB, K = 1, 2 218.0 / 217.1, 264.7 / 266.9.  The last of the fp8 and of the float rows lie
+// beyond kLongCopies: with 16 KB of copies a token and more the stores at device scope are level or gain.  (Quantised rows, at
+// device scope either way: level.)
+// Rows of at most 64 pieces have one wavefront in any case too and gain by the stores: us per step, several pieces / one, K = 1,
+// 2, 3, bf16 of 1 KB 48.7 / 49.7, 43.3 / 44.2, 49.6 / 50.5, of 512 bytes 46.4 / 47.7, 39.1 / 39.9, 40.6 / 41.7; fp8 of 1 KB
+// 59.9 / 60.0, 57.8 / 57.9, 67.8 / 68.6.
+constexpr uint32_t kLongCopies = 1024;   // pieces of a token's copies
+
+inline uint32_t pieces_per_lane(uint32_t topk, uint32_t chunks, bool quantize, bool by_column, uint32_t experts_per_rank) {
+    const bool held = chunks > 64 && chunks <= (experts_per_rank + 63) / 64 * 64;
+    if (held && topk * chunks < kLongCopies) return 1;
     if (topk == 1) return 4;
     if (topk <= 3) return chunks > 1024 ? 4 : 2;
     if (topk > 4 || by_column) return 1;

@@ -31,6 +31,16 @@ MOVED = [
     (4, 5120, FP8, 40, "col", 1),            # scales by column in workgroups of their own
     (4, 5120, FP8, 40, "row", 2),
 ]
+# top-k, ranks, experts, elements of a row, type, scales, layout of the scales, pieces: receivers of as many experts as a row
+# has pieces, or a piece more
+HELD = [
+    (1, 3, 384, 1024, BF16, None, "row", 1),
+    (1, 3, 384, 1032, BF16, None, "row", 4),
+    (2, 3, 1000, 2688, FP8, 21, "col", 1),    # 168 pieces, 334 experts: by column in workgroups of their own
+    (3, 2, 640, 5120, FP8, 40, "row", 1),     # 320 of each
+    (4, 2, 512, 1536, BF16, None, "row", 1),
+    (4, 2, 640, 2560, BF16, None, "row", 2),  # 320 of each, long copies
+]
 # top-k, hidden size of quantised rows, pieces
 QUANTISED = [(1, 128, 4), (1, 4224, 4), (2, 2176, 2), (3, 7168, 2), (4, 5120, 2), (4, 4096, 1)]
 
@@ -47,6 +57,18 @@ def test_rows_moved_as_they_are(topk, hidden, dtype, scales, layout, pieces):
     print(f"topk={topk} hidden={hidden} {dtype} tokens={tokens}", flush=True)
     out = BF16 if dtype == FP8 else dtype
     cfg = RefConfig("pieces", 3, 1, max(tokens), 17, hidden, scales, topk, dtype, out, F32 if scales else None, expert_padding=4)
+    world = [make_ref_rank(cfg, r, t) for r, t in enumerate(tokens)]
+    rows = rows_for(cfg, world)
+    routes = []
+    check(cfg, world, rows, run_gpu(cfg, world, rows, DEV, split=False, scale_layout=layout, routes=routes))
+    assert routes == [True]
+
+
+@pytest.mark.parametrize("topk,ranks,experts,hidden,dtype,scales,layout,pieces", HELD, ids=[f"k{s[0]}_h{s[3]}" for s in HELD])
+def test_rows_beside_many_local_experts(topk, ranks, experts, hidden, dtype, scales, layout, pieces):
+    tokens = [16384 // topk - 300, 301, 1][:ranks]
+    print(f"topk={topk} experts={experts} hidden={hidden} {dtype} tokens={tokens}", flush=True)
+    cfg = RefConfig("held", ranks, 1, max(tokens), experts, hidden, scales, topk, dtype, BF16, F32 if scales else None)
     world = [make_ref_rank(cfg, r, t) for r, t in enumerate(tokens)]
     rows = rows_for(cfg, world)
     routes = []

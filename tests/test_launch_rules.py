@@ -7,7 +7,7 @@ from pathlib import Path
 
 import pytest
 
-from test_gpu_pieces import GATHERS, MOVED, QUANTISED
+from test_gpu_pieces import GATHERS, HELD, MOVED, QUANTISED
 from test_gpu_shapes import STREAMED, copies_of
 from test_gpu_split import PIECES
 from test_gpu_written_through import STEPS
@@ -25,7 +25,10 @@ int written_through(uint64_t copies, uint32_t row_bytes, uint32_t k) {
     return a2a::copies_written_through(copies, row_bytes, k);
 }
 uint32_t pieces(uint32_t k, uint32_t chunks, int quantize, int by_column) {
-    return a2a::pieces_per_lane(k, chunks, quantize != 0, by_column != 0);
+    return a2a::pieces_per_lane(k, chunks, quantize != 0, by_column != 0, 1);
+}
+uint32_t pieces_beside(uint32_t k, uint32_t chunks, uint32_t experts) {
+    return a2a::pieces_per_lane(k, chunks, false, false, experts);
 }
 int two_pieces(uint32_t k, uint64_t slabs) { return a2a::two_pieces_a_lane(k, slabs); }
 int one_launch(uint32_t rows, uint32_t row_bytes, uint32_t items, uint32_t threads) {
@@ -101,6 +104,18 @@ def test_pieces_of_a_thread(rules):
         assert rules.pieces(k, hidden * dtype.itemsize // 16, 0, layout == "col") == pieces, (k, hidden)
     for k, hidden, pieces in QUANTISED:
         assert rules.pieces(k, hidden // 16, 1, 0) == pieces, (k, hidden)
+
+
+def test_pieces_of_a_thread_where_the_local_experts_hold_the_workgroup(rules):
+    # as many threads for experts as pieces: no wavefront fewer with several pieces, so one, with the stores it had
+    assert [rules.pieces_beside(1, chunks, 128) for chunks in (64, 65, 128, 129)] == [4, 1, 1, 4]
+    assert [rules.pieces_beside(2, 128, experts) for experts in (8, 64, 65, 96, 128, 1024)] == [2, 2, 1, 1, 1, 1]
+    # unless a token's copies are long
+    assert [rules.pieces_beside(2, chunks, 512) for chunks in (511, 512)] == [1, 2]
+    assert [rules.pieces_beside(4, chunks, 512) for chunks in (192, 255, 320)] == [1, 1, 2]
+    for topk, ranks, experts, hidden, dtype, scales, layout, pieces in HELD:
+        chunks = hidden * dtype.itemsize // 16
+        assert rules.pieces_beside(topk, chunks, -(-experts // ranks)) == pieces, (topk, hidden)
 
 
 def test_pieces_of_the_gather(rules):
