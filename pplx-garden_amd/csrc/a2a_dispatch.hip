@@ -2638,10 +2638,8 @@ hipError_t launch_dispatch_single(const PushArgs &args, const FinalizeArgs &fin,
 // are two registers' loads a piece: beyond two workgroups a compute unit they are moved in two rounds instead of four, and up to
 // three workgroups a compute unit (K = 1, hidden 2048, 8 x 640 28.7 / 21.6; 4096, 731 workgroups 41.2 / 36.7; K = 2 49.0 / 46.7; 914
 // workgroups 57.3 / 58.9; 5120, 694 workgroups 39.7 / 37.2, 853 45.3 / 46.3).  Where 256 workgroups do hold a step, two a compute unit
-// lose up to 12 % or gain up to 10, by how the rows divide among the wavefronts; with eight copies of more than 1024 tokens they
-// gain (one a compute unit / two: bf16 of 8 KB, 8 x 160 38.8 / 35.6, 8 x 208 4.8 %, one source of 1100 34.9 / 31.3, of 1500 42.6 / 40.3;
-// fp8 of 7 KB, 8 x 160 49.0 / 46.3, 8 x 240 1.7 %; quantised of 7 KB, 8 x 160 50.3 / 47.9, but with four tokens a workgroup 8 x 192
-// 57.4 / 60.0, 8 x 256 2.1 % slower).
+// lose up to 12 % or gain up to 10, by how the rows divide among the wavefronts; with eight copies of more than 1024 tokens it is
+// two_workgroups_a_unit (a2a_rules.h) that says which.  (Six and seven copies have one; two have not been measured there.)
 bool plan_dispatch_sources(const PushArgs &args, const Workspace &ws, bool quantize, uint32_t total_tokens, SourcesPlan &plan,
                            uint32_t &groups, uint32_t &threads, uint32_t &rounds) {
     constexpr uint32_t kComputeUnits = 256;
@@ -2663,25 +2661,28 @@ bool plan_dispatch_sources(const PushArgs &args, const Workspace &ws, bool quant
     if (most == 0) return false;
     plan.per_group = (total_tokens + kComputeUnits - 1) / kComputeUnits;
     const bool spread = plan.per_group > most;
-    // tokens of a workgroup when there are two per compute unit, the tables' one among them
-    uint32_t of_two = std::min(most, (total_tokens + 2 * kComputeUnits - 1) / (2 * kComputeUnits));
-    while (of_two < most && groups_of(of_two) >= 2 * kComputeUnits) ++of_two;
-    if (spread) {
-        plan.per_group = ws.topk * plan.units >= 8 ? of_two : most;
-        if (quantize && groups_of(plan.per_group) >= 2 * kComputeUnits)
-            plan.per_group = std::max(1u, std::min(most, kSourcesMaxUnits / 2 / plan.units));
-    } else if (ws.topk == 8 && plan.per_group > 4 && (!quantize || of_two <= 3)) {
-        plan.per_group = of_two;
-    }
-    plan.chunks = 0;
-    groups = groups_of(plan.per_group);
     uint32_t senders = 0;
+    plan.chunks = 0;
     for (uint32_t g = 0; g < ws.num_groups; ++g) {
         if (args.src[g].num_tokens == 0) continue;
         if (args.src[g].indices_stride != ws.topk) return false;
         ++senders;
         plan.chunks += (args.src[g].num_tokens * ws.topk + kSourcesChunk - 1) / kSourcesChunk;
     }
+    if (spread || (ws.topk == 8 && plan.per_group > 4)) {
+        // tokens of a workgroup when there are two per compute unit, the tables' one among them
+        uint32_t of_two = std::min(most, (total_tokens + 2 * kComputeUnits - 1) / (2 * kComputeUnits));
+        while (of_two < most && groups_of(of_two) >= 2 * kComputeUnits) ++of_two;
+        if (spread) {
+            plan.per_group = ws.topk * plan.units >= 8 ? of_two : most;
+            if (quantize && groups_of(plan.per_group) >= 2 * kComputeUnits)
+                plan.per_group = std::max(1u, std::min(most, kSourcesMaxUnits / 2 / plan.units));
+        } else if (two_workgroups_a_unit(quantize, args.hidden_dim_scale != 0, plan.per_group, of_two, plan.units,
+                                         ws.experts_per_rank, senders)) {
+            plan.per_group = of_two;
+        }
+    }
+    groups = groups_of(plan.per_group);
     if (senders == 1 && entries <= kSingleMaxEntries && pieces + kWave <= 1024) return false;
     if (spread && (quantize ? groups >= 3 * kComputeUnits : entries * groups > kSourcesMaxVisits)) return false;
     if (entries > kSingleMaxEntries && pieces * 16 < kSourcesMinRow) return false;

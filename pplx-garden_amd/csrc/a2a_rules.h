@@ -156,6 +156,35 @@ inline uint32_t pieces_per_lane(uint32_t topk, uint32_t chunks, bool quantize, b
     return !fills || (!quantize && waves == 2) ? 2 : 1;
 }
 
+// Whether a step of eight copies a token that the one launch of several sources can hold with a workgroup per compute unit, of
+// `one` > 4 tokens each, has two per compute unit instead, of `two` tokens.  With up to 32 routes a workgroup's resolver has two
+// lanes a route, with up to 64 one, and what a route waits for last is the sum over the earlier experts of its receiver, four of
+// them a lane and the others one after another.  So two workgroups gain the more the more experts a receiver has, and while
+// `two` <= 4.  Against that stand the tables that more workgroups count, and quantised rows, which want their tokens spread
+// evenly: six on a compute unit with two workgroups of three where one has five.  us per step, one / two:
+//   quantised 4 KB, E experts   8 x 130  E = 64 27.6 / 28.2, 256 28.7 / 26.6;  4 x 290  E = 64 29.9 / 29.5;
+//                               16 x 65  E = 64 27.8 / 28.5, 256 28.4 / 28.4;  8 x 159  E = 64 31.0 / 31.5, 256 32.0 / 29.8
+//             3 KB              8 x 130  E = 64 22.6 / 23.2, 256 23.7 / 22.0;  one source of 1400, E = 64 27.1 / 26.4
+//             5 KB              8 x 145  E = 64 34.6 / 35.1, 256 35.6 / 33.0;  8 x 180, E = 128 41.0 / 39.4
+//             2 KB, 6 KB, 7 KB  8 x 160  E = 64 20.5 / 20.3, 42.5 / 41.8, 48.6 / 46.8;  four tokens a workgroup, 7 KB 58.1 / 59.0
+//   bf16 2 KB, 4 KB, 7 KB, 8 KB 8 x 160  E = 64 15.7 / 14.2, 22.0 / 20.5, 33.8 / 31.6, 37.8 / 35.1
+//   fp8  2 KB, 5 KB, 7 KB       8 x 160  E = 64 19.8 / 18.4, 36.1 / 34.1, 47.0 / 46.3
+// (The few that lose all the same: uneven loads with few experts a receiver, one / two for 460, 0, 153, 1, ... tokens, E = 64, 3 KB
+// 25.4 / 25.1, 4 KB 30.7 / 30.4.)
+// Four tokens of four units each are two rounds of eight wavefronts, too few to count for many sources: bf16 of 4 KB, 8 x 220
+// 28.9 / 28.1, 16 x 110 28.3 / 28.8.  2048 tokens are more than two workgroups of four on each compute unit, and with five routes
+// have a lane each: short rows lose (8 x 256: bf16 of 2 KB 19.6 / 20.5, of 3 KB 25.4 / 25.8, 4 KB level, 5 KB 38.2 / 37.4, 7 KB
+// 50.0 / 49.7; fp8 of 2 KB 26.7 / 27.4; but 16 x 128, E = 384, bf16 of 2 KB 22.6 / 21.2, fp8 29.2 / 28.4), and with scales longer
+// ones whose receivers have few experts (fp8 of 4 KB, 8 x 256, E = 64 44.8 / 45.1, 256 46.2 / 45.6, 2 x 1024, E = 64 47.8 / 46.8;
+// 5 KB 53.4 / 54.2, 54.8 / 53.8, 53.9 / 52.8; 6 KB 60.7 / 61.4, 62.4 / 61.6, 62.6 / 61.9).
+inline bool two_workgroups_a_unit(bool quantize, bool scaled, uint32_t one, uint32_t two, uint32_t units, uint32_t experts_per_rank,
+                                  uint32_t senders) {
+    if (quantize) return two <= 3 && (one > 5 || experts_per_rank > 8 || units < 3 || units > 5);
+    if (two <= 4) return two * units != 16 || senders <= 8;
+    if (units < 4) return senders > 8 && experts_per_rank > 16;
+    return !scaled || units > 5 || experts_per_rank > 16;
+}
+
 // copies_past_cache for the recvs of the split calls, from kStreamReceived bytes of copies in all of a step's recvs on.  What this
 // keeps in the cache are the STAGED rows, which the recvs of all the ranks a token was routed to read, and the copies of the
 // first recvs are gone anyway by the time the last one has run.  Whole steps, us, copies kept / past the cache, with a

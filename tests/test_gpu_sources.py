@@ -197,3 +197,44 @@ def test_more_workgroups_than_compute_units_quantised(name):
     case, tokens, how = SPREAD_QUANTISED[name]
     print(f"{name} tokens={tokens}", flush=True)
     run_and_check(replace(case, name=name, num_tokens=max(tokens), seed=47_000), tokens, **how)
+
+
+# Steps of eight copies on both sides of the line between one workgroup a compute unit and two: tokens of a workgroup
+ONE_OR_TWO = {
+    "five_few_experts": (replace(BASE, num_experts=64, hidden_dim=4096), [131] + [130] * 7, dict(repeats=True)),
+    "three_many_experts": (replace(BASE, num_experts=251, hidden_dim=4096, expert_padding=16), [131] + [130] * 7, dict(repeats=True)),
+    "three_few_experts": (replace(BASE, num_experts=64, hidden_dim=3072), [171] + [170] * 7, dict(stray=True)),
+    "seven": (replace(BASE, num_experts=256, hidden_dim=2048), [1, 700, 0, 193, 0, 0, 700, 0], dict(repeats=True)),
+}
+
+
+@pytest.mark.parametrize("name", ONE_OR_TWO)
+def test_one_or_two_workgroups_a_compute_unit(name):
+    case, tokens, how = ONE_OR_TWO[name]
+    print(f"{name} tokens={tokens}", flush=True)
+    run_and_check(replace(case, name=name, num_tokens=max(tokens), seed=51_000), tokens, **how)
+
+
+# The same of rows moved as they are: ranks' tokens, experts, elements, type, scales
+ONE_OR_TWO_MOVED = {
+    "eight_2_kb": ([256] * 8, 64, 1024, BF16, None),
+    "five_5_kb": ([256] * 8, 64, 2560, BF16, None),
+    "eight_5_kb_scales": ([255] * 7 + [254], 64, 5120, FP8, 40),
+    "five_5_kb_scales_many_experts": ([256] * 8, 256, 5120, FP8, 40),
+    "five_2_kb_of_sixteen_many_experts": ([128] * 16, 384, 1024, BF16, None),
+    "five_6_kb_scales": ([2047, 1], 48, 6144, FP8, 48),
+    "seven_4_kb_of_sixteen": ([113] + [110] * 15, 128, 2048, BF16, None),
+    "four_4_kb_of_eight": ([223] + [220] * 7, 128, 2048, BF16, None),
+}
+
+
+@pytest.mark.parametrize("name", ONE_OR_TWO_MOVED)
+def test_one_or_two_workgroups_a_compute_unit_of_rows_as_they_are(name):
+    tokens, experts, hidden, dtype, scales = ONE_OR_TWO_MOVED[name]
+    print(f"{name} tokens={tokens}", flush=True)
+    cfg = RefConfig(name, len(tokens), 1, max(tokens), experts, hidden, scales, 8, dtype, BF16, F32 if scales else None)
+    world = [make_ref_rank(cfg, r, t) for r, t in enumerate(tokens)]
+    rows = rows_for(cfg, world)
+    routes = []
+    check(cfg, world, rows, run_gpu(cfg, world, rows, DEV, split=False, routes=routes))
+    assert routes == [False]

@@ -30,6 +30,9 @@ uint32_t pieces(uint32_t k, uint32_t chunks, int quantize, int by_column) {
 uint32_t pieces_beside(uint32_t k, uint32_t chunks, uint32_t experts) {
     return a2a::pieces_per_lane(k, chunks, false, false, experts);
 }
+int two_workgroups(int quantize, int scaled, uint32_t one, uint32_t two, uint32_t units, uint32_t experts, uint32_t senders) {
+    return a2a::two_workgroups_a_unit(quantize != 0, scaled != 0, one, two, units, experts, senders);
+}
 int two_pieces(uint32_t k, uint64_t slabs) { return a2a::two_pieces_a_lane(k, slabs); }
 int one_launch(uint32_t rows, uint32_t row_bytes, uint32_t items, uint32_t threads) {
     return a2a::first_recv_in_one_launch(rows, row_bytes, items, threads);
@@ -116,6 +119,22 @@ def test_pieces_of_a_thread_where_the_local_experts_hold_the_workgroup(rules):
     for topk, ranks, experts, hidden, dtype, scales, layout, pieces in HELD:
         chunks = hidden * dtype.itemsize // 16
         assert rules.pieces_beside(topk, chunks, -(-experts // ranks)) == pieces, (topk, hidden)
+
+
+def test_two_workgroups_a_compute_unit_where_they_gain(rules):
+    # quantised rows, five tokens a workgroup or three: receivers of many experts, or rows of few or many units
+    assert [rules.two_workgroups(1, 1, 5, 3, 4, le, 8) for le in (4, 8, 9, 32)] == [0, 0, 1, 1]
+    assert [rules.two_workgroups(1, 1, 5, 3, units, 8, 8) for units in range(1, 9)] == [1, 1, 0, 0, 0, 1, 1, 1]
+    # six on a compute unit either way; never four
+    assert rules.two_workgroups(1, 1, 6, 3, 4, 8, 8) and not rules.two_workgroups(1, 1, 6, 4, 2, 32, 8)
+    # rows as they are: always with up to four tokens, but for two rounds of eight wavefronts and many sources
+    assert all(rules.two_workgroups(0, 0, one, two, units, 8, 16) for one, two in ((5, 3), (6, 3), (7, 4)) for units in (1, 2, 3, 5, 7))
+    assert [rules.two_workgroups(0, 0, 7, 4, 4, 8, senders) for senders in (1, 8, 9, 16)] == [1, 1, 0, 0]
+    # with five, which have a lane a route, only rows of 4 KB and more, of 6 KB where they have scales and few experts
+    assert [rules.two_workgroups(0, 0, 8, 5, units, 8, 8) for units in range(1, 8)] == [0, 0, 0, 1, 1, 1, 1]
+    assert [rules.two_workgroups(0, 1, 8, 5, units, 8, 8) for units in range(1, 8)] == [0, 0, 0, 0, 0, 1, 1]
+    assert [rules.two_workgroups(0, 1, 8, 5, units, 17, 8) for units in range(1, 8)] == [0, 0, 0, 1, 1, 1, 1]
+    assert [rules.two_workgroups(0, 1, 8, 5, 2, 24, senders) for senders in (8, 9, 16)] == [0, 1, 1]
 
 
 def test_pieces_of_the_gather(rules):
