@@ -324,7 +324,7 @@ bool fused_routing_pays(const FinalizeArgs &fa, uint32_t world, uint32_t total_b
 }
 
 // Dimensions of the device workspace for steps of at most `max_tokens` tokens per
-// rank, and its tables carved out of `base` (256-byte aligned each).  With a null
+// rank, and its tables carved out of `base` (at multiples of kTableUnit each).  With a null
 // `base` only the dimensions are filled in.  Returns the bytes the tables take.
 size_t carve_workspace(const a2a_config &c, uint32_t max_tokens, uint8_t *base, Workspace &ws) {
     const uint32_t N = c.world_size, E = c.num_experts, K = c.num_experts_per_token;
@@ -343,7 +343,7 @@ size_t carve_workspace(const a2a_config &c, uint32_t max_tokens, uint8_t *base, 
     size_t off = 0;
     auto carve = [&off](size_t bytes) {
         const size_t at = off;
-        off = align_up(off + bytes, 256);
+        off = align_up(off + bytes, kTableUnit * sizeof(uint32_t));
         return at;
     };
     const size_t o_local = carve((size_t)N * ws.max_tk * sizeof(uint16_t));

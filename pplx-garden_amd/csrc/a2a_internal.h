@@ -5,6 +5,7 @@
 
 #include <hip/hip_runtime.h>
 #include <hip/hip_ext.h>
+#include <stddef.h>
 #include <stdint.h>
 
 #include "a2a.h"
@@ -17,6 +18,11 @@ constexpr int kWave = 64;
 constexpr int kRouteBlock = 1024;
 constexpr uint32_t kInvalidSlot = 0xFFFFFFFFu;
 constexpr int kMaxWorld = A2A_MAX_WORLD_SIZE;
+constexpr uint32_t kTableUnit = 64;   // words: the workspace's tables begin at multiples of it
+
+// Fields of packed words: whether values up to `most` fit `bits`, and whether this one does.
+constexpr bool holds(uint32_t bits, uint64_t most) { return most < (1ull << bits); }
+inline bool fits_field(ptrdiff_t value, uint32_t bits) { return value >= 0 && holds(bits, (uint64_t)value); }
 
 // Device workspace, shared by all logical ranks of a context.  Per-rank arrays
 // are laid out [world][...] with the strides below.
@@ -211,6 +217,7 @@ struct CombineSoleArgs {
     __device__ __forceinline__ bool accumulate() const { return sizes >> 29 != 0; }
 };
 static_assert(sizeof(CombineSoleArgs) <= kShortArguments, "");
+static_assert(holds(11, A2A_MAX_EXPERTS) && holds(7, A2A_MAX_EXPERTS_PER_TOKEN), "sizes");
 
 // Events a caller wants recorded when a kernel itself begins and ends (both
 // null: an ordinary launch).

@@ -56,8 +56,6 @@ struct StageSendArgs {
     uint32_t resolver_wave;   // resolving send: wavefront that resolves the routes (set by the launcher)
 };
 
-constexpr uint32_t kTableUnit = 64;   // words: the workspace's tables begin at multiples of it
-
 // What stage_send_quick_kernel needs (kShortArguments); buffers and tables are those of the sender's dp group.
 struct SendQuickArgs {
     const uint8_t *x;
@@ -84,6 +82,9 @@ struct SendQuickArgs {
     __device__ __forceinline__ uint32_t *flags() const { return num_routed + (distances >> 10); }
 };
 static_assert(sizeof(SendQuickArgs) <= kShortArguments, "");
+static_assert(holds(10, 1024 - kWave) && holds(11, A2A_MAX_EXPERTS) && holds(11, A2A_MAX_EXPERTS_PER_TOKEN), "sizes");
+constexpr uint32_t kSenderTable = (A2A_MAX_WORLD_SIZE * A2A_MAX_EXPERTS + kTableUnit - 1) / kTableUnit;   // of the largest, in kTableUnit
+static_assert(holds(10, kSenderTable) && holds(22, 3ull * kSenderTable * kTableUnit), "distances");
 
 // A grid of wavefronts over the pieces (128 sixteen-byte chunks) of a receiver's rows.
 struct PieceGrid {
@@ -138,6 +139,9 @@ struct RecvRowsArgs {
     __device__ __forceinline__ uint32_t *flags() const { return counts - to_flags; }
 };
 static_assert(sizeof(RecvRowsArgs) <= kShortArguments, "");
+// (the last receiver's first expert may lie up to a receiver's share behind the last one)
+static_assert(holds(11, A2A_MAX_EXPERTS) && holds(5, (A2A_MAX_EXPERTS + kTableUnit - 1) / kTableUnit) &&
+              holds(16, kTableUnit + A2A_MAX_EXPERTS + A2A_MAX_WORLD_SIZE), "num_local, to_first_rows, to_flags");
 
 struct CombineSendArgs {
     const uint8_t *y;

@@ -1994,7 +1994,10 @@ hipError_t launch_stage_send_small(const StageSendArgs &args, const Workspace &w
         q.num_tokens = args.src.num_tokens;
         q.num_scales = args.hidden_dim_scale;
         q.sizes = pieces | ws.num_experts << 10 | ws.topk << 21;
-        q.distances = (uint32_t)(ws.expert_offsets - ws.num_routed) / kTableUnit | (uint32_t)(ws.err - q.num_routed) << 10;
+        const ptrdiff_t to_offsets = ws.expert_offsets - ws.num_routed, to_flags = ws.err - q.num_routed;
+        if (to_offsets % kTableUnit != 0 || !fits_field(to_offsets / kTableUnit, 10) || !fits_field(to_flags, 22))
+            return hipErrorInvalidValue;
+        q.distances = (uint32_t)to_offsets / kTableUnit | (uint32_t)to_flags << 10;
 #define A2A_LAUNCH_SEND_QUICK(NB)                                                                                    \
     do {                                                                                                             \
         if (quantize)                                                                                                \
@@ -2193,8 +2196,11 @@ hipError_t launch_stage_recv(const StageRecvArgs &args, const Workspace &ws, con
     m.step_rows = grid.step_rows;
     m.step_pieces = grid.step_pieces;
     m.num_local = first >= ws.num_experts ? 0 : std::min(ws.num_experts - first, ws.experts_per_rank);
-    m.to_first_rows = (uint32_t)(ws.padded_offset - ws.tokens_per_expert) / kTableUnit;
-    m.to_flags = (uint32_t)(m.counts - ws.err);
+    const ptrdiff_t to_first_rows = ws.padded_offset - ws.tokens_per_expert, to_flags = m.counts - ws.err;
+    if (to_first_rows % kTableUnit != 0 || !fits_field(to_first_rows / kTableUnit, 5) || !fits_field(to_flags, 16))
+        return hipErrorInvalidValue;
+    m.to_first_rows = (uint32_t)to_first_rows / kTableUnit;
+    m.to_flags = (uint32_t)to_flags;
     // Scales by column: a wavefront for every kScaleColumns columns of 64 rows that the receiver typically gets.
     const bool columns = args.dst.out_x != nullptr && scales_by_column(args.dst) &&
                          (uint64_t)typical * args.hidden_dim_scale >= kColumnWords;

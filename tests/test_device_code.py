@@ -54,3 +54,20 @@ def test_kernels_of_short_arguments_take_no_hidden_ones():
             found.add(kind)
             assert not re.search(r"\b(blockDim|gridDim)\b", body), kind
     assert found == short
+
+
+@pytest.mark.skipif(not Path(HIPCC).exists(), reason="needs hipcc")
+@pytest.mark.parametrize("limit,largest,refused", [("EXPERTS", 1984, None), ("EXPERTS", 2048, "to_first_rows"),
+                                                   ("WORLD_SIZE", 64, "distances"), ("EXPERTS_PER_TOKEN", 128, "sizes")])
+def test_limits_that_packed_words_do_not_hold_are_refused(tmp_path, limit, largest, refused):
+    """The kernels of short arguments get sizes and distances in a few bits each: a larger limit has to end the build."""
+    header = (ROOT.parent / "include" / "a2a.h").read_text()
+    changed, count = re.subn(rf"(#define A2A_MAX_{limit}) \d+", rf"\1 {largest}", header)
+    assert count == 1
+    (tmp_path / "a2a.h").write_text(changed)
+    source = tmp_path / "limits.hip"
+    source.write_text('#include "a2a_staged.h"\n')
+    cmd = [HIPCC, "--offload-arch=gfx950", "-std=c++17", "-fsyntax-only", "-I", str(tmp_path), "-I", str(ROOT / "csrc"), str(source)]
+    result = subprocess.run(cmd, capture_output=True, text=True)
+    assert (result.returncode == 0) == (refused is None), result.stderr
+    assert refused is None or refused in result.stderr
