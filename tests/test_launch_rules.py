@@ -93,6 +93,7 @@ def test_rows_that_leave_much_of_their_last_4_kb_empty_are_not_written_through(r
 def test_the_gpu_tests_of_written_through_steps_lie_on_the_side_they_are_meant_for(rules, tokens, experts, topk, hidden, dtype,
                                                                                    through):
     row = hidden * dtype.itemsize
+    assert sum(tokens) * topk > 16384 and not rules.past_cache(sum(tokens) * topk * row, 0, topk)
     assert bool(rules.written_through(sum(tokens) * topk * row, row, topk)) == through
 
 
