@@ -29,6 +29,7 @@ GIVEN = [
     ([1300, 2500, 1], 1024, 6, 4096, 32),     # more experts than threads; a span that ends in its first chunk of entries
     ([16384, 16385, 3], 6, 1, 4096, 4),       # a copy a token: by column beside the rows
     ([2048, 2049, 3], 16, 8, 4096, 4),        # whole spans, and a token more; a single slice of columns
+    ([3277, 2048, 3], 16, 5, 4096, 4),        # a last span of one entry
 ]
 
 
