@@ -91,7 +91,7 @@ STREAMED = [
     (torch.float8_e4m3fn, 1152, 9, 8, (33000, 1900), True),   # 322 MB, 80 MB
     (torch.bfloat16, 1000, 0, 9, (17000, 1000), True),        # 324 MB, 36 MB: two groups of rows a token
     (torch.float32, 1004, 0, 40, (2000, 0), True),            # 321 MB, 8 MB: one sender, few enough tokens for its own gather
-    (torch.bfloat16, 1000, 0, 2, (80000, 2100), False),       # 328 MB of copies that stay ordinary, 164 MB
+    (torch.bfloat16, 1000, 0, 2, (80000, 2100), False),       # 328 MB of copies that do not (two pieces a thread), 164 MB
     (torch.bfloat16, 1000, 0, 5, (29000, 2000), False),       # 310 MB, 62 MB
 ]
 
@@ -100,12 +100,31 @@ def copies_of(row, hidden, k, tokens):
     return sum(tokens) * k * hidden * row.itemsize
 
 
+# The same of quantised rows, of which a thread moves several pieces: hidden, experts per token, tokens, pieces
+STREAMED_QUANTISED = [
+    (4224, 1, (70000, 6000), 4),      # 321 MB: 264 pieces of a row, the last of four rounds nearly empty
+    (7296, 2, (20000, 2100), 2),      # 322 MB: 456
+    (2176, 3, (45000, 4100), 2),      # 321 MB: 136
+    (4224, 4, (17000, 2000), 2),      # 321 MB: five wavefronts with a piece a thread, three here
+]
+
+
 @pytest.mark.parametrize("row,hidden,scales,k,tokens,streamed", STREAMED,
                          ids=lambda v: str(v).replace("torch.", "") if isinstance(v, torch.dtype) else None)
 def test_streamed_copies_and_tokens(row, hidden, scales, k, tokens, streamed):
+    group_and_split_calls_agree(row, hidden, scales, k, tokens)
+
+
+@pytest.mark.parametrize("hidden,k,tokens,pieces", STREAMED_QUANTISED)
+def test_streamed_quantised_rows(hidden, k, tokens, pieces):
+    group_and_split_calls_agree(torch.float8_e4m3fn, hidden, hidden // 128, k, tokens, quantise=True)
+
+
+def group_and_split_calls_agree(row, hidden, scales, k, tokens, quantise=False):
     from pplx_garden_amd.distributed.loopback import LoopbackWorld
     from pplx_garden_amd.kernels.p2p_all_to_all import P2PAllToAll
 
+    print(f"{row} hidden={hidden} k={k} tokens={tokens} quantise={quantise}", flush=True)
     device, N, E = torch.device("cuda:0"), 3, max(24, k + 2)
     out = torch.bfloat16 if scales else row
     world = LoopbackWorld(N, device=device)
@@ -119,8 +138,8 @@ def test_streamed_copies_and_tokens(row, hidden, scales, k, tokens, streamed):
     data = []
     for t in counts:
         data.append(dict(
-            dp_x=torch.randn((t, hidden), generator=gen, device=device).to(row),
-            dp_x_scale=torch.rand((t, scales), generator=gen, device=device) if scales else None,
+            dp_x=torch.randn((t, hidden), generator=gen, device=device).to(torch.bfloat16 if quantise else row),
+            dp_x_scale=torch.rand((t, scales), generator=gen, device=device) if scales and not quantise else None,
             indices=torch.rand((t, E), generator=gen, device=device).topk(k).indices.to(torch.int32).view(torch.uint32),
             weights=torch.rand((t, k), generator=gen, device=device)))
     expert_y = [torch.randn((rows, hidden), generator=gen, device=device).to(out) for _ in range(N)]

@@ -8,7 +8,7 @@ from pathlib import Path
 import pytest
 
 from test_gpu_pieces import GATHERS, HELD, MOVED, QUANTISED
-from test_gpu_shapes import STREAMED, copies_of
+from test_gpu_shapes import STREAMED, STREAMED_QUANTISED, copies_of
 from test_gpu_split import PIECES
 from test_gpu_written_through import STEPS
 
@@ -77,6 +77,12 @@ def test_copies_that_the_infinity_cache_can_hold_stay_there_for_their_reader(rul
 @pytest.mark.parametrize("row,hidden,scales,k,tokens,streamed", STREAMED)
 def test_the_gpu_tests_of_streamed_steps_lie_on_the_side_they_are_meant_for(rules, row, hidden, scales, k, tokens, streamed):
     assert bool(rules.past_cache(copies_of(row, hidden, k, tokens), 0, k)) == streamed
+
+
+def test_the_gpu_tests_of_streamed_quantised_rows_are_streamed_and_move_the_pieces_they_are_meant_for(rules):
+    for hidden, k, tokens, pieces in STREAMED_QUANTISED:
+        assert rules.past_cache(sum(tokens) * k * hidden, 1, k), (hidden, k)
+        assert rules.pieces(k, hidden // 16, 1, 0) == pieces, (hidden, k)
 
 
 def test_rows_that_leave_much_of_their_last_4_kb_empty_are_not_written_through(rules):
