@@ -2606,20 +2606,22 @@ hipError_t launch_dispatch_single(const PushArgs &args, const FinalizeArgs &fin,
     return hipGetLastError();
 }
 
-// Whether a step takes dispatch_sources_kernel, and its shape: tokens of a workgroup as in the kernels of one source
-// (about one workgroup per compute unit) as long as a workgroup can hold them, and otherwise, or where that is better, with about
-// two workgroups per compute unit (the tables' one among them: with 513 the last one starts when another has ended), or as
-// many as there are when each holds what it can; beside the resolver as many wavefronts as there are units to move or chunks
-// to count (8 x 32 tokens of hidden 2048, 2 units and 8 chunks: 6.6 us with 4 wavefronts, 4.6 with 8), in as few rounds
-// as 15 of them need.  The line at 16384 entries is the resolver's: with more than eight tokens of top-8 a workgroup has
-// more routes than its one resolving wavefront has lanes.  It is not the counting's, which costs every workgroup 0.16 us
-// per 1024 entries where the routing launch it replaces costs 5 to 6 us: level near 32 000 by these figures.  Larger steps
-// with two resolving wavefronts have not been measured.  Above 8192 entries rows of 2 KB, because with smaller ones the
-// counting is what is left (one source of 2048 tokens, hidden 1024: 21.5 us a step against 20.4; hidden 2048 and 1500
-// tokens: 23.2 against 23.9).  Steps of one source with up to kSingleMaxEntries entries have the two kernels that are made
-// for them (128 tokens 4.54 us against 4.77 here, 1024 tokens 15.4 against 16.1) unless a row's pieces leave these no
-// wavefront beside them: float rows of 16 KB and more, K = 8, us per step before / here: 4 tokens 9.6 / 8.5, 128 14.2 / 11.3, 400
-// 27.9 / 23.8; of 28 KB 10.8 / 10.0, 20.7 / 15.7, 48.5 / 41.0.
+// Whether a step takes dispatch_sources_kernel, and its shape: tokens of a workgroup as in the kernels of one source (about one
+// workgroup per compute unit) as long as a workgroup can hold them, and otherwise, or where that is better, with about two
+// workgroups per compute unit (the tables' one among them: with 513 the last one starts when another has ended), or as many as
+// there are when each holds what it can; beside the resolver as many wavefronts as there are units to move or chunks to count
+// (8 x 32 tokens of hidden 2048, 2 units and 8 chunks: 6.6 us with 4 wavefronts, 4.6 with 8), in as few rounds as 15 of them
+// need.  The line at 16384 entries: with a workgroup per compute unit it was the resolver's, whose wavefront has a lane for
+// each route of eight tokens of top-8.  It is none now that steps spread over more workgroups, nor the counting's, which costs
+// every workgroup 0.16 us per 1024 entries where the routing launch it replaces costs 5 to 6 us: up to 24576 entries and 511
+// workgroups one launch still gains (us per step, two launches / one, 8 x 420 fp8 of 7 KB, K = 6 102.8 / 88.3, 8 x 300 bf16 of
+// 8 KB, K = 8 70.5 / 66.3, quantised of 7 KB 90.0 / 88.4), and loses from some 25 600 on (scales by column 1.6 %) or with more
+// workgroups (572: 4.5 %).  It stands where it does because steps just above it are what the two launches' edge cases are
+// tested with.  Above 8192 entries rows of 2 KB, because with smaller ones the counting is what is left (one source of 2048
+// tokens, hidden 1024: 21.5 us a step against 20.4; hidden 2048 and 1500 tokens: 23.2 against 23.9).  Steps of one source with
+// up to kSingleMaxEntries entries have the two kernels that are made for them (128 tokens 4.54 us against 4.77 here, 1024
+// tokens 15.4 against 16.1) unless a row's pieces leave these no wavefront beside them: float rows of 16 KB and more, K = 8, us
+// per step before / here: 4 tokens 9.6 / 8.5, 128 14.2 / 11.3, 400 27.9 / 23.8; of 28 KB 10.8 / 10.0, 20.7 / 15.7, 48.5 / 41.0.
 // Steps of more tokens than 256 workgroups hold, us per step in two launches (or, below 3 * 2^19 visits, with the general
 // kernel) / here:
 //                      K = 1               K = 2               K = 4               K = 8
@@ -2633,6 +2635,9 @@ hipError_t launch_dispatch_single(const PushArgs &args, const FinalizeArgs &fin,
 //       28 KB  8 x 109   46.4 /  24.0        54.0 /  32.2        60.2 /  44.2        94.3 /  82.9
 //   fp8  7 KB  8 x 400   37.6 /  30.3        49.5 /  40.7        69.8 /  62.6
 //   quantised  8 x 300   34.7 /  31.4        43.5 /  39.0        59.3 /  52.1
+// and K = 3, 5, 6, 7: bf16 of 8 KB, 8 x 240 34.4 / 24.9, 42.7 / 34.8, 48.7 / 40.5, 54.0 / 46.5; quantised of 7 KB, 8 x 292 53.1 / 44.9,
+// 65.2 / 58.6, 73.4 / 67.4, 82.9 / 78.5.  Rows of less than 2 KB (up to 8192 entries): 8 x 1000, K = 1, bf16 of 256 bytes 18.3 / 18.1, of
+// 1 KB 21.9 / 19.9, of 1.5 KB 30.1 / 18.4, fp8 of 1 KB 26.7 / 21.9; 8 x 500, K = 2, bf16 of 1 KB 16.2 / 13.1, quantised 21.5 / 16.2.
 // What ends it is the counting, every entry by every workgroup: 1143 workgroups x 16 000 entries (bf16 8 KB, K = 2) 81.3 / 79.6,
 // 2000 x 16 000 (14 KB) 133.2 / 134.8, 1800 x 14 400 (fp8, K = 1) 116.4 / 119.3, 2057 x 14 400 (2 KB) 36.0 / 42.4.  Quantised rows
 // are two registers' loads a piece: beyond two workgroups a compute unit they are moved in two rounds instead of four, and up to

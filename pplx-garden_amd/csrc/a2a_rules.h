@@ -129,6 +129,9 @@ inline bool copies_written_through(uint64_t copies, uint32_t row_bytes, uint32_t
 // and with a sweep between dispatch and combine that reads the received rows, before / as it is: K = 1, bf16 rows of 14 KB
 // 535 / 385, quantised of 7 KB 372 / 316; K = 2, bf16 of 5.9 KB 169 / 144, fp8 of 7 KB 243 / 215; K = 4, fp8 of 5 KB
 // 125.5 / 120.7, bf16 of 14 KB 253 / 236.  (K = 2 with rows of 28 KB: two pieces 461, four 438.)
+// K = 3, 8 x 2000 tokens, before / as it is: bf16 of 2 KB 60.9 / 56.5, 5.9 KB 168 / 143, 14 KB 374 / 323; f32 of 16 KB 403 / 377; fp8 of
+// 5 KB 204 / 182; quantised of 4 KB 158.2 / 156.6, 7 KB 279 / 257.  Copies that go past the Infinity Cache: quantised of 7 KB,
+// 16 x 4096, K = 1 810 / 594, 8 x 3000, K = 3 413 / 380; fp8 of 5 KB, 8 x 4096, K = 3 406 / 342; bf16 of 5.9 KB, 8 x 4096, K = 4 396 / 358.
 // Four copies a token: two pieces where a piece a thread makes workgroups that do not fill a compute unit's 32 places for
 // wavefronts (3, 5, 6, 7, 14 of them, not 1, 4, 8 or 16), and for the shortest unquantised rows; not where scales go out by
 // column, which workgroups of fewer than 256 threads leave to the rows (fp8 rows of 2944 bytes 116.6 / 121.5, of 5120 level;
