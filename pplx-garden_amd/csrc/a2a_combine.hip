@@ -408,7 +408,8 @@ __global__ __launch_bounds__(kWave) void combine_staged_kernel(const CombineStag
 
 // The combine of a small step with one sender, whose launch is what it costs: the words of kShortArguments instead of every
 // rank's descriptors.  A receiver's rows are found by their distance from the first receiver's, which lane r holds for receiver r.
-// Steps of 128 tokens, host's pace: hidden 7168 10.5 -> 9.8 us, 2048 10.6 -> 9.9; other steps of one sender (bounds, strided rows,
+// Steps of 128 tokens, host's pace, medians of 14 processes a side in turn (which lie up to 10 % apart): hidden 7168 10.7 -> 9.8 us,
+// 2048 10.7 -> 9.9; other steps of one sender (bounds, strided rows,
 // more receivers, buffers of different lengths) keep the kernel above.
 template <typename T, typename U, int GROUP, int PIECES>
 __global__ __launch_bounds__(kWave) void combine_sole_kernel(const CombineSoleArgs args) {
